@@ -16,6 +16,7 @@ package.  Both libraries expose the same operations:
 
 import ctypes
 import os
+import unittest
 
 import numpy as np
 
@@ -260,6 +261,8 @@ class RefBasis:
     matrix (f1Xf1i_f1Oi)."""
 
     def __init__(self, Z, xyz_bohr, spec, spherical):
+        if not reference_available():
+            raise unittest.SkipTest("the compiled reference is not built")
         lib = reference().lib
         self.lib = lib
         f = lib.xcref_basis_setup
