@@ -5,17 +5,20 @@
 The library is written next to this file; it is git-ignored and travels with the source tree.
 """
 
+import concurrent.futures
 import os
 import subprocess
 import sys
+import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIBRARY = os.path.join(HERE, "libxcquad.so")
 SOURCES = ["xq_alloc.hip", "xq_api.hip", "xq_grid.hip", "xq_basis.hip", "xq_integrate.hip", "xq_f64.hip", "xq_mixed.hip",
-           "xq_gradients.hip", "xq_uks.hip", "xq_noalloc.hip", "qs_integrals.hip", "qs_dense.hip"]
+           "xq_gradients.hip", "xq_uks.hip", "xq_noalloc.hip", "qs_integrals.hip",
+           "qs_fit_low.hip", "qs_fit_dp.hip", "qs_fit_dd_sp.hip", "qs_fit_dd_d.hip", "qs_dense.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
-FLAGS = ["-O3", "-std=c++17", "-fPIC", "-shared", "--offload-arch=gfx950",
+FLAGS = ["-O3", "-std=c++17", "-fPIC", "--offload-arch=gfx950",
          # Packed FP32 instructions stay off: hipcc would otherwise form v_pk_* FP32 ops from plain float code.
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
          "-Wno-unused-result"]
@@ -23,12 +26,24 @@ FLAGS = ["-O3", "-std=c++17", "-fPIC", "-shared", "--offload-arch=gfx950",
 LIBS = ["-L/opt/rocm/lib", "-lrocsolver", "-lrocblas", "-Wl,-rpath,/opt/rocm/lib"]
 
 
-def build(verbose=False):
-    """Compile every HIP source into libxcquad.so; raises CalledProcessError on a compiler error."""
-    cmd = [HIPCC] + FLAGS + ["-o", LIBRARY + ".tmp"] + [os.path.join(CSRC, s) for s in SOURCES] + LIBS
+def _run(cmd, verbose):
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.run(cmd, check=True)
+
+
+def build(verbose=False):
+    """Compile every HIP source, several at a time, and link libxcquad.so; raises CalledProcessError on a compiler error."""
+    with tempfile.TemporaryDirectory() as objects:
+        def compiled(source):
+            out = os.path.join(objects, source + ".o")
+            _run([HIPCC] + FLAGS + ["-c", os.path.join(CSRC, source), "-o", out], verbose)
+            return out
+        # The files of the largest unrolled kernels first: they take the longest.
+        slow = sorted(SOURCES, key=lambda s: not s.startswith("qs_fit_"))
+        with concurrent.futures.ThreadPoolExecutor(min(8, os.cpu_count() or 1)) as pool:
+            files = list(pool.map(compiled, slow))
+        _run([HIPCC, "-shared", "-fPIC", "--offload-arch=gfx950", "-o", LIBRARY + ".tmp"] + files + LIBS, verbose)
     os.replace(LIBRARY + ".tmp", LIBRARY)
     return LIBRARY
 

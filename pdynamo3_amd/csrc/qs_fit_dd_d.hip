@@ -1,0 +1,9 @@
+// Electron-fit integral kernels of the pair classes dd with d fit shells.
+#define QS_FIT_KERNELS
+#include "qs_fit_kernels.h"
+
+namespace qs {
+
+template void launch_fit<2, 2, 2>(const FitLaunch &, const PairItem *, int);
+
+}  // namespace qs

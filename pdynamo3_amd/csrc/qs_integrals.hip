@@ -29,6 +29,7 @@
 #include <vector>
 
 #include "../../include/qcscf.h"
+#include "qs_fit_kernels.h"
 #include "qs_shells.h"
 #include "xq_c2s.h"
 #include "xq_internal.h"
@@ -70,19 +71,69 @@ int ensure_boys() {
     return kOK;
 }
 
+// The device address of the Boys table on the current GPU.
+int boys_address(const double **boys) {
+    void *p = nullptr;
+    XQ_CHECK(hipGetSymbolAddress(&p, HIP_SYMBOL(g_boys)));
+    *boys = static_cast<const double *>(p);
+    return kOK;
+}
 
 // ------------------------------------------------------------------------------------------------------------------------
-// One-electron matrices: one thread per shell pair (A >= B).
+// Shell pairs by class (qs_kernels.h): their records, one thread per pair, and the one-electron matrices.
 // ------------------------------------------------------------------------------------------------------------------------
-__global__ void __launch_bounds__(kThreads) one_electron_kernel(int nPairs, const QPair *__restrict__ pairs,
+template <int LA, int LB>
+__global__ void __launch_bounds__(kThreads) pair_records_kernel(int nPairs, PairItem *__restrict__ items,
                                                                 const QShell *__restrict__ shells,
                                                                 const double *__restrict__ exps,
-                                                                const double *__restrict__ coefs, int nAtoms,
-                                                                const double *__restrict__ atoms, int spherical,
-                                                                double *__restrict__ S,
-                                                                double *__restrict__ T, double *__restrict__ V) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < nPairs) one_electron_pair(k, pairs, shells, exps, coefs, nAtoms, atoms, spherical, g_boys, g_c2s, S, T, V);
+                                                                const double *__restrict__ coefs,
+                                                                double *__restrict__ records) {
+    const int k = blockIdx.x * kThreads + threadIdx.x;
+    if (k >= nPairs) return;
+    const PairItem it = items[k];
+    items[k].n = pair_records<LA, LB>(shells[it.a], shells[it.b], exps, coefs, records + it.first);
+}
+
+template <int LA, int LB>
+__global__ void __launch_bounds__(kThreads) overlap_kinetic_kernel(int nPairs, const PairItem *__restrict__ items,
+                                                                   const QShell *__restrict__ shells,
+                                                                   const double *__restrict__ exps,
+                                                                   const double *__restrict__ coefs, int spherical,
+                                                                   double *__restrict__ S, double *__restrict__ T) {
+    const int k = blockIdx.x * kThreads + threadIdx.x;
+    if (k >= nPairs) return;
+    const QShell A = shells[items[k].a], B = shells[items[k].b];
+    overlap_kinetic<LA, LB>(A, B, exps, coefs, spherical, [&](int i, int j, double overlap, double kinetic) {
+        const long long o = packed_index(A.f0 + i, B.f0 + j);
+        S[o] = overlap;
+        T[o] = kinetic;
+    });
+}
+
+// Nuclear attraction: one wave per pair, its lanes the nuclei; the lanes' blocks are summed over the wave.  With the pair's
+// integrals unrolled by class and its records shared by the lanes, S, T and V of (H2O)16 take 0.2 ms; one thread per pair
+// with loops over all angular momenta and 6 KB of private memory took 12.7 ms.
+template <int LA, int LB>
+__global__ void __launch_bounds__(256) nuclear_kernel(int nPairs, const PairItem *__restrict__ items,
+                                                      const QShell *__restrict__ shells,
+                                                      const double *__restrict__ records, int nAtoms,
+                                                      const double *__restrict__ atoms, int spherical,
+                                                      double *__restrict__ V) {
+    const int k = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x * 4 + (threadIdx.x >> 6)));
+    if (k >= nPairs) return;
+    const int lane = threadIdx.x & 63;
+    const PairItem it = items[k];
+    double acc[PairClass<LA, LB>::na * PairClass<LA, LB>::nb][1];
+    nuclear_block<LA, LB>(records + it.first, it.n, lane, 64, nAtoms, atoms, g_boys, acc);
+    static_for<PairClass<LA, LB>::na * PairClass<LA, LB>::nb>([&](auto ab) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) acc[ab][0] += __shfl_xor(acc[ab][0], o, 64);
+    });
+    const int fa = shells[it.a].f0, fb = shells[it.b].f0;
+    pair_functions<LA, LB, 1>(spherical, acc);
+    for_functions<LA, LB>(spherical, [&](int i, int j, auto ab) {
+        if (lane == 0) V[packed_index(fa + i, fb + j)] = acc[ab][0];
+    });
 }
 
 // ------------------------------------------------------------------------------------------------------------------------
@@ -95,20 +146,6 @@ __global__ void __launch_bounds__(kThreads) fit_matrix_kernel(int nPairs, const 
                                                               double *__restrict__ M) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k < nPairs) fit_matrix_pair(k, pairs, shells, exps, coefs, nFit, spherical, g_boys, g_c2s, M);
-}
-
-// ------------------------------------------------------------------------------------------------------------------------
-// Electron-fit integrals: one thread per (significant orbital shell pair, fit shell).
-// ------------------------------------------------------------------------------------------------------------------------
-__global__ void __launch_bounds__(kThreads) fit_integrals_kernel(
-    long long k0, long long nWork, int nFitShells, const PairEntry *__restrict__ pairs, const QShell *__restrict__ oShells,
-    const double *__restrict__ oExps, const double *__restrict__ oCoefs, int oSpherical,
-    const QShell *__restrict__ fShells, const double *__restrict__ fExps, const double *__restrict__ fCoefs, int fSpherical,
-    int nFit, double *__restrict__ B) {
-    const long long k = k0 + blockIdx.x * static_cast<long long>(blockDim.x) + threadIdx.x;
-    if (k < nWork)
-        fit_integrals_item(k, nFitShells, pairs, oShells, oExps, oCoefs, oSpherical, fShells, fExps, fCoefs, fSpherical, nFit,
-                           g_boys, g_c2s, B);
 }
 
 // ------------------------------------------------------------------------------------------------------------------------
@@ -176,6 +213,8 @@ struct qs_fit {
     int nFit = 0, nOrbital = 0;
     long long rows = 0, nPairs = 0;
     std::vector<qs::QPair> fitPairs;
+    std::vector<int> column;           // stored column of each fit function
+    std::vector<double> host;          // b and c in the order of the columns
     const qs_basis *orbital = nullptr, *fit = nullptr;
     double *d_B = nullptr;
     long long *d_rowPacked = nullptr;
@@ -206,21 +245,19 @@ void qs_release(T **p) {
     if (*p != nullptr) { (void)xq::cache_free(*p); *p = nullptr; }
 }
 
-// The integral kernels hold their McMurchie-Davidson tables in private memory (about 8 KB per lane for the fit
-// integrals), and the runtime gives every hardware queue that runs one its own scratch area sized for the whole
+// The fit matrix kernel holds its McMurchie-Davidson tables in private memory (3.7 KB per lane), and the runtime gives every hardware queue that runs one its own scratch area sized for the whole
 // device.  Two such kernels in flight at once on two queues (set-up threads of a request loop) made the second queue's
 // scratch allocation fail (HSA_STATUS_ERROR_OUT_OF_RESOURCES, queue abort), so at most one of them runs at a time in
 // the process: each holds this lock from its launch until its stream has drained.  The same allocation fails when the
 // device is nearly full (a request loop's caching allocator holds idle blocks), so each launch first makes sure that
-// kScratchHeadroom bytes are free: the fit-integral kernel's 8,368 bytes per lane at 3 waves per SIMD on 256 CUs take
-// about 1.6 GB.
+// kScratchHeadroom bytes are free.
 std::mutex g_integralKernels;
 constexpr size_t kScratchHeadroom = static_cast<size_t>(6) << 30;
 // The runtime's scratch areas belong to hardware queues and come from a pool of fixed size, separate from the free
 // device memory: several queues that each ran one of these kernels held areas sized for a whole-device dispatch and a
 // further request failed with HSA_STATUS_ERROR_OUT_OF_RESOURCES with 217 GB free.  So every launch of them goes to one
 // stream per device (one queue, one area), and no launch is larger than kSliceThreads threads, which bounds the area a
-// dispatch asks for (about 1.8 GB at 13,760 bytes per lane).
+// dispatch asks for.
 constexpr int kMaxDevices = 64;
 hipStream_t g_integralStream[kMaxDevices] = {};
 constexpr long long kSliceThreads = 2048LL * 64;
@@ -234,6 +271,57 @@ int integral_stream(hipStream_t *out) {
         XQ_CHECK(hipStreamCreateWithFlags(&g_integralStream[dev], hipStreamNonBlocking));
     *out = g_integralStream[dev];
     return kOK;
+}
+
+// Shell pairs sorted by class, and where each class starts; doubles of all their records.
+struct PairSet {
+    std::vector<PairItem> items;
+    int start[7] = {0, 0, 0, 0, 0, 0, 0};
+    long long doubles = 0;
+};
+
+int pair_class(const QShell &a, const QShell &b) {
+    const int la = std::max(a.l, b.l), lb = std::min(a.l, b.l);
+    return la * (la + 1) / 2 + lb;
+}
+
+// The pairs by class, in their order within a class; row: the first row of each pair's electron-fit integrals, or empty.
+PairSet pair_set(const QBasis *b, const std::vector<QPair> &pairs, const std::vector<long long> &row) {
+    PairSet set;
+    set.items.resize(pairs.size());
+    for (const QPair &q : pairs) set.start[pair_class(b->shells[q.x], b->shells[q.y]) + 1]++;
+    for (int c = 0; c < 6; c++) set.start[c + 1] += set.start[c];
+    int at[6];
+    for (int c = 0; c < 6; c++) at[c] = set.start[c];
+    for (size_t k = 0; k < pairs.size(); k++) {
+        const QShell &A = b->shells[pairs[k].x], &B = b->shells[pairs[k].y];
+        set.items[at[pair_class(A, B)]++] =
+            pair_item(b->shells.data(), pairs[k].x, pairs[k].y, row.empty() ? 0 : row[k], set.doubles);
+        set.doubles += record_room(A, B);
+    }
+    return set;
+}
+
+// launch(la, lb, items of the class, their number) for every class of the set that has pairs.
+template <class Launch>
+int for_classes(const PairSet &set, PairItem *d_items, const char *what, Launch launch) {
+    for (int la = 0, c = 0; la <= kMaxL; la++)
+        for (int lb = 0; lb <= la; lb++, c++) {
+            const int n = set.start[c + 1] - set.start[c];
+            if (n == 0) continue;
+            with_pair_class(la, lb, [&](auto A, auto B) { launch(A, B, d_items + set.start[c], n); });
+            XQ_TRY(check(hipGetLastError(), what));
+        }
+    return kOK;
+}
+
+inline dim3 groups(long long items, int perGroup) { return dim3(static_cast<unsigned>((items + perGroup - 1) / perGroup)); }
+
+int launch_records(const qs_basis *b, const PairSet &set, PairItem *d_items, double *d_records, hipStream_t s) {
+    return for_classes(set, d_items, "pair_records_kernel", [&](auto la, auto lb, PairItem *items, int n) {
+        hipLaunchKernelGGL((pair_records_kernel<la, lb>), groups(n, kThreads), dim3(kThreads), 0, s, n, items, b->d_shells,
+                           b->d_exps, b->d_coefs, d_records);
+    });
 }
 
 }  // namespace
@@ -296,22 +384,16 @@ int qs_one_electron(qs_basis *basis, double *S, double *T, double *V) {
         return kInvalidArgument;
     }
     const size_t n = static_cast<size_t>(basis->nFunctions), size = n * (n + 1) / 2;
-    std::vector<QPair> pairs = shell_pairs(basis, false);
-    // Pairs of one class (angular momenta and primitive counts) side by side, so that a wave's pairs share their loop
-    // bounds; each pair writes its own entries of S, T and V.
-    auto cls = [&](const QPair &q) {
-        const QShell &a = basis->shells[q.x], &b = basis->shells[q.y];
-        return ((a.l * 8 + b.l) * 64 + a.nPrim) * 64 + b.nPrim;
-    };
-    std::stable_sort(pairs.begin(), pairs.end(), [&](const QPair &u, const QPair &v) { return cls(u) < cls(v); });
+    const PairSet set = pair_set(basis, shell_pairs(basis, false), {});
     std::vector<double> atoms(4 * static_cast<size_t>(basis->nAtoms));
     for (int a = 0; a < basis->nAtoms; a++) {
         for (int c = 0; c < 3; c++) atoms[4 * a + c] = basis->xyz[3 * a + c];
         atoms[4 * a + 3] = static_cast<double>(basis->Z[a]);
     }
-    QPair *d_pairs = nullptr;
-    double *d_atoms = nullptr, *d_S = nullptr, *d_T = nullptr, *d_V = nullptr;
-    int status = qs_alloc(&d_pairs, pairs.size());
+    PairItem *d_items = nullptr;
+    double *d_records = nullptr, *d_atoms = nullptr, *d_S = nullptr, *d_T = nullptr, *d_V = nullptr;
+    int status = qs_alloc(&d_items, set.items.size());
+    if (status == kOK) status = qs_alloc(&d_records, static_cast<size_t>(set.doubles));
     if (status == kOK) status = qs_alloc(&d_atoms, atoms.size());
     if (status == kOK) status = qs_alloc(&d_S, size);
     if (status == kOK) status = qs_alloc(&d_T, size);
@@ -320,18 +402,18 @@ int qs_one_electron(qs_basis *basis, double *S, double *T, double *V) {
         std::lock_guard<std::mutex> lock(g_integralKernels);
         hipStream_t s = nullptr;
         if (status == kOK) status = integral_stream(&s);
-        if (status == kOK) status = check(hipMemcpyAsync(d_pairs, pairs.data(), pairs.size() * sizeof(QPair),
+        if (status == kOK) status = check(hipMemcpyAsync(d_items, set.items.data(), set.items.size() * sizeof(PairItem),
                                                          hipMemcpyHostToDevice, s), "copy pairs");
         if (status == kOK) status = check(hipMemcpyAsync(d_atoms, atoms.data(), atoms.size() * sizeof(double),
                                                          hipMemcpyHostToDevice, s), "copy atoms");
-        if (status == kOK && !pairs.empty()) status = xq::ensure_free_device_memory(kScratchHeadroom, "one-electron integrals");
-        for (long long k0 = 0; status == kOK && k0 < static_cast<long long>(pairs.size()); k0 += kSliceThreads) {
-            const long long m = std::min<long long>(kSliceThreads, static_cast<long long>(pairs.size()) - k0);
-            hipLaunchKernelGGL(one_electron_kernel, dim3(static_cast<unsigned>((m + kThreads - 1) / kThreads)),
-                               dim3(kThreads), 0, s, static_cast<int>(m), d_pairs + k0, basis->d_shells, basis->d_exps,
-                               basis->d_coefs, basis->nAtoms, d_atoms, basis->spherical, d_S, d_T, d_V);
-            status = check(hipGetLastError(), "one_electron_kernel");
-        }
+        if (status == kOK) status = launch_records(basis, set, d_items, d_records, s);
+        if (status == kOK)
+            status = for_classes(set, d_items, "one-electron kernels", [&](auto la, auto lb, PairItem *items, int n) {
+                hipLaunchKernelGGL((overlap_kinetic_kernel<la, lb>), groups(n, kThreads), dim3(kThreads), 0, s, n, items,
+                                   basis->d_shells, basis->d_exps, basis->d_coefs, basis->spherical, d_S, d_T);
+                hipLaunchKernelGGL((nuclear_kernel<la, lb>), groups(n, 4), dim3(256), 0, s, n, items, basis->d_shells,
+                                   d_records, basis->nAtoms, d_atoms, basis->spherical, d_V);
+            });
         if (status == kOK) status = check(hipMemcpyAsync(S, d_S, size * sizeof(double), hipMemcpyDeviceToHost, s), "copy S");
         if (status == kOK) status = check(hipMemcpyAsync(T, d_T, size * sizeof(double), hipMemcpyDeviceToHost, s), "copy T");
         if (status == kOK) status = check(hipMemcpyAsync(V, d_V, size * sizeof(double), hipMemcpyDeviceToHost, s), "copy V");
@@ -340,7 +422,8 @@ int qs_one_electron(qs_basis *basis, double *S, double *T, double *V) {
             if (status == kOK) status = drained;
         }
     }
-    qs_release(&d_pairs);
+    qs_release(&d_items);
+    qs_release(&d_records);
     qs_release(&d_atoms);
     qs_release(&d_S);
     qs_release(&d_T);
@@ -374,13 +457,13 @@ int qs_fit_create(const qs_basis *orbital, const qs_basis *fitBasis, qs_fit **ou
     int status = check(hipStreamCreateWithFlags(&F->stream, hipStreamNonBlocking), "hipStreamCreate");
     // Significant shell pairs and their rows.
     std::vector<QPair> sp = status == kOK ? shell_pairs(orbital, true) : std::vector<QPair>();
-    std::vector<PairEntry> pairs(sp.size());
+    std::vector<long long> row(sp.size());
     std::vector<long long> rowPacked;
     std::vector<unsigned char> rowDiag;
     long long rows = 0;
     for (size_t k = 0; k < sp.size(); k++) {
         const QShell &A = orbital->shells[sp[k].x], &B = orbital->shells[sp[k].y];
-        pairs[k] = PairEntry{sp[k].x, sp[k].y, rows};
+        row[k] = rows;
         for (int i = 0; i < A.nf; i++)
             for (int j = 0; j < B.nf; j++) {
                 const int mu = A.f0 + i, nu = B.f0 + j;
@@ -393,12 +476,32 @@ int qs_fit_create(const qs_basis *orbital, const qs_basis *fitBasis, qs_fit **ou
     F->nPairs = static_cast<long long>(sp.size());
     const size_t nOrbPacked = static_cast<size_t>(F->nOrbital) * (F->nOrbital + 1) / 2;
     const long long nChunks = (rows + kRowChunk - 1) / kRowChunk;
-    PairEntry *d_pairs = nullptr;
-    // The fit shells in order of angular momentum for the integral launch: the consecutive work items of a wave take
-    // one shell pair and consecutive fit shells, which then share their loop bounds (each shell writes its own
-    // functions, f0 .. f0 + nf - 1, wherever it sits in this list).
+    const PairSet set = pair_set(orbital, sp, row);
+    // The fit shells by angular momentum, and the stored column of every fit function: by angular momentum, then
+    // by function of the shell, then by shell.
     std::vector<QShell> fitSorted(fitBasis->shells);
     std::stable_sort(fitSorted.begin(), fitSorted.end(), [](const QShell &u, const QShell &v) { return u.l < v.l; });
+    FitLaunch launch{};
+    launch.oShells = orbital->d_shells;
+    launch.oSpherical = orbital->spherical;
+    launch.fSpherical = fitBasis->spherical;
+    launch.fExps = fitBasis->d_exps;
+    launch.fCoefs = fitBasis->d_coefs;
+    launch.nFit = F->nFit;
+    int *first = launch.first, *column = launch.column;
+    F->column.resize(static_cast<size_t>(F->nFit));
+    F->host.resize(static_cast<size_t>(F->nFit));
+    for (int l = 0; l <= kMaxL; l++) {
+        int n = 0;
+        while (first[l] + n < static_cast<int>(fitSorted.size()) && fitSorted[first[l] + n].l == l) n++;
+        const int nf = n > 0 ? fitSorted[first[l]].nf : 0;
+        for (int k = 0; k < n; k++)
+            for (int m = 0; m < nf; m++) F->column[fitSorted[first[l] + k].f0 + m] = column[l] + m * n + k;
+        first[l + 1] = first[l] + n;
+        column[l + 1] = column[l] + n * nf;
+    }
+    PairItem *d_items = nullptr;
+    double *d_records = nullptr;
     QShell *d_fitSorted = nullptr;
     if (status == kOK) status = qs_alloc(&F->d_B, static_cast<size_t>(rows) * F->nFit);
     if (status == kOK) status = qs_alloc(&F->d_rowPacked, rowPacked.size());
@@ -408,7 +511,8 @@ int qs_fit_create(const qs_basis *orbital, const qs_basis *fitBasis, qs_fit **ou
     if (status == kOK) status = qs_alloc(&F->d_b, F->nFit);
     if (status == kOK) status = qs_alloc(&F->d_c, F->nFit);
     if (status == kOK) status = qs_alloc(&F->d_partial, static_cast<size_t>(nChunks > 0 ? nChunks : 1) * F->nFit);
-    if (status == kOK) status = qs_alloc(&d_pairs, pairs.size());
+    if (status == kOK) status = qs_alloc(&d_items, set.items.size());
+    if (status == kOK) status = qs_alloc(&d_records, static_cast<size_t>(set.doubles));
     if (status == kOK) status = qs_alloc(&d_fitSorted, fitSorted.empty() ? 1 : fitSorted.size());
     if (status == kOK && !fitSorted.empty())
         status = check(hipMemcpy(d_fitSorted, fitSorted.data(), fitSorted.size() * sizeof(QShell), hipMemcpyHostToDevice),
@@ -418,28 +522,30 @@ int qs_fit_create(const qs_basis *orbital, const qs_basis *fitBasis, qs_fit **ou
                                  hipMemcpyHostToDevice), "copy rows");
         if (status == kOK) status = check(hipMemcpy(F->d_rowDiag, rowDiag.data(), rowDiag.size(), hipMemcpyHostToDevice),
                                           "copy rows");
-        if (status == kOK) status = check(hipMemcpy(d_pairs, pairs.data(), pairs.size() * sizeof(PairEntry),
+        if (status == kOK) status = check(hipMemcpy(d_items, set.items.data(), set.items.size() * sizeof(PairItem),
                                                     hipMemcpyHostToDevice), "copy pairs");
-        const long long nWork = F->nPairs * static_cast<long long>(fitBasis->shells.size());
         std::lock_guard<std::mutex> lock(g_integralKernels);
         hipStream_t is = nullptr;
         if (status == kOK) status = integral_stream(&is);
-        if (status == kOK && nWork > 0) status = xq::ensure_free_device_memory(kScratchHeadroom, "fit integrals");
-        for (long long k0 = 0; status == kOK && k0 < nWork; k0 += kSliceThreads) {
-            const long long m = std::min<long long>(kSliceThreads, nWork - k0);
-            hipLaunchKernelGGL(fit_integrals_kernel, dim3(static_cast<unsigned>((m + kThreads - 1) / kThreads)),
-                               dim3(kThreads), 0, is, k0, nWork, static_cast<int>(fitBasis->shells.size()), d_pairs,
-                               orbital->d_shells, orbital->d_exps, orbital->d_coefs, orbital->spherical,
-                               d_fitSorted, fitBasis->d_exps, fitBasis->d_coefs, fitBasis->spherical, F->nFit,
-                               F->d_B);
-            status = check(hipGetLastError(), "fit_integrals_kernel");
-        }
+        if (status == kOK) status = launch_records(orbital, set, d_items, d_records, is);
+        launch.stream = is;
+        launch.records = d_records;
+        launch.fShells = d_fitSorted;
+        launch.B = F->d_B;
+        if (status == kOK) status = boys_address(&launch.boys);
+        if (status == kOK)
+            status = for_classes(set, d_items, "fit_integrals_kernel", [&](auto la, auto lb, PairItem *items, int n) {
+                launch_fit<la, lb, 0>(launch, items, n);
+                launch_fit<la, lb, 1>(launch, items, n);
+                launch_fit<la, lb, 2>(launch, items, n);
+            });
         if (is != nullptr) {
             const int drained = check(hipStreamSynchronize(is), "fit integrals");
             if (status == kOK) status = drained;
         }
     }
-    qs_release(&d_pairs);
+    qs_release(&d_items);
+    qs_release(&d_records);
     qs_release(&d_fitSorted);
     if (status == kOK) F->fitPairs = shell_pairs(fitBasis, false);
     if (status != kOK) { qs_fit_free(F); return status; }
@@ -493,11 +599,10 @@ int qs_fit_b(qs_fit *fit, const double *P, double *b) {
         hipLaunchKernelGGL(fit_b_reduce_kernel, dim3((fit->nFit + 255) / 256), dim3(256), 0, s, nChunks, fit->nFit,
                            fit->d_partial, fit->d_b);
         XQ_CHECK(hipGetLastError());
-        XQ_CHECK(hipMemcpyAsync(b, fit->d_b, fit->nFit * sizeof(double), hipMemcpyDeviceToHost, s));
-    } else {
-        for (int k = 0; k < fit->nFit; k++) b[k] = 0.0;
+        XQ_CHECK(hipMemcpyAsync(fit->host.data(), fit->d_b, fit->nFit * sizeof(double), hipMemcpyDeviceToHost, s));
     }
     XQ_CHECK(hipStreamSynchronize(s));
+    for (int k = 0; k < fit->nFit; k++) b[k] = nChunks > 0 ? fit->host[fit->column[k]] : 0.0;
     return kOK;
 }
 
@@ -505,7 +610,8 @@ int qs_fit_fock(qs_fit *fit, const double *c, double *Fock) {
     if (fit == nullptr || c == nullptr || Fock == nullptr) { set_error("invalid fit arguments"); return kInvalidArgument; }
     const size_t nPacked = static_cast<size_t>(fit->nOrbital) * (fit->nOrbital + 1) / 2;
     hipStream_t s = fit->stream;
-    XQ_CHECK(hipMemcpyAsync(fit->d_c, c, fit->nFit * sizeof(double), hipMemcpyHostToDevice, s));
+    for (int k = 0; k < fit->nFit; k++) fit->host[fit->column[k]] = c[k];
+    XQ_CHECK(hipMemcpyAsync(fit->d_c, fit->host.data(), fit->nFit * sizeof(double), hipMemcpyHostToDevice, s));
     XQ_CHECK(hipMemcpyAsync(fit->d_F, Fock, nPacked * sizeof(double), hipMemcpyHostToDevice, s));
     if (fit->rows > 0) {
         const long long waves = fit->rows;
@@ -537,13 +643,16 @@ int qs_fit_estimate_bytes(int nAtoms, const int *Z, const double *xyzBohr, int n
     std::string err = build_shells(&orb, nSpec, spec);
     if (err.empty()) err = build_shells(&fit, nFitSpec, fitSpec);
     if (!err.empty()) { set_error(err); return kInvalidArgument; }
-    // The arrays qs_fit_create allocates: the integrals (rows x nFit), the row maps, P, F, b, c and the partial sums of b.
-    long long rows = 0;
-    for (const QPair &pq : shell_pairs(&orb, true))
+    // The arrays qs_fit_create allocates: the integrals (rows x nFit), the row maps, P, F, b, c, the partial sums of b, and
+    // the shell pairs' records during the set-up.
+    long long rows = 0, setup = 0;
+    for (const QPair &pq : shell_pairs(&orb, true)) {
         rows += static_cast<long long>(orb.shells[pq.x].nf) * orb.shells[pq.y].nf;
+        setup += 8 * record_room(orb.shells[pq.x], orb.shells[pq.y]) + static_cast<long long>(sizeof(PairItem));
+    }
     const long long nFit = fit.nFunctions, n = orb.nFunctions, nPacked = n * (n + 1) / 2;
     const long long nChunks = (rows + kRowChunk - 1) / kRowChunk;
-    *bytes = 8 * rows * nFit + 9 * rows + 16 * nPacked + 16 * nFit + 8 * (nChunks > 0 ? nChunks : 1) * nFit;
+    *bytes = 8 * rows * nFit + 9 * rows + 16 * nPacked + 16 * nFit + 8 * (nChunks > 0 ? nChunks : 1) * nFit + setup;
     return kOK;
 }
 
