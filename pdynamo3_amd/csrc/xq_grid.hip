@@ -378,303 +378,261 @@ void becke_pairs(const xq_grid *g, std::vector<double> &invR, std::vector<double
 // registers).
 constexpr int kMaxLaneAtoms = 16;
 
-// Screen of the weight-derivative terms.  The term of the ordered pair (k, m) is ifac = (ds_km/dmu) (A_k / s_km) fac_k, and
-// moves an atom or the point by at most |ifac| 2 / R_km.  |ds/dmu| <= 1.6875 x 2 = 3.375 (|ds/dnu| peaks at nu = 0 with
-// (3/2)^3 / 2, |dnu/dmu| = |1 - 2 a mu| <= 2); |A_k / s_km| <= Q_k, the product of k's factors without its smallest one;
-// |fac_k| = |eXC w| / sum_i A_i for k != g.  Atoms with Q_k < 2^-80 sum_i A_i (k != g) are outside the set K: the terms of
-// pairs (k, m) with k outside K and of pairs (m, k) with k outside K are each below 3.375 2^-80 |eXC w| 2 / R_km, and
-// are left out (below 1e-15 hartree/bohr in all for any molecule this kernel takes); every other pair term is computed.
-// sum_i A_i is taken over the atoms whose bound passes half the screen at max(A_g, A_near), A_near the product of the
-// atom nearest the point (K lies among them); each atom left out of it has A_i below 2^-81 max(A_g, A_near).
-constexpr double kWeightScreen = 0x1p-80;
-constexpr int kNearAtoms = 24;           // atoms whose factors bound a cell product (the point's atom and its nearest)
+// Screen of the weight-derivative terms: atoms whose cell product, and atoms whose factor of the derivative, is below this
+// share of their sum.  A cell factor s(nu) near its zero is s = c y^11 P with y = 1 - nu and a derivative of 11 s / y, so a
+// term that the screen drops is below 1e-16 of the point's energy over a bond length.
+constexpr double kWeightScreen = 0x1p-64;
 
-// Derivative polynomial of the cell function's polynomial: d_t = (2 t + 1) c_t, so that d/dnu sum_t c_t nu^(2t+1) =
-// sum_t d_t nu^(2t).
-__constant__ double c_beckeD[11] = {1.0 * 1.000000000000000e+00, 3.0 * -3.333333333333333e+00,
-                                    5.0 * 9.000000000000000e+00, 7.0 * -17.142857142857142e+00,
-                                    9.0 * 23.333333333333332e+00, 11.0 * -22.909090909090910e+00,
-                                    13.0 * 16.153846153846153e+00, 15.0 * -8.000000000000000e+00,
-                                    17.0 * 2.647058823529412e+00, 19.0 * -0.526315789473684e+00,
-                                    21.0 * 0.047619047619048e+00};
-
-// Atom k's cell-factor product with the factor s of one partner left out, from the product of its non-zero factors (of
-// either sign: a factor can round to a tiny negative value) and the count of its zero factors.  invS = 1 / s (used only
-// when no factor vanished, so s != 0).
-__device__ __forceinline__ double excluded_product(double prodNZ, int zeros, double s, double invS) {
-    if (zeros == 0) return prodNZ * invS;
-    return (zeros == 1 && s == 0.0) ? prodNZ : 0.0;
+// The cell function's small side: s = kBeckeA * integral of (1 - x^2)^10 from n to 1 for n = |nu|.  With y = 1 - n that is
+// kBeckeA y^11 sum_j e_j n^j, e_j = binom(10, j) * integral of t^(10 + j) (2 - t)^(10 - j) from 0 to 1: every e_j is
+// positive, so the form keeps its relative accuracy down to the smallest factors.
+__device__ __forceinline__ double becke_small(double n, double y) {
+    constexpr double e[11] = {0.27026018357287707, 1.9728620193016477, 6.8371721158098868, 14.627745835176176,
+                                21.197110423116616, 21.591331269349844, 15.57688338493292, 7.829573934837093,
+                                2.6165413533834587, 0.52380952380952384, 0.047619047619047616};
+    double p = e[10];
+#pragma unroll
+    for (int j = 9; j >= 0; j--) p = fma(p, n, e[j]);
+    const double y2 = y * y, y4 = y2 * y2;
+    return kBeckeA * p * (y4 * y4 * y2 * y);
 }
 
-// XC gradient weight terms (DFTGridWeights_Derivatives, DFTGridWeights.c:98-215).  One wave per point, WPG points per
-// round of a work-group; lane l owns atoms l, l + 64, ... (at most LA of them) and accumulates their gradient in
-// registers.  Per point (grid atom g, weight w, energy density eXC = eps rho): A_i = prod_j s_ij; p = A_g / sum_i A_i;
-// ew = eXC w / (p sum_i A_i); dA_i/dmu_ij = ds_ij prod_{k != j} s_ik; for every ordered pair (i, j) the reference adds
-// ifac = dA_i/dmu_ij fac_i, fac_i = ew (1 - p) for i = g and -ew p otherwise, times the derivatives of mu_ij with respect
-// to atom i, atom j and the point (which moves with atom g).  The pair loop runs over m in K (wave-uniform) and the
-// lane's atoms k, evaluating each pair once: the terms of (k, m) and (m, k) that move k, the point term of (k, m), and
-// for k outside K the terms of (m, k) that move m (summed over the wave) and the point; the reference's O(nAtoms^3)
-// update of dA/dmu becomes O(nAtoms^2) per point, and the screen (kWeightScreen) leaves O(|K| nAtoms): the atoms whose
-// cell product is not negligible at the point.  Both factors of a pair come from one polynomial (s_km and s_mk = 1 - s_km share nu), and
-// one division gives both 1 / s_km and 1 / s_mk.
-// LDS per wave: the distances R, their inverses and the non-zero products (3 nAtoms doubles), and the zero counts (nAtoms
-// bytes, after the doubles of all WPG waves).  WPG waves per work-group (4, or 2 for molecules whose per-wave LDS would
-// not fit four times in 64 KB); the waves share no LDS.
-template <int LA, int WPG>
+// 1 / x for normal x: the hardware's estimate with two Newton steps.
+__device__ __forceinline__ double reciprocal(double x) {
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(fma(-x, r, 1.0), r, r);
+    return fma(fma(-x, r, 1.0), r, r);
+}
+
+template <int GS>
+__device__ __forceinline__ double group_sum(double x) {
+#pragma unroll
+    for (int o = GS / 2; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
+    return x;
+}
+
+// LDS writes of a wave are in order; this keeps the compiler from moving accesses over it.
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// XC gradient weight terms (DFTGridWeights_Derivatives, DFTGridWeights.c:98-215).  A group of GS lanes takes a point (grid
+// atom g, weight w, energy density eXC = eps rho); lane l owns atoms l, l + GS, ... (at most LA of them) and accumulates
+// their gradient in registers.  With A_i = prod_j s_ij and S = sum_i A_i the point's term is
+//     eXC dw = sum_m c_m d ln A_m,   c_m = eXC w (delta_mg - A_m / S)   (w of the exact A_g),
+// and every pair of atoms m, k enters it as D dmu_mk with D = g (c_k / s_km - c_m / s_mk), g = -ds_mk / dmu_mk (the same for
+// both orders), mu_mk = (r_m - r_k) / R_mk.
+//   Products.  Row c evaluates the factors of atom c with every lane atom: s_ci for A_c and s_ic, which multiplies lane
+//   atom i's bound b_i >= A_i.  Rows are taken for g, then always for the atom of the largest bound, until no bound passes
+//   the screen at the largest product found: the atoms that matter at the point, and about one row more.
+//   Derivatives.  For each m whose c_m passes the screen, one row of pair terms: a pair of two such atoms is met from both
+//   sides and gives each side's own atom its force; a pair with another atom k (c_k = 0) gives both forces at once.
+//   The point moves with g, and its force is what makes the sum of a point's forces vanish.
+// Bound by FP64 arithmetic (about 35 operations a factor, 70 a pair term) and the wave reductions of each row.  Groups of 16
+// and 32 lanes keep small molecules' lanes busy.  pairs[m][k] = {1 / R_mk, a_mk} (square, so that a row is read in order;
+// a_km = -a_mk).  LDS: the coordinates, and per group each atom's distance and c.
+// Against one point a wave with bounds from the 24 atoms nearest g and a screen on products without their smallest factor
+// (which kept several times the atoms): (H2O)64, 2.4 million points, 102 -> 24 ms; (H2O)5, four points a wave, 2.5 -> 0.26 ms.
+template <int LA, int GS, int WPG>
 __global__ void __launch_bounds__(64 * WPG) weight_gradient_kernel(int nPoints,
                                                               const double *__restrict__ px, const double *__restrict__ py,
                                                               const double *__restrict__ pz, const double *__restrict__ pw,
                                                               const int *__restrict__ pointAtom,
                                                               const double *__restrict__ eXC, const double *__restrict__ xyz,
-                                                              int nAtoms, const double *__restrict__ invR,
-                                                              const double *__restrict__ aij,
-                                                              const int *__restrict__ nearAtoms, int nNear,
+                                                              int nAtoms, const double2 *__restrict__ pairs,
                                                               double *__restrict__ grad) {
+    static_assert(LA == 1 || GS == 64, "smaller groups hold one atom per lane");
+    constexpr int kGroups = 64 * WPG / GS;
     extern __shared__ double lds[];
-    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-    double *R = lds + static_cast<size_t>(wv) * 3 * nAtoms, *iR = R + nAtoms, *prodNZ = iR + nAtoms;
-    unsigned char *zeros = reinterpret_cast<unsigned char *>(lds + static_cast<size_t>(3 * WPG) * nAtoms) + wv * nAtoms;
+    const int t = threadIdx.x, gl = t & (GS - 1), gi = t / GS;
+    double *sxyz = lds, *rL = lds + static_cast<size_t>(3 + 2 * gi) * nAtoms, *cL = rL + nAtoms;
+    for (int i = t; i < 3 * nAtoms; i += 64 * WPG) sxyz[i] = xyz[i];
+    __syncthreads();
     double G[LA][3];
 #pragma unroll
     for (int a = 0; a < LA; a++) G[a][0] = G[a][1] = G[a][2] = 0.0;
-    // Work-group g takes the rounds g, g + gridDim.x, ... of WPG consecutive points (a point's cost depends on the atoms
+    // The group's lanes among the wave's ballot bits.
+    const int bit0 = t & 63 & ~(GS - 1);
+    const unsigned long long ones = GS == 64 ? ~0ull : ((1ull << (GS & 63)) - 1ull);
+    auto ballot = [&](bool x) { return (__ballot(x) >> bit0) & ones; };
+    // Work-group b takes the rounds b, b + gridDim.x, ... of kGroups consecutive points (a point's cost depends on the atoms
     // whose cells matter there, so contiguous ranges would differ in cost).
-    for (int base = blockIdx.x * WPG; base < nPoints; base += gridDim.x * WPG) {
-        const int p = base + wv;
-        const bool active = p < nPoints && eXC[p] != 0.0;
+    for (int base = blockIdx.x * kGroups; base < nPoints; base += gridDim.x * kGroups) {
+        const int p = base + gi;
+        const double e = p < nPoints ? eXC[p] : 0.0;
+        const bool active = e != 0.0;
+        if (!__any(active)) continue;
         const double rx = active ? px[p] : 0.0, ry = active ? py[p] : 0.0, rz = active ? pz[p] : 0.0;
-        if (active)
-            for (int i = lane; i < nAtoms; i += 64) {
-                const double dx = xyz[3 * i] - rx, dy = xyz[3 * i + 1] - ry, dz = xyz[3 * i + 2] - rz;
-                R[i] = sqrt(dx * dx + dy * dy + dz * dz);
-                iR[i] = 1.0 / R[i];
+        const int g = active ? pointAtom[p] : 0;
+        double r[LA], b[LA], A[LA];
+        bool done[LA];
+        wave_fence();
+#pragma unroll
+        for (int a = 0; a < LA; a++) {
+            const int i = gl + GS * a;
+            r[a] = 0.0;
+            if (i < nAtoms) {
+                const double dx = sxyz[3 * i] - rx, dy = sxyz[3 * i + 1] - ry, dz = sxyz[3 * i + 2] - rz;
+                r[a] = sqrt(dx * dx + dy * dy + dz * dz);
+                rL[i] = r[a];
             }
-        __syncthreads();
-        // Products of the cell factors, their zero counts, and the screened set K (flag 0x80 of the count).  A_g and the
-        // product of the atom nearest the point are lower bounds of sum_i A_i; the partial product of atom i over the
-        // atoms nearest g bounds every product of i with one factor left out (|s| <= 1), so an atom whose bound is below
-        // the screen at the larger of the two is outside K.  The
-        // remaining candidates take their full products with the factors spread over the wave.  The others keep a zero
-        // product and a count of 2, which leaves their terms out, as the screen leaves out those of the atoms outside K.
-        double sumA = 0.0;
-        int g = 0;
-        unsigned long long maskK[LA];   // the atoms of K among atoms 64 a .. 64 a + 63 (the same in every lane)
-#pragma unroll
-        for (int a = 0; a < LA; a++) maskK[a] = 0ull;
-        if (active) {
-            g = pointAtom[p];
-            auto full_product = [&](int i, double &prod, int &nz, double &minS) {
-                prod = 1.0;
-                minS = 1.0;
-                nz = 0;
-                for (int j = lane; j < nAtoms; j += 64) {
-                    if (j == i) continue;
-                    const int ij = pair_index(i, j);
-                    const double s = becke_factor_of(i > j, R[i], R[j], invR[ij], aij[ij]);
-                    if (s == 0.0) nz++;
-                    else {
-                        prod *= s;
-                        minS = fmin(minS, fabs(s));
-                    }
-                }
-                // Butterfly reductions: every lane ends with the same bits.
-#pragma unroll
-                for (int o = 32; o > 0; o >>= 1) {
-                    prod *= __shfl_xor(prod, o, 64);
-                    minS = fmin(minS, __shfl_xor(minS, o, 64));
-                    nz += __shfl_xor(nz, o, 64);
-                }
-            };
-            double pg, mg;
-            int zg;
-            full_product(g, pg, zg, mg);
-            // The atom nearest the point other than g (the wave's arg-min of R, ties to the lower index) and its product:
-            // sum_i A_i >= max(A_g, A_near), which bounds the screen for points deep in another atom's cell too.
-            double dn = 0.0;
-            int near = -1;
-            for (int j = lane; j < nAtoms; j += 64)
-                if (j != g && (near < 0 || R[j] < dn)) { dn = R[j]; near = j; }
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) {
-                const double od = __shfl_xor(dn, o, 64);
-                const int on = __shfl_xor(near, o, 64);
-                if (on >= 0 && (near < 0 || od < dn || (od == dn && on < near))) { dn = od; near = on; }
-            }
-            double pn = 0.0, mn = 1.0;
-            int zn = 2;
-            if (near >= 0) full_product(near, pn, zn, mn);
-            const double bound = 0x1p-81 * fmax(zg == 0 ? fabs(pg) : 0.0, zn == 0 ? fabs(pn) : 0.0);   // half the screen
-            const int *nearList = nearAtoms + static_cast<size_t>(g) * nNear;
-            bool cand[LA];
-            double Q[LA];
-#pragma unroll
-            for (int a = 0; a < LA; a++) {
-                const int i = lane + 64 * a;
-                cand[a] = false;
-                Q[a] = 0.0;
-                if (i >= nAtoms) continue;
-                if (i != g) {
-                    double pp = 1.0, mp = 1.0;
-                    int zp = 0;
-                    for (int q = 0; q < nNear; q++) {
-                        const int j = nearList[q];
-                        if (j == i) continue;
-                        const int ij = pair_index(i, j);
-                        const double s = fabs(becke_factor_of(i > j, R[i], R[j], invR[ij], aij[ij]));
-                        if (s == 0.0) zp++;
-                        else {
-                            pp *= s;
-                            mp = fmin(mp, s);
-                        }
-                    }
-                    const double qp = zp == 0 ? pp / mp : (zp == 1 ? pp : 0.0);
-                    cand[a] = !(qp < bound);
-                }
-                prodNZ[i] = 0.0;
-                zeros[i] = 2;
-            }
-#pragma unroll
-            for (int a = 0; a < LA; a++) {
-                unsigned long long mask = __ballot(cand[a] || lane + 64 * a == g || lane + 64 * a == near);
-                while (mask != 0ull) {
-                    const int bit = __ffsll(static_cast<long long>(mask)) - 1;
-                    mask &= mask - 1ull;
-                    const int c = 64 * a + bit;
-                    double pc = pg, mc = mg;
-                    int zc = zg;
-                    if (c == near) { pc = pn; mc = mn; zc = zn; }
-                    else if (c != g) full_product(c, pc, zc, mc);
-                    if (zc == 0) sumA += pc;
-                    if (lane == bit) {
-                        cand[a] = true;
-                        prodNZ[c] = pc;
-                        zeros[c] = static_cast<unsigned char>(zc < 2 ? zc : 2);
-                        Q[a] = zc == 0 ? fabs(pc) / mc : (zc == 1 ? fabs(pc) : 0.0);
-                    }
-                }
-            }
-#pragma unroll
-            for (int a = 0; a < LA; a++) {
-                const int i = lane + 64 * a;
-                const bool inK = i < nAtoms && cand[a] && (i == g || !(Q[a] < kWeightScreen * sumA));
-                if (inK) zeros[i] |= 0x80;
-                maskK[a] = __ballot(inK);
-            }
+            b[a] = 1.0;
+            A[a] = 0.0;
+            done[a] = i >= nAtoms;
         }
-        __syncthreads();
-        if (active) {
-            const double Ag = (zeros[g] & 0x7f) == 0 ? prodNZ[g] : 0.0;
-            const double pW = Ag / sumA;
-            const double ew = eXC[p] * pw[p] / (pW * sumA);
-            double gs[3] = {0.0, 0.0, 0.0};
-            // The lane's atoms k (their data held in registers across the pair loop).
-            double kR[LA], kP[LA], kf[LA];
-            int kNZ[LA];
-            bool kIn[LA];
+        wave_fence();
+        // A_g from the cell factors as the weight w was made from them (candidate_points_kernel): deep in another atom's cell
+        // they are rounding, and w with them.
+        double made = 1.0;
+        const double rg = rL[g];
+#pragma unroll
+        for (int a = 0; a < LA; a++) {
+            const int i = gl + GS * a;
+            if (i >= nAtoms || i == g) continue;
+            const double2 q = pairs[static_cast<size_t>(g) * nAtoms + i];
+            made *= becke_factor_of(g > i, rg, r[a], q.x, g > i ? q.y : -q.y);
+        }
+#pragma unroll
+        for (int o = GS / 2; o > 0; o >>= 1) made *= __shfl_xor(made, o, 64);
+        // Products.
+        bool run = active;
+        int c = g;
+        double most = 0.0;
+        do {
+            const double rc = rL[c];
+            double prod = 1.0;
 #pragma unroll
             for (int a = 0; a < LA; a++) {
-                const int k = lane + 64 * a < nAtoms ? lane + 64 * a : 0;
-                kR[a] = R[k];
-                kP[a] = prodNZ[k];
-                kNZ[a] = zeros[k] & 0x7f;
-                kIn[a] = (zeros[k] & 0x80) != 0;
-                kf[a] = k == g ? ew * (1.0 - pW) : -ew * pW;
-            }
-            // Every pair (k, m) with m in K and k a lane atom, each evaluated once: the terms of (k, m) and (m, k) that
-            // move k and the point term of (k, m); for k outside K also the terms of (m, k) that move m and the point
-            // (the terms of (k, m) that move m are below the screen), summed over the wave for m.
-            for (int a2 = 0; a2 < LA; a2++)
-            for (unsigned long long mk = maskK[a2]; mk != 0ull; mk &= mk - 1ull) {
-                const int m = 64 * a2 + __ffsll(static_cast<long long>(mk)) - 1;
-                const int nzm = zeros[m] & 0x7f;
-                const double xm = xyz[3 * m], ym = xyz[3 * m + 1], zmc = xyz[3 * m + 2];
-                const double Rm = R[m], pm = prodNZ[m], iRm = iR[m];
-                const double emx = (xm - rx) * iRm, emy = (ym - ry) * iRm, emz = (zmc - rz) * iRm;
-                const double fm = m == g ? ew * (1.0 - pW) : -ew * pW;
-                double hx = 0.0, hy = 0.0, hz = 0.0;
-#pragma unroll
-                for (int a = 0; a < LA; a++) {
-                    const int k = lane + 64 * a;
-                    if (k >= nAtoms || k == m) continue;
-                    const int km = pair_index(k, m);
-                    const double r = invR[km], am = aij[km];
-                    const bool kHigh = k > m;
-                    // mu and nu of the pair stored as (max, min), as the cell factors take them.
-                    const double muP = (kHigh ? kR[a] - Rm : Rm - kR[a]) * r;
-                    const double nu = muP + am * (1.0 - muP * muP), nu2 = nu * nu;
-                    const double S = kBeckeA * becke_poly(nu);
-                    const double skm = kHigh ? 0.5 - S : 0.5 + S, smk = kHigh ? 0.5 + S : 0.5 - S;
-                    double dsum = c_beckeD[10];
-#pragma unroll
-                    for (int tt = 9; tt >= 0; tt--) dsum = dsum * nu2 + c_beckeD[tt];
-                    dsum *= -kBeckeA * (1.0 - 2.0 * am * muP);
-                    const double sProd = skm * smk;
-                    double invKM, invMK;
-                    if (fabs(sProd) >= 0x1p-1000) {
-                        const double inv = 1.0 / sProd;
-                        invKM = smk * inv;
-                        invMK = skm * inv;
-                    } else {
-                        invKM = 1.0 / skm;
-                        invMK = 1.0 / smk;
-                    }
-                    const double ifKM = dsum * excluded_product(kP[a], kNZ[a], skm, invKM) * kf[a];
-                    const double ifMK = dsum * excluded_product(pm, nzm, smk, invMK) * fm;
-                    const double mu = kHigh ? muP : -muP, mr2 = mu * r * r;
-                    const double xk = xyz[3 * k], yk = xyz[3 * k + 1], zk = xyz[3 * k + 2], iRk = iR[k];
-                    const double kex = (xk - rx) * iRk, key = (yk - ry) * iRk, kez = (zk - rz) * iRk;
-                    const double dx = xk - xm, dy = yk - ym, dz = zk - zmc;
-                    // Pair (k, m) moves atom k through d mu / d r_k and the point through -(d mu / d r_k + d mu / d r_m);
-                    // pair (m, k) moves atom k through its second atom: both along r (e_k) - mu r^2 (r_k - r_m).
-                    const double d = ifKM - ifMK;
-                    G[a][0] += d * (kex * r - dx * mr2);
-                    G[a][1] += d * (key * r - dy * mr2);
-                    G[a][2] += d * (kez * r - dz * mr2);
-                    double wr = ifKM * r;
-                    if (!kIn[a]) {
-                        // Pair (m, k) moves atom m along r (e_m) - (-mu) r^2 (r_m - r_k) = r (e_m) - mu r^2 (r_k - r_m).
-                        hx += ifMK * (emx * r - dx * mr2);
-                        hy += ifMK * (emy * r - dy * mr2);
-                        hz += ifMK * (emz * r - dz * mr2);
-                        wr -= ifMK * r;
-                    }
-                    gs[0] += wr * (emx - kex);
-                    gs[1] += wr * (emy - key);
-                    gs[2] += wr * (emz - kez);
-                }
-#pragma unroll
-                for (int o = 32; o > 0; o >>= 1) {
-                    hx += __shfl_xor(hx, o, 64);
-                    hy += __shfl_xor(hy, o, 64);
-                    hz += __shfl_xor(hz, o, 64);
-                }
-                if (lane == (m & 63)) {
-#pragma unroll
-                    for (int a = 0; a < LA; a++)
-                        if (a == (m >> 6)) { G[a][0] += hx; G[a][1] += hy; G[a][2] += hz; }
-                }
+                const int i = gl + GS * a;
+                if (i >= nAtoms || i == c) continue;
+                const double2 q = pairs[static_cast<size_t>(c) * nAtoms + i];
+                const double mu = (rc - r[a]) * q.x, nu = fma(q.y, fma(-mu, mu, 1.0), mu), n = fabs(nu);
+                const double small = becke_small(n, fmax(1.0 - n, 0.0)), large = 1.0 - small;
+                prod *= nu > 0.0 ? small : large;
+                b[a] *= nu > 0.0 ? large : small;
             }
 #pragma unroll
-            for (int d = 0; d < 3; d++)
-#pragma unroll
-                for (int o = 32; o > 0; o >>= 1) gs[d] += __shfl_xor(gs[d], o, 64);
-            if (lane == (g & 63)) {
+            for (int o = GS / 2; o > 0; o >>= 1) prod *= __shfl_xor(prod, o, 64);
+            if (run) {
+                most = fmax(most, prod);
 #pragma unroll
                 for (int a = 0; a < LA; a++)
-                    if (a == (g >> 6)) { G[a][0] += gs[0]; G[a][1] += gs[1]; G[a][2] += gs[2]; }
+                    if (gl + GS * a == c) { A[a] = prod; done[a] = true; }
+            }
+            double best = -1.0;
+            int bi = 0;
+#pragma unroll
+            for (int a = 0; a < LA; a++)
+                if (!done[a] && b[a] > best) { best = b[a]; bi = gl + GS * a; }
+            double top = best;
+#pragma unroll
+            for (int o = GS / 2; o > 0; o >>= 1) top = fmax(top, __shfl_xor(top, o, 64));
+            run = run && top >= kWeightScreen * most && top > 0.0;
+            const unsigned long long at = ballot(best == top);
+            c = __shfl(bi, bit0 + __ffsll(static_cast<long long>(at)) - 1, 64);
+        } while (__any(run));
+        // c_m; that of g from the others' share, which keeps its accuracy where g's cell holds almost all.
+        double others = 0.0, own = 0.0;
+#pragma unroll
+        for (int a = 0; a < LA; a++) {
+            if (gl + GS * a == g) own = A[a];
+            else others += A[a];
+        }
+        others = group_sum<GS>(others);
+        own = group_sum<GS>(own);
+        const double ew = active ? e * pw[p] * (own / made) : 0.0, scale = active ? ew / (own + others) : 0.0;
+        double cf[LA];
+        unsigned long long maskK[LA], anyK = 0ull;
+#pragma unroll
+        for (int a = 0; a < LA; a++) {
+            const int i = gl + GS * a;
+            cf[a] = i == g ? scale * others : -scale * A[a];
+            if (!(fabs(cf[a]) >= kWeightScreen * fabs(ew)) || !active) cf[a] = 0.0;
+            if (i < nAtoms) cL[i] = cf[a];
+            maskK[a] = ballot(cf[a] != 0.0);
+            anyK |= maskK[a];
+        }
+        if (!__any(anyK != 0ull)) continue;
+        wave_fence();
+        // Derivatives.  ir: 1 / distance of the lane's atoms.
+        double ir[LA], gs[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+        for (int a = 0; a < LA; a++) ir[a] = gl + GS * a < nAtoms ? reciprocal(r[a]) : 0.0;
+#pragma unroll 1
+        for (int a2 = 0; a2 < LA; a2++) {
+            unsigned long long mk = 0ull;
+#pragma unroll
+            for (int a = 0; a < LA; a++)
+                if (a == a2) mk = maskK[a];
+            while (__any(mk != 0ull)) {
+                const bool some = mk != 0ull;
+                const int m = some ? GS * a2 + __ffsll(static_cast<long long>(mk)) - 1 : 0;
+                mk &= mk - 1ull;
+                const double xm = sxyz[3 * m], ym = sxyz[3 * m + 1], zm = sxyz[3 * m + 2], rm = rL[m];
+                const double cm = some ? cL[m] : 0.0, irm = reciprocal(rm);
+                const double ex = (xm - rx) * irm, ey = (ym - ry) * irm, ez = (zm - rz) * irm;
+                double h[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+                for (int a = 0; a < LA; a++) {
+                    const int k = gl + GS * a;
+                    if (k >= nAtoms || k == m || !some) continue;
+                    const double2 q = pairs[static_cast<size_t>(m) * nAtoms + k];
+                    const double mu = (rm - r[a]) * q.x, nu = fma(q.y, fma(-mu, mu, 1.0), mu), n = fabs(nu);
+                    const double y = fmax(1.0 - n, 0.0), small = becke_small(n, y), large = 1.0 - small;
+                    const double smk = nu > 0.0 ? small : large, skm = nu > 0.0 ? large : small;
+                    // 1 - nu^2 = y (2 - y); dnu / dmu = 1 - 2 a mu.
+                    const double u = y * (2.0 - y), u2 = u * u, u4 = u2 * u2;
+                    const double d = kBeckeA * (u4 * u4 * u2) * fma(-2.0 * q.y, mu, 1.0) * (cf[a] * smk - cm * skm) *
+                                     reciprocal(fmax(small * large, 0x1p-1000));
+                    // d mu_mk / d r_k = -e_k / R - mu (r_k - r_m) / R^2, d mu_mk / d r_m = e_m / R + mu (r_k - r_m) / R^2.
+                    const double al = d * q.x, be = al * q.x * mu, ak = al * ir[a];
+                    const double xk = sxyz[3 * k], yk = sxyz[3 * k + 1], zk = sxyz[3 * k + 2];
+                    const double bx = be * (xk - xm), by = be * (yk - ym), bz = be * (zk - zm);
+                    const double fx = -fma(ak, xk - rx, bx), fy = -fma(ak, yk - ry, by), fz = -fma(ak, zk - rz, bz);
+                    G[a][0] += fx;
+                    G[a][1] += fy;
+                    G[a][2] += fz;
+                    gs[0] += fx;
+                    gs[1] += fy;
+                    gs[2] += fz;
+                    if (cf[a] == 0.0) {
+                        h[0] += fma(al, ex, bx);
+                        h[1] += fma(al, ey, by);
+                        h[2] += fma(al, ez, bz);
+                    }
+                }
+#pragma unroll
+                for (int x = 0; x < 3; x++) h[x] = group_sum<GS>(h[x]);
+                if (some && gl == (m & (GS - 1))) {
+#pragma unroll
+                    for (int a = 0; a < LA; a++)
+                        if (a == a2) { G[a][0] += h[0]; G[a][1] += h[1]; G[a][2] += h[2]; }
+                    gs[0] += h[0];
+                    gs[1] += h[1];
+                    gs[2] += h[2];
+                }
             }
         }
-        __syncthreads();
+#pragma unroll
+        for (int x = 0; x < 3; x++) gs[x] = group_sum<GS>(gs[x]);
+#pragma unroll
+        for (int a = 0; a < LA; a++)
+            if (active && gl + GS * a == g) { G[a][0] -= gs[0]; G[a][1] -= gs[1]; G[a][2] -= gs[2]; }
     }
+    // The work-group's groups summed in LDS (the coordinates' place), then one addition per atom and component.
+    __syncthreads();
+    for (int i = t; i < 3 * nAtoms; i += 64 * WPG) sxyz[i] = 0.0;
+    __syncthreads();
 #pragma unroll
     for (int a = 0; a < LA; a++) {
-        const int k = lane + 64 * a;
-        if (k < nAtoms) {
-            atomicAdd(&grad[3 * k], G[a][0]);
-            atomicAdd(&grad[3 * k + 1], G[a][1]);
-            atomicAdd(&grad[3 * k + 2], G[a][2]);
-        }
+        const int k = gl + GS * a;
+        if (k < nAtoms)
+#pragma unroll
+            for (int x = 0; x < 3; x++) atomicAdd(&sxyz[3 * k + x], G[a][x]);
     }
+    __syncthreads();
+    for (int i = t; i < 3 * nAtoms; i += 64 * WPG) atomicAdd(&grad[i], sxyz[i]);
 }
 
 }  // namespace
@@ -895,50 +853,36 @@ long long estimated_points(int accuracy, int nAtoms, const int *Z) {
 int weight_gradients(xq_grid *g, const double *d_eXC, double *d_grad, hipStream_t s) {
     const int nA = g->nAtoms, G = g->nPoints;
     if (G <= 0 || nA < 2) return kOK;
-    // Waves per work-group: four up to 640 atoms, two above (each wave needs 25 bytes of LDS per atom: 4 x 25 x 640 and
-    // 2 x 25 x 1024 bytes both fit in 64 KB).  The kernel instance below takes the same count.
-    const size_t perWave = (3 * sizeof(double) + 1) * static_cast<size_t>(nA);
-    const int wpg = nA <= 640 ? 4 : 2;
-    const size_t lds = wpg * perWave;
+    // Waves per work-group: four up to 640 atoms, two above (the coordinates and 16 bytes of LDS per atom and wave: 11 x 8 x
+    // 640 and 7 x 8 x 1024 bytes both fit in 64 KB).  Up to 16 atoms four points share a wave, up to 32 two.
+    const int wpg = nA <= 640 ? 4 : 2, group = nA <= 16 ? 16 : (nA <= 32 ? 32 : 64);
+    const size_t lds = (3 + 2 * static_cast<size_t>(64 * wpg / group)) * sizeof(double) * static_cast<size_t>(nA);
     if (nA > 64 * kMaxLaneAtoms || lds > 64 * 1024) {
         set_error("XC gradients support at most " + std::to_string(64 * kMaxLaneAtoms) + " atoms");
         return kInvalidArgument;
     }
     std::vector<double> invR, aij;
     becke_pairs(g, invR, aij);
+    // Square pair table, [m][k] = {1 / R_mk, a_mk}.
+    std::vector<double2> pairs(static_cast<size_t>(nA) * nA, make_double2(0.0, 0.0));
+    for (int i = 0, ij = 0; i < nA; i++)
+        for (int j = 0; j < i; j++, ij++) {
+            pairs[static_cast<size_t>(i) * nA + j] = make_double2(invR[ij], aij[ij]);
+            pairs[static_cast<size_t>(j) * nA + i] = make_double2(invR[ij], -aij[ij]);
+        }
     std::vector<int> pointAtom(static_cast<size_t>(G), 0);
     for (const DevBlock &b : g->blocks)
         for (int k = 0; k < b.nPoints; k++) pointAtom[static_cast<size_t>(b.pStart) + k] = b.atom;
-    // Per atom: itself and the atoms nearest it (the partial products that bound the cell products of a point).
-    const int nNear = std::min(kNearAtoms, nA);
-    std::vector<int> nearAtoms(static_cast<size_t>(nA) * nNear), order(nA);
-    for (int a = 0; a < nA; a++) {
-        std::vector<double> d2(nA);
-        for (int j = 0; j < nA; j++) {
-            const double dx = g->xyz[3 * j] - g->xyz[3 * a], dy = g->xyz[3 * j + 1] - g->xyz[3 * a + 1],
-                         dz = g->xyz[3 * j + 2] - g->xyz[3 * a + 2];
-            d2[j] = j == a ? -1.0 : dx * dx + dy * dy + dz * dz;
-            order[j] = j;
-        }
-        std::partial_sort(order.begin(), order.begin() + nNear, order.end(),
-                          [&](int u, int v) { return d2[u] < d2[v] || (d2[u] == d2[v] && u < v); });
-        for (int q = 0; q < nNear; q++) nearAtoms[static_cast<size_t>(a) * nNear + q] = order[q];
-    }
-    double *d_invR = nullptr, *d_aij = nullptr, *d_xyz = nullptr;
-    int *d_pointAtom = nullptr, *d_near = nullptr;
+    double2 *d_pairs = nullptr;
+    double *d_xyz = nullptr;
+    int *d_pointAtom = nullptr;
     int status = kOK;
     do {
-        if ((status = dev_alloc(g, &d_invR, invR.size())) != kOK) break;
-        if ((status = dev_alloc(g, &d_aij, aij.size())) != kOK) break;
+        if ((status = dev_alloc(g, &d_pairs, pairs.size())) != kOK) break;
         if ((status = dev_alloc(g, &d_xyz, g->xyz.size())) != kOK) break;
         if ((status = dev_alloc(g, &d_pointAtom, pointAtom.size())) != kOK) break;
-        if ((status = dev_alloc(g, &d_near, nearAtoms.size())) != kOK) break;
-        if ((status = check(hipMemcpyAsync(d_near, nearAtoms.data(), nearAtoms.size() * sizeof(int),
-                                           hipMemcpyHostToDevice, s), "copy near atoms")) != kOK) break;
-        if ((status = check(hipMemcpyAsync(d_invR, invR.data(), invR.size() * sizeof(double), hipMemcpyHostToDevice, s),
-                            "copy invR")) != kOK) break;
-        if ((status = check(hipMemcpyAsync(d_aij, aij.data(), aij.size() * sizeof(double), hipMemcpyHostToDevice, s),
-                            "copy aij")) != kOK) break;
+        if ((status = check(hipMemcpyAsync(d_pairs, pairs.data(), pairs.size() * sizeof(double2), hipMemcpyHostToDevice, s),
+                            "copy pairs")) != kOK) break;
         if ((status = check(hipMemcpyAsync(d_xyz, g->xyz.data(), g->xyz.size() * sizeof(double), hipMemcpyHostToDevice, s),
                             "copy xyz")) != kOK) break;
         if ((status = check(hipMemcpyAsync(d_pointAtom, pointAtom.data(), pointAtom.size() * sizeof(int),
@@ -946,25 +890,25 @@ int weight_gradients(xq_grid *g, const double *d_eXC, double *d_grad, hipStream_
         const int nGroups = std::min(2048 * 4 / wpg, (G + 63) / 64);
         auto launch = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(nGroups), dim3(64 * wpg), lds, s, G, g->d_x, g->d_y, g->d_z,
-                               g->d_w, d_pointAtom, d_eXC, d_xyz, nA, d_invR, d_aij, d_near, nNear, d_grad);
+                               g->d_w, d_pointAtom, d_eXC, d_xyz, nA, d_pairs, d_grad);
         };
         // Atoms per lane: the smallest instance that covers nAtoms (fewer registers for small systems).
-        if (nA <= 64) launch(weight_gradient_kernel<1, 4>);
-        else if (nA <= 128) launch(weight_gradient_kernel<2, 4>);
-        else if (nA <= 192) launch(weight_gradient_kernel<3, 4>);
-        else if (nA <= 256) launch(weight_gradient_kernel<4, 4>);
-        else if (nA <= 384) launch(weight_gradient_kernel<6, 4>);
-        else if (nA <= 640) launch(weight_gradient_kernel<10, 4>);
-        else launch(weight_gradient_kernel<kMaxLaneAtoms, 2>);
+        if (nA <= 16) launch(weight_gradient_kernel<1, 16, 4>);
+        else if (nA <= 32) launch(weight_gradient_kernel<1, 32, 4>);
+        else if (nA <= 64) launch(weight_gradient_kernel<1, 64, 4>);
+        else if (nA <= 128) launch(weight_gradient_kernel<2, 64, 4>);
+        else if (nA <= 192) launch(weight_gradient_kernel<3, 64, 4>);
+        else if (nA <= 256) launch(weight_gradient_kernel<4, 64, 4>);
+        else if (nA <= 384) launch(weight_gradient_kernel<6, 64, 4>);
+        else if (nA <= 640) launch(weight_gradient_kernel<10, 64, 4>);
+        else launch(weight_gradient_kernel<kMaxLaneAtoms, 64, 2>);
         if ((status = check(hipGetLastError(), "weight_gradient_kernel")) != kOK) break;
         status = check(hipStreamSynchronize(s), "gradient sync");
     } while (false);
     (void)hipStreamSynchronize(s);
-    dev_free(g, &d_invR);
-    dev_free(g, &d_aij);
+    dev_free(g, &d_pairs);
     dev_free(g, &d_xyz);
     dev_free(g, &d_pointAtom);
-    dev_free(g, &d_near);
     return status;
 }
 
