@@ -189,8 +189,8 @@ int xq_estimate_bytes(long long nPoints, int nFunctions, double meanKeptFunction
         // exponents, P digits.
         b += 1.1 * (18.0 + 1.15 * 17.0) * values + 512.0 * blocks + 8.0 * n * n + 4.0 * n;
     else
-        // Phi in two operand orders, grad Phi, W (48 bytes per stored value).
-        b += 1.1 * 48.0 * values;
+        // Phi in two operand orders, grad Phi, W (48 bytes per stored value) and the density's row-chunk shares (1 byte).
+        b += 1.1 * 49.0 * values;
     *bytes = static_cast<long long>(b);
     return kOK;
 }

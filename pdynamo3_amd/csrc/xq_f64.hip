@@ -3,9 +3,9 @@
 //   X = P_red Phi, rho = sum Phi X, grad rho = 2 sum grad Phi X, functional, W = (w vrho / 2) Phi + 2 w vsigma
 //   (grad rho . grad Phi), V += Phi W^T + W Phi^T (lower triangle).
 // The basis values are stored once per geometry in the lane order the products consume, so every operand load is one
-// coalesced 512-byte row per wave.  The kernels follow the mixed path's structure (xq_mixed.hip): a per-block density
-// kernel with P_red staged in LDS by row panels, a per-chunk W kernel, and a Fock kernel over a flat list of
-// lower-triangle tiles with FP64 atomics; all read the same job table, so one launch serves one job or a batch.
+// coalesced 512-byte row per wave.  The kernels follow the mixed path's structure (xq_mixed.hip): a density kernel per row
+// chunk of a block with P_red staged in LDS, the functional per block, a per-chunk W kernel, and a Fock kernel over a flat
+// list of lower-triangle tiles with FP64 atomics; all read the same job table, so one launch serves one job or a batch.
 //
 // MFMA lane layout (16 x 16 x 4, FP64): lane l supplies A[l % 16][l / 16] and B[l / 16][l % 16] and receives
 // D[4 v + l / 16][l % 16] for v = 0..3.
@@ -33,8 +33,7 @@ namespace {
 
 constexpr int kC = 32;                   // chunk rows
 constexpr int kChunk = 4096;             // doubles per chunk plane
-constexpr int kPanelF = 4;               // chunks of P_red columns staged at once
-constexpr int kPanelPitch = kPanelF * kC + 2;   // LDS row pitch in doubles (padded against bank conflicts)
+constexpr int kRowPitch = kC + 4;        // LDS row pitch of a staged P_red chunk in doubles (padded against bank conflicts)
 constexpr int kIdxCache = 1024;          // kept-function indices of a block cached in LDS by the density kernel
 
 __device__ __forceinline__ v4d mfma_f64(double a, double b, const v4d &c) {
@@ -78,176 +77,107 @@ __global__ void __launch_bounds__(256) f64_prepare_kernel(
     }
 }
 
-// Density kernel (per block, 256 threads = 4 waves; wave wv owns points 32 wv .. + 31): X = P_red Phi on FP64 MFMA in
-// 32 x 32 tiles (2 x 2 MFMA tiles per wave), rho and grad rho, the functional, E_xc / N_e block sums and the W
-// coefficients per point.  P_red is staged in LDS by row panels of kPanelF chunks; the Phi operands of the next chunk
-// are loaded while the current one is multiplied.
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
-density_kernel_f64(const MixedJob *__restrict__ jobs, int nJobs) {
-    __shared__ double sPf[kC][kPanelPitch];
+// Density rows (one row chunk I of one block per work-group, 256 threads = 4 waves; wave wv owns points 32 wv .. + 31):
+// X = P_red Phi for the chunk's 32 rows on FP64 MFMA (2 x 2 MFMA tiles per wave), then the chunk's share of rho and grad rho
+// at the block's points, stored in part[chunk][4][point]; density_functional_kernel (xq_mixed.hip) sums the shares.  Each
+// step multiplies one 32 x 32 chunk of P_red, gathered by all threads and staged in one of two LDS buffers (one barrier per
+// step), with the matching Phi chunk, whose operands go straight to registers; both are fetched one step ahead.  The row
+// chunks of a block are consecutive items of one XCD, so that Phi comes from HBM about once per block.
+// Bound by the FP64 matrix cores and the gathers' latency.  One work-group per block, which read Phi once per row chunk from
+// HBM and waited for each panel of gathers, took 8.26 ms on (H2O)64 (1.3e11 operations, 9.6 GB); this
+// takes 4.13 ms and the functional 0.21 ms.
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
+density_rows_kernel_f64(const MixedJob *__restrict__ jobs, int nJobs, int interleaved) {
+    __shared__ double sP[2][kC][kRowPitch];
     __shared__ int sIdx[kIdxCache];
-    __shared__ double rsum[4][kBlockSize];
-    __shared__ double wsum[4][2];
-    // Work-group g runs on XCD x = g % 8 and takes slot g / 8 of that XCD's list: the jobs' block ranges x in job order
-    // (each a contiguous region of its molecule, so that the XCD's L2 holds the P rows its blocks gather; the ranges
-    // of one job have equal estimated cost), each range's blocks in order of decreasing cost.
+    // Work-group g runs on XCD x = g % 8 and takes slot g / 8 of that XCD's item list, as the mixed density rows.
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-    const MixedJob &J = jobs[job_of(jobs, nJobs, slot, [xcd](const MixedJob &j) { return j.xcdBase[xcd]; })];
-    const int local = slot - J.xcdBase[xcd];
-    if (local >= J.xcdStart[xcd + 1] - J.xcdStart[xcd]) return;
-    const int b = J.order[J.xcdStart[xcd] + local].x;
-    const DevBlock blk = J.blocks[b];
-    const int nb = blk.nKept, np = blk.nPoints, n = J.n;
+    const MixedJob &J = interleaved ? jobs[slot & 1]
+                                    : jobs[job_of(jobs, nJobs, slot, [xcd](const MixedJob &j) { return j.itemBase[xcd]; })];
+    const int local = interleaved ? slot >> 1 : slot - J.itemBase[xcd];
+    if (local >= J.itemStart[xcd + 1] - J.itemStart[xcd]) return;
+    // {chunk, kept functions x 1024 + row chunk, first kept index, block}.
+    const int4 ent = J.items[J.itemStart[xcd] + local];
+    const size_t CI = static_cast<size_t>(ent.x);
+    const int nb = ent.y >> 10, I = ent.y & 1023, n = J.n;
+    const size_t C = CI - I;
+    const int nChunks = (nb + kC - 1) / kC;
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6, l16 = lane & 15, l4 = lane >> 4;
-    if (nb <= 0) {
-        if (t == 0) { J.blockEN[2 * b] = 0.0; J.blockEN[2 * b + 1] = 0.0; J.skip[b] = 1; }
-        if (J.rhoOut != nullptr && t < np)
-            for (int c = 0; c < 4; c++) J.rhoOut[4 * (static_cast<size_t>(blk.pStart) + t) + c] = 0.0;
-        return;
-    }
     // The block's kept-function indices, cached in LDS for the P_red gathers (blocks with more kept functions than the
     // cache read them from memory).
-    const int *idxG = J.idx + blk.iOffset;
+    const int *idxG = J.idx + ent.z;
     for (int k = t; k < nb && k < kIdxCache; k += 256) sIdx[k] = idxG[k];
     __syncthreads();
     const int *idx = nb <= kIdxCache ? sIdx : idxG;
-    const size_t C = static_cast<size_t>(J.chunkOffset[b]);
-    const int nChunks = (nb + kC - 1) / kC;
     const double *__restrict__ P = J.P;
     const double *__restrict__ FPB = J.FPB;
     const double *__restrict__ GPB = J.GPB;
     // Operand entry (s, h) of this lane within a chunk plane of FPB / GPB.
     auto op = [&](int s, int h) { return ((wv * 8 + s) * 2 + h) * 64 + lane; };
-    auto fetchB = [&](int c, double (&bq)[8][2]) {
+    // Staging: row sr, columns 8 j + s8 (eight lanes read eight consecutive kept functions).
+    const int sr = t >> 3, s8 = t & 7, r = kC * I + sr;
+    const size_t rowOff = r < nb ? static_cast<size_t>(idx[r]) * n : 0;
+    double pv[4], bnext[8][2];
+    auto fetch = [&](int c) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int k = kC * c + 8 * j + s8;
+            pv[j] = r < nb && k < nb ? P[rowOff + idx[k]] : 0.0;
+        }
 #pragma unroll
         for (int s = 0; s < 8; s++)
 #pragma unroll
-            for (int h = 0; h < 2; h++) bq[s][h] = FPB[(C + c) * kChunk + op(s, h)];
+            for (int h = 0; h < 2; h++) bnext[s][h] = FPB[(C + c) * kChunk + op(s, h)];
     };
-    const int sr = t >> 3, s8 = t & 7;     // staging: row sr, columns 4 s8 .. + 3 of each chunk of the panel
-    double bnext[8][2];
-    fetchB(0, bnext);
-    double pr[2] = {0.0, 0.0}, pgx[2] = {0.0, 0.0}, pgy[2] = {0.0, 0.0}, pgz[2] = {0.0, 0.0};
-    for (int I = 0; I < nChunks; I++) {
-        v4d acc[2][2];
-        const int r = kC * I + sr;
-        const size_t rowOff = r < nb ? static_cast<size_t>(idx[r]) * n : 0;
-        for (int c0 = 0; c0 < nChunks; c0 += kPanelF) {
-            const int nc = nChunks - c0 < kPanelF ? nChunks - c0 : kPanelF;
-            double pv[kPanelF][4];
+    v4d acc[2][2];
 #pragma unroll
-            for (int m = 0; m < kPanelF; m++)
+    for (int hm = 0; hm < 2; hm++)
 #pragma unroll
-                for (int jj = 0; jj < 4; jj++) {
-                    const int k = kC * (c0 + m) + 4 * s8 + jj;
-                    pv[m][jj] = (m < nc && r < nb && k < nb) ? P[rowOff + idx[k]] : 0.0;
-                }
-            __syncthreads();   // every wave is done with the previous panel
+        for (int hn = 0; hn < 2; hn++) acc[hm][hn] = v4d{0.0, 0.0, 0.0, 0.0};
+    fetch(0);
+#pragma unroll 2
+    for (int c = 0; c < nChunks; c++) {
+        double (&buf)[kC][kRowPitch] = sP[c & 1];
 #pragma unroll
-            for (int m = 0; m < kPanelF; m++)
+        for (int j = 0; j < 4; j++) buf[sr][8 * j + s8] = pv[j];
+        double bq[8][2];
 #pragma unroll
-                for (int jj = 0; jj < 4; jj++) sPf[sr][kC * m + 4 * s8 + jj] = pv[m][jj];
-            if (c0 == 0) {
+        for (int s = 0; s < 8; s++) { bq[s][0] = bnext[s][0]; bq[s][1] = bnext[s][1]; }
+        // A wave writes this buffer again two steps on, after the next barrier, which every wave reaches done with it.
+        __syncthreads();
+        if (c + 1 < nChunks) fetch(c + 1);
 #pragma unroll
-                for (int hm = 0; hm < 2; hm++)
-#pragma unroll
-                    for (int hn = 0; hn < 2; hn++) acc[hm][hn] = v4d{0.0, 0.0, 0.0, 0.0};
-            }
-            __syncthreads();
-            for (int cl = 0; cl < nc; cl++) {
-                const int c = c0 + cl;
-                double bq[8][2];
-#pragma unroll
-                for (int s = 0; s < 8; s++) { bq[s][0] = bnext[s][0]; bq[s][1] = bnext[s][1]; }
-                if (c + 1 < nChunks) fetchB(c + 1, bnext);
-                else if (I + 1 < nChunks) fetchB(0, bnext);
-#pragma unroll
-                for (int s = 0; s < 8; s++) {
-                    const double a0 = sPf[l16][kC * cl + 4 * s + l4], a1 = sPf[16 + l16][kC * cl + 4 * s + l4];
-                    acc[0][0] = mfma_f64(a0, bq[s][0], acc[0][0]);
-                    acc[0][1] = mfma_f64(a0, bq[s][1], acc[0][1]);
-                    acc[1][0] = mfma_f64(a1, bq[s][0], acc[1][0]);
-                    acc[1][1] = mfma_f64(a1, bq[s][1], acc[1][1]);
-                }
-            }
+        for (int s = 0; s < 8; s++) {
+            const double a0 = buf[l16][4 * s + l4], a1 = buf[16 + l16][4 * s + l4];
+            acc[0][0] = mfma_f64(a0, bq[s][0], acc[0][0]);
+            acc[0][1] = mfma_f64(a0, bq[s][1], acc[0][1]);
+            acc[1][0] = mfma_f64(a1, bq[s][0], acc[1][0]);
+            acc[1][1] = mfma_f64(a1, bq[s][1], acc[1][1]);
         }
-        // Epilogue: register v of (hm, hn) is row 16 hm + 4 v + l / 16 of chunk I at point 32 wv + 16 hn + l % 16.
+    }
+    // Epilogue: register v of (hm, hn) is row 16 hm + 4 v + l / 16 of chunk I at point 32 wv + 16 hn + l % 16.
+    double pr[4][2] = {};
+#pragma unroll
+    for (int x = 0; x < 4; x++) {
+        const double *plane = x == 0 ? FPB + CI * kChunk : GPB + (3 * CI + (x - 1)) * kChunk;
 #pragma unroll
         for (int hm = 0; hm < 2; hm++)
 #pragma unroll
             for (int v = 0; v < 4; v++)
 #pragma unroll
-                for (int hn = 0; hn < 2; hn++) {
-                    const int o = op(4 * hm + v, hn);
-                    const double x = acc[hm][hn][v];
-                    pr[hn] += FPB[(C + I) * kChunk + o] * x;
-                    pgx[hn] += GPB[3 * (C + I) * kChunk + o] * x;
-                    pgy[hn] += GPB[(3 * (C + I) + 1) * kChunk + o] * x;
-                    pgz[hn] += GPB[(3 * (C + I) + 2) * kChunk + o] * x;
-                }
+                for (int hn = 0; hn < 2; hn++) pr[x][hn] += plane[op(4 * hm + v, hn)] * acc[hm][hn][v];
     }
-    // Sum over the four lanes that share a point (l / 16 = 0..3).
+    double *q = J.part + CI * 4 * kBlockSize;
 #pragma unroll
-    for (int hn = 0; hn < 2; hn++) {
+    for (int hn = 0; hn < 2; hn++)
 #pragma unroll
-        for (int o = 16; o < 64; o <<= 1) {
-            pr[hn] += __shfl_xor(pr[hn], o, 64);
-            pgx[hn] += __shfl_xor(pgx[hn], o, 64);
-            pgy[hn] += __shfl_xor(pgy[hn], o, 64);
-            pgz[hn] += __shfl_xor(pgz[hn], o, 64);
+        for (int x = 0; x < 4; x++) {
+            // Sum over the four lanes that share a point (l / 16 = 0..3).
+            double e = pr[x][hn];
+            e += __shfl_xor(e, 16, 64);
+            e += __shfl_xor(e, 32, 64);
+            if (l4 == 0) q[x * kBlockSize + kC * wv + 16 * hn + l16] = e;
         }
-        if (l4 == 0) {
-            const int p = kC * wv + 16 * hn + l16;
-            rsum[0][p] = pr[hn];
-            rsum[1][p] = pgx[hn];
-            rsum[2][p] = pgy[hn];
-            rsum[3][p] = pgz[hn];
-        }
-    }
-    __syncthreads();
-    double rho = 0.0, gx = 0.0, gy = 0.0, gz = 0.0;
-    if (t < np) { rho = rsum[0][t]; gx = 2.0 * rsum[1][t]; gy = 2.0 * rsum[2][t]; gz = 2.0 * rsum[3][t]; }
-    if (J.rhoOut != nullptr) {   // one spin of an unrestricted quadrature: the functional follows in its own kernel
-        if (t < np) {
-            double *o = J.rhoOut + 4 * (static_cast<size_t>(blk.pStart) + t);
-            o[0] = rho; o[1] = gx; o[2] = gy; o[3] = gz;
-        }
-        return;
-    }
-    double mx = t < np ? fabs(rho) : 0.0;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, 64));
-    if (lane == 0) wsum[wv][0] = mx;
-    __syncthreads();
-    const bool skipped = !(fmax(fmax(wsum[0][0], wsum[1][0]), fmax(wsum[2][0], wsum[3][0])) > J.rhoTol);
-    __syncthreads();
-    double e = 0.0, ne = 0.0;
-    if (t < np) {
-        double vr = 0.0, vs = 0.0;
-        if (!skipped) {
-            double eps;
-            evaluate_functional(J.fs, rho, gx * gx + gy * gy + gz * gz, eps, vr, vs);
-            const double ww = J.w[blk.pStart + t];
-            vr *= ww;
-            vs *= ww;
-            e = eps * rho * ww;
-            ne = rho * ww;
-        }
-        double *cw = J.wcoef + 4 * (static_cast<size_t>(blk.pStart) + t);
-        cw[0] = 0.5 * vr;
-        cw[1] = 2.0 * vs * gx;
-        cw[2] = 2.0 * vs * gy;
-        cw[3] = 2.0 * vs * gz;
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) { e += __shfl_xor(e, o, 64); ne += __shfl_xor(ne, o, 64); }
-    if (lane == 0) { wsum[wv][0] = e; wsum[wv][1] = ne; }
-    __syncthreads();
-    if (t == 0) {
-        J.blockEN[2 * b] = ((wsum[0][0] + wsum[1][0]) + wsum[2][0]) + wsum[3][0];
-        J.blockEN[2 * b + 1] = ((wsum[0][1] + wsum[1][1]) + wsum[2][1]) + wsum[3][1];
-        J.skip[b] = skipped ? 1 : 0;
-    }
 }
 
 // W (one chunk per work-group, 256 threads): W_rp = c0_p Phi_rp + c_p . grad Phi_rp from the density-order planes,
@@ -349,6 +279,7 @@ int prepare_f64(xq_grid *g, const double *f, const double *fx, const double *fy,
     XQ_TRY(dev_alloc(g, &g->d_FPA, nc * kChunk));
     XQ_TRY(dev_alloc(g, &g->d_WPA, nc * kChunk));
     XQ_TRY(dev_alloc(g, &g->d_wcoef, 4 * static_cast<size_t>(g->nPoints > 0 ? g->nPoints : 1)));
+    XQ_TRY(dev_alloc(g, &g->d_part, nc * 4 * kBlockSize));
     hipStream_t s = g->stream;
     if (g->nChunks > 0)
         hipLaunchKernelGGL(f64_prepare_kernel, dim3(static_cast<unsigned>(g->nChunks)), dim3(256), 0, s, g->d_blocks,
@@ -358,12 +289,20 @@ int prepare_f64(xq_grid *g, const double *f, const double *fx, const double *fy,
     return kOK;
 }
 
-// Per-step W planes of a second job on the handle (the beta spin of an unrestricted quadrature).
+// Per-step arrays of a second job on the handle (the beta spin of an unrestricted quadrature): W planes and the density's
+// row-chunk shares.  Complete or released.
 int alloc_step_f64(xq_grid *g, StepArrays *a) {
-    return dev_alloc(g, &a->WPA, static_cast<size_t>(g->nChunks > 0 ? g->nChunks : 1) * kChunk);
+    const size_t nc = static_cast<size_t>(g->nChunks > 0 ? g->nChunks : 1);
+    int status = dev_alloc(g, &a->WPA, nc * kChunk);
+    if (status == kOK) status = dev_alloc(g, &a->part, nc * 4 * kBlockSize);
+    if (status != kOK) free_step_f64(g, a);
+    return status;
 }
 
-void free_step_f64(xq_grid *g, StepArrays *a) { dev_free(g, &a->WPA); }
+void free_step_f64(xq_grid *g, StepArrays *a) {
+    dev_free(g, &a->WPA);
+    dev_free(g, &a->part);
+}
 
 void free_f64(xq_grid *g) {
     dev_free(g, &g->d_FPB);
@@ -374,17 +313,21 @@ void free_f64(xq_grid *g) {
 
 int launch_f64(hipStream_t s, const StageEvents &ev, int nJobs, xq_grid *const *grids, const FunctionalSet *fs,
                MixedJob *h_table, MixedJob *d_table, int stages, const StepArrays *over) {
-    long long rows, blocks, chunks, groups, blockSlots;
-    fill_jobs(nJobs, grids, fs, h_table, &rows, &blocks, &chunks, &groups, over, &blockSlots);
-    if (blocks > INT32_MAX / 2 || chunks > INT32_MAX / 2 || groups > INT32_MAX / 16) {
+    long long rows, blocks, chunks, groups, itemSlots;
+    fill_jobs(nJobs, grids, fs, h_table, &rows, &blocks, &chunks, &groups, over, &itemSlots);
+    if (blocks > INT32_MAX / 2 || chunks > INT32_MAX / 2 || groups > INT32_MAX / 16 || itemSlots > INT32_MAX / 16) {
         set_error("batch too large for one launch");
         return kInvalidArgument;
     }
     XQ_CHECK(hipMemcpyAsync(d_table, h_table, nJobs * sizeof(MixedJob), hipMemcpyHostToDevice, s));
     XQ_CHECK(hipEventRecord(ev.evRho0, s));
     if ((stages & kStageDensity) && blocks > 0) {
-        hipLaunchKernelGGL(density_kernel_f64, dim3(static_cast<unsigned>(8 * blockSlots)), dim3(256), 0, s, d_table,
-                           nJobs);
+        // The two spins of one handle (an unrestricted quadrature) run interleaved item by item.
+        const int interleaved = nJobs == 2 && grids[0] == grids[1] ? 1 : 0;
+        if (itemSlots > 0)
+            hipLaunchKernelGGL(density_rows_kernel_f64, dim3(static_cast<unsigned>(8 * itemSlots)), dim3(256), 0, s, d_table,
+                               nJobs, interleaved);
+        launch_density_functional(s, nJobs, blocks, h_table[0].rhoOut != nullptr, d_table);
     }
     XQ_CHECK(hipEventRecord(ev.evDens1, s));
     XQ_CHECK(hipEventRecord(ev.evRho1, s));

@@ -414,7 +414,7 @@ __global__ void __launch_bounds__(256) sum_copies_kernel(int nEntries, const dou
 namespace {
 
 // The launch order of the batch b0 .. b1 - 1, written to order[b0 .. b1): as the density launch's (xq_mixed.hip,
-// build_block_order), 8 contiguous ranges of equal estimated cost (T^2 + T + 1 for a block of T row chunks), one per
+// build_density_items), 8 contiguous ranges of equal estimated cost (T^2 + T + 1 for a block of T row chunks), one per
 // XCD, each sorted by decreasing cost, so that the batch's longest blocks do not start last.
 XcdRanges batch_order(const xq_grid *g, int b0, int b1, std::vector<int> &order) {
     std::vector<double> cost(static_cast<size_t>(b1 - b0));

@@ -77,13 +77,9 @@ struct MixedJob {
     double rhoTol;
     int n, nBlocks, nChunks, nTiles;
     int rowBase, blockBase, chunkBase, groupBase;
-    // Density launch: blocks order[xcdStart[x] .. xcdStart[x + 1]) run on XCD x, at that XCD's slots from xcdBase[x];
-    // each entry {block, first chunk, first kept index, kept functions x 256 + points}.
-    const int4 *order;
-    int xcdStart[9], xcdBase[8];
-    // Mixed density launch: one work-group per row chunk of a block; items[itemStart[x] .. itemStart[x + 1]) run on
-    // XCD x from slot itemBase[x], each {chunk, kept functions x 1024 + row chunk, first kept index, block}; part
-    // receives each chunk's share of rho and grad rho, [chunk][4][point].
+    // Density launches: one work-group per row chunk of a block; items[itemStart[x] .. itemStart[x + 1]) run on XCD x from
+    // slot itemBase[x], each {chunk, kept functions x 1024 + row chunk, first kept index, block}; part receives each chunk's
+    // share of rho and grad rho, [chunk][4][point].
     const int4 *items;
     int itemStart[9], itemBase[8];
     double *part;
@@ -107,13 +103,9 @@ struct xq_grid {
     std::vector<xq::DevBlock> blocks;     // host copy
     double *d_x = nullptr, *d_y = nullptr, *d_z = nullptr, *d_w = nullptr;
     xq::DevBlock *d_blocks = nullptr;
-    // Density launch order: the blocks cut into 8 contiguous ranges of equal estimated cost (one per XCD, so that each
-    // XCD's L2 holds one region's P rows), each range in order of decreasing cost (the longest blocks start first).
-    std::vector<int4> h_order;
-    int4 *d_order = nullptr;
-    int xcdStart[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    // The mixed density launch's items: each block of the order above cut into its row chunks, consecutive on the
-    // block's XCD; per chunk, its share of rho and grad rho (d_part).
+    // The density launches' items: the blocks cut into 8 contiguous ranges of equal estimated cost (one per XCD, so that
+    // each XCD's L2 holds one region's P rows), each range in order of decreasing cost (the longest blocks start first),
+    // every block cut into its row chunks; per chunk, its share of rho and grad rho (d_part).
     std::vector<int4> h_items;
     int4 *d_items = nullptr;
     int itemStart[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
@@ -263,14 +255,13 @@ void launch_expand(int n, const double *packed, double *dense, hipStream_t s);
 void launch_zero(int n, double *dense, hipStream_t s);
 void launch_pack(int n, const double *dense, double *packed, hipStream_t s);
 // Shared by both precisions: the job table entries of the given handles, the per-block chunk tables and Fock tile list.
-// blockSlots (optional): the density launch's work-groups per XCD, the largest over the XCDs of the jobs' summed block
-// ranges; itemSlots (optional): the same for the mixed density launch's row-chunk items.
+// itemSlots (optional): the density launches' work-groups per XCD, the largest over the XCDs of the jobs' summed items.
 void fill_jobs(int nJobs, xq_grid *const *grids, const FunctionalSet *fs, MixedJob *h_table, long long *rows,
                long long *blocks, long long *chunks, long long *groups, const StepArrays *over = nullptr,
-               long long *blockSlots = nullptr, long long *itemSlots = nullptr);
-// The density launch's block order (d_order, xcdStart) and the mixed launch's row-chunk items (d_items, itemStart),
-// from the blocks' kept-function counts; at basis set-up.
-int build_block_order(xq_grid *g, hipStream_t s);
+               long long *itemSlots = nullptr);
+// The density launches' row-chunk items (d_items, itemStart), from the blocks' kept-function counts; at basis set-up.
+int build_density_items(xq_grid *g, hipStream_t s);
+void launch_density_functional(hipStream_t s, int nJobs, long long blocks, bool rhoOut, const MixedJob *d_table);
 int chunk_tables(xq_grid *g);
 int prepare_f64(xq_grid *g, const double *f, const double *fx, const double *fy, const double *fz);
 void free_f64(xq_grid *g);

@@ -773,15 +773,15 @@ int chunk_tables(xq_grid *g) {
         XQ_CHECK(hipMemcpyAsync(g->d_tiles, tiles.data(), tiles.size() * sizeof(int4), hipMemcpyHostToDevice, s));
     // The host vectors must outlive the copies.
     XQ_CHECK(hipStreamSynchronize(s));
-    return build_block_order(g, s);
+    return build_density_items(g, s);
 }
 
-// The density launch's block order.  A block of T row chunks costs about T^2 MFMA steps of the density kernel, plus
+// The density launches' items.  A block of T row chunks costs about T^2 MFMA steps of the density kernel, plus
 // one epilogue per row chunk and the functional (counted as one step each, and one for a block without kept
 // functions).  The blocks are cut into 8 contiguous ranges of equal summed cost, one per XCD, each sorted by decreasing
 // cost: on (H2O)64 the largest blocks take about 28 times the mean, and started last they set the length of the launch.
-// The mixed density launch takes the same order with each block cut into its row chunks, consecutive on its XCD.
-int build_block_order(xq_grid *g, hipStream_t s) {
+// Each block is cut into its row chunks, consecutive on its XCD.
+int build_density_items(xq_grid *g, hipStream_t s) {
     const int nB = g->nBlocks;
     std::vector<double> cost(static_cast<size_t>(nB > 0 ? nB : 1), 0.0);
     double total = 0.0;
@@ -790,15 +790,14 @@ int build_block_order(xq_grid *g, hipStream_t s) {
         cost[b] = T * T + T + 1.0;
         total += cost[b];
     }
-    g->xcdStart[0] = 0;
+    int start[9] = {0, 0, 0, 0, 0, 0, 0, 0, nB};
     int b = 0;
     double acc = 0.0;
     for (int x = 1; x < 8; x++) {
         const double target = total * x / 8.0;
         while (b < nB && acc + 0.5 * cost[b] < target) acc += cost[b++];
-        g->xcdStart[x] = b;
+        start[x] = b;
     }
-    g->xcdStart[8] = nB;
     std::vector<int> order(static_cast<size_t>(nB > 0 ? nB : 1), 0), firstChunk(static_cast<size_t>(nB > 0 ? nB : 1), 0);
     for (int i = 0, c = 0; i < nB; i++) {
         order[i] = i;
@@ -806,24 +805,20 @@ int build_block_order(xq_grid *g, hipStream_t s) {
         c += (g->blocks[i].nKept + kC - 1) / kC;
     }
     for (int x = 0; x < 8; x++)
-        std::stable_sort(order.begin() + g->xcdStart[x], order.begin() + g->xcdStart[x + 1],
+        std::stable_sort(order.begin() + start[x], order.begin() + start[x + 1],
                          [&](int u, int v) { return cost[u] > cost[v]; });
-    g->h_order.assign(order.size(), make_int4(0, 0, 0, 0));
     g->h_items.clear();
     for (int x = 0; x < 8; x++) {
         g->itemStart[x] = static_cast<int>(g->h_items.size());
-        for (int i = g->xcdStart[x]; i < g->xcdStart[x + 1]; i++) {
+        for (int i = start[x]; i < start[x + 1]; i++) {
             const xq::DevBlock &blk = g->blocks[order[i]];
-            g->h_order[i] = make_int4(order[i], firstChunk[order[i]], blk.iOffset, blk.nKept * 256 + blk.nPoints);
             // The block's row chunks, one item each (nKept <= 26000, so that row chunk I < 1024 fits beside it).
             for (int I = 0; I < (blk.nKept + kC - 1) / kC; I++)
                 g->h_items.push_back(make_int4(firstChunk[order[i]] + I, blk.nKept * 1024 + I, blk.iOffset, order[i]));
         }
     }
     g->itemStart[8] = static_cast<int>(g->h_items.size());
-    XQ_TRY(dev_alloc(g, &g->d_order, g->h_order.size()));
     XQ_TRY(dev_alloc(g, &g->d_items, g->h_items.empty() ? 1 : g->h_items.size()));
-    XQ_CHECK(hipMemcpyAsync(g->d_order, g->h_order.data(), g->h_order.size() * sizeof(int4), hipMemcpyHostToDevice, s));
     if (!g->h_items.empty())
         XQ_CHECK(hipMemcpyAsync(g->d_items, g->h_items.data(), g->h_items.size() * sizeof(int4), hipMemcpyHostToDevice,
                                 s));
@@ -976,12 +971,10 @@ void free_step_mixed(xq_grid *g, StepArrays *a) {
 }
 
 void free_mixed(xq_grid *g) {
-    dev_free(g, &g->d_order);
     dev_free(g, &g->d_items);
     dev_free(g, &g->d_part);
-    g->h_order.clear();
     g->h_items.clear();
-    for (int x = 0; x <= 8; x++) g->xcdStart[x] = g->itemStart[x] = 0;
+    for (int x = 0; x <= 8; x++) g->itemStart[x] = 0;
     dev_free(g, &g->d_chunkOffset);
     dev_free(g, &g->d_chunkBlock);
     dev_free(g, &g->d_tiles);
@@ -1016,19 +1009,13 @@ void free_mixed(xq_grid *g) {
 // The job table entries of the given handles (each with its functional) and each stage's total work-groups.
 void fill_jobs(int nJobs, xq_grid *const *grids, const FunctionalSet *fs, MixedJob *h_table, long long *rowsOut,
                long long *blocksOut, long long *chunksOut, long long *groupsOut, const StepArrays *over,
-               long long *blockSlotsOut, long long *itemSlotsOut) {
-    long long rows = 0, blocks = 0, chunks = 0, groups = 0, slots[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+               long long *itemSlotsOut) {
+    long long rows = 0, blocks = 0, chunks = 0, groups = 0;
     long long itemSlots[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     for (int j = 0; j < nJobs; j++) {
         const xq_grid *g = grids[j];
         MixedJob &J = h_table[j];
         J.blocks = g->d_blocks;
-        J.order = g->d_order;
-        for (int x = 0; x <= 8; x++) J.xcdStart[x] = g->xcdStart[x];
-        for (int x = 0; x < 8; x++) {
-            J.xcdBase[x] = static_cast<int>(slots[x]);
-            slots[x] += g->xcdStart[x + 1] - g->xcdStart[x];
-        }
         J.items = g->d_items;
         J.part = g->d_part;
         for (int x = 0; x <= 8; x++) J.itemStart[x] = g->itemStart[x];
@@ -1100,10 +1087,17 @@ void fill_jobs(int nJobs, xq_grid *const *grids, const FunctionalSet *fs, MixedJ
     }
     *rowsOut = rows;
     *blocksOut = blocks;
-    if (blockSlotsOut != nullptr) *blockSlotsOut = *std::max_element(slots, slots + 8);
     if (itemSlotsOut != nullptr) *itemSlotsOut = *std::max_element(itemSlots, itemSlots + 8);
     *chunksOut = chunks;
     *groupsOut = groups;
+}
+
+// The functional of every block of the jobs after their density rows (either precision); rhoOut: the density stage of one
+// spin of an unrestricted quadrature (every job of the call).
+void launch_density_functional(hipStream_t s, int nJobs, long long blocks, bool rhoOut, const MixedJob *d_table) {
+    const dim3 grid(static_cast<unsigned>(blocks));
+    if (rhoOut) hipLaunchKernelGGL(density_functional_kernel<true>, grid, dim3(kBlockSize), 0, s, d_table, nJobs);
+    else hipLaunchKernelGGL(density_functional_kernel<false>, grid, dim3(kBlockSize), 0, s, d_table, nJobs);
 }
 
 // The four stage launches of the mixed path, each one launch over all the jobs.  h_table (pinned) and d_table hold at
@@ -1111,7 +1105,7 @@ void fill_jobs(int nJobs, xq_grid *const *grids, const FunctionalSet *fs, MixedJ
 int launch_mixed(hipStream_t s, const StageEvents &ev, int nJobs, xq_grid *const *grids, const FunctionalSet *fs,
                  MixedJob *h_table, MixedJob *d_table, int stages, const StepArrays *over) {
     long long rows, blocks, chunks, groups, itemSlots;
-    fill_jobs(nJobs, grids, fs, h_table, &rows, &blocks, &chunks, &groups, over, nullptr, &itemSlots);
+    fill_jobs(nJobs, grids, fs, h_table, &rows, &blocks, &chunks, &groups, over, &itemSlots);
     if (rows > INT32_MAX / 2 || blocks > INT32_MAX / 2 || chunks > INT32_MAX / 2 || groups > INT32_MAX / 16 ||
         itemSlots > INT32_MAX / 16) {
         set_error("batch too large for one launch");
@@ -1130,13 +1124,7 @@ int launch_mixed(hipStream_t s, const StageEvents &ev, int nJobs, xq_grid *const
             hipLaunchKernelGGL(density_rows_kernel, dim3(static_cast<unsigned>(8 * itemSlots)), dim3(256), 0, s, d_table,
                                nJobs, interleaved);
         XQ_CHECK(hipEventRecord(ev.evDens1, s));
-        if (h_table[0].rhoOut != nullptr) {   // the density stage of one spin (every job of the call)
-            hipLaunchKernelGGL(density_functional_kernel<true>, dim3(static_cast<unsigned>(blocks)), dim3(kBlockSize), 0,
-                               s, d_table, nJobs);
-        } else {
-            hipLaunchKernelGGL(density_functional_kernel<false>, dim3(static_cast<unsigned>(blocks)), dim3(kBlockSize),
-                               0, s, d_table, nJobs);
-        }
+        launch_density_functional(s, nJobs, blocks, h_table[0].rhoOut != nullptr, d_table);
     } else {
         XQ_CHECK(hipEventRecord(ev.evDens1, s));
     }
