@@ -6,16 +6,15 @@
 // csource/Lebedev.c:62-193), the octahedral orbit expansion order (Lebedev.c:1565-1719) and the Becke weight
 // (DFTGridWeights.c:43-80, 220-258).
 //
-// Device layout: every radial shell (atom, radius) is one work-group; each thread computes the Becke weight of one angular
-// point in FP64.  Candidate points of one atom are contiguous and ordered (radial shell, angular index) exactly as the
+// Device layout: a group of 16 to 64 lanes of a radial shell's (atom, radius) work-groups computes the Becke weight of one
+// angular point in FP64, the atoms spread over its lanes.  Candidate points of one atom are contiguous and ordered (radial shell, angular index) exactly as the
 // reference orders them, so the order-preserving cull reproduces the reference's point and block order.
 //
-// Becke weight: P_A / sum_i P_i with P_i = prod_{j != i} s(nu_ij).  P_A (the point's own atom) is formed in full.  For
-// i != A the product is formed factor by factor, starting with the factors from atom A and from the atom nearest the
-// point, then the others nearest atom to A first (the factors that can make it vanish come early), and stops once it falls below 2^-64 max(|P_A|, |P_near|), P_near
-// the product of the atom nearest the point: all later factors lie in [0, 1], so the dropped part of sum_i P_i is below
-// nAtoms * 2^-64 of max(P_A, P_near) <= the sum.  This turns the reference's O(nAtoms^2) pair loop per point into
-// O(nAtoms) for points that sit in their own atom's cell or in the cell of the atom nearest them.
+// Becke weight: P_A / sum_i P_i with P_i = prod_{j != i} s(nu_ij).  P_A (the point's own atom) is formed first, then the
+// product of the atom whose factors with the atoms done so far leave the largest bound, and so on until every remaining
+// atom's bound is below 2^-64 of the largest product: each cell function lies in [0, 1], so what is left out of the sum is
+// below nAtoms * 2^-64 of it.  This turns the reference's O(nAtoms^2) pair loop per point into O(nAtoms) for each of the
+// few atoms whose cells matter at the point.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -160,121 +159,136 @@ __device__ __forceinline__ double becke_poly(double nu) {
     return sum;
 }
 
-// Factor of P_k from the pair (k, m), k != m, given the pair's 1/R and size adjustment (stored once for the ordered pair
-// (max, min)): s(nu) for k > m, 1 - s(nu) for k < m, with mu = (r_max - r_min) / R.
-__device__ __forceinline__ double becke_factor_of(bool kHigh, double rk, double rm, double invR, double a) {
-    const double rhi = kHigh ? rk : rm, rlo = kHigh ? rm : rk;
-    const double mu = (rhi - rlo) * invR;
-    const double nu = mu + a * (1.0 - mu * mu);
-    const double s = kBeckeA * becke_poly(nu);
-    return kHigh ? (0.5 - s) : (0.5 + s);
+template <int GS>
+__device__ __forceinline__ double group_sum(double x) {
+#pragma unroll
+    for (int o = GS / 2; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
+    return x;
+}
+template <int GS>
+__device__ __forceinline__ double group_product(double x) {
+#pragma unroll
+    for (int o = GS / 2; o > 0; o >>= 1) x *= __shfl_xor(x, o, 64);
+    return x;
 }
 
-__device__ __forceinline__ int pair_index(int k, int m) {
-    const int hi = k > m ? k : m, lo = k > m ? m : k;
-    return (hi * (hi - 1)) / 2 + lo;
+// LDS writes of a wave are in order; this keeps the compiler from moving accesses over it.
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 
-// Candidate points of one radial shell per work-group (thread = angular point) and their Becke weights
-// w = 4 pi w_r w_ang P_A / sum_i P_i (DFTGrid.c:158-211, DFTGridWeights.c:220-258).  P_A and the product of the atom
-// nearest the point come first; when even P_A / (P_A + P_near) leaves the weight below half the cull tolerance (or
-// P_A = 0), the point is culled (as the reference culls it) without the other products.  The atom coordinates, the pair
-// data of the shell's atom A (row A of 1/R and a) and the atoms in order of distance from A are staged in LDS.  P_A is
-// computed in full; each other P_i takes its factors with A and the nearest atom, then the others nearest A first, and
-// stops once it falls below 2^-64 of max(|P_A|, |P_near|) (both <= the sum), where it no longer changes the sum beyond
-// rounding.  Each factor is the reference's cell function of the same mu and nu, rounded as the reference rounds it (so factors that vanish there vanish here); the products are taken in another
-// order, so weights agree with the reference's to rounding and the same points pass the cull.
-__global__ void __launch_bounds__(256) candidate_points_kernel(const RadialShell *__restrict__ shells,
-                                                               const double *__restrict__ rules,
-                                                               const double *__restrict__ xyz, int nAtoms,
-                                                               const double *__restrict__ invR,
-                                                               const double *__restrict__ aij,
-                                                               const int *__restrict__ order,
-                                                               double *__restrict__ cx, double *__restrict__ cy,
-                                                               double *__restrict__ cz, double *__restrict__ cw,
-                                                               int *__restrict__ keep) {
+// The group's ballot bits (group at lane bit0 of its wave), lowest first.
+template <int GS>
+__device__ __forceinline__ unsigned long long group_ballot(bool x, int bit0) {
+    return (__ballot(x) >> bit0) & (GS == 64 ? ~0ull : ((1ull << (GS & 63)) - 1ull));
+}
+
+// The atom (lane atoms gl + GS a, not done) of the largest bound of a group, and that bound (-1 if all are done).
+template <int LA, int GS>
+__device__ __forceinline__ int next_atom(const double (&b)[LA], const bool (&done)[LA], int gl, int bit0, double &top) {
+    double best = -1.0;
+    int bi = 0;
+#pragma unroll
+    for (int a = 0; a < LA; a++)
+        if (!done[a] && b[a] > best) { best = b[a]; bi = gl + GS * a; }
+    top = best;
+#pragma unroll
+    for (int o = GS / 2; o > 0; o >>= 1) top = fmax(top, __shfl_xor(top, o, 64));
+    return __shfl(bi, bit0 + __ffsll(static_cast<long long>(group_ballot<GS>(best == top, bit0))) - 1, 64);
+}
+
+// Share of the largest cell product at a point below which an atom's product does not count: in the sum of the products, and
+// in the derivatives, where a factor s = c y^11 P (y = 1 - nu) near its zero has a derivative of 11 s / y, so that a dropped
+// term is below 1e-16 of the point's energy over a bond length.
+constexpr double kCellScreen = 0x1p-64;
+
+// Candidate points of one radial shell and their Becke weights w = 4 pi w_r w_ang P_A / sum_i P_i (DFTGrid.c:158-211,
+// DFTGridWeights.c:220-258).  A group of GS lanes takes a point, lane l the atoms l, l + GS, ... (at most LA).  Row c
+// evaluates the pairs of atom c with every lane atom: s_ci for P_c and s_ic for the lane atoms' bounds.  Rows are taken for
+// the shell's atom A, then always for the atom of the largest bound, until none passes the screen or the point's weight
+// cannot pass the cull.  Each factor is the reference's cell function of the same mu and nu, rounded as the reference rounds
+// it (so factors that vanish there vanish here, and the same points pass the cull); products and sums are taken in another
+// order, so weights agree with the reference's to rounding.  pairs[i][j] = {1 / R_ij, a_ij} (a_ji = -a_ij: -nu and its
+// polynomial are exact negatives).  The shell's points are dealt to gridDim.y work-groups.
+// Bound by FP64 arithmetic (45 operations a factor).  One point per thread, whose lanes lay in all directions from A and
+// so took nearly every factor of every atom between them, took 7.4 ms on (H2O)24 and 48 ms on (H2O)64; this GRIDMS.
+template <int LA, int GS, int WPG>
+__global__ void __launch_bounds__(64 * WPG) candidate_points_kernel(const RadialShell *__restrict__ shells,
+                                                                    const double *__restrict__ rules,
+                                                                    const double *__restrict__ xyz, int nAtoms,
+                                                                    const double2 *__restrict__ pairs,
+                                                                    double *__restrict__ cx, double *__restrict__ cy,
+                                                                    double *__restrict__ cz, double *__restrict__ cw,
+                                                                    int *__restrict__ keep) {
+    constexpr int kGroups = 64 * WPG / GS;
     extern __shared__ double lds[];
-    double *sx = lds, *sy = lds + nAtoms, *sz = lds + 2 * nAtoms, *sInv = lds + 3 * nAtoms, *sA = lds + 4 * nAtoms;
-    int *sOrd = reinterpret_cast<int *>(lds + 5 * nAtoms);
+    const int t = threadIdx.x, gl = t & (GS - 1), gi = t / GS, bit0 = t & 63 & ~(GS - 1);
+    double *sxyz = lds, *rL = lds + static_cast<size_t>(3 + gi) * nAtoms;
+    for (int i = t; i < 3 * nAtoms; i += 64 * WPG) sxyz[i] = xyz[i];
+    __syncthreads();
     const RadialShell sh = shells[blockIdx.x];
     const int A = sh.atom;
-    for (int j = threadIdx.x; j < nAtoms; j += blockDim.x) {
-        sOrd[j] = order[static_cast<size_t>(A) * nAtoms + j];
-        sx[j] = xyz[3 * j];
-        sy[j] = xyz[3 * j + 1];
-        sz[j] = xyz[3 * j + 2];
-        const int ij = j == A ? 0 : pair_index(A, j);
-        sInv[j] = j == A ? 0.0 : invR[ij];
-        sA[j] = j == A ? 0.0 : aij[ij];
-    }
-    __syncthreads();
-    auto dist = [&](int i, double px, double py, double pz) {
-        const double dx = sx[i] - px, dy = sy[i] - py, dz = sz[i] - pz;
-        return sqrt(dx * dx + dy * dy + dz * dz);
-    };
-    const double ax = sx[A], ay = sy[A], az = sz[A];
-    for (int k = threadIdx.x; k < sh.nAng; k += blockDim.x) {
-        const double *u = rules + 4 * (sh.rule + k);
-        const double px = u[0] * sh.r + ax, py = u[1] * sh.r + ay, pz = u[2] * sh.r + az;
-        const double rA = dist(A, px, py, pz);
-        // P_A in full.
-        double PA = 1.0;
-        for (int j = 0; j < nAtoms; j++) {
-            if (j == A) continue;
-            PA *= becke_factor_of(A > j, rA, dist(j, px, py, pz), sInv[j], sA[j]);
-        }
-        // Products below 2^-64 of max(|P_A|, |P_near|) <= sum_i P_i no longer change the sum beyond rounding.
-        double floor = fabs(PA) * 0x1p-64;
+    for (int k0 = blockIdx.y * kGroups; k0 < sh.nAng; k0 += gridDim.y * kGroups) {
+        const int k = k0 + gi;
+        const bool active = k < sh.nAng;
+        const double *u = rules + 4 * (sh.rule + (active ? k : 0));
+        const double px = u[0] * sh.r + sxyz[3 * A], py = u[1] * sh.r + sxyz[3 * A + 1], pz = u[2] * sh.r + sxyz[3 * A + 2];
         const double wru = sh.wr * u[3];
-        const int o = sh.out + k;
-        cx[o] = px;
-        cy[o] = py;
-        cz[o] = pz;
-        // The atom nearest the point (other than A) gets its full product first: sum_i P_i >= P_A + P_near, so a point
-        // whose weight cannot exceed half the cull tolerance even then is culled without the other products.
-        int near = -1;
-        double dNear = 0.0;
-        for (int j = 0; j < nAtoms; j++) {
-            if (j == A) continue;
-            const double dx = sx[j] - px, dy = sy[j] - py, dz = sz[j] - pz, d2 = dx * dx + dy * dy + dz * dz;
-            if (near < 0 || d2 < dNear) { near = j; dNear = d2; }
+        double r[LA], b[LA];
+        bool done[LA];
+        wave_fence();
+#pragma unroll
+        for (int a = 0; a < LA; a++) {
+            const int i = gl + GS * a;
+            r[a] = 0.0;
+            if (i < nAtoms) {
+                const double dx = sxyz[3 * i] - px, dy = sxyz[3 * i + 1] - py, dz = sxyz[3 * i + 2] - pz;
+                r[a] = sqrt(dx * dx + dy * dy + dz * dz);
+                rL[i] = r[a];
+            }
+            b[a] = 1.0;
+            done[a] = i >= nAtoms;
         }
-        double sum = PA, rn = 0.0;
-        if (near >= 0) {
-            rn = dist(near, px, py, pz);
-            double Pn = becke_factor_of(near > A, rn, rA, sInv[near], sA[near]);
-            for (int j = 0; j < nAtoms; j++) {
-                if (j == near || j == A) continue;
-                const int ij = pair_index(near, j);
-                Pn *= becke_factor_of(near > j, rn, dist(j, px, py, pz), invR[ij], aij[ij]);
+        wave_fence();
+        bool run = active;
+        int c = A;
+        double PA = 0.0, sum = 0.0, most = 0.0;
+        do {
+            const double rc = rL[c];
+            double prod = 1.0;
+#pragma unroll
+            for (int a = 0; a < LA; a++) {
+                const int i = gl + GS * a;
+                if (i >= nAtoms || i == c) continue;
+                const double2 q = pairs[static_cast<size_t>(c) * nAtoms + i];
+                const double mu = (rc - r[a]) * q.x, nu = mu + q.y * (1.0 - mu * mu), S = kBeckeA * becke_poly(nu);
+                prod *= 0.5 - S;
+                b[a] *= fabs(0.5 + S);
             }
-            sum += Pn;
-            floor = fmax(floor, fabs(Pn) * 0x1p-64);
-            if (PA == 0.0 || (sum > 0.0 && fabs(wru) * (fabs(PA) / sum) < 0.5 * kWeightTol)) {
-                cw[o] = 0.0;
-                keep[o] = 0;
-                continue;
+            prod = group_product<GS>(prod);
+            if (run) {
+                if (c == A) PA = prod;
+                sum += prod;
+                most = fmax(most, fabs(prod));
+#pragma unroll
+                for (int a = 0; a < LA; a++) done[a] = done[a] || gl + GS * a == c;
+                // A point whose weight cannot exceed half the cull tolerance with the products so far is culled.
+                run = PA != 0.0 && !(sum > 0.0 && fabs(wru) * (fabs(PA) / sum) < 0.5 * kWeightTol);
             }
+            double top;
+            c = next_atom<LA, GS>(b, done, gl, bit0, top);
+            run = run && top >= kCellScreen * most && top > 0.0;
+        } while (__any(run));
+        if (active && gl == 0) {
+            const int o = sh.out + k;
+            const double w = PA != 0.0 ? wru * (PA / sum) : 0.0;
+            cx[o] = px;
+            cy[o] = py;
+            cz[o] = pz;
+            cw[o] = w;
+            keep[o] = fabs(w) > kWeightTol ? 1 : 0;
         }
-        for (int i = 0; i < nAtoms; i++) {
-            if (i == A || i == near) continue;
-            const double ri = dist(i, px, py, pz);
-            double Pi = becke_factor_of(i > A, ri, rA, sInv[i], sA[i]);
-            if (near >= 0 && fabs(Pi) >= floor) {   // then the atom nearest the point
-                const int in = pair_index(i, near);
-                Pi *= becke_factor_of(i > near, ri, rn, invR[in], aij[in]);
-            }
-            for (int jj = 0; jj < nAtoms && fabs(Pi) >= floor; jj++) {
-                const int j = sOrd[jj];
-                if (j == i || j == A || j == near) continue;
-                const int ij = pair_index(i, j);
-                Pi *= becke_factor_of(i > j, ri, dist(j, px, py, pz), invR[ij], aij[ij]);
-            }
-            if (fabs(Pi) >= floor) sum += Pi;
-        }
-        const double w = wru * (PA / sum);
-        cw[o] = w;
-        keep[o] = fabs(w) > kWeightTol ? 1 : 0;
     }
 }
 
@@ -356,32 +370,34 @@ __global__ void __launch_bounds__(256) scan_apply_kernel(int n, const int *__res
     }
 }
 
-// Becke pair data (DFTGridWeights.c:43-80): 1/R_ij and the size adjustment a_ij for i > j, packed as pair_index.
-void becke_pairs(const xq_grid *g, std::vector<double> &invR, std::vector<double> &aij) {
-    const int nA = g->nAtoms;
-    const size_t nPairs = nA > 1 ? static_cast<size_t>(nA) * (nA - 1) / 2 : 1;
-    invR.assign(nPairs, 0.0);
-    aij.assign(nPairs, 0.0);
-    for (int i = 0, ij = 0; i < nA; i++) {
-        for (int j = 0; j < i; j++, ij++) {
-            double dx = g->xyz[3 * i] - g->xyz[3 * j], dy = g->xyz[3 * i + 1] - g->xyz[3 * j + 1],
-                   dz = g->xyz[3 * i + 2] - g->xyz[3 * j + 2];
-            double chi = bragg_radius(g->Z[i]) / bragg_radius(g->Z[j]);
-            double u = (chi - 1.0) / (chi + 1.0), a = u / (u * u - 1.0);
-            invR[ij] = 1.0 / std::sqrt(dx * dx + dy * dy + dz * dz);
-            aij[ij] = a > 0.5 ? 0.5 : (a < -0.5 ? -0.5 : a);
+// start[a] = kept points before atom a's first candidate (a <= nAtoms).
+__global__ void __launch_bounds__(256) atom_starts_kernel(int nAtoms, int nCand, const int *__restrict__ atomFirst,
+                                                          const int *__restrict__ dst, const int *__restrict__ total,
+                                                          int *__restrict__ start) {
+    const int a = blockIdx.x * 256 + threadIdx.x;
+    if (a <= nAtoms) start[a] = atomFirst[a] < nCand ? dst[atomFirst[a]] : *total;
+}
+
+// Becke pair data (DFTGridWeights.c:43-80): pairs[i][j] = {1 / R_ij, a_ij}, a_ij the size adjustment (a_ji = -a_ij).
+std::vector<double2> becke_pairs(const xq_grid *g) {
+    const size_t nA = static_cast<size_t>(g->nAtoms);
+    std::vector<double2> pairs(nA * nA, make_double2(0.0, 0.0));
+    for (size_t i = 0; i < nA; i++)
+        for (size_t j = 0; j < i; j++) {
+            const double dx = g->xyz[3 * i] - g->xyz[3 * j], dy = g->xyz[3 * i + 1] - g->xyz[3 * j + 1],
+                         dz = g->xyz[3 * i + 2] - g->xyz[3 * j + 2];
+            const double chi = bragg_radius(g->Z[i]) / bragg_radius(g->Z[j]);
+            const double u = (chi - 1.0) / (chi + 1.0), a = u / (u * u - 1.0);
+            const double invR = 1.0 / std::sqrt(dx * dx + dy * dy + dz * dz), adj = a > 0.5 ? 0.5 : (a < -0.5 ? -0.5 : a);
+            pairs[i * nA + j] = make_double2(invR, adj);
+            pairs[j * nA + i] = make_double2(invR, -adj);
         }
-    }
+    return pairs;
 }
 
 // Largest number of atoms per lane of the weight-derivative kernel: 64 x 16 = 1024 atoms (more atoms per lane spill
 // registers).
 constexpr int kMaxLaneAtoms = 16;
-
-// Screen of the weight-derivative terms: atoms whose cell product, and atoms whose factor of the derivative, is below this
-// share of their sum.  A cell factor s(nu) near its zero is s = c y^11 P with y = 1 - nu and a derivative of 11 s / y, so a
-// term that the screen drops is below 1e-16 of the point's energy over a bond length.
-constexpr double kWeightScreen = 0x1p-64;
 
 // The cell function's small side: s = kBeckeA * integral of (1 - x^2)^10 from n to 1 for n = |nu|.  With y = 1 - n that is
 // kBeckeA y^11 sum_j e_j n^j, e_j = binom(10, j) * integral of t^(10 + j) (2 - t)^(10 - j) from 0 to 1: every e_j is
@@ -402,19 +418,6 @@ __device__ __forceinline__ double reciprocal(double x) {
     double r = __builtin_amdgcn_rcp(x);
     r = fma(fma(-x, r, 1.0), r, r);
     return fma(fma(-x, r, 1.0), r, r);
-}
-
-template <int GS>
-__device__ __forceinline__ double group_sum(double x) {
-#pragma unroll
-    for (int o = GS / 2; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
-    return x;
-}
-
-// LDS writes of a wave are in order; this keeps the compiler from moving accesses over it.
-__device__ __forceinline__ void wave_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
 }
 
 // XC gradient weight terms (DFTGridWeights_Derivatives, DFTGridWeights.c:98-215).  A group of GS lanes takes a point (grid
@@ -452,10 +455,7 @@ __global__ void __launch_bounds__(64 * WPG) weight_gradient_kernel(int nPoints,
     double G[LA][3];
 #pragma unroll
     for (int a = 0; a < LA; a++) G[a][0] = G[a][1] = G[a][2] = 0.0;
-    // The group's lanes among the wave's ballot bits.
-    const int bit0 = t & 63 & ~(GS - 1);
-    const unsigned long long ones = GS == 64 ? ~0ull : ((1ull << (GS & 63)) - 1ull);
-    auto ballot = [&](bool x) { return (__ballot(x) >> bit0) & ones; };
+    const int bit0 = t & 63 & ~(GS - 1);   // the group's place in its wave
     // Work-group b takes the rounds b, b + gridDim.x, ... of kGroups consecutive points (a point's cost depends on the atoms
     // whose cells matter there, so contiguous ranges would differ in cost).
     for (int base = blockIdx.x * kGroups; base < nPoints; base += gridDim.x * kGroups) {
@@ -491,10 +491,10 @@ __global__ void __launch_bounds__(64 * WPG) weight_gradient_kernel(int nPoints,
             const int i = gl + GS * a;
             if (i >= nAtoms || i == g) continue;
             const double2 q = pairs[static_cast<size_t>(g) * nAtoms + i];
-            made *= becke_factor_of(g > i, rg, r[a], q.x, g > i ? q.y : -q.y);
+            const double mu = (rg - r[a]) * q.x;
+            made *= 0.5 - kBeckeA * becke_poly(mu + q.y * (1.0 - mu * mu));
         }
-#pragma unroll
-        for (int o = GS / 2; o > 0; o >>= 1) made *= __shfl_xor(made, o, 64);
+        made = group_product<GS>(made);
         // Products.
         bool run = active;
         int c = g;
@@ -512,25 +512,16 @@ __global__ void __launch_bounds__(64 * WPG) weight_gradient_kernel(int nPoints,
                 prod *= nu > 0.0 ? small : large;
                 b[a] *= nu > 0.0 ? large : small;
             }
-#pragma unroll
-            for (int o = GS / 2; o > 0; o >>= 1) prod *= __shfl_xor(prod, o, 64);
+            prod = group_product<GS>(prod);
             if (run) {
                 most = fmax(most, prod);
 #pragma unroll
                 for (int a = 0; a < LA; a++)
                     if (gl + GS * a == c) { A[a] = prod; done[a] = true; }
             }
-            double best = -1.0;
-            int bi = 0;
-#pragma unroll
-            for (int a = 0; a < LA; a++)
-                if (!done[a] && b[a] > best) { best = b[a]; bi = gl + GS * a; }
-            double top = best;
-#pragma unroll
-            for (int o = GS / 2; o > 0; o >>= 1) top = fmax(top, __shfl_xor(top, o, 64));
-            run = run && top >= kWeightScreen * most && top > 0.0;
-            const unsigned long long at = ballot(best == top);
-            c = __shfl(bi, bit0 + __ffsll(static_cast<long long>(at)) - 1, 64);
+            double top;
+            c = next_atom<LA, GS>(b, done, gl, bit0, top);
+            run = run && top >= kCellScreen * most && top > 0.0;
         } while (__any(run));
         // c_m; that of g from the others' share, which keeps its accuracy where g's cell holds almost all.
         double others = 0.0, own = 0.0;
@@ -548,9 +539,9 @@ __global__ void __launch_bounds__(64 * WPG) weight_gradient_kernel(int nPoints,
         for (int a = 0; a < LA; a++) {
             const int i = gl + GS * a;
             cf[a] = i == g ? scale * others : -scale * A[a];
-            if (!(fabs(cf[a]) >= kWeightScreen * fabs(ew)) || !active) cf[a] = 0.0;
+            if (!(fabs(cf[a]) >= kCellScreen * fabs(ew)) || !active) cf[a] = 0.0;
             if (i < nAtoms) cL[i] = cf[a];
-            maskK[a] = ballot(cf[a] != 0.0);
+            maskK[a] = group_ballot<GS>(cf[a] != 0.0, bit0);
             anyK |= maskK[a];
         }
         if (!__any(anyK != 0ull)) continue;
@@ -690,44 +681,28 @@ int build_grid(xq_grid *g) {
         }
     }
     atomFirst[nA] = nCand;
-    // Becke pair data (DFTGridWeights.c:43-80): 1/R_ij and the size adjustment a_ij, for i > j.
-    const size_t nPairs = nA > 1 ? static_cast<size_t>(nA) * (nA - 1) / 2 : 1;
-    std::vector<double> invR, aij;
-    becke_pairs(g, invR, aij);
+    const std::vector<double2> pairs = becke_pairs(g);
     // Device work.
     RadialShell *d_shells = nullptr;
-    double *d_rules = nullptr, *d_xyz = nullptr, *d_invR = nullptr, *d_aij = nullptr;
-    int *d_order = nullptr;
+    double *d_rules = nullptr, *d_xyz = nullptr;
+    double2 *d_pairs = nullptr;
     double *cx = nullptr, *cy = nullptr, *cz = nullptr, *cw = nullptr;
-    int *keep = nullptr, *dst = nullptr, *total = nullptr, *tileSums = nullptr;
-    // LDS of the candidate kernel: atom coordinates, the shell atom's pair row and its distance order (44 bytes per
-    // atom).
-    const size_t lds = (5 * sizeof(double) + sizeof(int)) * static_cast<size_t>(nA);
-    if (lds > 64 * 1024) {
+    int *keep = nullptr, *dst = nullptr, *total = nullptr, *tileSums = nullptr, *d_atomFirst = nullptr, *d_atomStart = nullptr;
+    // Waves per work-group of the candidate kernel: four up to 640 atoms, two above (the coordinates and 8 bytes of LDS per
+    // atom and group: 7 x 8 x 640 and 5 x 8 x 1489 bytes both fit in 64 KB).  Up to 16 atoms four points share a wave, up to
+    // 32 two.
+    const int wpg = nA <= 640 ? 4 : 2, group = nA <= 16 ? 16 : (nA <= 32 ? 32 : 64);
+    const size_t lds = (3 + static_cast<size_t>(64 * wpg / group)) * sizeof(double) * static_cast<size_t>(nA);
+    if (nA > 1489) {
         set_error("grid construction supports at most 1489 atoms");
         return kInvalidArgument;
-    }
-    // Per atom A, all atoms in order of distance from A (A first).
-    std::vector<int> order(static_cast<size_t>(nA) * nA);
-    {
-        std::vector<double> d2(nA);
-        for (int a = 0; a < nA; a++) {
-            int *row = order.data() + static_cast<size_t>(a) * nA;
-            for (int j = 0; j < nA; j++) {
-                const double dx = g->xyz[3 * a] - g->xyz[3 * j], dy = g->xyz[3 * a + 1] - g->xyz[3 * j + 1],
-                             dz = g->xyz[3 * a + 2] - g->xyz[3 * j + 2];
-                d2[j] = dx * dx + dy * dy + dz * dz;
-                row[j] = j;
-            }
-            std::stable_sort(row, row + nA, [&](int p, int q) { return d2[p] < d2[q]; });
-        }
     }
     int status = kOK;
     auto cleanup = [&]() {
         // The kernels that use these arrays must be done before the arrays are reused.
         (void)hipStreamSynchronize(g->stream);
-        dev_free(g, &d_shells); dev_free(g, &d_rules); dev_free(g, &d_xyz); dev_free(g, &d_invR); dev_free(g, &d_aij);
-        dev_free(g, &d_order);
+        dev_free(g, &d_shells); dev_free(g, &d_rules); dev_free(g, &d_xyz); dev_free(g, &d_pairs);
+        dev_free(g, &d_atomFirst); dev_free(g, &d_atomStart);
         dev_free(g, &cx); dev_free(g, &cy); dev_free(g, &cz); dev_free(g, &cw); dev_free(g, &keep); dev_free(g, &dst); dev_free(g, &total);
         dev_free(g, &tileSums);
     };
@@ -735,9 +710,9 @@ int build_grid(xq_grid *g) {
         if ((status = dev_alloc(g, &d_shells, shells.size())) != kOK) break;
         if ((status = dev_alloc(g, &d_rules, rules.size())) != kOK) break;
         if ((status = dev_alloc(g, &d_xyz, g->xyz.size())) != kOK) break;
-        if ((status = dev_alloc(g, &d_invR, nPairs)) != kOK) break;
-        if ((status = dev_alloc(g, &d_aij, nPairs)) != kOK) break;
-        if ((status = dev_alloc(g, &d_order, order.size())) != kOK) break;
+        if ((status = dev_alloc(g, &d_pairs, pairs.size())) != kOK) break;
+        if ((status = dev_alloc(g, &d_atomFirst, atomFirst.size())) != kOK) break;
+        if ((status = dev_alloc(g, &d_atomStart, atomFirst.size())) != kOK) break;
         if ((status = dev_alloc(g, &cx, nCand)) != kOK) break;
         if ((status = dev_alloc(g, &cy, nCand)) != kOK) break;
         if ((status = dev_alloc(g, &cz, nCand)) != kOK) break;
@@ -753,36 +728,48 @@ int build_grid(xq_grid *g) {
                             "copy rules")) != kOK) break;
         if ((status = check(hipMemcpyAsync(d_xyz, g->xyz.data(), g->xyz.size() * sizeof(double), hipMemcpyHostToDevice, s),
                             "copy xyz")) != kOK) break;
-        if ((status = check(hipMemcpyAsync(d_invR, invR.data(), nPairs * sizeof(double), hipMemcpyHostToDevice, s),
-                            "copy invR")) != kOK) break;
-        if ((status = check(hipMemcpyAsync(d_aij, aij.data(), nPairs * sizeof(double), hipMemcpyHostToDevice, s),
-                            "copy aij")) != kOK) break;
-        if ((status = check(hipMemcpyAsync(d_order, order.data(), order.size() * sizeof(int), hipMemcpyHostToDevice, s),
-                            "copy order")) != kOK) break;
+        if ((status = check(hipMemcpyAsync(d_pairs, pairs.data(), pairs.size() * sizeof(double2), hipMemcpyHostToDevice, s),
+                            "copy pairs")) != kOK) break;
+        if ((status = check(hipMemcpyAsync(d_atomFirst, atomFirst.data(), atomFirst.size() * sizeof(int),
+                                           hipMemcpyHostToDevice, s), "copy atoms")) != kOK) break;
         if (!shells.empty()) {
-            hipLaunchKernelGGL(candidate_points_kernel, dim3(shells.size()), dim3(256), lds, s, d_shells, d_rules, d_xyz, nA,
-                               d_invR, d_aij, d_order, cx, cy, cz, cw, keep);
+            // A shell's points go to enough work-groups to fill the chip (8 x 256 of them), at most one round each.
+            const unsigned rounds = static_cast<unsigned>((lebedev_size_for_l(65) * group + 64 * wpg - 1) / (64 * wpg));
+            const unsigned split = std::min<unsigned>(rounds, static_cast<unsigned>(2048 / shells.size()) + 1);
+            auto launch = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(shells.size()), split), dim3(64 * wpg), lds, s,
+                                   d_shells, d_rules, d_xyz, nA, d_pairs, cx, cy, cz, cw, keep);
+            };
+            // Atoms per lane: the smallest instance that covers nAtoms.
+            if (nA <= 16) launch(candidate_points_kernel<1, 16, 4>);
+            else if (nA <= 32) launch(candidate_points_kernel<1, 32, 4>);
+            else if (nA <= 64) launch(candidate_points_kernel<1, 64, 4>);
+            else if (nA <= 128) launch(candidate_points_kernel<2, 64, 4>);
+            else if (nA <= 192) launch(candidate_points_kernel<3, 64, 4>);
+            else if (nA <= 256) launch(candidate_points_kernel<4, 64, 4>);
+            else if (nA <= 384) launch(candidate_points_kernel<6, 64, 4>);
+            else if (nA <= 640) launch(candidate_points_kernel<10, 64, 4>);
+            else if (nA <= 1024) launch(candidate_points_kernel<16, 64, 2>);
+            else launch(candidate_points_kernel<24, 64, 2>);
             if ((status = check(hipGetLastError(), "candidate_points_kernel")) != kOK) break;
             const int nTiles = (nCand + kScanTile - 1) / kScanTile;
             hipLaunchKernelGGL(scan_tile_sums_kernel, dim3(nTiles), dim3(256), 0, s, nCand, keep, tileSums);
             hipLaunchKernelGGL(scan_sums_kernel, dim3(1), dim3(256), 0, s, nTiles, tileSums, total);
             hipLaunchKernelGGL(scan_apply_kernel, dim3(nTiles), dim3(256), 0, s, nCand, keep, tileSums, dst);
+            // Each atom's first kept point: the scan at the atom boundaries (the end's is the total).
+            hipLaunchKernelGGL(atom_starts_kernel, dim3((nA + 256) / 256), dim3(256), 0, s, nA, nCand, d_atomFirst, dst, total,
+                               d_atomStart);
             if ((status = check(hipGetLastError(), "scan kernels")) != kOK) break;
         }
-        // Per-atom kept counts from the scan at the atom boundaries.
-        std::vector<int> scanned(nCand > 0 ? nCand : 1, 0), kept(nCand > 0 ? nCand : 1, 0);
-        int nKept = 0;
+        std::vector<int> atomStart(static_cast<size_t>(nA) + 1, 0);
         if (nCand > 0) {
             // Wait for the kernels first: a pageable copy that waits for its stream holds the runtime's staging path.
             if ((status = check(hipStreamSynchronize(s), "grid sync")) != kOK) break;
-            if ((status = check(hipMemcpyAsync(scanned.data(), dst, nCand * sizeof(int), hipMemcpyDeviceToHost, s),
-                                "copy scan")) != kOK) break;
-            if ((status = check(hipMemcpyAsync(kept.data(), keep, nCand * sizeof(int), hipMemcpyDeviceToHost, s),
-                                "copy keep")) != kOK) break;
-            if ((status = check(hipMemcpyAsync(&nKept, total, sizeof(int), hipMemcpyDeviceToHost, s), "copy total")) != kOK)
-                break;
+            if ((status = check(hipMemcpyAsync(atomStart.data(), d_atomStart, atomStart.size() * sizeof(int),
+                                               hipMemcpyDeviceToHost, s), "copy scan")) != kOK) break;
             if ((status = check(hipStreamSynchronize(s), "grid sync")) != kOK) break;
         }
+        const int nKept = atomStart[nA];
         g->nPoints = nKept;
         if ((status = dev_alloc(g, &g->d_x, nKept)) != kOK) break;
         if ((status = dev_alloc(g, &g->d_y, nKept)) != kOK) break;
@@ -796,10 +783,7 @@ int build_grid(xq_grid *g) {
         // Blocks of at most kBlockSize consecutive points per atom.
         g->blocks.clear();
         for (int a = 0; a < nA; a++) {
-            const int c0 = atomFirst[a], c1 = atomFirst[a + 1];
-            if (c1 <= c0) continue;
-            const int p0 = scanned[c0];
-            const int p1 = scanned[c1 - 1] + kept[c1 - 1];
+            const int p0 = atomStart[a], p1 = atomStart[a + 1];
             for (int p = p0; p < p1; p += kBlockSize) {
                 DevBlock b;
                 b.atom = a;
@@ -861,15 +845,7 @@ int weight_gradients(xq_grid *g, const double *d_eXC, double *d_grad, hipStream_
         set_error("XC gradients support at most " + std::to_string(64 * kMaxLaneAtoms) + " atoms");
         return kInvalidArgument;
     }
-    std::vector<double> invR, aij;
-    becke_pairs(g, invR, aij);
-    // Square pair table, [m][k] = {1 / R_mk, a_mk}.
-    std::vector<double2> pairs(static_cast<size_t>(nA) * nA, make_double2(0.0, 0.0));
-    for (int i = 0, ij = 0; i < nA; i++)
-        for (int j = 0; j < i; j++, ij++) {
-            pairs[static_cast<size_t>(i) * nA + j] = make_double2(invR[ij], aij[ij]);
-            pairs[static_cast<size_t>(j) * nA + i] = make_double2(invR[ij], -aij[ij]);
-        }
+    const std::vector<double2> pairs = becke_pairs(g);
     std::vector<int> pointAtom(static_cast<size_t>(G), 0);
     for (const DevBlock &b : g->blocks)
         for (int k = 0; k < b.nPoints; k++) pointAtom[static_cast<size_t>(b.pStart) + k] = b.atom;
