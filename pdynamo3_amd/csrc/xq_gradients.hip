@@ -35,8 +35,7 @@ namespace {
 // larger batches than 131,072 rows took 3.6 ms off an (H2O)64 gradient call: fewer launches, each with its own tail.
 constexpr long long kBatchRows = 524288;
 constexpr int kC = 32;                           // rows per chunk (two 16-row MFMA tiles)
-constexpr int kPanelF = 4;                       // chunks of P_red columns staged in LDS at once
-constexpr int kPanelPitch = kPanelF * kC + 2;    // LDS row pitch in doubles (padded against bank conflicts)
+constexpr int kRowPitch = kC + 4;                // LDS row pitch of a staged P_red chunk in doubles (padded against bank conflicts)
 constexpr int kIdxCache = 1024;                  // kept-function indices cached in LDS
 constexpr int kGradCopies = 64;                  // copies of the gradient array that spread the atomics
 
@@ -46,70 +45,60 @@ __device__ __forceinline__ v4d mfma_f64(double a, double b, const v4d &c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
-// P_red Bp for one block on FP64 MFMA (v_mfma_f64_16x16x4f64: lane l supplies A[l % 16][l / 16] and B[l / 16][l % 16]
-// and receives D[4 v + l / 16][l % 16]).  256 threads; wave wv owns points 32 wv .. + 31 (two 16-point tiles); for each
-// chunk I of 32 rows, epi(I, acc) receives acc[hm][hn][v] = (P_red Bp)[32 I + 16 hm + 4 v + l / 16][32 wv + 16 hn + l % 16].
-// P_red is staged in LDS by panels of kPanelF chunks of columns; Bp is the block's first row of a plane of rows of 128
-// points (rows >= nb are not read).  Row chunks I0 .. I1 - 1.
-template <typename Epi>
+// P_red Bp for row chunk I of one block on FP64 MFMA (v_mfma_f64_16x16x4f64: lane l supplies A[l % 16][l / 16] and
+// B[l / 16][l % 16] and receives D[4 v + l / 16][l % 16]).  256 threads; wave wv owns points 32 wv .. + 31 (two 16-point
+// tiles): acc[hm][hn][v] = (P_red Bp)[32 I + 16 hm + 4 v + l / 16][32 wv + 16 hn + l % 16].  Bp is the block's first row of
+// a plane of rows of 128 points (rows >= nb are not read).  Each step multiplies one 32 x 32 chunk of P_red, gathered by
+// all threads and staged in one of two LDS buffers (one barrier per step), with 32 rows of Bp; both are fetched one step
+// ahead.  Staged panels of four chunks, each waited for, took 7.2 ms (X pass) and 9.3 ms (Z pass) per call on
+// (H2O)64; this takes 4.1 and 6.1 ms.
 __device__ __forceinline__ void reduced_product(const double *__restrict__ P, int n, const int *idx, int nb,
-                                                const double *__restrict__ Bp, double (&sPf)[kC][kPanelPitch], int I0,
-                                                int I1, Epi epi) {
+                                                const double *__restrict__ Bp, double (&sP)[2][kC][kRowPitch], int I,
+                                                v4d (&acc)[2][2]) {
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6, l16 = lane & 15, l4 = lane >> 4;
     const int nChunks = (nb + kC - 1) / kC;
-    const int sr = t >> 3, s8 = t & 7;     // staging: row sr, columns 4 s8 .. + 3 of each chunk of the panel
-    auto fetchB = [&](int c, double (&bq)[8][2]) {
+    // Staging: row sr, columns 8 j + s8 (eight lanes read eight consecutive kept functions).
+    const int sr = t >> 3, s8 = t & 7, r = kC * I + sr;
+    const size_t rowOff = r < nb ? static_cast<size_t>(idx[r]) * n : 0;
+    double pv[4], bnext[8][2];
+    auto fetch = [&](int c) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int k = kC * c + 8 * j + s8;
+            pv[j] = r < nb && k < nb ? P[rowOff + idx[k]] : 0.0;
+        }
 #pragma unroll
         for (int s = 0; s < 8; s++) {
             const int k = kC * c + 4 * s + l4;
 #pragma unroll
             for (int h = 0; h < 2; h++)
-                bq[s][h] = k < nb ? Bp[static_cast<size_t>(k) * kBlockSize + kC * wv + 16 * h + l16] : 0.0;
+                bnext[s][h] = k < nb ? Bp[static_cast<size_t>(k) * kBlockSize + kC * wv + 16 * h + l16] : 0.0;
         }
     };
-    for (int I = I0; I < I1; I++) {
-        v4d acc[2][2];
 #pragma unroll
-        for (int hm = 0; hm < 2; hm++)
+    for (int hm = 0; hm < 2; hm++)
 #pragma unroll
-            for (int hn = 0; hn < 2; hn++) acc[hm][hn] = v4d{0.0, 0.0, 0.0, 0.0};
-        double bnext[8][2];
-        fetchB(0, bnext);
-        const int r = kC * I + sr;
-        const size_t rowOff = r < nb ? static_cast<size_t>(idx[r]) * n : 0;
-        for (int c0 = 0; c0 < nChunks; c0 += kPanelF) {
-            const int nc = nChunks - c0 < kPanelF ? nChunks - c0 : kPanelF;
-            double pv[kPanelF][4];
+        for (int hn = 0; hn < 2; hn++) acc[hm][hn] = v4d{0.0, 0.0, 0.0, 0.0};
+    fetch(0);
+#pragma unroll 2
+    for (int c = 0; c < nChunks; c++) {
+        double (&buf)[kC][kRowPitch] = sP[c & 1];
 #pragma unroll
-            for (int m = 0; m < kPanelF; m++)
+        for (int j = 0; j < 4; j++) buf[sr][8 * j + s8] = pv[j];
+        double bq[8][2];
 #pragma unroll
-                for (int jj = 0; jj < 4; jj++) {
-                    const int k = kC * (c0 + m) + 4 * s8 + jj;
-                    pv[m][jj] = (m < nc && r < nb && k < nb) ? P[rowOff + idx[k]] : 0.0;
-                }
-            __syncthreads();   // every wave is done with the previous panel
+        for (int s = 0; s < 8; s++) { bq[s][0] = bnext[s][0]; bq[s][1] = bnext[s][1]; }
+        // A wave writes this buffer again two steps on, after the next barrier, which every wave reaches done with it.
+        __syncthreads();
+        if (c + 1 < nChunks) fetch(c + 1);
 #pragma unroll
-            for (int m = 0; m < kPanelF; m++)
-#pragma unroll
-                for (int jj = 0; jj < 4; jj++) sPf[sr][kC * m + 4 * s8 + jj] = pv[m][jj];
-            __syncthreads();
-            for (int cl = 0; cl < nc; cl++) {
-                const int c = c0 + cl;
-                double bq[8][2];
-#pragma unroll
-                for (int s = 0; s < 8; s++) { bq[s][0] = bnext[s][0]; bq[s][1] = bnext[s][1]; }
-                if (c + 1 < nChunks) fetchB(c + 1, bnext);
-#pragma unroll
-                for (int s = 0; s < 8; s++) {
-                    const double a0 = sPf[l16][kC * cl + 4 * s + l4], a1 = sPf[16 + l16][kC * cl + 4 * s + l4];
-                    acc[0][0] = mfma_f64(a0, bq[s][0], acc[0][0]);
-                    acc[0][1] = mfma_f64(a0, bq[s][1], acc[0][1]);
-                    acc[1][0] = mfma_f64(a1, bq[s][0], acc[1][0]);
-                    acc[1][1] = mfma_f64(a1, bq[s][1], acc[1][1]);
-                }
-            }
+        for (int s = 0; s < 8; s++) {
+            const double a0 = buf[l16][4 * s + l4], a1 = buf[16 + l16][4 * s + l4];
+            acc[0][0] = mfma_f64(a0, bq[s][0], acc[0][0]);
+            acc[0][1] = mfma_f64(a0, bq[s][1], acc[0][1]);
+            acc[1][0] = mfma_f64(a1, bq[s][0], acc[1][0]);
+            acc[1][1] = mfma_f64(a1, bq[s][1], acc[1][1]);
         }
-        epi(I, acc);
     }
 }
 
@@ -132,7 +121,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) g
     const int4 *__restrict__ items, XcdRanges xr, long long rowBase, const DevBlock *__restrict__ blocks,
     const int *__restrict__ idxAll, int n, const double *__restrict__ P0, const double *__restrict__ P1, Planes10 B,
     double *__restrict__ Xp0, double *__restrict__ Xp1, double *__restrict__ part, int nSpins) {
-    __shared__ double sPf[kC][kPanelPitch];
+    __shared__ double sP[2][kC][kRowPitch];
     __shared__ int sIdx[kIdxCache];
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
     if (slot >= xr.start[xcd + 1] - xr.start[xcd]) return;
@@ -151,26 +140,26 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) g
     {
         double *X = (sp == 0 ? Xp0 : Xp1) + R0;
         double pr[2] = {0.0, 0.0}, pgx[2] = {0.0, 0.0}, pgy[2] = {0.0, 0.0}, pgz[2] = {0.0, 0.0};
-        reduced_product(sp == 0 ? P0 : P1, n, idx, nb, F, sPf, I, I + 1, [&](int, v4d (&acc)[2][2]) {
+        v4d acc[2][2];
+        reduced_product(sp == 0 ? P0 : P1, n, idx, nb, F, sP, I, acc);
 #pragma unroll
-            for (int hm = 0; hm < 2; hm++)
+        for (int hm = 0; hm < 2; hm++)
 #pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    const int i = kC * I + 16 * hm + 4 * v + l4;
-                    if (i < nb) {
+            for (int v = 0; v < 4; v++) {
+                const int i = kC * I + 16 * hm + 4 * v + l4;
+                if (i < nb) {
 #pragma unroll
-                        for (int hn = 0; hn < 2; hn++) {
-                            const size_t o = static_cast<size_t>(i) * kBlockSize + kC * wv + 16 * hn + l16;
-                            const double x = acc[hm][hn][v];
-                            X[o] = x;
-                            pr[hn] += F[o] * x;
-                            pgx[hn] += Fx[o] * x;
-                            pgy[hn] += Fy[o] * x;
-                            pgz[hn] += Fz[o] * x;
-                        }
+                    for (int hn = 0; hn < 2; hn++) {
+                        const size_t o = static_cast<size_t>(i) * kBlockSize + kC * wv + 16 * hn + l16;
+                        const double x = acc[hm][hn][v];
+                        X[o] = x;
+                        pr[hn] += F[o] * x;
+                        pgx[hn] += Fx[o] * x;
+                        pgy[hn] += Fy[o] * x;
+                        pgz[hn] += Fz[o] * x;
                     }
                 }
-        });
+            }
         double *q = part + (static_cast<size_t>(it.z) * nSpins + sp) * 4 * kBlockSize;
 #pragma unroll
         for (int hn = 0; hn < 2; hn++) {
@@ -305,7 +294,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) g
     const double *__restrict__ P1, Planes10 B, const double *__restrict__ Xp0, const double *__restrict__ Xp1,
     const double *__restrict__ Up0, const double *__restrict__ Up1, const double *__restrict__ coef,
     const int *__restrict__ skip, double *__restrict__ gradCopies, int nAtoms, int nSpins) {
-    __shared__ double sPf[kC][kPanelPitch];
+    __shared__ double sP[2][kC][kRowPitch];
     __shared__ int sIdx[kIdxCache];
     __shared__ double sCoef[3][kBlockSize];
     __shared__ double sRed[4][kC][3];
@@ -336,56 +325,56 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) g
     {
         const double *X = (sp == 0 ? Xp0 : Xp1) + R0;
         const double *sA = sCoef[0], *sB = sCoef[1], *sC = sCoef[2];
-        reduced_product(sp == 0 ? P0 : P1, n, idx, nb, (sp == 0 ? Up0 : Up1) + R0, sPf, I, I + 1, [&](int, v4d (&acc)[2][2]) {
-            double c[2][4][3];
+        v4d acc[2][2];
+        reduced_product(sp == 0 ? P0 : P1, n, idx, nb, (sp == 0 ? Up0 : Up1) + R0, sP, I, acc);
+        double c[2][4][3];
 #pragma unroll
-            for (int hm = 0; hm < 2; hm++)
+        for (int hm = 0; hm < 2; hm++)
 #pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    c[hm][v][0] = c[hm][v][1] = c[hm][v][2] = 0.0;
-                    const int i = kC * I + 16 * hm + 4 * v + l4;
-                    if (i < nb) {
+            for (int v = 0; v < 4; v++) {
+                c[hm][v][0] = c[hm][v][1] = c[hm][v][2] = 0.0;
+                const int i = kC * I + 16 * hm + 4 * v + l4;
+                if (i < nb) {
 #pragma unroll
-                        for (int hn = 0; hn < 2; hn++) {
-                            const int p = kC * wv + 16 * hn + l16;
-                            if (p < np) {
-                                const size_t o = static_cast<size_t>(i) * kBlockSize + p;
-                                const double z = acc[hm][hn][v], x = X[o];
-                                const double ax = sA[p], ay = sB[p], az = sC[p];
-                                const double hxy = Hxy[o], hxz = Hxz[o], hyz = Hyz[o];
-                                c[hm][v][0] += z * Fx[o] + x * (Hxx[o] * ax + hxy * ay + hxz * az);
-                                c[hm][v][1] += z * Fy[o] + x * (hxy * ax + Hyy[o] * ay + hyz * az);
-                                c[hm][v][2] += z * Fz[o] + x * (hxz * ax + hyz * ay + Hzz[o] * az);
-                            }
+                    for (int hn = 0; hn < 2; hn++) {
+                        const int p = kC * wv + 16 * hn + l16;
+                        if (p < np) {
+                            const size_t o = static_cast<size_t>(i) * kBlockSize + p;
+                            const double z = acc[hm][hn][v], x = X[o];
+                            const double ax = sA[p], ay = sB[p], az = sC[p];
+                            const double hxy = Hxy[o], hxz = Hxz[o], hyz = Hyz[o];
+                            c[hm][v][0] += z * Fx[o] + x * (Hxx[o] * ax + hxy * ay + hxz * az);
+                            c[hm][v][1] += z * Fy[o] + x * (hxy * ax + Hyy[o] * ay + hyz * az);
+                            c[hm][v][2] += z * Fz[o] + x * (hxz * ax + hyz * ay + Hzz[o] * az);
                         }
                     }
                 }
-            // Sum over the 16 points of each lane group, then over the four waves.
+            }
+        // Sum over the 16 points of each lane group, then over the four waves.
 #pragma unroll
-            for (int hm = 0; hm < 2; hm++)
+        for (int hm = 0; hm < 2; hm++)
 #pragma unroll
-                for (int v = 0; v < 4; v++)
+            for (int v = 0; v < 4; v++)
 #pragma unroll
-                    for (int d = 0; d < 3; d++) {
-                        double e = c[hm][v][d];
+                for (int d = 0; d < 3; d++) {
+                    double e = c[hm][v][d];
 #pragma unroll
-                        for (int o = 1; o < 16; o <<= 1) e += __shfl_xor(e, o, 64);
-                        if (l16 == 0) sRed[wv][16 * hm + 4 * v + l4][d] = e;
-                    }
-            __syncthreads();
-            if (t < kC) {
-                const int i = kC * I + t;
-                if (i < nb) {
-                    const int atom = atomOf[idxG[i]];
+                    for (int o = 1; o < 16; o <<= 1) e += __shfl_xor(e, o, 64);
+                    if (l16 == 0) sRed[wv][16 * hm + 4 * v + l4][d] = e;
+                }
+        __syncthreads();
+        if (t < kC) {
+            const int i = kC * I + t;
+            if (i < nb) {
+                const int atom = atomOf[idxG[i]];
 #pragma unroll
-                    for (int d = 0; d < 3; d++) {
-                        const double gi = ((sRed[0][t][d] + sRed[1][t][d]) + sRed[2][t][d]) + sRed[3][t][d];
-                        atomicAdd(&grad[3 * atom + d], -gi);
-                        gs[d] += gi;
-                    }
+                for (int d = 0; d < 3; d++) {
+                    const double gi = ((sRed[0][t][d] + sRed[1][t][d]) + sRed[2][t][d]) + sRed[3][t][d];
+                    atomicAdd(&grad[3 * atom + d], -gi);
+                    gs[d] += gi;
                 }
             }
-        });
+        }
     }
     // The grid moves with the block's atom (UGradientContributions :909-941): it receives the sum of the row terms.
     if (wv == 0) {
