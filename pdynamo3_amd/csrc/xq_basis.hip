@@ -14,6 +14,7 @@
 // The kept sets are exactly the reference's: screening removes only functions whose bound is below the tolerance.
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 #include <hip/hip_runtime.h>
 
 #include "xq_internal.h"
@@ -56,6 +57,24 @@ struct ShellDims {
     static constexpr int nCBF = cart_offset(LH + 1) - cart_offset(LL);
     static constexpr int nSph = (LH + 1) * (LH + 1) - LL * LL;
 };
+
+// f(lLow, lHigh, spherical) as compile-time constants for the shell's type.
+template <typename F>
+__device__ __forceinline__ void for_shell_type(const xq::DevShell &sh, bool sph, F f) {
+    using std::integral_constant;
+    auto type = [&](auto ll, auto lh) {
+        if (sph) f(ll, lh, std::true_type{});
+        else f(ll, lh, std::false_type{});
+    };
+    switch (sh.lLow * 4 + sh.lHigh) {
+        case 0: type(integral_constant<int, 0>{}, integral_constant<int, 0>{}); break;
+        case 5: type(integral_constant<int, 1>{}, integral_constant<int, 1>{}); break;
+        case 1: type(integral_constant<int, 0>{}, integral_constant<int, 1>{}); break;
+        case 10: type(integral_constant<int, 2>{}, integral_constant<int, 2>{}); break;
+        case 15: type(integral_constant<int, 3>{}, integral_constant<int, 3>{}); break;
+        default: break;
+    }
+}
 
 template <int LL, int LH, bool SPH, bool GRAD>
 __device__ __forceinline__ void shell_eval(const xq::DevShell &sh, const double *__restrict__ coef,
@@ -120,31 +139,18 @@ __device__ __forceinline__ void shell_eval(const xq::DevShell &sh, const double 
     }
 }
 
-// Dispatch on the shell type; calls body(nBasis, v, vx, vy, vz).  Supported: S, P, D, F, SP.
+// Dispatch on the shell type; calls body(N, v, vx, vy, vz), N the shell's functions as a compile-time constant (so that the
+// arrays stay in registers).  Supported: S, P, D, F, SP.
 template <bool GRAD, typename Body>
 __device__ __forceinline__ void with_shell(const xq::DevShell &sh, bool sph, const double *coef, const double *trans,
                                            double dx, double dy, double dz, Body body) {
-    double v[16], vx[16], vy[16], vz[16];
-    const int key = sh.lLow * 4 + sh.lHigh;
-    if (sph) {
-        switch (key) {
-            case 0: shell_eval<0, 0, true, GRAD>(sh, coef, trans, dx, dy, dz, v, vx, vy, vz); body(1, v, vx, vy, vz); break;
-            case 5: shell_eval<1, 1, true, GRAD>(sh, coef, trans, dx, dy, dz, v, vx, vy, vz); body(3, v, vx, vy, vz); break;
-            case 1: shell_eval<0, 1, true, GRAD>(sh, coef, trans, dx, dy, dz, v, vx, vy, vz); body(4, v, vx, vy, vz); break;
-            case 10: shell_eval<2, 2, true, GRAD>(sh, coef, trans, dx, dy, dz, v, vx, vy, vz); body(5, v, vx, vy, vz); break;
-            case 15: shell_eval<3, 3, true, GRAD>(sh, coef, trans, dx, dy, dz, v, vx, vy, vz); body(7, v, vx, vy, vz); break;
-            default: break;
-        }
-    } else {
-        switch (key) {
-            case 0: shell_eval<0, 0, false, GRAD>(sh, coef, trans, dx, dy, dz, v, vx, vy, vz); body(1, v, vx, vy, vz); break;
-            case 5: shell_eval<1, 1, false, GRAD>(sh, coef, trans, dx, dy, dz, v, vx, vy, vz); body(3, v, vx, vy, vz); break;
-            case 1: shell_eval<0, 1, false, GRAD>(sh, coef, trans, dx, dy, dz, v, vx, vy, vz); body(4, v, vx, vy, vz); break;
-            case 10: shell_eval<2, 2, false, GRAD>(sh, coef, trans, dx, dy, dz, v, vx, vy, vz); body(6, v, vx, vy, vz); break;
-            case 15: shell_eval<3, 3, false, GRAD>(sh, coef, trans, dx, dy, dz, v, vx, vy, vz); body(10, v, vx, vy, vz); break;
-            default: break;
-        }
-    }
+    auto shell = [&](auto ll, auto lh, auto s) {
+        constexpr int N = s ? ShellDims<ll, lh>::nSph : ShellDims<ll, lh>::nCBF;
+        double v[N], vx[N], vy[N], vz[N];
+        shell_eval<ll, lh, s, GRAD>(sh, coef, trans, dx, dy, dz, v, vx, vy, vz);
+        body(std::integral_constant<int, N>{}, v, vx, vy, vz);
+    };
+    for_shell_type(sh, sph, shell);
 }
 
 __device__ __forceinline__ double wave_max(double v) {
@@ -168,15 +174,19 @@ __device__ __forceinline__ double radial_bound(int L, double a, double d) {
 }
 
 // Work-group of kBlockSize threads, one thread per point.  Writes the kept functions of block b to tmpIdx[b * nF ...] and
-// their count to counts[b].
+// their count to counts[b].  mask (dynamic LDS, two shells a word): per shell, bit 15 if its bound reaches bfTol on the
+// block's sphere, bits 0 .. 9 its functions that pass bfTol at some point.  Each wave evaluates the candidate shells at its
+// 64 points and marks the functions that pass there (one ballot each), and the marked functions are written in order after
+// one barrier; a maximum over the work-group with two barriers per function took 0.61 ms on (H2O)24, this
+// takes 0.30 ms.
 __global__ void __launch_bounds__(kBlockSize) basis_count_kernel(
     int nBlocks, const xq::DevBlock *__restrict__ blocks, const double *__restrict__ px, const double *__restrict__ py,
     const double *__restrict__ pz, int nShells, const xq::DevShell *__restrict__ shells, const double *__restrict__ coef,
     const double *__restrict__ trans, int spherical, int nF, double bfTol, int *__restrict__ tmpIdx,
     int *__restrict__ counts) {
-    __shared__ unsigned char cand[kMaxShellsLDS];
+    extern __shared__ unsigned mask[];
     __shared__ double red[4][2];
-    __shared__ int nKeptS;
+    __shared__ int waveKept[2];
     const int b = blockIdx.x;
     const xq::DevBlock blk = blocks[b];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
@@ -186,6 +196,7 @@ __global__ void __launch_bounds__(kBlockSize) basis_count_kernel(
     // Bounding sphere: centroid and largest distance.
     double sx = wave_sum(x), sy = wave_sum(y), sz = wave_sum(z);
     if (lane == 0) { red[wave][0] = sx; red[wave][1] = sy; red[wave + 2][0] = sz; }
+    for (int w = t; w < (nShells + 1) / 2; w += kBlockSize) mask[w] = 0u;
     __syncthreads();
     const double inv = 1.0 / blk.nPoints;
     const double cx = (red[0][0] + red[1][0]) * inv, cy = (red[0][1] + red[1][1]) * inv, cz = (red[2][0] + red[3][0]) * inv;
@@ -196,7 +207,7 @@ __global__ void __launch_bounds__(kBlockSize) basis_count_kernel(
     __syncthreads();
     const double radius = fmax(red[0][0], red[1][0]);
     // Candidate shells.
-    for (int s = t; s < nShells; s += blockDim.x) {
+    for (int s = t; s < nShells; s += kBlockSize) {
         const xq::DevShell &sh = shells[s];
         const double dd = sqrt((sh.x - cx) * (sh.x - cx) + (sh.y - cy) * (sh.y - cy) + (sh.z - cz) * (sh.z - cz)) - radius;
         const double d = dd > 0.0 ? dd : 0.0;
@@ -204,37 +215,52 @@ __global__ void __launch_bounds__(kBlockSize) basis_count_kernel(
         const double *ex = coef + sh.coef;
         for (int q = 0; q < sh.nPrim; q++)
             for (int L = sh.lLow; L <= sh.lHigh; L++) bound += sh.bound[q] * radial_bound(L, ex[q], d);
-        cand[s] = bound * (1.0 + 1.0e-12) > bfTol ? 1 : 0;
+        if (bound * (1.0 + 1.0e-12) > bfTol) atomicOr(&mask[s >> 1], 0x8000u << (16 * (s & 1)));
     }
-    if (t == 0) nKeptS = 0;
     __syncthreads();
-    int *out = tmpIdx + static_cast<size_t>(b) * nF;
-    for (int s = 0; s < nShells; s++) {
-        if (!cand[s]) continue;
-        const xq::DevShell sh = shells[s];
-        with_shell<false>(sh, spherical != 0, coef, trans, x - sh.x, y - sh.y, z - sh.z,
-                          [&](int nB, const double *v, const double *, const double *, const double *) {
-                              for (int k = 0; k < nB; k++) {
-                                  double m = wave_max(valid ? fabs(v[k]) : 0.0);
-                                  if (lane == 0) red[wave][0] = m;
-                                  __syncthreads();
-                                  if (t == 0 && fmax(red[0][0], red[1][0]) > bfTol) out[nKeptS++] = sh.fStart + k;
-                                  __syncthreads();
-                              }
-                          });
+    auto bits = [&](int s) { return s < nShells ? (mask[s >> 1] >> (16 * (s & 1))) & 0xffffu : 0u; };
+    for (int s0 = 0; s0 < nShells; s0 += 64)
+        for (unsigned long long cand = __ballot((bits(s0 + lane) & 0x8000u) != 0u); cand != 0ull; cand &= cand - 1ull) {
+            const int s = s0 + __ffsll(static_cast<long long>(cand)) - 1;
+            const xq::DevShell &sh = shells[s];
+            with_shell<false>(sh, spherical != 0, coef, trans, x - sh.x, y - sh.y, z - sh.z,
+                              [&](auto n, const double *v, const double *, const double *, const double *) {
+                                  unsigned pass = 0u;
+#pragma unroll
+                                  for (int k = 0; k < n; k++)
+                                      if (__ballot(valid && fabs(v[k]) > bfTol) != 0ull) pass |= 1u << k;
+                                  if (lane == 0 && pass != 0u) atomicOr(&mask[s >> 1], pass << (16 * (s & 1)));
+                              });
+        }
+    __syncthreads();
+    // Thread t lists the functions of the shells t * per .. + per - 1.
+    const int per = (nShells + kBlockSize - 1) / kBlockSize, s1 = t * per;
+    int kept = 0;
+    for (int s = s1; s < s1 + per; s++) kept += __popc(bits(s) & 0x7fffu);
+    int before = kept;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int u = __shfl_up(before, o, 64);
+        if (lane >= o) before += u;
     }
-    if (t == 0) counts[b] = nKeptS;
+    if (lane == 63) waveKept[wave] = before;
+    __syncthreads();
+    int o = before - kept + (wave == 1 ? waveKept[0] : 0);
+    int *out = tmpIdx + static_cast<size_t>(b) * nF;
+    for (int s = s1; s < s1 + per; s++)
+        for (unsigned m = bits(s) & 0x7fffu; m != 0u; m &= m - 1u) out[o++] = shells[s].fStart + __ffs(static_cast<int>(m)) - 1;
+    if (t == 0) counts[b] = waveKept[0] + waveKept[1];
 }
 
 // Values and gradients of the kept functions of block b into rows [vOffset, vOffset + nKept) of f, fx, fy, fz (row stride
-// kBlockSize; entries past the block's points are zero).  T is the storage type.
-template <typename T>
+// kBlockSize; entries past the block's points are zero).  EB, EG (mixed precision, else null): per point, the powers of two
+// above max |phi| and above max |d phi / dx_c| over the block's kept functions.
 __global__ void __launch_bounds__(kBlockSize) basis_eval_kernel(
     const xq::DevBlock *__restrict__ blocks, const double *__restrict__ px, const double *__restrict__ py,
     const double *__restrict__ pz, const xq::DevShell *__restrict__ shells, const int *__restrict__ shellOf,
     const double *__restrict__ coef, const double *__restrict__ trans, int spherical, int nF,
-    const int *__restrict__ tmpIdx, int *__restrict__ idx, T *__restrict__ f, T *__restrict__ fx, T *__restrict__ fy,
-    T *__restrict__ fz) {
+    const int *__restrict__ tmpIdx, int *__restrict__ idx, double *__restrict__ f, double *__restrict__ fx,
+    double *__restrict__ fy, double *__restrict__ fz, signed char *__restrict__ EB, signed char *__restrict__ EG) {
     const int b = blockIdx.x;
     const xq::DevBlock blk = blocks[b];
     const int t = threadIdx.x;
@@ -243,22 +269,34 @@ __global__ void __launch_bounds__(kBlockSize) basis_eval_kernel(
                  z = valid ? pz[blk.pStart + t] : 0.0;
     const int *kept = tmpIdx + static_cast<size_t>(b) * nF;
     for (int k = t; k < blk.nKept; k += blockDim.x) idx[blk.iOffset + k] = kept[k];
+    double m[4] = {0.0, 0.0, 0.0, 0.0};
     int k = 0;
     while (k < blk.nKept) {
-        const xq::DevShell sh = shells[shellOf[kept[k]]];
+        const xq::DevShell &sh = shells[shellOf[kept[k]]];
         with_shell<true>(sh, spherical != 0, coef, trans, x - sh.x, y - sh.y, z - sh.z,
-                         [&](int nB, const double *v, const double *vx, const double *vy, const double *vz) {
-                             for (int j = 0; j < nB; j++) {
+                         [&](auto n, const double *v, const double *vx, const double *vy, const double *vz) {
+#pragma unroll
+                             for (int j = 0; j < n; j++) {
                                  if (k < blk.nKept && kept[k] == sh.fStart + j) {
                                      const size_t o = static_cast<size_t>(blk.vOffset + k) * kBlockSize + t;
-                                     f[o] = static_cast<T>(valid ? v[j] : 0.0);
-                                     fx[o] = static_cast<T>(valid ? vx[j] : 0.0);
-                                     fy[o] = static_cast<T>(valid ? vy[j] : 0.0);
-                                     fz[o] = static_cast<T>(valid ? vz[j] : 0.0);
+                                     f[o] = valid ? v[j] : 0.0;
+                                     fx[o] = valid ? vx[j] : 0.0;
+                                     fy[o] = valid ? vy[j] : 0.0;
+                                     fz[o] = valid ? vz[j] : 0.0;
+                                     m[0] = fmax(m[0], fabs(v[j]));
+                                     m[1] = fmax(m[1], fabs(vx[j]));
+                                     m[2] = fmax(m[2], fabs(vy[j]));
+                                     m[3] = fmax(m[3], fabs(vz[j]));
                                      k++;
                                  }
                              }
                          });
+    }
+    if (EB != nullptr) {
+        EB[static_cast<size_t>(b) * kBlockSize + t] = static_cast<signed char>(valid ? stored_exponent(m[0]) : 0);
+        for (int c = 0; c < 3; c++)
+            EG[(static_cast<size_t>(b) * 3 + c) * kBlockSize + t] =
+                static_cast<signed char>(valid ? stored_exponent(m[c + 1]) : 0);
     }
 }
 
@@ -269,7 +307,7 @@ __global__ void __launch_bounds__(kBlockSize) basis_eval_kernel(
 template <int LL, int LH, bool SPH>
 __device__ __forceinline__ void shell_eval2(const xq::DevShell &sh, const double *__restrict__ coef,
                                             const double *__restrict__ trans, double dx, double dy, double dz,
-                                            double (*out)[16]) {
+                                            double (*out)[SPH ? ShellDims<LL, LH>::nSph : ShellDims<LL, LH>::nCBF]) {
     constexpr int NC = ShellDims<LL, LH>::nCBF;
     constexpr int NB = SPH ? ShellDims<LL, LH>::nSph : NC;
     constexpr int C0 = cart_offset(LL);
@@ -331,31 +369,16 @@ __device__ __forceinline__ void shell_eval2(const xq::DevShell &sh, const double
     }
 }
 
-// Dispatch on the shell type; calls body(nBasis, out).
+// Dispatch on the shell type; calls body(N, out), N the shell's functions as a compile-time constant.
 template <typename Body>
 __device__ __forceinline__ void with_shell2(const xq::DevShell &sh, bool sph, const double *coef, const double *trans,
                                             double dx, double dy, double dz, Body body) {
-    double out[10][16];
-    const int key = sh.lLow * 4 + sh.lHigh;
-    if (sph) {
-        switch (key) {
-            case 0: shell_eval2<0, 0, true>(sh, coef, trans, dx, dy, dz, out); body(1, out); break;
-            case 5: shell_eval2<1, 1, true>(sh, coef, trans, dx, dy, dz, out); body(3, out); break;
-            case 1: shell_eval2<0, 1, true>(sh, coef, trans, dx, dy, dz, out); body(4, out); break;
-            case 10: shell_eval2<2, 2, true>(sh, coef, trans, dx, dy, dz, out); body(5, out); break;
-            case 15: shell_eval2<3, 3, true>(sh, coef, trans, dx, dy, dz, out); body(7, out); break;
-            default: break;
-        }
-    } else {
-        switch (key) {
-            case 0: shell_eval2<0, 0, false>(sh, coef, trans, dx, dy, dz, out); body(1, out); break;
-            case 5: shell_eval2<1, 1, false>(sh, coef, trans, dx, dy, dz, out); body(3, out); break;
-            case 1: shell_eval2<0, 1, false>(sh, coef, trans, dx, dy, dz, out); body(4, out); break;
-            case 10: shell_eval2<2, 2, false>(sh, coef, trans, dx, dy, dz, out); body(6, out); break;
-            case 15: shell_eval2<3, 3, false>(sh, coef, trans, dx, dy, dz, out); body(10, out); break;
-            default: break;
-        }
-    }
+    for_shell_type(sh, sph, [&](auto ll, auto lh, auto s) {
+        constexpr int N = s ? ShellDims<ll, lh>::nSph : ShellDims<ll, lh>::nCBF;
+        double out[10][N];
+        shell_eval2<ll, lh, s>(sh, coef, trans, dx, dy, dz, out);
+        body(std::integral_constant<int, N>{}, out);
+    });
 }
 
 // Values and first and second derivatives of the kept functions of blocks b0 + blockIdx.x into rows
@@ -378,9 +401,10 @@ __global__ void __launch_bounds__(kBlockSize) basis_eval2_kernel(
     const int k1 = static_cast<int>((static_cast<long long>(h) + 1) * blk.nKept / S);
     int k = static_cast<int>(static_cast<long long>(h) * blk.nKept / S);
     while (k < k1) {
-        const xq::DevShell sh = shells[shellOf[kept[k]]];
-        with_shell2(sh, spherical != 0, coef, trans, x - sh.x, y - sh.y, z - sh.z, [&](int nB, const double (*v)[16]) {
-            for (int j = 0; j < nB; j++) {
+        const xq::DevShell &sh = shells[shellOf[kept[k]]];
+        with_shell2(sh, spherical != 0, coef, trans, x - sh.x, y - sh.y, z - sh.z, [&](auto n, const auto &v) {
+#pragma unroll
+            for (int j = 0; j < n; j++) {
                 if (k < k1 && kept[k] == sh.fStart + j) {
                     const size_t o = static_cast<size_t>(blk.vOffset - rowBase + k) * kBlockSize + t;
 #pragma unroll
@@ -537,7 +561,8 @@ int set_basis(xq_grid *g, int nSpec, const double *spec, int spherical, int prec
         if ((status = check(hipMemcpyAsync(d_shellOf, shellOf.data(), shellOf.size() * sizeof(int), hipMemcpyHostToDevice, s),
                             "copy shellOf")) != kOK) break;
         if (g->nBlocks > 0) {
-            hipLaunchKernelGGL(basis_count_kernel, dim3(g->nBlocks), dim3(kBlockSize), 0, s, g->nBlocks, g->d_blocks, g->d_x,
+            const size_t mask = sizeof(unsigned) * ((static_cast<size_t>(g->nShells) + 1) / 2);
+            hipLaunchKernelGGL(basis_count_kernel, dim3(g->nBlocks), dim3(kBlockSize), mask, s, g->nBlocks, g->d_blocks, g->d_x,
                                g->d_y, g->d_z, g->nShells, g->d_shells, g->d_coef, g->d_trans, g->spherical, f, g->bfTol,
                                tmpIdx, counts);
             if ((status = check(hipGetLastError(), "basis_count_kernel")) != kOK) break;
@@ -577,11 +602,16 @@ int set_basis(xq_grid *g, int nSpec, const double *spec, int spherical, int prec
             g->deviceBytes += static_cast<long long>(nVal * elt);
         }
         if (status != kOK) break;
+        if (precision == XQ_PRECISION_MIXED) {
+            const size_t nB = static_cast<size_t>(g->nBlocks > 0 ? g->nBlocks : 1);
+            if ((status = dev_alloc(g, &g->d_EB, nB * kBlockSize)) != kOK) break;
+            if ((status = dev_alloc(g, &g->d_EG, 3 * nB * kBlockSize)) != kOK) break;
+        }
         if (g->nBlocks > 0) {
-            hipLaunchKernelGGL(basis_eval_kernel<double>, dim3(g->nBlocks), dim3(kBlockSize), 0, s, g->d_blocks, g->d_x,
+            hipLaunchKernelGGL(basis_eval_kernel, dim3(g->nBlocks), dim3(kBlockSize), 0, s, g->d_blocks, g->d_x,
                                g->d_y, g->d_z, g->d_shells, d_shellOf, g->d_coef, g->d_trans, g->spherical, f, tmpIdx,
                                g->d_idx, static_cast<double *>(g->d_f), static_cast<double *>(g->d_fx),
-                               static_cast<double *>(g->d_fy), static_cast<double *>(g->d_fz));
+                               static_cast<double *>(g->d_fy), static_cast<double *>(g->d_fz), g->d_EB, g->d_EG);
             if ((status = check(hipGetLastError(), "basis_eval_kernel")) != kOK) break;
         }
         // The operand-order planes of the chosen precision replace the FP64 rows.

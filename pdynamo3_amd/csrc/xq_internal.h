@@ -23,6 +23,17 @@ constexpr int kMaxCBF = 20;
 constexpr int kMaxPrim = 16;
 constexpr int kMaxL = 3;
 
+// Exponents of the mixed path's digit groups are int8.  A group whose largest magnitude is below 2^-100 (contributions below
+// 1e-30 of unit-sized terms) gets exponent 0, which rounds all its digits to zero.  Magnitudes here stay far below 2^127.
+constexpr int kMinStoredExponent = -100;
+
+// Power of two strictly above max|x| (frexp exponent), clamped as described above.
+__device__ __forceinline__ int stored_exponent(double amax) {
+    int e = 0;
+    if (amax > 0.0) (void)frexp(amax, &e);
+    return e < kMinStoredExponent ? 0 : e;
+}
+
 void set_error(const std::string &message);
 
 // Shell description on the device (one per shell of every atom).

@@ -84,19 +84,8 @@ constexpr int kPRowDwords = 12;         // one staged P_red row in LDS: 8 words 
 constexpr int kIdxCache = 1024;         // kept-function indices of a block cached in LDS by the density kernel
 constexpr int kSuper = 4;               // blocks per superblock of the Fock product
 
-// Stored exponents are int8.  A group whose largest magnitude is below 2^-100 (contributions below 1e-30 of unit-sized
-// terms) gets exponent 0, which rounds all its digits to zero.  Magnitudes here stay far below 2^127.
-constexpr int kMinStoredExponent = -100;
-
 __device__ __forceinline__ v16i mfma_i8(const v4i &a, const v4i &b, const v16i &c) {
     return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);
-}
-
-// Power of two strictly above max|x| (frexp exponent), clamped as described above.
-__device__ __forceinline__ int stored_exponent(double amax) {
-    int e = 0;
-    if (amax > 0.0) (void)frexp(amax, &e);
-    return e < kMinStoredExponent ? 0 : e;
 }
 
 template <int D>
@@ -188,30 +177,6 @@ __device__ __forceinline__ int job_of(const xq::MixedJob *jobs, int nJobs, int g
 // ------------------------------------------------------------------------------------------------------------------------
 // Set-up, once per geometry.
 // ------------------------------------------------------------------------------------------------------------------------
-// EB and EG: per point of a block, the powers of two above max |Phi| and above max |d Phi / dx_c| over the block's kept
-// functions (128 threads = points).
-__global__ void __launch_bounds__(kBlockSize) point_exponent_kernel(
-    const xq::DevBlock *__restrict__ blocks, const double *__restrict__ f, const double *__restrict__ fx,
-    const double *__restrict__ fy, const double *__restrict__ fz, signed char *__restrict__ EB,
-    signed char *__restrict__ EG) {
-    const int b = blockIdx.x, t = threadIdx.x;
-    const xq::DevBlock blk = blocks[b];
-    const size_t R = static_cast<size_t>(blk.vOffset);
-    double m = 0.0, mx = 0.0, my = 0.0, mz = 0.0;
-    for (int r = 0; r < blk.nKept; r++) {
-        const size_t o = (R + r) * kBlockSize + t;
-        m = fmax(m, fabs(f[o]));
-        mx = fmax(mx, fabs(fx[o]));
-        my = fmax(my, fabs(fy[o]));
-        mz = fmax(mz, fabs(fz[o]));
-    }
-    EB[static_cast<size_t>(b) * kBlockSize + t] = static_cast<signed char>(stored_exponent(m));
-    signed char *eg = EG + static_cast<size_t>(b) * 3 * kBlockSize + t;
-    eg[0] = static_cast<signed char>(stored_exponent(mx));
-    eg[kBlockSize] = static_cast<signed char>(stored_exponent(my));
-    eg[2 * kBlockSize] = static_cast<signed char>(stored_exponent(mz));
-}
-
 // One union chunk per work-group (256 threads): EA, DA, GHU and GLU of the chunk's 32 union rows from the FP64 values of
 // the block's kept rows (zero for the rows the block does not keep).
 __global__ void __launch_bounds__(256) fock_operand_prepare_kernel(
@@ -911,6 +876,7 @@ static int union_tables(xq_grid *g) {
     return kOK;
 }
 
+// The operand planes from the FP64 values (the point exponents EB and EG are there, xq_basis.hip).
 int prepare_mixed(xq_grid *g, const double *f, const double *fx, const double *fy, const double *fz) {
     XQ_TRY(chunk_tables(g));
     XQ_TRY(union_tables(g));
@@ -919,9 +885,7 @@ int prepare_mixed(xq_grid *g, const double *f, const double *fx, const double *f
     XQ_TRY(dev_alloc(g, &g->d_DA, ncU * kChunkBytes));
     XQ_TRY(dev_alloc(g, &g->d_EA, ncU * kC));
     XQ_TRY(dev_alloc(g, &g->d_DB, nc * kChunkBytesB));
-    XQ_TRY(dev_alloc(g, &g->d_EB, static_cast<size_t>(g->nBlocks > 0 ? g->nBlocks : 1) * kBlockSize));
     XQ_TRY(dev_alloc(g, &g->d_GF, nc * kChunkGrad));
-    XQ_TRY(dev_alloc(g, &g->d_EG, static_cast<size_t>(g->nBlocks > 0 ? g->nBlocks : 1) * 3 * kBlockSize));
     XQ_TRY(dev_alloc(g, &g->d_DW, ncU * kChunkBytes));
     XQ_TRY(dev_alloc(g, &g->d_GHU, ncU * kChunkGrad));
     XQ_TRY(dev_alloc(g, &g->d_GLU, ncU * kChunkGrad));
@@ -931,9 +895,6 @@ int prepare_mixed(xq_grid *g, const double *f, const double *fx, const double *f
     XQ_TRY(dev_alloc(g, &g->d_wcoef, 4 * static_cast<size_t>(g->nPoints > 0 ? g->nPoints : 1)));
     XQ_TRY(dev_alloc(g, &g->d_part, nc * 4 * kBlockSize));
     hipStream_t s = g->stream;
-    if (g->nBlocks > 0)
-        hipLaunchKernelGGL(point_exponent_kernel, dim3(g->nBlocks), dim3(kBlockSize), 0, s, g->d_blocks, f, fx, fy, fz,
-                           g->d_EB, g->d_EG);
     if (chunks > 0)
         hipLaunchKernelGGL(density_operand_prepare_kernel, dim3(static_cast<unsigned>(chunks)), dim3(256), 0, s,
                            g->d_blocks, g->d_chunkOffset, g->d_chunkBlock, f, fx, fy, fz, g->d_EB, g->d_EG, g->d_DB,
