@@ -88,15 +88,24 @@ __device__ __forceinline__ v16i mfma_i8(const v4i &a, const v4i &b, const v16i &
     return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);
 }
 
+// The D digits of x in a group of power of two e.  The integer Q = round(x 2^(7D - e)) is exact in FP64; its first four digits
+// come from one 32-bit word and a fifth from the remainder, so that nothing is converted to 64-bit integers (which takes
+// about ten instructions).
 template <int D>
 __device__ __forceinline__ void slice(double x, int e, signed char *d) {
-    const long long Q = static_cast<long long>(rint(ldexp(x, 7 * D - e)));
+    static_assert(D == 4 || D == 5, "four digits fill one word");
+    const double Q = rint(ldexp(x, 7 * D - e));
     // |x| < 2^e, so |Q| <= 2^(7D); the one value that rounds up to 2^(7D) is clamped to the largest D-digit magnitude.
-    unsigned long long a = static_cast<unsigned long long>(Q < 0 ? -Q : Q);
-    a = a < (1ull << (7 * D)) ? a : (1ull << (7 * D)) - 1ull;
-    const int sign = Q < 0 ? -1 : 1;
+    const double a = fmin(fabs(Q), static_cast<double>((1ull << (7 * D)) - 1ull));
+    const int s = Q < 0.0 ? -1 : 0;      // (digit ^ s) - s is the digit with Q's sign
+    unsigned u;
+    if constexpr (D == 4) u = static_cast<unsigned>(static_cast<int>(a));
+    else {
+        u = static_cast<unsigned>(static_cast<int>(a * 0x1p-7));
+        d[4] = static_cast<signed char>((static_cast<int>(fma(-128.0, static_cast<double>(static_cast<int>(u)), a)) ^ s) - s);
+    }
 #pragma unroll
-    for (int k = 0; k < D; k++) d[k] = static_cast<signed char>(sign * static_cast<int>((a >> (7 * (D - 1 - k))) & 127ull));
+    for (int k = 0; k < 4; k++) d[k] = static_cast<signed char>((static_cast<int>((u >> (7 * (3 - k))) & 127u) ^ s) - s);
 }
 
 // Exact combination of digit-order accumulators: sum_s acc_s 128^(S-1-s) as a 64-bit integer.
@@ -146,13 +155,11 @@ __device__ __forceinline__ int ubyte_of(const v4i &x, int v) {
 // Element v (0..15) of sixteen int32 held in four 16-byte operands.
 __device__ __forceinline__ double int_of(const v4i (&g)[4], int v) { return static_cast<double>(g[v >> 2][v & 3]); }
 
-// B-bit fixed point of g with |g| < 2^e: round(g 2^(B - e)) in [-(2^B - 1), 2^B - 1].
+// B-bit fixed point of g with |g| < 2^e: round(g 2^(B - e)) in [-(2^B - 1), 2^B - 1] (B <= 31).
 template <int B>
 __device__ __forceinline__ int grad_encode(double g, int e) {
-    long long Q = static_cast<long long>(rint(ldexp(g, B - e)));
-    const long long lim = (1ll << B) - 1;
-    Q = Q > lim ? lim : (Q < -lim ? -lim : Q);
-    return static_cast<int>(Q);
+    constexpr double lim = static_cast<double>((1ll << B) - 1);
+    return static_cast<int>(fmin(fmax(rint(ldexp(g, B - e)), -lim), lim));
 }
 
 // Row of a chunk held at density position 16 h + v (K position 4 q + j holds row 8 j + q).
@@ -178,47 +185,49 @@ __device__ __forceinline__ int job_of(const xq::MixedJob *jobs, int nJobs, int g
 // Set-up, once per geometry.
 // ------------------------------------------------------------------------------------------------------------------------
 // One union chunk per work-group (256 threads): EA, DA, GHU and GLU of the chunk's 32 union rows from the FP64 values of
-// the block's kept rows (zero for the rows the block does not keep).
+// the block's kept rows (zero for the rows the block does not keep).  Each plane's 32 rows are read in order into LDS, from
+// which thread (q, lane) takes its 16 points of one row; reading those 16 points from memory took 2.14 ms on (H2O)24
+// (2.7 GB in, 1.1 GB out) where this takes 1.08 ms.
 __global__ void __launch_bounds__(256) fock_operand_prepare_kernel(
     const xq::DevBlock *__restrict__ blocks, const int *__restrict__ uChunkBlock, const int *__restrict__ uRow,
     const double *__restrict__ f, const double *__restrict__ fx, const double *__restrict__ fy,
     const double *__restrict__ fz, const signed char *__restrict__ EG, signed char *__restrict__ DA,
     signed char *__restrict__ EA, short *__restrict__ GHU, unsigned char *__restrict__ GLU) {
-    __shared__ int sE[kC];
-    __shared__ int sRow[kC];
+    __shared__ double sv[kC][kBlockSize + 1];
+    __shared__ int sRow[kC], sE[3][kBlockSize];
     const size_t C = blockIdx.x;
     const int b = uChunkBlock[C];
-    const xq::DevBlock blk = blocks[b];
-    const int t = threadIdx.x;
-    const size_t R = static_cast<size_t>(blk.vOffset);
+    const int t = threadIdx.x, q = t >> 6, lane = t & 63, lr = lane & 31, lh = lane >> 5;
+    const size_t R = static_cast<size_t>(blocks[b].vOffset);
     if (t < kC) sRow[t] = uRow[C * kC + t];
+    for (int k = t; k < 3 * kBlockSize; k += 256) sE[k / kBlockSize][k % kBlockSize] = EG[static_cast<size_t>(b) * 3 * kBlockSize + k];
     __syncthreads();
-    auto value = [&](const double *a, int i, int p) -> double {
-        const int k = sRow[i];
-        return k >= 0 ? a[(R + k) * kBlockSize + p] : 0.0;
-    };
-    // EA: row i = t / 8 of the chunk, eight threads per row with 16 points each.
-    {
-        const int i = t >> 3, part = t & 7;
-        double m = 0.0;
-#pragma unroll 4
-        for (int k = 0; k < 16; k++) m = fmax(m, fabs(value(f, i, 16 * part + k)));
+    // Plane a's rows into LDS: two rows at a time, a thread per point.
+    auto stage = [&](const double *__restrict__ a) {
 #pragma unroll
-        for (int o = 4; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 8));
-        if (part == 0) {
-            const int e = stored_exponent(m);
-            sE[i] = e;
-            EA[C * kC + i] = static_cast<signed char>(e);
+        for (int r = 0; r < kC; r += 2) {
+            const int i = r + (t >> 7), k = sRow[i];
+            sv[i][t & (kBlockSize - 1)] = k >= 0 ? a[(R + k) * kBlockSize + (t & (kBlockSize - 1))] : 0.0;
         }
-    }
+        __syncthreads();
+    };
+    const double *mine = &sv[lr][kC * q + 16 * lh];
+    stage(f);
+    // EA: the row's largest value, over the 8 threads (q, lh) that share it.
+    double m = 0.0;
+#pragma unroll
+    for (int k = 0; k < 16; k++) m = fmax(m, fabs(mine[k]));
+    m = fmax(m, __shfl_xor(m, 32, 64));
+    __shared__ double sm[4][kC];
+    if (lh == 0) sm[q][lr] = m;
     __syncthreads();
-    // DA: thread = (q, lane).
-    const int q = t >> 6, lane = t & 63, lr = lane & 31, lh = lane >> 5, e = sE[lr];
+    const int e = stored_exponent(fmax(fmax(sm[0][lr], sm[1][lr]), fmax(sm[2][lr], sm[3][lr])));
+    if (q == 0 && lh == 0) EA[C * kC + lr] = static_cast<signed char>(e);
     signed char d[kDPhi][16];
 #pragma unroll
     for (int k = 0; k < 16; k++) {
         signed char dd[kDPhi];
-        slice<kDPhi>(value(f, lr, kC * q + 16 * lh + k), e, dd);
+        slice<kDPhi>(mine[k], e, dd);
 #pragma unroll
         for (int j = 0; j < kDPhi; j++) d[j][k] = dd[j];
     }
@@ -227,14 +236,13 @@ __global__ void __launch_bounds__(256) fock_operand_prepare_kernel(
         *reinterpret_cast<v4i *>(&DA[C * kChunkBytes + (q * kDPhi + j) * 1024 + lane * 16]) = pack16(d[j]);
     // GHU, GLU: the same thread's 16 values of each gradient component, scaled by each point's component exponent.
     const double *grads[3] = {fx, fy, fz};
-#pragma unroll
+#pragma unroll 1
     for (int c = 0; c < 3; c++) {
+        __syncthreads();      // every thread is done with the plane before
+        stage(grads[c]);
         int Q[16];
 #pragma unroll
-        for (int k = 0; k < 16; k++) {
-            const int p = kC * q + 16 * lh + k;
-            Q[k] = grad_encode<kGradBitsW>(value(grads[c], lr, p), EG[(static_cast<size_t>(b) * 3 + c) * kBlockSize + p]);
-        }
+        for (int k = 0; k < 16; k++) Q[k] = grad_encode<kGradBitsW>(mine[k], sE[c][kC * q + 16 * lh + k]);
         // Q = 256 hi + lo with lo in [0, 255]: hi = Q >> 8 (arithmetic), lo = Q & 255.
         v4i hq[2], lq;
 #pragma unroll
@@ -253,46 +261,60 @@ __global__ void __launch_bounds__(256) fock_operand_prepare_kernel(
     }
 }
 
-// One chunk per work-group (256 threads): DB and GF from the FP64 values of the chunk's rows.
+// One chunk per work-group (256 threads): DB and GF from the FP64 values of the chunk's rows.  Each plane's 32 rows are read
+// in order into LDS, and consecutive threads write consecutive 16-byte pieces of the operands; threads that each wrote 64
+// bytes of their own took 1.32 ms on (H2O)24 (2.5 GB in, 1.4 GB out) where this takes 1.17 ms.
 __global__ void __launch_bounds__(256) density_operand_prepare_kernel(
     const xq::DevBlock *__restrict__ blocks, const int *__restrict__ chunkOffset, const int *__restrict__ chunkBlock,
     const double *__restrict__ f, const double *__restrict__ fx, const double *__restrict__ fy,
     const double *__restrict__ fz, const signed char *__restrict__ EB, const signed char *__restrict__ EG,
     signed char *__restrict__ DB, int *__restrict__ GF) {
+    __shared__ double sv[kC][kBlockSize + 8];     // padded so that 8 points of 4 rows lie in different banks
     const size_t C = blockIdx.x;
     const int b = chunkBlock[C];
     const xq::DevBlock blk = blocks[b];
     const int nb = blk.nKept, rc = static_cast<int>(C) - chunkOffset[b], t = threadIdx.x;
-    const size_t R = static_cast<size_t>(blk.vOffset);
-    auto value = [&](const double *a, int row, int p) -> double {
-        return row < nb ? a[(R + row) * kBlockSize + p] : 0.0;
+    const size_t R = static_cast<size_t>(blk.vOffset) + static_cast<size_t>(kC) * rc;
+    auto stage = [&](const double *__restrict__ a) {
+#pragma unroll
+        for (int r = 0; r < kC; r += 2) {
+            const int i = r + (t >> 7), p = t & (kBlockSize - 1);
+            sv[i][p] = kC * rc + i < nb ? a[(R + i) * kBlockSize + p] : 0.0;
+        }
+        __syncthreads();
     };
-    // DB and GF: thread = (point p, half h) with the 16 rows chunk_fun(h, 0..15).
+    stage(f);
+    // DB: thread = (point p, half h) with the 16 rows chunk_fun(h, 0..15).
     {
-        const int p = t & (kBlockSize - 1), h = t >> 7;
+        const int p = t >> 1, h = t & 1;
         const int e = EB[static_cast<size_t>(b) * kBlockSize + p];
         signed char d[kDB][16];
 #pragma unroll
         for (int v = 0; v < 16; v++) {
             signed char dd[kDB];
-            slice<kDB>(value(f, kC * rc + chunk_fun(h, v), p), e, dd);
+            slice<kDB>(sv[chunk_fun(h, v)][p], e, dd);
 #pragma unroll
             for (int j = 0; j < kDB; j++) d[j][v] = dd[j];
         }
 #pragma unroll
         for (int j = 0; j < kDB; j++)
             *reinterpret_cast<v4i *>(&DB[C * kChunkBytesB + (j * kBlockSize + p) * kC + 16 * h]) = pack16(d[j]);
-        const double *grads[3] = {fx, fy, fz};
+    }
+    // GF: thread = (points t / 8 + 32 i, positions 4 w .. + 3).
+    const double *grads[3] = {fx, fy, fz};
+    const int w = t & 7, h = w >> 2, v0 = 4 * (w & 3);
+#pragma unroll 1
+    for (int c = 0; c < 3; c++) {
+        __syncthreads();      // every thread is done with the plane before
+        stage(grads[c]);
 #pragma unroll
-        for (int c = 0; c < 3; c++) {
+        for (int i = 0; i < 4; i++) {
+            const int p = 32 * i + (t >> 3);
             const int eg = EG[(static_cast<size_t>(b) * 3 + c) * kBlockSize + p];
-            v4i gq[4];
+            v4i g;
 #pragma unroll
-            for (int v = 0; v < 16; v++)
-                gq[v >> 2][v & 3] = grad_encode<kGradBits>(value(grads[c], kC * rc + chunk_fun(h, v), p), eg);
-            const size_t o = C * kChunkGrad + (c * kBlockSize + p) * kC + 16 * h;
-#pragma unroll
-            for (int w = 0; w < 4; w++) *reinterpret_cast<v4i *>(GF + o + 4 * w) = gq[w];
+            for (int v = 0; v < 4; v++) g[v] = grad_encode<kGradBits>(sv[chunk_fun(h, v0 + v)][p], eg);
+            *reinterpret_cast<v4i *>(GF + C * kChunkGrad + (c * kBlockSize + p) * kC + 4 * w) = g;
         }
     }
 }
