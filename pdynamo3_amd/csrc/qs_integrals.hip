@@ -152,48 +152,83 @@ __global__ void __launch_bounds__(kThreads) fit_matrix_kernel(int nPairs, const 
 // Per SCF iteration: b = sum_rows w_row P_row B_row (partial sums over row chunks, then a fixed-order reduction) and
 // F_row += B_row . c (one wave per row).  w_row = 2 off the diagonal, 1 on it, 0 for a duplicate row.
 // ------------------------------------------------------------------------------------------------------------------------
-constexpr int kRowChunk = 1024;
+constexpr int kRowChunk = 256;
 
+// Partial sums of b over kRowChunk rows: a thread per fit function, the rows' weights w_row P_row gathered once into LDS and
+// the rows' loads independent of each other.  Bound by reading the integrals: 1.7 GB on (H2O)48 in 0.29 ms, against 0.61
+// with chunks of 1,024 rows whose every load waited for the row's index and density; on (H2O)16, which had too few
+// chunks to fill the chip, 0.37 -> 0.02 ms.
 __global__ void __launch_bounds__(256) fit_b_partial_kernel(long long rows, int nFit, const double *__restrict__ B,
                                                            const long long *__restrict__ rowPacked,
                                                            const unsigned char *__restrict__ rowDiag,
                                                            const double *__restrict__ P, double *__restrict__ partial) {
-    const int col = blockIdx.x * 256 + threadIdx.x;
+    __shared__ double sw[kRowChunk];
     const long long r0 = static_cast<long long>(blockIdx.y) * kRowChunk;
-    const long long r1 = r0 + kRowChunk < rows ? r0 + kRowChunk : rows;
-    double acc = 0.0;
-    if (col < nFit)
-        for (long long r = r0; r < r1; r++) {
-            const long long o = rowPacked[r];
-            if (o < 0) continue;
-            acc += (rowDiag[r] ? 1.0 : 2.0) * P[o] * B[r * nFit + col];
-        }
-    if (col < nFit) partial[static_cast<size_t>(blockIdx.y) * nFit + col] = acc;
-}
-
-__global__ void __launch_bounds__(256) fit_b_reduce_kernel(int nChunks, int nFit, const double *__restrict__ partial,
-                                                          double *__restrict__ b) {
+    const int n = static_cast<int>(rows - r0 < kRowChunk ? rows - r0 : kRowChunk);
+    for (int k = threadIdx.x; k < n; k += 256) {
+        const long long o = rowPacked[r0 + k];
+        sw[k] = o < 0 ? 0.0 : (rowDiag[r0 + k] ? 1.0 : 2.0) * P[o];
+    }
+    __syncthreads();
     const int col = blockIdx.x * 256 + threadIdx.x;
     if (col >= nFit) return;
+    const double *row = B + r0 * nFit + col;
     double acc = 0.0;
-    for (int k = 0; k < nChunks; k++) acc += partial[static_cast<size_t>(k) * nFit + col];
-    b[col] = acc;
+#pragma unroll 8
+    for (int k = 0; k < n; k++) acc = fma(sw[k], row[static_cast<size_t>(k) * nFit], acc);
+    partial[static_cast<size_t>(blockIdx.y) * nFit + col] = acc;
 }
+
+// b from the partial sums: 64 fit functions per work-group, 16 threads each (chunks j, j + 16, ...), then their 16 sums in
+// order.
+__global__ void __launch_bounds__(1024) fit_b_reduce_kernel(int nChunks, int nFit, const double *__restrict__ partial,
+                                                            double *__restrict__ b) {
+    __shared__ double s[16][64];
+    const int c = threadIdx.x & 63, j = threadIdx.x >> 6, col = blockIdx.x * 64 + c;
+    double acc = 0.0;
+    if (col < nFit) {
+#pragma unroll 4
+        for (int k = j; k < nChunks; k += 16) acc += partial[static_cast<size_t>(k) * nFit + col];
+    }
+    s[j][c] = acc;
+    __syncthreads();
+    if (j == 0 && col < nFit) {
+        for (int k = 1; k < 16; k++) acc += s[k][c];
+        b[col] = acc;
+    }
+}
+
+// F_row += B_row . c, four rows per wave: each value of c serves four loads.  Bound by reading the integrals ((H2O)48: one row
+// per wave 0.37 ms, this 0.29 ms).
+constexpr int kFockRows = 4;
 
 __global__ void __launch_bounds__(256) fit_fock_kernel(long long rows, int nFit, const double *__restrict__ B,
                                                       const long long *__restrict__ rowPacked,
                                                       const double *__restrict__ c, double *__restrict__ F) {
-    const long long r = (blockIdx.x * 256LL + threadIdx.x) / 64;
+    const long long r0 = (blockIdx.x * 256LL + threadIdx.x) / 64 * kFockRows;
     const int lane = threadIdx.x & 63;
-    if (r >= rows) return;
-    const long long o = rowPacked[r];
-    if (o < 0) return;                  // wave-uniform: the whole wave leaves together
-    const double *row = B + r * nFit;
-    double acc = 0.0;
-    for (int k = lane; k < nFit; k += 64) acc += row[k] * c[k];
+    if (r0 >= rows) return;
+    const int n = static_cast<int>(rows - r0 < kFockRows ? rows - r0 : kFockRows);
+    const double *row[kFockRows];
+    double acc[kFockRows];
 #pragma unroll
-    for (int s = 32; s > 0; s >>= 1) acc += __shfl_xor(acc, s, 64);
-    if (lane == 0) F[o] += acc;
+    for (int i = 0; i < kFockRows; i++) {
+        row[i] = B + (r0 + (i < n ? i : 0)) * nFit;     // the last rows' waves repeat a row
+        acc[i] = 0.0;
+    }
+#pragma unroll 2
+    for (int k = lane; k < nFit; k += 64) {
+        const double x = c[k];
+#pragma unroll
+        for (int i = 0; i < kFockRows; i++) acc[i] = fma(row[i][k], x, acc[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < kFockRows; i++) {
+#pragma unroll
+        for (int s = 32; s > 0; s >>= 1) acc[i] += __shfl_xor(acc[i], s, 64);
+        const long long o = i < n ? rowPacked[r0 + i] : -1;
+        if (lane == 0 && o >= 0) F[o] += acc[i];
+    }
 }
 
 }  // namespace
@@ -596,7 +631,7 @@ int qs_fit_b(qs_fit *fit, const double *P, double *b) {
     if (nChunks > 0) {
         hipLaunchKernelGGL(fit_b_partial_kernel, dim3((fit->nFit + 255) / 256, nChunks), dim3(256), 0, s, fit->rows,
                            fit->nFit, fit->d_B, fit->d_rowPacked, fit->d_rowDiag, fit->d_P, fit->d_partial);
-        hipLaunchKernelGGL(fit_b_reduce_kernel, dim3((fit->nFit + 255) / 256), dim3(256), 0, s, nChunks, fit->nFit,
+        hipLaunchKernelGGL(fit_b_reduce_kernel, dim3((fit->nFit + 63) / 64), dim3(1024), 0, s, nChunks, fit->nFit,
                            fit->d_partial, fit->d_b);
         XQ_CHECK(hipGetLastError());
         XQ_CHECK(hipMemcpyAsync(fit->host.data(), fit->d_b, fit->nFit * sizeof(double), hipMemcpyDeviceToHost, s));
@@ -614,7 +649,7 @@ int qs_fit_fock(qs_fit *fit, const double *c, double *Fock) {
     XQ_CHECK(hipMemcpyAsync(fit->d_c, fit->host.data(), fit->nFit * sizeof(double), hipMemcpyHostToDevice, s));
     XQ_CHECK(hipMemcpyAsync(fit->d_F, Fock, nPacked * sizeof(double), hipMemcpyHostToDevice, s));
     if (fit->rows > 0) {
-        const long long waves = fit->rows;
+        const long long waves = (fit->rows + kFockRows - 1) / kFockRows;
         hipLaunchKernelGGL(fit_fock_kernel, dim3(static_cast<unsigned>((waves * 64 + 255) / 256)), dim3(256), 0, s,
                            fit->rows, fit->nFit, fit->d_B, fit->d_rowPacked, fit->d_c, fit->d_F);
         XQ_CHECK(hipGetLastError());
