@@ -8,7 +8,7 @@
 
 namespace qs {
 
-// What the launches of one qs_fit_create share.
+// What the launches of one qs_fit_create or qs_fit_matrix share.
 struct FitLaunch {
     hipStream_t stream;
     const QShell *oShells;
@@ -20,6 +20,7 @@ struct FitLaunch {
     int column[kMaxL + 2];
     const double *fExps, *fCoefs, *boys;
     int nFit;
+    double cut;                     // integrals not above it in magnitude are stored as zero; negative for none
     double *B;
 };
 
@@ -43,7 +44,7 @@ __global__ void __launch_bounds__(256) fit_integrals_kernel(int nPairs, const Pa
                                                             const double *__restrict__ fExps,
                                                             const double *__restrict__ fCoefs,
                                                             const double *__restrict__ boysTable, int column, int nFit,
-                                                            double *__restrict__ B) {
+                                                            double cut, double *__restrict__ B) {
     const int chunks = (nFitShells + 63) / 64;
     const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x * 4 + (threadIdx.x >> 6)));
     const int k = w / chunks, c = (w - k * chunks) * 64 + static_cast<int>(threadIdx.x & 63);
@@ -57,7 +58,7 @@ __global__ void __launch_bounds__(256) fit_integrals_kernel(int nPairs, const Pa
     for_functions<LA, LB>(oSpherical, [&](int i, int j, auto ab) {
         double *row = out + pair_row(it, i, j, ma, mb) * nFit;
         fit_functions<LC, M0, NM>(fSpherical, acc[ab], [&](int f, double x) {
-            row[f * nFitShells] = fabs(x) > kUnderFlow ? x : 0.0;
+            row[f * nFitShells] = cut >= 0.0 && !(fabs(x) > cut) ? 0.0 : x;
         });
     });
 }
@@ -72,7 +73,7 @@ void launch_fit(const FitLaunch &f, const PairItem *items, int n) {
     static_for<cartesians(LC) / NM>([&](auto group) {
         hipLaunchKernelGGL((fit_integrals_kernel<LA, LB, LC, group * NM, NM>), grid, dim3(256), 0, f.stream, n, items,
                            f.oShells, f.oSpherical, f.records, shells, f.fShells + f.first[LC], f.fSpherical, f.fExps,
-                           f.fCoefs, f.boys, f.column[LC], f.nFit, f.B);
+                           f.fCoefs, f.boys, f.column[LC], f.nFit, f.cut, f.B);
     });
 }
 

@@ -44,8 +44,6 @@ namespace qs {
 
 // The Boys function table, one copy per GPU (filled once per device by the first basis created on it).
 __device__ double g_boys[kBoysPoints * kBoysTable];
-// The c2s transformations of l = 0..2 ([l][6][5]), one copy per GPU.
-__device__ double g_c2s[3 * 6 * 5];
 
 namespace {
 
@@ -54,7 +52,7 @@ constexpr int kThreads = 128;
 std::mutex g_boysMutex;
 bool g_boysReady[64] = {};
 
-// The Boys table and the c2s transformations on the current GPU (once per device) from ensure_boys.
+// The Boys table on the current GPU (once per device).
 int ensure_boys() {
     int device = 0;
     XQ_CHECK(hipGetDevice(&device));
@@ -64,9 +62,6 @@ int ensure_boys() {
     std::vector<double> t;
     boys_table(t);
     XQ_CHECK(hipMemcpyToSymbol(HIP_SYMBOL(g_boys), t.data(), t.size() * sizeof(double)));
-    double c2s[90];
-    c2s_table(c2s);
-    XQ_CHECK(hipMemcpyToSymbol(HIP_SYMBOL(g_c2s), c2s, sizeof(c2s)));
     g_boysReady[device] = true;
     return kOK;
 }
@@ -137,15 +132,28 @@ __global__ void __launch_bounds__(256) nuclear_kernel(int nPairs, const PairItem
 }
 
 // ------------------------------------------------------------------------------------------------------------------------
-// Fit matrix: (C|D) for fit shell pairs C >= D, one thread each; the fit functions' integrals in the last row.
+// Fit matrix: its integrals are the electron-fit integrals of pairs of a fit shell with the unit shell (qs_kernels.h), dense
+// with the fit functions' stored columns; here the lower triangle is packed, with the functions' own integrals in the last
+// row.  One thread per entry, and per fit shell.
 // ------------------------------------------------------------------------------------------------------------------------
-__global__ void __launch_bounds__(kThreads) fit_matrix_kernel(int nPairs, const QPair *__restrict__ pairs,
-                                                              const QShell *__restrict__ shells,
-                                                              const double *__restrict__ exps,
-                                                              const double *__restrict__ coefs, int nFit, int spherical,
-                                                              double *__restrict__ M) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < nPairs) fit_matrix_pair(k, pairs, shells, exps, coefs, nFit, spherical, g_boys, g_c2s, M);
+__global__ void __launch_bounds__(256) fit_matrix_pack_kernel(int nFit, const double *__restrict__ dense,
+                                                              const int *__restrict__ column, double *__restrict__ M) {
+    const int q = blockIdx.x * 256 + threadIdx.x;
+    for (int p = blockIdx.y; p < nFit; p += gridDim.y)
+        if (q <= p) M[packed_index(p, q)] = dense[static_cast<size_t>(p) * nFit + column[q]];
+}
+
+template <int LA>
+__global__ void __launch_bounds__(kThreads) fit_charges_kernel(int nShells, const PairItem *__restrict__ items,
+                                                               const QShell *__restrict__ shells,
+                                                               const double *__restrict__ exps,
+                                                               const double *__restrict__ coefs, int spherical,
+                                                               double *__restrict__ charges) {
+    const int k = blockIdx.x * kThreads + threadIdx.x;
+    if (k >= nShells) return;
+    const QShell A = shells[items[k].a];
+    overlap_kinetic<LA, 0>(A, shells[items[k].b], exps, coefs, spherical,
+                           [&](int i, int, double s, double) { charges[A.f0 + i] = s; });
 }
 
 // ------------------------------------------------------------------------------------------------------------------------
@@ -247,7 +255,8 @@ struct qs_basis : qs::QBasis {
 struct qs_fit {
     int nFit = 0, nOrbital = 0;
     long long rows = 0, nPairs = 0;
-    std::vector<qs::QPair> fitPairs;
+    qs::FitLaunch launch = {};         // the fit shells and functions in the order of the columns
+    qs::QShell *d_fitSorted = nullptr;
     std::vector<int> column;           // stored column of each fit function
     std::vector<double> host;          // b and c in the order of the columns
     const qs_basis *orbital = nullptr, *fit = nullptr;
@@ -278,34 +287,6 @@ int qs_alloc(T **p, size_t n) {
 template <typename T>
 void qs_release(T **p) {
     if (*p != nullptr) { (void)xq::cache_free(*p); *p = nullptr; }
-}
-
-// The fit matrix kernel holds its McMurchie-Davidson tables in private memory (3.7 KB per lane), and the runtime gives every hardware queue that runs one its own scratch area sized for the whole
-// device.  Two such kernels in flight at once on two queues (set-up threads of a request loop) made the second queue's
-// scratch allocation fail (HSA_STATUS_ERROR_OUT_OF_RESOURCES, queue abort), so at most one of them runs at a time in
-// the process: each holds this lock from its launch until its stream has drained.  The same allocation fails when the
-// device is nearly full (a request loop's caching allocator holds idle blocks), so each launch first makes sure that
-// kScratchHeadroom bytes are free.
-std::mutex g_integralKernels;
-constexpr size_t kScratchHeadroom = static_cast<size_t>(6) << 30;
-// The runtime's scratch areas belong to hardware queues and come from a pool of fixed size, separate from the free
-// device memory: several queues that each ran one of these kernels held areas sized for a whole-device dispatch and a
-// further request failed with HSA_STATUS_ERROR_OUT_OF_RESOURCES with 217 GB free.  So every launch of them goes to one
-// stream per device (one queue, one area), and no launch is larger than kSliceThreads threads, which bounds the area a
-// dispatch asks for.
-constexpr int kMaxDevices = 64;
-hipStream_t g_integralStream[kMaxDevices] = {};
-constexpr long long kSliceThreads = 2048LL * 64;
-
-// The integral stream of the current device (created on first use); the caller holds g_integralKernels.
-int integral_stream(hipStream_t *out) {
-    int dev = 0;
-    XQ_CHECK(hipGetDevice(&dev));
-    if (dev < 0 || dev >= kMaxDevices) { set_error("device index out of range"); return kInvalidArgument; }
-    if (g_integralStream[dev] == nullptr)
-        XQ_CHECK(hipStreamCreateWithFlags(&g_integralStream[dev], hipStreamNonBlocking));
-    *out = g_integralStream[dev];
-    return kOK;
 }
 
 // Shell pairs sorted by class, and where each class starts; doubles of all their records.
@@ -383,14 +364,20 @@ int qs_basis_create(int nAtoms, const int *Z, const double *xyzBohr, int nSpec, 
     int status = kOK;
     if (!err.empty()) { set_error(err); status = kInvalidArgument; }
     if (status == kOK) status = check(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking), "hipStreamCreate");
-    if (status == kOK) status = qs_alloc(&b->d_shells, b->shells.size());
-    if (status == kOK) status = qs_alloc(&b->d_exps, b->exps.size());
-    if (status == kOK) status = qs_alloc(&b->d_coefs, b->coefs.size());
-    if (status == kOK) status = check(hipMemcpyAsync(b->d_shells, b->shells.data(), b->shells.size() * sizeof(QShell),
+    // On the device the unit shell and its primitive follow the basis's own.
+    std::vector<QShell> shells(b->shells);
+    std::vector<double> exps(b->exps), coefs(b->coefs);
+    shells.push_back(unit_shell(static_cast<int>(exps.size())));
+    exps.push_back(0.0);
+    coefs.push_back(1.0);
+    if (status == kOK) status = qs_alloc(&b->d_shells, shells.size());
+    if (status == kOK) status = qs_alloc(&b->d_exps, exps.size());
+    if (status == kOK) status = qs_alloc(&b->d_coefs, coefs.size());
+    if (status == kOK) status = check(hipMemcpyAsync(b->d_shells, shells.data(), shells.size() * sizeof(QShell),
                                                      hipMemcpyHostToDevice, b->stream), "copy shells");
-    if (status == kOK) status = check(hipMemcpyAsync(b->d_exps, b->exps.data(), b->exps.size() * sizeof(double),
+    if (status == kOK) status = check(hipMemcpyAsync(b->d_exps, exps.data(), exps.size() * sizeof(double),
                                                      hipMemcpyHostToDevice, b->stream), "copy exponents");
-    if (status == kOK) status = check(hipMemcpyAsync(b->d_coefs, b->coefs.data(), b->coefs.size() * sizeof(double),
+    if (status == kOK) status = check(hipMemcpyAsync(b->d_coefs, coefs.data(), coefs.size() * sizeof(double),
                                                      hipMemcpyHostToDevice, b->stream), "copy coefficients");
     if (status == kOK) status = check(hipStreamSynchronize(b->stream), "copy basis");
     if (status != kOK) { qs_basis_free(b); return status; }
@@ -433,30 +420,24 @@ int qs_one_electron(qs_basis *basis, double *S, double *T, double *V) {
     if (status == kOK) status = qs_alloc(&d_S, size);
     if (status == kOK) status = qs_alloc(&d_T, size);
     if (status == kOK) status = qs_alloc(&d_V, size);
-    {
-        std::lock_guard<std::mutex> lock(g_integralKernels);
-        hipStream_t s = nullptr;
-        if (status == kOK) status = integral_stream(&s);
-        if (status == kOK) status = check(hipMemcpyAsync(d_items, set.items.data(), set.items.size() * sizeof(PairItem),
-                                                         hipMemcpyHostToDevice, s), "copy pairs");
-        if (status == kOK) status = check(hipMemcpyAsync(d_atoms, atoms.data(), atoms.size() * sizeof(double),
-                                                         hipMemcpyHostToDevice, s), "copy atoms");
-        if (status == kOK) status = launch_records(basis, set, d_items, d_records, s);
-        if (status == kOK)
-            status = for_classes(set, d_items, "one-electron kernels", [&](auto la, auto lb, PairItem *items, int n) {
-                hipLaunchKernelGGL((overlap_kinetic_kernel<la, lb>), groups(n, kThreads), dim3(kThreads), 0, s, n, items,
-                                   basis->d_shells, basis->d_exps, basis->d_coefs, basis->spherical, d_S, d_T);
-                hipLaunchKernelGGL((nuclear_kernel<la, lb>), groups(n, 4), dim3(256), 0, s, n, items, basis->d_shells,
-                                   d_records, basis->nAtoms, d_atoms, basis->spherical, d_V);
-            });
-        if (status == kOK) status = check(hipMemcpyAsync(S, d_S, size * sizeof(double), hipMemcpyDeviceToHost, s), "copy S");
-        if (status == kOK) status = check(hipMemcpyAsync(T, d_T, size * sizeof(double), hipMemcpyDeviceToHost, s), "copy T");
-        if (status == kOK) status = check(hipMemcpyAsync(V, d_V, size * sizeof(double), hipMemcpyDeviceToHost, s), "copy V");
-        if (s != nullptr) {
-            const int drained = check(hipStreamSynchronize(s), "one-electron integrals");
-            if (status == kOK) status = drained;
-        }
-    }
+    hipStream_t s = basis->stream;
+    if (status == kOK) status = check(hipMemcpyAsync(d_items, set.items.data(), set.items.size() * sizeof(PairItem),
+                                                     hipMemcpyHostToDevice, s), "copy pairs");
+    if (status == kOK) status = check(hipMemcpyAsync(d_atoms, atoms.data(), atoms.size() * sizeof(double),
+                                                     hipMemcpyHostToDevice, s), "copy atoms");
+    if (status == kOK) status = launch_records(basis, set, d_items, d_records, s);
+    if (status == kOK)
+        status = for_classes(set, d_items, "one-electron kernels", [&](auto la, auto lb, PairItem *items, int n) {
+            hipLaunchKernelGGL((overlap_kinetic_kernel<la, lb>), groups(n, kThreads), dim3(kThreads), 0, s, n, items,
+                               basis->d_shells, basis->d_exps, basis->d_coefs, basis->spherical, d_S, d_T);
+            hipLaunchKernelGGL((nuclear_kernel<la, lb>), groups(n, 4), dim3(256), 0, s, n, items, basis->d_shells,
+                               d_records, basis->nAtoms, d_atoms, basis->spherical, d_V);
+        });
+    if (status == kOK) status = check(hipMemcpyAsync(S, d_S, size * sizeof(double), hipMemcpyDeviceToHost, s), "copy S");
+    if (status == kOK) status = check(hipMemcpyAsync(T, d_T, size * sizeof(double), hipMemcpyDeviceToHost, s), "copy T");
+    if (status == kOK) status = check(hipMemcpyAsync(V, d_V, size * sizeof(double), hipMemcpyDeviceToHost, s), "copy V");
+    const int drained = check(hipStreamSynchronize(s), "one-electron integrals");
+    if (status == kOK) status = drained;
     qs_release(&d_items);
     qs_release(&d_records);
     qs_release(&d_atoms);
@@ -477,6 +458,7 @@ void qs_fit_free(qs_fit *fit) {
     qs_release(&fit->d_b);
     qs_release(&fit->d_c);
     qs_release(&fit->d_partial);
+    qs_release(&fit->d_fitSorted);
     if (fit->stream) (void)hipStreamDestroy(fit->stream);
     delete fit;
 }
@@ -516,7 +498,9 @@ int qs_fit_create(const qs_basis *orbital, const qs_basis *fitBasis, qs_fit **ou
     // by function of the shell, then by shell.
     std::vector<QShell> fitSorted(fitBasis->shells);
     std::stable_sort(fitSorted.begin(), fitSorted.end(), [](const QShell &u, const QShell &v) { return u.l < v.l; });
-    FitLaunch launch{};
+    FitLaunch &launch = F->launch;     // records and B differ between the set-up and the fit matrix
+    launch.stream = F->stream;
+    launch.cut = kUnderFlow;
     launch.oShells = orbital->d_shells;
     launch.oSpherical = orbital->spherical;
     launch.fSpherical = fitBasis->spherical;
@@ -537,7 +521,6 @@ int qs_fit_create(const qs_basis *orbital, const qs_basis *fitBasis, qs_fit **ou
     }
     PairItem *d_items = nullptr;
     double *d_records = nullptr;
-    QShell *d_fitSorted = nullptr;
     if (status == kOK) status = qs_alloc(&F->d_B, static_cast<size_t>(rows) * F->nFit);
     if (status == kOK) status = qs_alloc(&F->d_rowPacked, rowPacked.size());
     if (status == kOK) status = qs_alloc(&F->d_rowDiag, rowDiag.size());
@@ -548,10 +531,12 @@ int qs_fit_create(const qs_basis *orbital, const qs_basis *fitBasis, qs_fit **ou
     if (status == kOK) status = qs_alloc(&F->d_partial, static_cast<size_t>(nChunks > 0 ? nChunks : 1) * F->nFit);
     if (status == kOK) status = qs_alloc(&d_items, set.items.size());
     if (status == kOK) status = qs_alloc(&d_records, static_cast<size_t>(set.doubles));
-    if (status == kOK) status = qs_alloc(&d_fitSorted, fitSorted.empty() ? 1 : fitSorted.size());
+    if (status == kOK) status = qs_alloc(&F->d_fitSorted, fitSorted.size());
     if (status == kOK && !fitSorted.empty())
-        status = check(hipMemcpy(d_fitSorted, fitSorted.data(), fitSorted.size() * sizeof(QShell), hipMemcpyHostToDevice),
+        status = check(hipMemcpy(F->d_fitSorted, fitSorted.data(), fitSorted.size() * sizeof(QShell), hipMemcpyHostToDevice),
                        "copy fit shells");
+    launch.fShells = F->d_fitSorted;
+    if (status == kOK) status = boys_address(&launch.boys);
     if (status == kOK && rows > 0) {
         status = check(hipMemcpy(F->d_rowPacked, rowPacked.data(), rowPacked.size() * sizeof(long long),
                                  hipMemcpyHostToDevice), "copy rows");
@@ -559,30 +544,20 @@ int qs_fit_create(const qs_basis *orbital, const qs_basis *fitBasis, qs_fit **ou
                                           "copy rows");
         if (status == kOK) status = check(hipMemcpy(d_items, set.items.data(), set.items.size() * sizeof(PairItem),
                                                     hipMemcpyHostToDevice), "copy pairs");
-        std::lock_guard<std::mutex> lock(g_integralKernels);
-        hipStream_t is = nullptr;
-        if (status == kOK) status = integral_stream(&is);
-        if (status == kOK) status = launch_records(orbital, set, d_items, d_records, is);
-        launch.stream = is;
+        if (status == kOK) status = launch_records(orbital, set, d_items, d_records, F->stream);
         launch.records = d_records;
-        launch.fShells = d_fitSorted;
         launch.B = F->d_B;
-        if (status == kOK) status = boys_address(&launch.boys);
         if (status == kOK)
             status = for_classes(set, d_items, "fit_integrals_kernel", [&](auto la, auto lb, PairItem *items, int n) {
                 launch_fit<la, lb, 0>(launch, items, n);
                 launch_fit<la, lb, 1>(launch, items, n);
                 launch_fit<la, lb, 2>(launch, items, n);
             });
-        if (is != nullptr) {
-            const int drained = check(hipStreamSynchronize(is), "fit integrals");
-            if (status == kOK) status = drained;
-        }
+        const int drained = check(hipStreamSynchronize(F->stream), "fit integrals");
+        if (status == kOK) status = drained;
     }
     qs_release(&d_items);
     qs_release(&d_records);
-    qs_release(&d_fitSorted);
-    if (status == kOK) F->fitPairs = shell_pairs(fitBasis, false);
     if (status != kOK) { qs_fit_free(F); return status; }
     *out = F;
     return kOK;
@@ -590,35 +565,65 @@ int qs_fit_create(const qs_basis *orbital, const qs_basis *fitBasis, qs_fit **ou
 
 int qs_fit_matrix(qs_fit *fit, double *M) {
     if (fit == nullptr || M == nullptr) { set_error("invalid fit matrix arguments"); return kInvalidArgument; }
-    const size_t n = static_cast<size_t>(fit->nFit) + 1, size = n * (n + 1) / 2;
-    double *d_M = nullptr;
-    QPair *d_pairs = nullptr;
-    int status = qs_alloc(&d_M, size);
-    if (status == kOK) status = qs_alloc(&d_pairs, fit->fitPairs.size());
-    if (status == kOK) status = check(hipMemcpy(d_pairs, fit->fitPairs.data(), fit->fitPairs.size() * sizeof(QPair),
-                                                hipMemcpyHostToDevice), "copy fit pairs");
-    {
-        std::lock_guard<std::mutex> lock(g_integralKernels);
-        hipStream_t is = nullptr;
-        if (status == kOK) status = integral_stream(&is);
-        if (status == kOK) status = check(hipMemsetAsync(d_M, 0, size * sizeof(double), is), "clear M");
-        if (status == kOK && !fit->fitPairs.empty()) status = xq::ensure_free_device_memory(kScratchHeadroom, "fit matrix");
-        const long long nPairs = static_cast<long long>(fit->fitPairs.size());
-        for (long long k0 = 0; status == kOK && k0 < nPairs; k0 += kSliceThreads) {
-            const long long m = std::min<long long>(kSliceThreads, nPairs - k0);
-            hipLaunchKernelGGL(fit_matrix_kernel, dim3(static_cast<unsigned>((m + kThreads - 1) / kThreads)),
-                               dim3(kThreads), 0, is, static_cast<int>(m), d_pairs + k0, fit->fit->d_shells,
-                               fit->fit->d_exps, fit->fit->d_coefs, fit->nFit, fit->fit->spherical, d_M);
-            status = check(hipGetLastError(), "fit_matrix_kernel");
-        }
-        if (is != nullptr) {
-            const int drained = check(hipStreamSynchronize(is), "fit matrix");
-            if (status == kOK) status = drained;
-        }
+    const size_t nFit = static_cast<size_t>(fit->nFit), size = (nFit + 1) * (nFit + 2) / 2;
+    const qs_basis *basis = fit->fit;
+    // One pair of every fit shell with the unit shell; a shell's rows are its functions.
+    std::vector<QPair> pairs(basis->shells.size());
+    std::vector<long long> row(pairs.size());
+    for (size_t k = 0; k < pairs.size(); k++) {
+        pairs[k] = QPair{static_cast<int>(k), static_cast<int>(basis->shells.size())};
+        row[k] = basis->shells[k].f0;
     }
+    QBasis withUnit;
+    withUnit.shells = basis->shells;
+    withUnit.shells.push_back(unit_shell(static_cast<int>(basis->exps.size())));
+    const PairSet set = pair_set(&withUnit, pairs, row);
+    PairItem *d_items = nullptr;
+    double *d_records = nullptr, *d_dense = nullptr, *d_M = nullptr;
+    int *d_column = nullptr;
+    const hipStream_t s = fit->stream;
+    int status = qs_alloc(&d_M, size);
+    if (status == kOK) status = qs_alloc(&d_dense, nFit * nFit);
+    if (status == kOK) status = qs_alloc(&d_column, nFit);
+    if (status == kOK) status = qs_alloc(&d_items, set.items.size());
+    if (status == kOK) status = qs_alloc(&d_records, static_cast<size_t>(set.doubles));
+    if (status == kOK) status = check(hipMemcpyAsync(d_items, set.items.data(), set.items.size() * sizeof(PairItem),
+                                                     hipMemcpyHostToDevice, s), "copy fit shells");
+    if (status == kOK) status = check(hipMemcpyAsync(d_column, fit->column.data(), nFit * sizeof(int),
+                                                     hipMemcpyHostToDevice, s), "copy columns");
+    if (status == kOK) status = launch_records(basis, set, d_items, d_records, s);
+    FitLaunch launch = fit->launch;
+    launch.oShells = basis->d_shells;
+    launch.oSpherical = basis->spherical;
+    launch.records = d_records;
+    launch.cut = -1.0;
+    launch.B = d_dense;
+    if (status == kOK)
+        status = for_classes(set, d_items, "fit matrix kernels", [&](auto la, auto lb, PairItem *items, int n) {
+            if constexpr (lb == 0) {     // the unit shell is the second of every pair
+                launch_fit<la, 0, 0>(launch, items, n);
+                launch_fit<la, 0, 1>(launch, items, n);
+                launch_fit<la, 0, 2>(launch, items, n);
+                hipLaunchKernelGGL(fit_charges_kernel<la>, groups(n, kThreads), dim3(kThreads), 0, s, n, items,
+                                   basis->d_shells, basis->d_exps, basis->d_coefs, basis->spherical,
+                                   d_M + nFit * (nFit + 1) / 2);
+            }
+        });
+    if (status == kOK && nFit > 0) {
+        hipLaunchKernelGGL(fit_matrix_pack_kernel, dim3(static_cast<unsigned>((nFit + 255) / 256),
+                                                        static_cast<unsigned>(std::min<size_t>(nFit, 65535))),
+                           dim3(256), 0, s, fit->nFit, d_dense, d_column, d_M);
+        status = check(hipGetLastError(), "fit_matrix_pack_kernel");
+    }
+    const int drained = check(hipStreamSynchronize(s), "fit matrix");
+    if (status == kOK) status = drained;
     if (status == kOK) status = check(hipMemcpy(M, d_M, size * sizeof(double), hipMemcpyDeviceToHost), "copy M");
+    if (status == kOK) M[size - 1] = 0.0;      // the constraint's own entry
     qs_release(&d_M);
-    qs_release(&d_pairs);
+    qs_release(&d_dense);
+    qs_release(&d_column);
+    qs_release(&d_items);
+    qs_release(&d_records);
     return status;
 }
 

@@ -49,29 +49,6 @@ constexpr double kUnderFlow = 1.0e-12;    // electron-fit integrals dropped by t
 constexpr double kNuclearWidth = 1.0e-4;
 constexpr double kNuclearExponent = 4.0 / (kNuclearWidth * kNuclearWidth * M_PI);
 
-// Cartesian factor of component c of angular momentum l: sqrt((2l-1)!! / ((2x-1)!! (2y-1)!! (2z-1)!!)).
-QS_HD double cart_factor(int l, int c) {
-    int x, y, z;
-    cart_powers(l, c, x, y, z);
-    auto of = [](int m) { double f = 1.0; for (int i = 3; i <= m; i += 2) f *= i; return f; };
-    return sqrt(of(2 * l - 1) / (of(2 * x - 1) * of(2 * y - 1) * of(2 * z - 1)));
-}
-
-// Transform a Cartesian block in place along one index: [outer][ncart(l)][inner] -> [outer][2l+1][inner]; c2s holds
-// the transformation of l = 0..2 as [l][6][5].  Used only when the basis is spherical.
-QS_HD void to_spherical(int l, const double *c2s, double *blk, int outer, int inner, double *tmp) {
-    const int nc = ncart(l), ns = 2 * l + 1;
-    for (int o = 0; o < outer; o++)
-        for (int i = 0; i < inner; i++) {
-            for (int s = 0; s < ns; s++) {
-                double v = 0.0;
-                for (int c = 0; c < nc; c++) v += c2s[(l * 6 + c) * 5 + s] * blk[(o * nc + c) * inner + i];
-                tmp[s] = v;
-            }
-            for (int s = 0; s < ns; s++) blk[(o * ns + s) * inner + i] = tmp[s];
-        }
-}
-
 QS_HD long long packed_index(int i, int j) {
     return i >= j ? static_cast<long long>(i) * (i + 1) / 2 + j : static_cast<long long>(j) * (j + 1) / 2 + i;
 }
@@ -95,6 +72,9 @@ QS_HD constexpr Powers powers_of(int l, int c) {
     return Powers{0, 0, 0};
 }
 QS_HD constexpr int cartesians(int l) { return (l + 1) * (l + 2) / 2; }
+// Cartesian factor of component c of angular momentum l: sqrt((2l-1)!! / ((2x-1)!! (2y-1)!! (2z-1)!!)), which is sqrt(3) for
+// xy, xz and yz and 1 otherwise (l <= 2).
+QS_HD constexpr double cart_factor(int l, int c) { return l == 2 && (c == 1 || c == 3 || c == 4) ? 1.7320508075688772935 : 1.0; }
 
 // Hermite coefficients of a pair of the class: component pair ab = (ia, ib) has (x + 1)(y + 1)(z + 1) of them, x, y and z
 // the summed powers, from at[ab]; size is the doubles of a record (p, 1 / p, P, coefficients).  The tables are constants
@@ -516,85 +496,19 @@ inline long long record_room(const QShell &A, const QShell &B) {
     return size * A.nPrim * B.nPrim;
 }
 
+// The unit function as an s shell whose one primitive, of exponent 0 and coefficient 1, is at prim: a pair with it is the
+// other shell alone.
+inline QShell unit_shell(int prim) {
+    QShell u{};
+    u.nPrim = 1;
+    u.prim = prim;
+    u.nf = 1;
+    return u;
+}
+
 // Row of function i of the first role and j of the second (mb functions of the pair's second shell B).
 QS_HD long long pair_row(const PairItem &it, int i, int j, int ma, int mb) {
     return it.row + (it.swapped ? static_cast<long long>(j) * ma + i : static_cast<long long>(i) * mb + j);
-}
-
-// (C|D) of fit shell pair k (C >= D) into the packed fit matrix; the diagonal pair also writes its functions' integrals
-// into row nFit.
-QS_HD void fit_matrix_pair(int k, const QPair *__restrict__ pairs, const QShell *__restrict__ shells,
-                           const double *__restrict__ exps, const double *__restrict__ coefs, int nFit, int spherical,
-                           const double *__restrict__ boysTable, const double *__restrict__ c2s, double *__restrict__ M) {
-    const QShell C = shells[pairs[k].x], D = shells[pairs[k].y];
-    const int nc = ncart(C.l), nd = ncart(D.l);
-    double blk[36], tmp[6], Gc[3][9], Gd[3][9], R[kRD * kRD * kRD];
-    for (int i = 0; i < 36; i++) blk[i] = 0.0;
-    for (int qc = 0; qc < C.nPrim; qc++)
-        for (int qd = 0; qd < D.nPrim; qd++) {
-            const double g = exps[C.prim + qc], d = exps[D.prim + qd];
-            const double alpha = g * d / (g + d);
-            const double pref = 2.0 * pow(M_PI, 2.5) / (g * d * sqrt(g + d)) * coefs[C.prim + qc] * coefs[D.prim + qd];
-            for (int dim = 0; dim < 3; dim++) { hermite_single(C.l, g, Gc[dim]); hermite_single(D.l, d, Gd[dim]); }
-            hermite_r(C.l + D.l, alpha, C.x - D.x, C.y - D.y, C.z - D.z, boysTable, R);
-            for (int ic = 0; ic < nc; ic++) {
-                int xc, yc, zc;
-                cart_powers(C.l, ic, xc, yc, zc);
-                for (int id = 0; id < nd; id++) {
-                    int xd, yd, zd;
-                    cart_powers(D.l, id, xd, yd, zd);
-                    double acc = 0.0;
-                    for (int t1 = 0; t1 <= xc; t1++)
-                        for (int u1 = 0; u1 <= yc; u1++)
-                            for (int v1 = 0; v1 <= zc; v1++) {
-                                const double e1 = Gc[0][xc * 3 + t1] * Gc[1][yc * 3 + u1] * Gc[2][zc * 3 + v1];
-                                if (e1 == 0.0) continue;
-                                for (int t2 = 0; t2 <= xd; t2++)
-                                    for (int u2 = 0; u2 <= yd; u2++)
-                                        for (int v2 = 0; v2 <= zd; v2++) {
-                                            const double e2 = Gd[0][xd * 3 + t2] * Gd[1][yd * 3 + u2] * Gd[2][zd * 3 + v2];
-                                            const double sg = ((t2 + u2 + v2) & 1) ? -1.0 : 1.0;
-                                            acc += e1 * e2 * sg * R[ridx(t1 + t2, u1 + u2, v1 + v2)];
-                                        }
-                            }
-                    blk[ic * nd + id] += pref * cart_factor(C.l, ic) * cart_factor(D.l, id) * acc;
-                }
-            }
-        }
-    int mc = nc, md = nd;
-    if (spherical) {
-        to_spherical(C.l, c2s, blk, 1, nd, tmp);
-        to_spherical(D.l, c2s, blk, 2 * C.l + 1, 1, tmp);
-        mc = 2 * C.l + 1;
-        md = 2 * D.l + 1;
-    }
-    for (int i = 0; i < mc; i++)
-        for (int j = 0; j < md; j++) {
-            const int p = C.f0 + i, q = D.f0 + j;
-            if (p < q) continue;
-            M[packed_index(p, q)] = blk[i * md + j];
-        }
-    // The fit functions' integrals (int chi_P dr) into row nFit, computed by the diagonal pair's thread.
-    if (pairs[k].x == pairs[k].y) {
-        double ov[6];
-        for (int ic = 0; ic < nc; ic++) {
-            int x, y, z;
-            cart_powers(C.l, ic, x, y, z);
-            double acc = 0.0;
-            for (int q = 0; q < C.nPrim; q++) {
-                const double g = exps[C.prim + q];
-                double G[9];
-                hermite_single(C.l, g, G);
-                acc += coefs[C.prim + q] * pow(M_PI / g, 1.5) * G[x * 3] * G[y * 3] * G[z * 3];
-            }
-            ov[ic] = acc * cart_factor(C.l, ic);
-        }
-        if (spherical) {
-            to_spherical(C.l, c2s, ov, 1, 1, tmp);
-            mc = 2 * C.l + 1;
-        }
-        for (int i = 0; i < mc; i++) M[packed_index(nFit, C.f0 + i)] = ov[i];
-    }
 }
 
 // ------------------------------------------------------------------------------------------------------------------------
@@ -620,6 +534,43 @@ inline void one_electron_pair(int k, const QPair *pairs, const QShell *shells, c
         pair_functions<la, lb, 1>(spherical, acc);
         for_functions<la, lb>(spherical, [&](int i, int j, auto ab) { at(V, i, j) = acc[ab][0]; });
     });
+}
+
+// (C|D) of fit shell pair k (C >= D) into the packed fit matrix; the diagonal pair also writes its functions' integrals into
+// row nFit.  C is taken as a pair with the unit shell.
+inline void fit_matrix_pair(int k, const QPair *pairs, const QShell *shells, const double *exps, const double *coefs, int nFit,
+                            int spherical, const double *boysTable, const double *, double *M) {
+    QShell C = shells[pairs[k].x];
+    const QShell &D = shells[pairs[k].y];
+    std::vector<double> e(exps + C.prim, exps + C.prim + C.nPrim), c(coefs + C.prim, coefs + C.prim + C.nPrim);
+    C.prim = 0;
+    const QShell unit = unit_shell(C.nPrim);
+    e.push_back(0.0);
+    c.push_back(1.0);
+    std::vector<double> records(static_cast<size_t>(record_room(C, unit)));
+    auto left = [&](auto la) {
+        const int n = pair_records<la, 0>(C, unit, e.data(), c.data(), records.data());
+        auto item = [&](auto lc, auto m0) {
+            constexpr int NM = fit_group<la, 0, lc>(), M0 = m0;
+            double acc[PairClass<la, 0>::na][NM];
+            fit_block<la, 0, lc, M0, NM>(records.data(), n, D, exps, coefs, boysTable, acc);
+            pair_functions<la, 0, NM>(spherical, acc);
+            for_functions<la, 0>(spherical, [&](int i, int, auto ab) {
+                fit_functions<lc, M0, NM>(spherical, acc[ab], [&](int f, double x) { M[packed_index(C.f0 + i, D.f0 + f)] = x; });
+            });
+        };
+        using std::integral_constant;
+        const integral_constant<int, 0> zero;
+        if (D.l == 0) item(zero, zero);
+        else if (D.l == 1) item(integral_constant<int, 1>{}, zero);
+        else item(integral_constant<int, 2>{}, zero);
+        if (pairs[k].x == pairs[k].y)
+            overlap_kinetic<la, 0>(C, unit, e.data(), c.data(), spherical,
+                                   [&](int i, int, double s, double) { M[packed_index(nFit, C.f0 + i)] = s; });
+    };
+    if (C.l == 0) left(std::integral_constant<int, 0>{});
+    else if (C.l == 1) left(std::integral_constant<int, 1>{});
+    else left(std::integral_constant<int, 2>{});
 }
 
 // (mu nu|P) of item k = (significant orbital shell pair k / nFitShells, fit shell k % nFitShells) into its rows of B

@@ -44,9 +44,9 @@ inline void boys_table(std::vector<double> &t) {
 inline void c2s_table(double *t) {
     for (int k = 0; k < 90; k++) t[k] = 0.0;
     for (int l = 0; l <= 2; l++) {
-        std::vector<double> m(static_cast<size_t>(ncart(l)) * (2 * l + 1), 0.0);
+        std::vector<double> m(static_cast<size_t>(cartesians(l)) * (2 * l + 1), 0.0);
         xq::c2s_block(l, m.data(), 2 * l + 1, 0, 0);
-        for (int c = 0; c < ncart(l); c++)
+        for (int c = 0; c < cartesians(l); c++)
             for (int sI = 0; sI < 2 * l + 1; sI++) t[(l * 6 + c) * 5 + sI] = m[static_cast<size_t>(c) * (2 * l + 1) + sI];
     }
 }
@@ -86,7 +86,7 @@ inline std::string build_shells(QBasis *b, int nSpec, const double *spec) {
                 sh.nPrim = np;
                 sh.prim = static_cast<int>(b->exps.size());
                 sh.f0 = f;
-                sh.nf = b->spherical ? 2 * l + 1 : ncart(l);
+                sh.nf = b->spherical ? 2 * l + 1 : cartesians(l);
                 sh.atom = a;
                 for (int q = 0; q < np; q++) {
                     const double alpha = spec[p + q * rowLen];

@@ -134,22 +134,4 @@ void cache_release() {
     release_cached_locked();
 }
 
-int ensure_free_device_memory(size_t bytes, const char *what) {
-    size_t freeB = 0, totalB = 0;
-    if (hipMemGetInfo(&freeB, &totalB) != hipSuccess) {
-        set_error(std::string(what) + ": hipMemGetInfo failed");
-        return kAlgorithmError;
-    }
-    if (freeB >= bytes) return kOK;
-    cache_release();   // idle blocks of the cache go back to the device
-    if (hipMemGetInfo(&freeB, &totalB) != hipSuccess) {
-        set_error(std::string(what) + ": hipMemGetInfo failed");
-        return kAlgorithmError;
-    }
-    if (freeB >= bytes) return kOK;
-    set_error(std::string(what) + ": " + std::to_string(freeB >> 20) + " MiB of device memory free, " +
-              std::to_string(bytes >> 20) + " MiB needed for the kernel's private memory");
-    return kOutOfMemory;
-}
-
 }  // namespace xq

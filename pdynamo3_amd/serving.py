@@ -189,8 +189,7 @@ class Server:
         self.energy_tolerance = energy_tolerance
         self.density_tolerance = density_tolerance
         if hbm_budget is None:
-            # 90% of the free memory, less room for the runtime's own allocations: the private memory of the SCF
-            # integral kernels (a few GB per launch) is allocated by the runtime at dispatch.
+            # 90% of the free memory, less room for the runtime's own allocations and the set-ups' temporary ones.
             free, _ = integrator.device_memory()
             hbm_budget = max(int(0.9 * free) - (16 << 30), int(0.5 * free))
         self.hbm_budget = int(hbm_budget)

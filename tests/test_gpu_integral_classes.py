@@ -78,3 +78,31 @@ def test_def2_svp_equals_the_host_work_items(spherical):
         g.fit_fock(np.eye(g.n_fit)[k], F)
         assert np.max(np.abs(F - D[:, k])) < 1.1e-12
     g.close()
+
+
+@pytest.mark.parametrize("waters", [1, 7])
+def test_cartesian_fit_matrix_contains_the_spherical_one(waters):
+    """Fit functions of one launch block of the packing kernel and of one and a part; 36 products of entries up to 1e2."""
+    from perf import cases
+    from pdynamo3_amd import basis, densities, scf
+    Z, xyz, spec, _ = cases._molecules(cases._case("integrals", waters), 3)[0]
+    fit = basis.load_basis(cases.FIT)
+    f = basis.element_spec(fit, Z)
+    M = {}
+    for spherical in (True, False):
+        g = scf.GPUIntegrals(Z, xyz, spec, True, f, spherical)
+        full = np.zeros((g.n_fit + 1, g.n_fit + 1))
+        full[np.tril_indices(g.n_fit + 1)] = g.fit_matrix()
+        M[spherical] = full + np.tril(full, -1).T
+        g.close()
+    T = np.zeros((M[False].shape[0], M[True].shape[0]))
+    at, to = 0, 0
+    for z in Z:
+        for shell in fit["elements"][str(int(z))]["shells"]:
+            for l in range(shell["lLow"], shell["lHigh"] + 1):
+                t = densities.c2s(l)
+                T[at:at + t.shape[0], to:to + t.shape[1]] = t
+                at, to = at + t.shape[0], to + t.shape[1]
+    T[at, to] = 1.0
+    assert (at + 1, to + 1) == T.shape
+    assert np.max(np.abs(T.T @ M[False] @ T - M[True])) < 1e-10
