@@ -159,18 +159,55 @@ __device__ __forceinline__ double becke_poly(double nu) {
     return sum;
 }
 
-template <int GS>
-__device__ __forceinline__ double group_sum(double x) {
-#pragma unroll
-    for (int o = GS / 2; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
+// Reductions over groups of GS = 16, 32 or 64 lanes, every lane receiving the result.  The lane exchanges are register
+// moves (DPP within a row of 16 lanes, row and half swaps above): with shuffles through the LDS crossbar, six dependent ones
+// per reduction, the weight derivatives of (H2O)64 took 24 ms instead of 20, its grid weights 14 instead of 12.
+template <int kControl>
+__device__ __forceinline__ unsigned row_move(unsigned x) {
+    return static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), kControl, 0xf, 0xf, true));
+}
+template <int kControl>
+__device__ __forceinline__ double row_move(double x) {
+    return __hiloint2double(static_cast<int>(row_move<kControl>(static_cast<unsigned>(__double2hiint(x)))),
+                            static_cast<int>(row_move<kControl>(static_cast<unsigned>(__double2loint(x)))));
+}
+// The even and the odd rows of 16 lanes (kRows = 1), or the halves of the wave (kRows = 2), each in place of both.
+template <int kRows>
+__device__ __forceinline__ void spread(unsigned x, unsigned &even, unsigned &odd) {
+    if constexpr (kRows == 1) {
+        const auto p = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+        even = p[0];
+        odd = p[1];
+    } else {
+        const auto p = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+        even = p[0];
+        odd = p[1];
+    }
+}
+template <int kRows>
+__device__ __forceinline__ void spread(double x, double &even, double &odd) {
+    unsigned eh, oh, el, ol;
+    spread<kRows>(static_cast<unsigned>(__double2hiint(x)), eh, oh);
+    spread<kRows>(static_cast<unsigned>(__double2loint(x)), el, ol);
+    even = __hiloint2double(static_cast<int>(eh), static_cast<int>(el));
+    odd = __hiloint2double(static_cast<int>(oh), static_cast<int>(ol));
+}
+template <int GS, class T, class Op>
+__device__ __forceinline__ T group_reduce(T x, Op op) {
+    static_assert(GS == 16 || GS == 32 || GS == 64, "groups of whole rows");
+    x = op(x, row_move<0xB1>(x));       // lanes 1, 0, 3, 2 of each four
+    x = op(x, row_move<0x4E>(x));       // lanes 2, 3, 0, 1
+    x = op(x, row_move<0x141>(x));      // each eight lanes reversed
+    x = op(x, row_move<0x140>(x));      // each sixteen lanes reversed
+    T even, odd;
+    if constexpr (GS >= 32) { spread<1>(x, even, odd); x = op(even, odd); }
+    if constexpr (GS == 64) { spread<2>(x, even, odd); x = op(even, odd); }
     return x;
 }
 template <int GS>
-__device__ __forceinline__ double group_product(double x) {
-#pragma unroll
-    for (int o = GS / 2; o > 0; o >>= 1) x *= __shfl_xor(x, o, 64);
-    return x;
-}
+__device__ __forceinline__ double group_sum(double x) { return group_reduce<GS>(x, [](double u, double v) { return u + v; }); }
+template <int GS>
+__device__ __forceinline__ double group_product(double x) { return group_reduce<GS>(x, [](double u, double v) { return u * v; }); }
 
 // LDS writes of a wave are in order; this keeps the compiler from moving accesses over it.
 __device__ __forceinline__ void wave_fence() {
@@ -184,19 +221,42 @@ __device__ __forceinline__ unsigned long long group_ballot(bool x, int bit0) {
     return (__ballot(x) >> bit0) & (GS == 64 ? ~0ull : ((1ull << (GS & 63)) - 1ull));
 }
 
-// The atom (lane atoms gl + GS a, not done) of the largest bound of a group, and that bound (-1 if all are done).
+// The atom (lane atoms gl + GS a, not done) of the largest bound of a group by the bounds' upper words, and that bound or
+// the next larger double with these upper words (0 if all are done or vanish).
 template <int LA, int GS>
 __device__ __forceinline__ int next_atom(const double (&b)[LA], const bool (&done)[LA], int gl, int bit0, double &top) {
-    double best = -1.0;
-    int bi = 0;
+    unsigned best = 0u;
+    int bi = gl;
 #pragma unroll
-    for (int a = 0; a < LA; a++)
-        if (!done[a] && b[a] > best) { best = b[a]; bi = gl + GS * a; }
-    top = best;
-#pragma unroll
-    for (int o = GS / 2; o > 0; o >>= 1) top = fmax(top, __shfl_xor(top, o, 64));
-    return __shfl(bi, bit0 + __ffsll(static_cast<long long>(group_ballot<GS>(best == top, bit0))) - 1, 64);
+    for (int a = 0; a < LA; a++) {
+        const unsigned key = done[a] ? 0u : static_cast<unsigned>(__double2hiint(b[a]));
+        if (key > best) { best = key; bi = gl + GS * a; }
+    }
+    const unsigned most = group_reduce<GS>(best, [](unsigned u, unsigned v) { return u > v ? u : v; });
+    top = most == 0u ? 0.0 : __hiloint2double(static_cast<int>(most), -1);
+    const int first = __ffsll(static_cast<long long>(group_ballot<GS>(best == most, bit0))) - 1;
+    if constexpr (GS == 64) return __builtin_amdgcn_readlane(bi, first);
+    else return __shfl(bi, bit0 + first, 64);
 }
+
+// The pairs of atom c with the lane atoms.  With up to four atoms per lane they are loaded when c is known, before the
+// reductions that end the row before; more would cost too many registers, and are read in place.
+template <int LA, int GS>
+struct PairRow {
+    static constexpr int kAhead = LA <= 4 ? LA : 1;
+    const double2 *__restrict__ row;
+    double2 q[kAhead];
+    __device__ __forceinline__ void load(const double2 *__restrict__ pairs, int c, int gl, int nAtoms) {
+        row = pairs + static_cast<size_t>(c) * nAtoms + gl;
+        if constexpr (kAhead == LA)
+#pragma unroll
+            for (int a = 0; a < LA; a++) q[a] = gl + GS * a < nAtoms ? row[GS * a] : make_double2(0.0, 0.0);
+    }
+    __device__ __forceinline__ double2 operator[](int a) const {
+        if constexpr (kAhead == LA) return q[a];
+        else return row[GS * a];
+    }
+};
 
 // Share of the largest cell product at a point below which an atom's product does not count: in the sum of the products, and
 // in the derivatives, where a factor s = c y^11 P (y = 1 - nu) near its zero has a derivative of 11 s / y, so that a dropped
@@ -213,7 +273,7 @@ constexpr double kCellScreen = 0x1p-64;
 // polynomial are exact negatives).  The shell's points are dealt to gridDim.y work-groups.
 // Bound by FP64 arithmetic (45 operations a factor).  One point per thread, whose lanes lay in all directions from A and
 // so took nearly every factor of every atom between them, took 7.4 ms on (H2O)24 and 48 ms on (H2O)64; this
-// takes 4.6 and 14 ms.
+// takes 2.7 and 11 ms.  Each row's pairs are fetched before the product that ends the row before.
 template <int LA, int GS, int WPG>
 __global__ void __launch_bounds__(64 * WPG) candidate_points_kernel(const RadialShell *__restrict__ shells,
                                                                     const double *__restrict__ rules,
@@ -254,32 +314,36 @@ __global__ void __launch_bounds__(64 * WPG) candidate_points_kernel(const Radial
         wave_fence();
         bool run = active;
         int c = A;
-        double PA = 0.0, sum = 0.0, most = 0.0;
+        double PA = 0.0, sum = 0.0, most = 0.0, rc = rL[A];
+        PairRow<LA, GS> row;
+        row.load(pairs, c, gl, nAtoms);
         do {
-            const double rc = rL[c];
             double prod = 1.0;
 #pragma unroll
             for (int a = 0; a < LA; a++) {
                 const int i = gl + GS * a;
                 if (i >= nAtoms || i == c) continue;
-                const double2 q = pairs[static_cast<size_t>(c) * nAtoms + i];
+                const double2 q = row[a];
                 const double mu = (rc - r[a]) * q.x, nu = mu + q.y * (1.0 - mu * mu), S = kBeckeA * becke_poly(nu);
                 prod *= 0.5 - S;
                 b[a] *= fabs(0.5 + S);
             }
-            prod = group_product<GS>(prod);
-            if (run) {
-                if (c == A) PA = prod;
-                sum += prod;
-                most = fmax(most, fabs(prod));
+            const bool first = c == A;
 #pragma unroll
-                for (int a = 0; a < LA; a++) done[a] = done[a] || gl + GS * a == c;
-                // A point whose weight cannot exceed half the cull tolerance with the products so far is culled.
-                run = PA != 0.0 && !(sum > 0.0 && fabs(wru) * (fabs(PA) / sum) < 0.5 * kWeightTol);
-            }
+            for (int a = 0; a < LA; a++) done[a] = done[a] || gl + GS * a == c;
             double top;
             c = next_atom<LA, GS>(b, done, gl, bit0, top);
-            run = run && top >= kCellScreen * most && top > 0.0;
+            rc = rL[c];
+            row.load(pairs, c, gl, nAtoms);
+            prod = group_product<GS>(prod);
+            if (run) {
+                if (first) PA = prod;
+                sum += prod;
+                most = fmax(most, fabs(prod));
+                // A point whose weight cannot exceed half the cull tolerance with the products so far is culled.
+                run = PA != 0.0 && !(sum > 0.0 && fabs(wru) * (fabs(PA) / sum) < 0.5 * kWeightTol) &&
+                      top >= kCellScreen * most && top > 0.0;
+            }
         } while (__any(run));
         if (active && gl == 0) {
             const int o = sh.out + k;
@@ -433,11 +497,12 @@ __device__ __forceinline__ double reciprocal(double x) {
 //   Derivatives.  For each m whose c_m passes the screen, one row of pair terms: a pair of two such atoms is met from both
 //   sides and gives each side's own atom its force; a pair with another atom k (c_k = 0) gives both forces at once.
 //   The point moves with g, and its force is what makes the sum of a point's forces vanish.
-// Bound by FP64 arithmetic (about 35 operations a factor, 70 a pair term) and the wave reductions of each row.  Groups of 16
+// Bound by FP64 arithmetic (about 35 operations a factor, 70 a pair term, 4,300 instructions a point of (H2O)64: the vector
+// units are busy for nine tenths of the time); a row's pairs are fetched while the row before is reduced.  Groups of 16
 // and 32 lanes keep small molecules' lanes busy.  pairs[m][k] = {1 / R_mk, a_mk} (square, so that a row is read in order;
 // a_km = -a_mk).  LDS: the coordinates, and per group each atom's distance and c.
 // Against one point a wave with bounds from the 24 atoms nearest g and a screen on products without their smallest factor
-// (which kept several times the atoms): (H2O)64, 2.4 million points, 102 -> 24 ms; (H2O)5, four points a wave, 2.5 -> 0.26 ms.
+// (which kept several times the atoms): (H2O)64, 2.4 million points, 102 -> 19 ms; (H2O)5, four points a wave, 2.5 -> 0.19 ms.
 template <int LA, int GS, int WPG>
 __global__ void __launch_bounds__(64 * WPG) weight_gradient_kernel(int nPoints,
                                                               const double *__restrict__ px, const double *__restrict__ py,
@@ -483,16 +548,17 @@ __global__ void __launch_bounds__(64 * WPG) weight_gradient_kernel(int nPoints,
             done[a] = i >= nAtoms;
         }
         wave_fence();
+        PairRow<LA, GS> row;
+        row.load(pairs, g, gl, nAtoms);
         // A_g from the cell factors as the weight w was made from them (candidate_points_kernel): deep in another atom's cell
         // they are rounding, and w with them.
-        double made = 1.0;
-        const double rg = rL[g];
+        double made = 1.0, rc = rL[g];
 #pragma unroll
         for (int a = 0; a < LA; a++) {
             const int i = gl + GS * a;
             if (i >= nAtoms || i == g) continue;
-            const double2 q = pairs[static_cast<size_t>(g) * nAtoms + i];
-            const double mu = (rg - r[a]) * q.x;
+            const double2 q = row[a];
+            const double mu = (rc - r[a]) * q.x;
             made *= 0.5 - kBeckeA * becke_poly(mu + q.y * (1.0 - mu * mu));
         }
         made = group_product<GS>(made);
@@ -501,28 +567,32 @@ __global__ void __launch_bounds__(64 * WPG) weight_gradient_kernel(int nPoints,
         int c = g;
         double most = 0.0;
         do {
-            const double rc = rL[c];
             double prod = 1.0;
 #pragma unroll
             for (int a = 0; a < LA; a++) {
                 const int i = gl + GS * a;
                 if (i >= nAtoms || i == c) continue;
-                const double2 q = pairs[static_cast<size_t>(c) * nAtoms + i];
+                const double2 q = row[a];
                 const double mu = (rc - r[a]) * q.x, nu = fma(q.y, fma(-mu, mu, 1.0), mu), n = fabs(nu);
                 const double small = becke_small(n, fmax(1.0 - n, 0.0)), large = 1.0 - small;
                 prod *= nu > 0.0 ? small : large;
                 b[a] *= nu > 0.0 ? large : small;
             }
+            const int taken = c;
+#pragma unroll
+            for (int a = 0; a < LA; a++) done[a] = done[a] || gl + GS * a == taken;
+            double top;
+            c = next_atom<LA, GS>(b, done, gl, bit0, top);
+            rc = rL[c];
+            row.load(pairs, c, gl, nAtoms);
             prod = group_product<GS>(prod);
             if (run) {
                 most = fmax(most, prod);
 #pragma unroll
                 for (int a = 0; a < LA; a++)
-                    if (gl + GS * a == c) { A[a] = prod; done[a] = true; }
+                    if (gl + GS * a == taken) A[a] = prod;
+                run = top >= kCellScreen * most && top > 0.0;
             }
-            double top;
-            c = next_atom<LA, GS>(b, done, gl, bit0, top);
-            run = run && top >= kCellScreen * most && top > 0.0;
         } while (__any(run));
         // c_m; that of g from the others' share, which keeps its accuracy where g's cell holds almost all.
         double others = 0.0, own = 0.0;
@@ -551,59 +621,66 @@ __global__ void __launch_bounds__(64 * WPG) weight_gradient_kernel(int nPoints,
         double ir[LA], gs[3] = {0.0, 0.0, 0.0};
 #pragma unroll
         for (int a = 0; a < LA; a++) ir[a] = gl + GS * a < nAtoms ? reciprocal(r[a]) : 0.0;
-#pragma unroll 1
-        for (int a2 = 0; a2 < LA; a2++) {
-            unsigned long long mk = 0ull;
+        // The next atom m of a group, -1 after the last.
+        auto take = [&]() {
+            int m = -1;
 #pragma unroll
             for (int a = 0; a < LA; a++)
-                if (a == a2) mk = maskK[a];
-            while (__any(mk != 0ull)) {
-                const bool some = mk != 0ull;
-                const int m = some ? GS * a2 + __ffsll(static_cast<long long>(mk)) - 1 : 0;
-                mk &= mk - 1ull;
-                const double xm = sxyz[3 * m], ym = sxyz[3 * m + 1], zm = sxyz[3 * m + 2], rm = rL[m];
-                const double cm = some ? cL[m] : 0.0, irm = reciprocal(rm);
-                const double ex = (xm - rx) * irm, ey = (ym - ry) * irm, ez = (zm - rz) * irm;
-                double h[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-                for (int a = 0; a < LA; a++) {
-                    const int k = gl + GS * a;
-                    if (k >= nAtoms || k == m || !some) continue;
-                    const double2 q = pairs[static_cast<size_t>(m) * nAtoms + k];
-                    const double mu = (rm - r[a]) * q.x, nu = fma(q.y, fma(-mu, mu, 1.0), mu), n = fabs(nu);
-                    const double y = fmax(1.0 - n, 0.0), small = becke_small(n, y), large = 1.0 - small;
-                    const double smk = nu > 0.0 ? small : large, skm = nu > 0.0 ? large : small;
-                    // 1 - nu^2 = y (2 - y); dnu / dmu = 1 - 2 a mu.
-                    const double u = y * (2.0 - y), u2 = u * u, u4 = u2 * u2;
-                    const double d = kBeckeA * (u4 * u4 * u2) * fma(-2.0 * q.y, mu, 1.0) * (cf[a] * smk - cm * skm) *
-                                     reciprocal(fmax(small * large, 0x1p-1000));
-                    // d mu_mk / d r_k = -e_k / R - mu (r_k - r_m) / R^2, d mu_mk / d r_m = e_m / R + mu (r_k - r_m) / R^2.
-                    const double al = d * q.x, be = al * q.x * mu, ak = al * ir[a];
-                    const double xk = sxyz[3 * k], yk = sxyz[3 * k + 1], zk = sxyz[3 * k + 2];
-                    const double bx = be * (xk - xm), by = be * (yk - ym), bz = be * (zk - zm);
-                    const double fx = -fma(ak, xk - rx, bx), fy = -fma(ak, yk - ry, by), fz = -fma(ak, zk - rz, bz);
-                    G[a][0] += fx;
-                    G[a][1] += fy;
-                    G[a][2] += fz;
-                    gs[0] += fx;
-                    gs[1] += fy;
-                    gs[2] += fz;
-                    if (cf[a] == 0.0) {
-                        h[0] += fma(al, ex, bx);
-                        h[1] += fma(al, ey, by);
-                        h[2] += fma(al, ez, bz);
-                    }
+                if (m < 0 && maskK[a] != 0ull) {
+                    m = GS * a + __ffsll(static_cast<long long>(maskK[a])) - 1;
+                    maskK[a] &= maskK[a] - 1ull;
                 }
+            return m;
+        };
+        int next = take();
+        row.load(pairs, next < 0 ? 0 : next, gl, nAtoms);
+        while (__any(next >= 0)) {
+            const bool some = next >= 0;
+            const int m = some ? next : 0;
+            const double xm = sxyz[3 * m], ym = sxyz[3 * m + 1], zm = sxyz[3 * m + 2], rm = rL[m];
+            const double cm = some ? cL[m] : 0.0, irm = reciprocal(rm);
+            const double ex = (xm - rx) * irm, ey = (ym - ry) * irm, ez = (zm - rz) * irm;
+            double h[3] = {0.0, 0.0, 0.0};
 #pragma unroll
-                for (int x = 0; x < 3; x++) h[x] = group_sum<GS>(h[x]);
-                if (some && gl == (m & (GS - 1))) {
-#pragma unroll
-                    for (int a = 0; a < LA; a++)
-                        if (a == a2) { G[a][0] += h[0]; G[a][1] += h[1]; G[a][2] += h[2]; }
-                    gs[0] += h[0];
-                    gs[1] += h[1];
-                    gs[2] += h[2];
+            for (int a = 0; a < LA; a++) {
+                const int k = gl + GS * a;
+                if (k >= nAtoms || k == m || !some) continue;
+                const double2 q = row[a];
+                const double mu = (rm - r[a]) * q.x, nu = fma(q.y, fma(-mu, mu, 1.0), mu), n = fabs(nu);
+                const double y = fmax(1.0 - n, 0.0), small = becke_small(n, y), large = 1.0 - small;
+                const double smk = nu > 0.0 ? small : large, skm = nu > 0.0 ? large : small;
+                // 1 - nu^2 = y (2 - y); dnu / dmu = 1 - 2 a mu.
+                const double u = y * (2.0 - y), u2 = u * u, u4 = u2 * u2;
+                const double d = kBeckeA * (u4 * u4 * u2) * fma(-2.0 * q.y, mu, 1.0) * (cf[a] * smk - cm * skm) *
+                                 reciprocal(fmax(small * large, 0x1p-1000));
+                // d mu_mk / d r_k = -e_k / R - mu (r_k - r_m) / R^2, d mu_mk / d r_m = e_m / R + mu (r_k - r_m) / R^2.
+                const double al = d * q.x, be = al * q.x * mu, ak = al * ir[a];
+                const double xk = sxyz[3 * k], yk = sxyz[3 * k + 1], zk = sxyz[3 * k + 2];
+                const double bx = be * (xk - xm), by = be * (yk - ym), bz = be * (zk - zm);
+                const double fx = -fma(ak, xk - rx, bx), fy = -fma(ak, yk - ry, by), fz = -fma(ak, zk - rz, bz);
+                G[a][0] += fx;
+                G[a][1] += fy;
+                G[a][2] += fz;
+                gs[0] += fx;
+                gs[1] += fy;
+                gs[2] += fz;
+                if (cf[a] == 0.0) {
+                    h[0] += fma(al, ex, bx);
+                    h[1] += fma(al, ey, by);
+                    h[2] += fma(al, ez, bz);
                 }
+            }
+            next = take();
+            row.load(pairs, next < 0 ? 0 : next, gl, nAtoms);
+#pragma unroll
+            for (int x = 0; x < 3; x++) h[x] = group_sum<GS>(h[x]);
+            if (some && gl == (m & (GS - 1))) {
+#pragma unroll
+                for (int a = 0; a < LA; a++)
+                    if (a == m / GS) { G[a][0] += h[0]; G[a][1] += h[1]; G[a][2] += h[2]; }
+                gs[0] += h[0];
+                gs[1] += h[1];
+                gs[2] += h[2];
             }
         }
 #pragma unroll
@@ -734,9 +811,10 @@ int build_grid(xq_grid *g) {
         if ((status = check(hipMemcpyAsync(d_atomFirst, atomFirst.data(), atomFirst.size() * sizeof(int),
                                            hipMemcpyHostToDevice, s), "copy atoms")) != kOK) break;
         if (!shells.empty()) {
-            // A shell's points go to enough work-groups to fill the chip (8 x 256 of them), at most one round each.
+            // A shell's points go to several work-groups (at most one per round of points), some 32768 in all: their costs
+            // differ, and with 2048 the chip stood idle for a third of the kernel ((H2O)24: 4.0 ms against 2.7).
             const unsigned rounds = static_cast<unsigned>((lebedev_size_for_l(65) * group + 64 * wpg - 1) / (64 * wpg));
-            const unsigned split = std::min<unsigned>(rounds, static_cast<unsigned>(2048 / shells.size()) + 1);
+            const unsigned split = std::min<unsigned>(rounds, static_cast<unsigned>(32768 / shells.size()) + 1);
             auto launch = [&](auto kernel) {
                 hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(shells.size()), split), dim3(64 * wpg), lds, s,
                                    d_shells, d_rules, d_xyz, nA, d_pairs, cx, cy, cz, cw, keep);
@@ -864,7 +942,8 @@ int weight_gradients(xq_grid *g, const double *d_eXC, double *d_grad, hipStream_
                             "copy xyz")) != kOK) break;
         if ((status = check(hipMemcpyAsync(d_pointAtom, pointAtom.data(), pointAtom.size() * sizeof(int),
                                            hipMemcpyHostToDevice, s), "copy point atoms")) != kOK) break;
-        const int nGroups = std::min(2048 * 4 / wpg, (G + 63) / 64);
+        // Enough work-groups to even their costs out ((H2O)64: 19.9 ms with 2048, 18.9 with 8192).
+        const int nGroups = std::min(8192 * 4 / wpg, (G + 63) / 64);
         auto launch = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(nGroups), dim3(64 * wpg), lds, s, G, g->d_x, g->d_y, g->d_z,
                                g->d_w, d_pointAtom, d_eXC, d_xyz, nA, d_pairs, d_grad);
