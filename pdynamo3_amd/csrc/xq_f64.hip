@@ -20,6 +20,7 @@
 #include <hip/hip_runtime.h>
 
 #include <climits>
+#include <type_traits>
 #include <vector>
 
 #include "xq_functional.h"
@@ -81,12 +82,14 @@ __global__ void __launch_bounds__(256) f64_prepare_kernel(
 // X = P_red Phi for the chunk's 32 rows on FP64 MFMA (2 x 2 MFMA tiles per wave), then the chunk's share of rho and grad rho
 // at the block's points, stored in part[chunk][4][point]; density_functional_kernel (xq_mixed.hip) sums the shares.  Each
 // step multiplies one 32 x 32 chunk of P_red, gathered by all threads and staged in one of two LDS buffers (one barrier per
-// step), with the matching Phi chunk, whose operands go straight to registers; both are fetched one step ahead.  The row
+// step), with the matching Phi chunk, whose operands go straight to registers; the words of P_red are fetched one step
+// ahead, and each Phi operand for the next step as soon as its products of this step are issued, into the same registers:
+// four work-groups per CU instead of three with a second set of operand registers (3.62 ms against 4.13).  The row
 // chunks of a block are consecutive items of one XCD, so that Phi comes from HBM about once per block.
-// Bound by the FP64 matrix cores and the gathers' latency.  One work-group per block, which read Phi once per row chunk from
-// HBM and waited for each panel of gathers, took 8.26 ms on (H2O)64 (1.3e11 operations, 9.6 GB); this
-// takes 4.13 ms and the functional 0.21 ms.
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
+// Bound by HBM (Phi and grad Phi once, 10.7 GB on (H2O)64, and the gathers of P_red) and the FP64 matrix cores (busy for
+// half of the time).  One work-group per block, which read Phi once per row chunk from HBM and waited for each panel of
+// gathers, took 8.26 ms on (H2O)64 (1.3e11 operations); this takes 3.62 ms and the functional 0.21 ms.
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
 density_rows_kernel_f64(const MixedJob *__restrict__ jobs, int nJobs, int interleaved) {
     __shared__ double sP[2][kC][kRowPitch];
     __shared__ int sIdx[kIdxCache];
@@ -117,35 +120,34 @@ density_rows_kernel_f64(const MixedJob *__restrict__ jobs, int nJobs, int interl
     // Staging: row sr, columns 8 j + s8 (eight lanes read eight consecutive kept functions).
     const int sr = t >> 3, s8 = t & 7, r = kC * I + sr;
     const size_t rowOff = r < nb ? static_cast<size_t>(idx[r]) * n : 0;
-    double pv[4], bnext[8][2];
-    auto fetch = [&](int c) {
+    double pv[4], bq[8][2];
+    auto fetch_p = [&](int c) {
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const int k = kC * c + 8 * j + s8;
             pv[j] = r < nb && k < nb ? P[rowOff + idx[k]] : 0.0;
         }
+    };
+    const double *__restrict__ bp = FPB + C * kChunk + op(0, 0);    // operands of the chunk to fetch
+    auto fetch_b = [&](int s) {
 #pragma unroll
-        for (int s = 0; s < 8; s++)
-#pragma unroll
-            for (int h = 0; h < 2; h++) bnext[s][h] = FPB[(C + c) * kChunk + op(s, h)];
+        for (int h = 0; h < 2; h++) bq[s][h] = bp[(2 * s + h) * 64];
     };
     v4d acc[2][2];
 #pragma unroll
     for (int hm = 0; hm < 2; hm++)
 #pragma unroll
         for (int hn = 0; hn < 2; hn++) acc[hm][hn] = v4d{0.0, 0.0, 0.0, 0.0};
-    fetch(0);
-#pragma unroll 2
-    for (int c = 0; c < nChunks; c++) {
+    auto step = [&](int c, auto more) {
         double (&buf)[kC][kRowPitch] = sP[c & 1];
 #pragma unroll
         for (int j = 0; j < 4; j++) buf[sr][8 * j + s8] = pv[j];
-        double bq[8][2];
-#pragma unroll
-        for (int s = 0; s < 8; s++) { bq[s][0] = bnext[s][0]; bq[s][1] = bnext[s][1]; }
         // A wave writes this buffer again two steps on, after the next barrier, which every wave reaches done with it.
         __syncthreads();
-        if (c + 1 < nChunks) fetch(c + 1);
+        if constexpr (more) {
+            fetch_p(c + 1);
+            bp += kChunk;
+        }
 #pragma unroll
         for (int s = 0; s < 8; s++) {
             const double a0 = buf[l16][4 * s + l4], a1 = buf[16 + l16][4 * s + l4];
@@ -153,31 +155,36 @@ density_rows_kernel_f64(const MixedJob *__restrict__ jobs, int nJobs, int interl
             acc[0][1] = mfma_f64(a0, bq[s][1], acc[0][1]);
             acc[1][0] = mfma_f64(a1, bq[s][0], acc[1][0]);
             acc[1][1] = mfma_f64(a1, bq[s][1], acc[1][1]);
+            if constexpr (more) fetch_b(s);
         }
-    }
-    // Epilogue: register v of (hm, hn) is row 16 hm + 4 v + l / 16 of chunk I at point 32 wv + 16 hn + l % 16.
-    double pr[4][2] = {};
+    };
+    fetch_p(0);
 #pragma unroll
+    for (int s = 0; s < 8; s++) fetch_b(s);
+#pragma unroll 1
+    for (int c = 0; c + 1 < nChunks; c++) step(c, std::true_type{});
+    step(nChunks - 1, std::false_type{});
+    // Epilogue: register v of (hm, hn) is row 16 hm + 4 v + l / 16 of chunk I at point 32 wv + 16 hn + l % 16.
+    double *q = J.part + CI * 4 * kBlockSize;
+#pragma unroll 1
     for (int x = 0; x < 4; x++) {
-        const double *plane = x == 0 ? FPB + CI * kChunk : GPB + (3 * CI + (x - 1)) * kChunk;
+        const double *__restrict__ plane = (x == 0 ? FPB + CI * kChunk : GPB + (3 * CI + (x - 1)) * kChunk) + op(0, 0);
+        double pr[2] = {};
 #pragma unroll
         for (int hm = 0; hm < 2; hm++)
 #pragma unroll
             for (int v = 0; v < 4; v++)
 #pragma unroll
-                for (int hn = 0; hn < 2; hn++) pr[x][hn] += plane[op(4 * hm + v, hn)] * acc[hm][hn][v];
-    }
-    double *q = J.part + CI * 4 * kBlockSize;
+                for (int hn = 0; hn < 2; hn++) pr[hn] += plane[(2 * (4 * hm + v) + hn) * 64] * acc[hm][hn][v];
+        // Sum over the four lanes that share a point (l / 16 = 0..3).
 #pragma unroll
-    for (int hn = 0; hn < 2; hn++)
-#pragma unroll
-        for (int x = 0; x < 4; x++) {
-            // Sum over the four lanes that share a point (l / 16 = 0..3).
-            double e = pr[x][hn];
+        for (int hn = 0; hn < 2; hn++) {
+            double e = pr[hn];
             e += __shfl_xor(e, 16, 64);
             e += __shfl_xor(e, 32, 64);
             if (l4 == 0) q[x * kBlockSize + kC * wv + 16 * hn + l16] = e;
         }
+    }
 }
 
 // W (one chunk per work-group, 256 threads): W_rp = c0_p Phi_rp + c_p . grad Phi_rp from the density-order planes,

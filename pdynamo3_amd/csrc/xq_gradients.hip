@@ -22,6 +22,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 #include "xq_functional.h"
@@ -49,9 +50,10 @@ __device__ __forceinline__ v4d mfma_f64(double a, double b, const v4d &c) {
 // B[l / 16][l % 16] and receives D[4 v + l / 16][l % 16]).  256 threads; wave wv owns points 32 wv .. + 31 (two 16-point
 // tiles): acc[hm][hn][v] = (P_red Bp)[32 I + 16 hm + 4 v + l / 16][32 wv + 16 hn + l % 16].  Bp is the block's first row of
 // a plane of rows of 128 points (rows >= nb are not read).  Each step multiplies one 32 x 32 chunk of P_red, gathered by
-// all threads and staged in one of two LDS buffers (one barrier per step), with 32 rows of Bp; both are fetched one step
-// ahead.  Staged panels of four chunks, each waited for, took 7.2 ms (X pass) and 9.3 ms (Z pass) per call on
-// (H2O)64; this takes 4.1 and 6.1 ms.
+// all threads and staged in one of two LDS buffers (one barrier per step), with 32 rows of Bp; the words of P_red are
+// fetched one step ahead, each operand of Bp for the next step as soon as its products of this step are issued.  Staged
+// panels of four chunks, each waited for, took 7.2 ms (X pass) and 9.3 ms (Z pass) per call on (H2O)64; this takes 3.8 and
+// 5.9 ms.
 __device__ __forceinline__ void reduced_product(const double *__restrict__ P, int n, const int *idx, int nb,
                                                 const double *__restrict__ Bp, double (&sP)[2][kC][kRowPitch], int I,
                                                 v4d (&acc)[2][2]) {
@@ -60,37 +62,33 @@ __device__ __forceinline__ void reduced_product(const double *__restrict__ P, in
     // Staging: row sr, columns 8 j + s8 (eight lanes read eight consecutive kept functions).
     const int sr = t >> 3, s8 = t & 7, r = kC * I + sr;
     const size_t rowOff = r < nb ? static_cast<size_t>(idx[r]) * n : 0;
-    double pv[4], bnext[8][2];
-    auto fetch = [&](int c) {
+    double pv[4], bq[8][2];
+    auto fetch_p = [&](int c) {
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const int k = kC * c + 8 * j + s8;
             pv[j] = r < nb && k < nb ? P[rowOff + idx[k]] : 0.0;
         }
+    };
+    const double *__restrict__ bp = Bp + l4 * kBlockSize + kC * wv + l16;
+    auto fetch_b = [&](int c, int s) {
 #pragma unroll
-        for (int s = 0; s < 8; s++) {
-            const int k = kC * c + 4 * s + l4;
-#pragma unroll
-            for (int h = 0; h < 2; h++)
-                bnext[s][h] = k < nb ? Bp[static_cast<size_t>(k) * kBlockSize + kC * wv + 16 * h + l16] : 0.0;
-        }
+        for (int h = 0; h < 2; h++) bq[s][h] = kC * c + 4 * s + l4 < nb ? bp[4 * s * kBlockSize + 16 * h] : 0.0;
     };
 #pragma unroll
     for (int hm = 0; hm < 2; hm++)
 #pragma unroll
         for (int hn = 0; hn < 2; hn++) acc[hm][hn] = v4d{0.0, 0.0, 0.0, 0.0};
-    fetch(0);
-#pragma unroll 2
-    for (int c = 0; c < nChunks; c++) {
+    auto step = [&](int c, auto more) {
         double (&buf)[kC][kRowPitch] = sP[c & 1];
 #pragma unroll
         for (int j = 0; j < 4; j++) buf[sr][8 * j + s8] = pv[j];
-        double bq[8][2];
-#pragma unroll
-        for (int s = 0; s < 8; s++) { bq[s][0] = bnext[s][0]; bq[s][1] = bnext[s][1]; }
         // A wave writes this buffer again two steps on, after the next barrier, which every wave reaches done with it.
         __syncthreads();
-        if (c + 1 < nChunks) fetch(c + 1);
+        if constexpr (more) {
+            fetch_p(c + 1);
+            bp += kC * kBlockSize;
+        }
 #pragma unroll
         for (int s = 0; s < 8; s++) {
             const double a0 = buf[l16][4 * s + l4], a1 = buf[16 + l16][4 * s + l4];
@@ -98,8 +96,15 @@ __device__ __forceinline__ void reduced_product(const double *__restrict__ P, in
             acc[0][1] = mfma_f64(a0, bq[s][1], acc[0][1]);
             acc[1][0] = mfma_f64(a1, bq[s][0], acc[1][0]);
             acc[1][1] = mfma_f64(a1, bq[s][1], acc[1][1]);
+            if constexpr (more) fetch_b(c + 1, s);
         }
-    }
+    };
+    fetch_p(0);
+#pragma unroll
+    for (int s = 0; s < 8; s++) fetch_b(0, s);
+#pragma unroll 1
+    for (int c = 0; c + 1 < nChunks; c++) step(c, std::true_type{});
+    step(nChunks - 1, std::false_type{});
 }
 
 // XCD ranges of a launch: XCD x takes entries start[x] .. start[x + 1] - 1 of its list.
