@@ -160,30 +160,38 @@ __global__ void __launch_bounds__(kThreads) fit_charges_kernel(int nShells, cons
 // Per SCF iteration: b = sum_rows w_row P_row B_row (partial sums over row chunks, then a fixed-order reduction) and
 // F_row += B_row . c (one wave per row).  w_row = 2 off the diagonal, 1 on it, 0 for a duplicate row.
 // ------------------------------------------------------------------------------------------------------------------------
-constexpr int kRowChunk = 256;
+constexpr int kRowChunk = 1024;
 
-// Partial sums of b over kRowChunk rows: a thread per fit function, the rows' weights w_row P_row gathered once into LDS and
-// the rows' loads independent of each other.  Bound by reading the integrals: 1.7 GB on (H2O)48 in 0.29 ms, against 0.61
-// with chunks of 1,024 rows whose every load waited for the row's index and density; on (H2O)16, which had too few
-// chunks to fill the chip, 0.37 -> 0.02 ms.
-__global__ void __launch_bounds__(256) fit_b_partial_kernel(long long rows, int nFit, const double *__restrict__ B,
-                                                           const long long *__restrict__ rowPacked,
-                                                           const unsigned char *__restrict__ rowDiag,
-                                                           const double *__restrict__ P, double *__restrict__ partial) {
+// Partial sums of b over kRowChunk rows: 16 waves per work-group, each 64 rows and the same 64 fit functions, their sums
+// added in order.  The rows' weights w_row P_row are gathered once into LDS, so that the rows' loads are independent of
+// each other.  Bound by reading the integrals: 1.7 GB on (H2O)48 in 0.29 ms, against 0.61 with a thread for 1,024 rows,
+// whose every load waited for the row's index and density, and on (H2O)16, whose chunks then were too few to
+// fill the chip, 0.02 ms against 0.37.
+__global__ void __launch_bounds__(1024) fit_b_partial_kernel(long long rows, int nFit, const double *__restrict__ B,
+                                                            const long long *__restrict__ rowPacked,
+                                                            const unsigned char *__restrict__ rowDiag,
+                                                            const double *__restrict__ P, double *__restrict__ partial) {
     __shared__ double sw[kRowChunk];
+    __shared__ double sums[16][64];
     const long long r0 = static_cast<long long>(blockIdx.y) * kRowChunk;
     const int n = static_cast<int>(rows - r0 < kRowChunk ? rows - r0 : kRowChunk);
-    for (int k = threadIdx.x; k < n; k += 256) {
+    for (int k = threadIdx.x; k < n; k += 1024) {
         const long long o = rowPacked[r0 + k];
         sw[k] = o < 0 ? 0.0 : (rowDiag[r0 + k] ? 1.0 : 2.0) * P[o];
     }
     __syncthreads();
-    const int col = blockIdx.x * 256 + threadIdx.x;
-    if (col >= nFit) return;
-    const double *row = B + r0 * nFit + col;
+    const int c = threadIdx.x & 63, wv = threadIdx.x >> 6, col = blockIdx.x * 64 + c;
+    const int k0 = wv * (kRowChunk / 16), k1 = k0 + kRowChunk / 16 < n ? k0 + kRowChunk / 16 : n;
     double acc = 0.0;
+    if (col < nFit) {
+        const double *row = B + r0 * nFit + col;
 #pragma unroll 8
-    for (int k = 0; k < n; k++) acc = fma(sw[k], row[static_cast<size_t>(k) * nFit], acc);
+        for (int k = k0; k < k1; k++) acc = fma(sw[k], row[static_cast<size_t>(k) * nFit], acc);
+    }
+    sums[wv][c] = acc;
+    __syncthreads();
+    if (wv != 0 || col >= nFit) return;
+    for (int k = 1; k < 16; k++) acc += sums[k][c];
     partial[static_cast<size_t>(blockIdx.y) * nFit + col] = acc;
 }
 
@@ -634,7 +642,7 @@ int qs_fit_b(qs_fit *fit, const double *P, double *b) {
     hipStream_t s = fit->stream;
     XQ_CHECK(hipMemcpyAsync(fit->d_P, P, nPacked * sizeof(double), hipMemcpyHostToDevice, s));
     if (nChunks > 0) {
-        hipLaunchKernelGGL(fit_b_partial_kernel, dim3((fit->nFit + 255) / 256, nChunks), dim3(256), 0, s, fit->rows,
+        hipLaunchKernelGGL(fit_b_partial_kernel, dim3((fit->nFit + 63) / 64, nChunks), dim3(1024), 0, s, fit->rows,
                            fit->nFit, fit->d_B, fit->d_rowPacked, fit->d_rowDiag, fit->d_P, fit->d_partial);
         hipLaunchKernelGGL(fit_b_reduce_kernel, dim3((fit->nFit + 63) / 64), dim3(1024), 0, s, nChunks, fit->nFit,
                            fit->d_partial, fit->d_b);
@@ -683,16 +691,13 @@ int qs_fit_estimate_bytes(int nAtoms, const int *Z, const double *xyzBohr, int n
     std::string err = build_shells(&orb, nSpec, spec);
     if (err.empty()) err = build_shells(&fit, nFitSpec, fitSpec);
     if (!err.empty()) { set_error(err); return kInvalidArgument; }
-    // The arrays qs_fit_create allocates: the integrals (rows x nFit), the row maps, P, F, b, c, the partial sums of b, and
-    // the shell pairs' records during the set-up.
-    long long rows = 0, setup = 0;
-    for (const QPair &pq : shell_pairs(&orb, true)) {
+    // The arrays that stay: the integrals (rows x nFit), the row maps, P, F, b, c and the partial sums of b.
+    long long rows = 0;
+    for (const QPair &pq : shell_pairs(&orb, true))
         rows += static_cast<long long>(orb.shells[pq.x].nf) * orb.shells[pq.y].nf;
-        setup += 8 * record_room(orb.shells[pq.x], orb.shells[pq.y]) + static_cast<long long>(sizeof(PairItem));
-    }
     const long long nFit = fit.nFunctions, n = orb.nFunctions, nPacked = n * (n + 1) / 2;
     const long long nChunks = (rows + kRowChunk - 1) / kRowChunk;
-    *bytes = 8 * rows * nFit + 9 * rows + 16 * nPacked + 16 * nFit + 8 * (nChunks > 0 ? nChunks : 1) * nFit + setup;
+    *bytes = 8 * rows * nFit + 9 * rows + 16 * nPacked + 16 * nFit + 8 * (nChunks > 0 ? nChunks : 1) * nFit;
     return kOK;
 }
 
