@@ -4,8 +4,9 @@
 // quadratures run would stall them at every release.  Freed blocks are kept instead and handed out again: a request
 // takes the smallest cached block of at least its size and at most a quarter larger (sizes are rounded up to 512 bytes,
 // and to 2 MiB above 1 MiB), so a loop whose jobs come and go reuses device memory without runtime calls.  When
-// hipMalloc fails, every cached block is released (hipFree) and the allocation is tried once more.  A block is cached
-// only after the work that used it has completed: every caller synchronises the owning stream before it frees.
+// hipMalloc fails, every cached block is released (hipFree) and the allocation is tried once more; they are released as
+// well before an allocation that would leave less than kRuntimeBytes of free device memory.  A block is cached only after
+// the work that used it has completed: every caller synchronises the owning stream before it frees.
 // Pinned host blocks (the staging of P and V) are cached the same way, since hipHostFree synchronises the device too.
 #include <hip/hip_runtime.h>
 
@@ -29,6 +30,10 @@ size_t g_cachedBytes = 0;
 long long g_failAfter = -1;                        // test hook: allocations left before one fails (-1: none fails)
 std::multimap<size_t, void *> g_hostCached;        // pinned host blocks, as above
 std::unordered_map<void *, size_t> g_hostLive;
+
+// Device memory left to the runtime, which allocates the private memory of a kernel at its dispatch (rocSOLVER's kernels have
+// some) and aborts the process when it cannot: idle blocks must not hold it.
+constexpr size_t kRuntimeBytes = size_t(6) << 30;
 
 size_t rounded(size_t bytes) {
     if (bytes == 0) bytes = 1;
@@ -59,6 +64,9 @@ hipError_t cache_alloc(void **ptr, size_t bytes) {
         g_cached.erase(it);
         return hipSuccess;
     }
+    size_t freeB = 0, totalB = 0;
+    if (!g_cached.empty() && hipMemGetInfo(&freeB, &totalB) == hipSuccess && freeB < size + kRuntimeBytes)
+        release_cached_locked();
     hipError_t e = hipMalloc(ptr, size);
     if (e != hipSuccess && !g_cached.empty()) {
         (void)hipGetLastError();
