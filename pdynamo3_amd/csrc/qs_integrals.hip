@@ -214,7 +214,11 @@ __global__ void __launch_bounds__(1024) fit_b_reduce_kernel(int nChunks, int nFi
     }
 }
 
-// F_row += B_row . c, four rows per wave: each value of c serves four loads.  Bound by reading the integrals ((H2O)48: one row
+__global__ void __launch_bounds__(256) zero_packed_kernel(size_t n, double *__restrict__ F) {
+    for (size_t k = blockIdx.x * 256ull + threadIdx.x; k < n; k += gridDim.x * 256ull) F[k] = 0.0;
+}
+
+// F_row = B_row . c, four rows per wave: each value of c serves four loads.  Bound by reading the integrals ((H2O)48: one row
 // per wave 0.37 ms, this 0.29 ms).
 constexpr int kFockRows = 4;
 
@@ -243,7 +247,7 @@ __global__ void __launch_bounds__(256) fit_fock_kernel(long long rows, int nFit,
 #pragma unroll
         for (int s = 32; s > 0; s >>= 1) acc[i] += __shfl_xor(acc[i], s, 64);
         const long long o = i < n ? rowPacked[r0 + i] : -1;
-        if (lane == 0 && o >= 0) F[o] += acc[i];
+        if (lane == 0 && o >= 0) F[o] = acc[i];
     }
 }
 
@@ -266,7 +270,7 @@ struct qs_fit {
     qs::FitLaunch launch = {};         // the fit shells and functions in the order of the columns
     qs::QShell *d_fitSorted = nullptr;
     std::vector<int> column;           // stored column of each fit function
-    std::vector<double> host;          // b and c in the order of the columns
+    double *staging = nullptr;         // pinned: b or c in the order of the columns (nFit), then packed P or F
     const qs_basis *orbital = nullptr, *fit = nullptr;
     double *d_B = nullptr;
     long long *d_rowPacked = nullptr;
@@ -467,6 +471,7 @@ void qs_fit_free(qs_fit *fit) {
     qs_release(&fit->d_c);
     qs_release(&fit->d_partial);
     qs_release(&fit->d_fitSorted);
+    if (fit->staging != nullptr) xq::cache_host_free(fit->staging);
     if (fit->stream) (void)hipStreamDestroy(fit->stream);
     delete fit;
 }
@@ -517,7 +522,6 @@ int qs_fit_create(const qs_basis *orbital, const qs_basis *fitBasis, qs_fit **ou
     launch.nFit = F->nFit;
     int *first = launch.first, *column = launch.column;
     F->column.resize(static_cast<size_t>(F->nFit));
-    F->host.resize(static_cast<size_t>(F->nFit));
     for (int l = 0; l <= kMaxL; l++) {
         int n = 0;
         while (first[l] + n < static_cast<int>(fitSorted.size()) && fitSorted[first[l] + n].l == l) n++;
@@ -540,6 +544,10 @@ int qs_fit_create(const qs_basis *orbital, const qs_basis *fitBasis, qs_fit **ou
     if (status == kOK) status = qs_alloc(&d_items, set.items.size());
     if (status == kOK) status = qs_alloc(&d_records, static_cast<size_t>(set.doubles));
     if (status == kOK) status = qs_alloc(&F->d_fitSorted, fitSorted.size());
+    if (status == kOK)
+        status = check(xq::cache_host_alloc(reinterpret_cast<void **>(&F->staging),
+                                            (static_cast<size_t>(F->nFit) + nOrbPacked) * sizeof(double) + 8),
+                       "hipHostMalloc");
     if (status == kOK && !fitSorted.empty())
         status = check(hipMemcpy(F->d_fitSorted, fitSorted.data(), fitSorted.size() * sizeof(QShell), hipMemcpyHostToDevice),
                        "copy fit shells");
@@ -639,36 +647,53 @@ int qs_fit_b(qs_fit *fit, const double *P, double *b) {
     if (fit == nullptr || P == nullptr || b == nullptr) { set_error("invalid fit arguments"); return kInvalidArgument; }
     const size_t nPacked = static_cast<size_t>(fit->nOrbital) * (fit->nOrbital + 1) / 2;
     const int nChunks = static_cast<int>((fit->rows + kRowChunk - 1) / kRowChunk);
+    if (nChunks == 0) {
+        for (int k = 0; k < fit->nFit; k++) b[k] = 0.0;
+        return kOK;
+    }
     hipStream_t s = fit->stream;
-    XQ_CHECK(hipMemcpyAsync(fit->d_P, P, nPacked * sizeof(double), hipMemcpyHostToDevice, s));
-    if (nChunks > 0) {
+    double *packed = fit->staging + fit->nFit;
+    xq::host_copy(packed, P, nPacked);
+    auto queue = [&]() -> int {
+        XQ_CHECK(hipMemcpyAsync(fit->d_P, packed, nPacked * sizeof(double), hipMemcpyHostToDevice, s));
         hipLaunchKernelGGL(fit_b_partial_kernel, dim3((fit->nFit + 63) / 64, nChunks), dim3(1024), 0, s, fit->rows,
                            fit->nFit, fit->d_B, fit->d_rowPacked, fit->d_rowDiag, fit->d_P, fit->d_partial);
         hipLaunchKernelGGL(fit_b_reduce_kernel, dim3((fit->nFit + 63) / 64), dim3(1024), 0, s, nChunks, fit->nFit,
                            fit->d_partial, fit->d_b);
         XQ_CHECK(hipGetLastError());
-        XQ_CHECK(hipMemcpyAsync(fit->host.data(), fit->d_b, fit->nFit * sizeof(double), hipMemcpyDeviceToHost, s));
-    }
-    XQ_CHECK(hipStreamSynchronize(s));
-    for (int k = 0; k < fit->nFit; k++) b[k] = nChunks > 0 ? fit->host[fit->column[k]] : 0.0;
+        XQ_CHECK(hipMemcpyAsync(fit->staging, fit->d_b, fit->nFit * sizeof(double), hipMemcpyDeviceToHost, s));
+        return kOK;
+    };
+    const int status = queue(), drained = check(hipStreamSynchronize(s), "fit b");
+    if (status != kOK) return status;
+    if (drained != kOK) return drained;
+    for (int k = 0; k < fit->nFit; k++) b[k] = fit->staging[fit->column[k]];
     return kOK;
 }
 
 int qs_fit_fock(qs_fit *fit, const double *c, double *Fock) {
     if (fit == nullptr || c == nullptr || Fock == nullptr) { set_error("invalid fit arguments"); return kInvalidArgument; }
     const size_t nPacked = static_cast<size_t>(fit->nOrbital) * (fit->nOrbital + 1) / 2;
+    if (fit->rows == 0) return kOK;
     hipStream_t s = fit->stream;
-    for (int k = 0; k < fit->nFit; k++) fit->host[fit->column[k]] = c[k];
-    XQ_CHECK(hipMemcpyAsync(fit->d_c, fit->host.data(), fit->nFit * sizeof(double), hipMemcpyHostToDevice, s));
-    XQ_CHECK(hipMemcpyAsync(fit->d_F, Fock, nPacked * sizeof(double), hipMemcpyHostToDevice, s));
-    if (fit->rows > 0) {
+    double *packed = fit->staging + fit->nFit;
+    for (int k = 0; k < fit->nFit; k++) fit->staging[fit->column[k]] = c[k];
+    // The term is formed from zero and added on the host: F itself does not cross to the GPU.
+    auto queue = [&]() -> int {
+        XQ_CHECK(hipMemcpyAsync(fit->d_c, fit->staging, fit->nFit * sizeof(double), hipMemcpyHostToDevice, s));
+        hipLaunchKernelGGL(zero_packed_kernel, dim3(static_cast<unsigned>(std::min<size_t>((nPacked + 255) / 256, 4096))),
+                           dim3(256), 0, s, nPacked, fit->d_F);
         const long long waves = (fit->rows + kFockRows - 1) / kFockRows;
         hipLaunchKernelGGL(fit_fock_kernel, dim3(static_cast<unsigned>((waves * 64 + 255) / 256)), dim3(256), 0, s,
                            fit->rows, fit->nFit, fit->d_B, fit->d_rowPacked, fit->d_c, fit->d_F);
         XQ_CHECK(hipGetLastError());
-    }
-    XQ_CHECK(hipMemcpyAsync(Fock, fit->d_F, nPacked * sizeof(double), hipMemcpyDeviceToHost, s));
-    XQ_CHECK(hipStreamSynchronize(s));
+        XQ_CHECK(hipMemcpyAsync(packed, fit->d_F, nPacked * sizeof(double), hipMemcpyDeviceToHost, s));
+        return kOK;
+    };
+    const int status = queue(), drained = check(hipStreamSynchronize(s), "fit Fock");
+    if (status != kOK) return status;
+    if (drained != kOK) return drained;
+    xq::host_add(Fock, packed, nPacked);
     return kOK;
 }
 

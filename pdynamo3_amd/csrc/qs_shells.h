@@ -109,21 +109,44 @@ inline std::string build_shells(QBasis *b, int nSpec, const double *spec) {
 }
 
 
-// Shell pairs A >= B whose largest primitive prefactor |c_a c_b| exp(-mu R^2) (pi/p)^(3/2) reaches the screen.
+// Shell pairs A >= B whose largest primitive prefactor |c_a c_b| exp(-mu R^2) (pi/p)^(3/2) max(1, 1/p) passes the screen
+// (all of them without screening).  A pair is settled by the first primitives that pass, the most diffuse ones being the
+// last of a shell as a rule, or by the bound from its shells' largest coefficients and smallest exponents, of which mu and
+// (pi/p)^(3/2) are monotonic: one or two exponentials a pair instead of one for each primitive pair.
 inline std::vector<QPair> shell_pairs(const QBasis *b, bool screen) {
+    const int n = static_cast<int>(b->shells.size());
     std::vector<QPair> out;
-    for (int A = 0; A < static_cast<int>(b->shells.size()); A++)
+    out.reserve(screen ? static_cast<size_t>(n) : static_cast<size_t>(n) * (n + 1) / 2);
+    if (!screen) {
+        for (int A = 0; A < n; A++)
+            for (int B = 0; B <= A; B++) out.push_back(QPair{A, B});
+        return out;
+    }
+    auto prefactor = [](double c, double a, double e, double r2) {
+        const double p = a + e, x = M_PI / p;
+        return c * std::exp(-a * e / p * r2) * (x * std::sqrt(x)) * std::max(1.0, 1.0 / p);
+    };
+    std::vector<double> most(b->shells.size(), 0.0), least(b->shells.size(), 0.0);
+    for (int A = 0; A < n; A++) {
+        const QShell &s = b->shells[A];
+        least[A] = b->exps[s.prim];
+        for (int q = 0; q < s.nPrim; q++) {
+            most[A] = std::max(most[A], std::fabs(b->coefs[s.prim + q]));
+            least[A] = std::min(least[A], b->exps[s.prim + q]);
+        }
+    }
+    for (int A = 0; A < n; A++)
         for (int B = 0; B <= A; B++) {
             const QShell &sa = b->shells[A], &sb = b->shells[B];
             const double dx = sa.x - sb.x, dy = sa.y - sb.y, dz = sa.z - sb.z, r2 = dx * dx + dy * dy + dz * dz;
-            double m = 0.0;
-            for (int qa = 0; qa < sa.nPrim; qa++)
-                for (int qb = 0; qb < sb.nPrim; qb++) {
-                    const double a = b->exps[sa.prim + qa], c = b->exps[sb.prim + qb], p = a + c;
-                    m = std::max(m, std::fabs(b->coefs[sa.prim + qa] * b->coefs[sb.prim + qb]) * std::exp(-a * c / p * r2) *
-                                        std::pow(M_PI / p, 1.5) * std::max(1.0, 1.0 / p));
-                }
-            if (!screen || m > kPairScreen) out.push_back(QPair{A, B});
+            // The bound's own rounding is far below the factor.
+            if (1.000001 * prefactor(most[A] * most[B], least[A], least[B], r2) <= kPairScreen) continue;
+            bool passes = false;
+            for (int qa = sa.nPrim - 1; qa >= 0 && !passes; qa--)
+                for (int qb = sb.nPrim - 1; qb >= 0 && !passes; qb--)
+                    passes = prefactor(std::fabs(b->coefs[sa.prim + qa] * b->coefs[sb.prim + qb]), b->exps[sa.prim + qa],
+                                       b->exps[sb.prim + qb], r2) > kPairScreen;
+            if (passes) out.push_back(QPair{A, B});
         }
     return out;
 }

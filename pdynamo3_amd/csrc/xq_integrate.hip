@@ -12,8 +12,11 @@
 // (int8 matrix cores).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "xq_functional.h"
@@ -95,10 +98,44 @@ void launch_pack_V(xq_grid *g, hipStream_t s) {
                        g->d_packed);
 }
 
+// f(begin, end) over 0 .. n - 1, cut between threads; what no thread could be started for runs here.
+template <typename F>
+static void in_ranges(size_t n, F f) {
+    constexpr size_t kPerThread = size_t{1} << 18;      // doubles: 2 MB
+    const size_t parts = std::min<size_t>({4, n / kPerThread, std::max<size_t>(1, std::thread::hardware_concurrency())});
+    if (parts <= 1) { f(size_t{0}, n); return; }
+    std::thread threads[3];
+    size_t done = n / parts;            // the first part is this thread's
+    const size_t own = done;
+    for (size_t k = 1; k < parts; k++) {
+        const size_t end = n * (k + 1) / parts;
+        try {
+            threads[k - 1] = std::thread(f, done, end);
+        } catch (const std::system_error &) {
+            break;
+        }
+        done = end;
+    }
+    f(size_t{0}, own);
+    f(done, n);
+    for (std::thread &t : threads)
+        if (t.joinable()) t.join();
+}
+
+void host_copy(double *to, const double *from, size_t n) {
+    in_ranges(n, [=](size_t a, size_t b) { std::memcpy(to + a, from + a, (b - a) * sizeof(double)); });
+}
+
+void host_add(double *to, const double *from, size_t n) {
+    in_ranges(n, [=](size_t a, size_t b) {
+        for (size_t k = a; k < b; k++) to[k] += from[k];
+    });
+}
+
 int upload_density(xq_grid *g, const double *Ppacked, hipStream_t s) {
     XQ_TRY(ensure_work(g));
     const size_t n = static_cast<size_t>(g->nFunctions), nPacked = n * (n + 1) / 2;
-    std::memcpy(g->h_stage, Ppacked, nPacked * sizeof(double));
+    host_copy(g->h_stage, Ppacked, nPacked);
     XQ_CHECK(hipMemcpyAsync(g->d_packed, g->h_stage, nPacked * sizeof(double), hipMemcpyHostToDevice, s));
     const int grid = static_cast<int>(std::min<size_t>((n * n + 255) / 256, 16384));
     hipLaunchKernelGGL(expand_packed_kernel, dim3(grid > 0 ? grid : 1), dim3(256), 0, s, g->nFunctions, g->d_packed, g->d_P);
@@ -227,7 +264,7 @@ static int integrate_jobs_queued(hipStream_t s, const StageEvents &ev, int nJobs
     for (int j = 0; j < nJobs; j++) {
         const xq_grid *g = grids[j];
         const size_t n = static_cast<size_t>(g->nFunctions), nPacked = n * (n + 1) / 2;
-        std::memcpy(g->h_stage, Ppacked[j], nPacked * sizeof(double));
+        host_copy(g->h_stage, Ppacked[j], nPacked);
         XQ_CHECK(hipMemcpyAsync(g->d_packed, g->h_stage, nPacked * sizeof(double), hipMemcpyHostToDevice, s));
     }
     XQ_CHECK(hipEventRecord(ev.ev0, s));
@@ -279,7 +316,7 @@ static int integrate_jobs_queued(hipStream_t s, const StageEvents &ev, int nJobs
             if (g->h_skip[b] && g->blocks[b].nKept > 0) skipped++;
         }
         const size_t n = static_cast<size_t>(g->nFunctions), nPacked = n * (n + 1) / 2;
-        for (size_t k = 0; k < nPacked; k++) V[j][k] += g->h_stage[k];
+        host_add(V[j], g->h_stage, nPacked);
         eXC[j] = e;
         nE[j] = ne;
         bfv += g->bfValues;

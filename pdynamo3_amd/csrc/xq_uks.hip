@@ -121,8 +121,8 @@ int integrate_uks(xq_grid *g, int nIDs, const int *ids, const double *Pa, const 
         beta.P = Pbd;
         beta.V = Vbd;
         // Both densities in, expanded to dense matrices.
-        std::memcpy(g->h_stage, Pa, nPacked * sizeof(double));
-        std::memcpy(stageB, Pb, nPacked * sizeof(double));
+        host_copy(g->h_stage, Pa, nPacked);
+        host_copy(stageB, Pb, nPacked);
         if ((status = check(hipEventRecord(g->ev0, s), "event")) != kOK) break;
         if ((status = check(hipMemcpyAsync(g->d_packed, g->h_stage, nPacked * sizeof(double), hipMemcpyHostToDevice, s),
                             "copy P alpha")) != kOK) break;
@@ -166,8 +166,8 @@ int integrate_uks(xq_grid *g, int nIDs, const int *ids, const double *Pa, const 
                                 "copy skips")) != kOK) break;
         }
         if ((status = check(hipStreamSynchronize(s), "unrestricted quadrature")) != kOK) break;
-        for (size_t k = 0; k < nPacked; k++) Va[k] += g->h_stage[k];
-        for (size_t k = 0; k < nPacked; k++) Vb[k] += stageB[k];
+        host_add(Va, g->h_stage, nPacked);
+        host_add(Vb, stageB, nPacked);
         // FP64 reductions in block order (DFTIntegrator.c:350-352).
         double e = 0.0, ne = 0.0;
         long long skipped = 0;
