@@ -58,6 +58,7 @@
 #include <algorithm>
 #include <climits>
 #include <cstdint>
+#include <type_traits>
 #include <vector>
 
 #include "xq_functional.h"
@@ -117,6 +118,31 @@ __device__ __forceinline__ long long combine(const int *acc) {
     return t;
 }
 
+// The same of five accumulators as the nearest double: both parts are exact (below 2^46 and 2^39), so that only their sum is
+// rounded, as the 64-bit integer's conversion would be, in half the operations.
+__device__ __forceinline__ double combined(int s0, int s1, int s2, int s3, int s4) {
+    const double hi = fma(fma(static_cast<double>(s0), 128.0, static_cast<double>(s1)), 128.0, static_cast<double>(s2));
+    return fma(hi, 16384.0, fma(static_cast<double>(s3), 128.0, static_cast<double>(s4)));
+}
+
+// Byte j of four 64-bit words as one 32-bit word, for the five digits of P.
+__device__ __forceinline__ void words_to_digits(const unsigned long long (&w)[4], unsigned (&digit)[5]) {
+    unsigned lo[4], hi[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        lo[k] = static_cast<unsigned>(w[k]);
+        hi[k] = static_cast<unsigned>(w[k] >> 32);
+    }
+    // perm(a, b, s): selector bytes 0 .. 3 take bytes of b, 4 .. 7 of a, 0xc zero.
+    const unsigned a01 = __builtin_amdgcn_perm(lo[1], lo[0], 0x05010400u), a23 = __builtin_amdgcn_perm(lo[3], lo[2], 0x05010400u);
+    const unsigned b01 = __builtin_amdgcn_perm(lo[1], lo[0], 0x07030602u), b23 = __builtin_amdgcn_perm(lo[3], lo[2], 0x07030602u);
+    digit[0] = __builtin_amdgcn_perm(a23, a01, 0x05040100u);
+    digit[1] = __builtin_amdgcn_perm(a23, a01, 0x07060302u);
+    digit[2] = __builtin_amdgcn_perm(b23, b01, 0x05040100u);
+    digit[3] = __builtin_amdgcn_perm(b23, b01, 0x07060302u);
+    digit[4] = __builtin_amdgcn_perm(hi[1], hi[0], 0x0c0c0400u) | __builtin_amdgcn_perm(hi[3], hi[2], 0x04000c0cu);
+}
+
 // Signed byte v (0..15) of a 16-byte operand, and 16 bytes packed into one.
 __device__ __forceinline__ int byte_of(const v4i &x, int v) {
     return static_cast<int>(static_cast<unsigned>(x[v >> 2]) << (24 - 8 * (v & 3))) >> 24;
@@ -138,9 +164,9 @@ __device__ __forceinline__ int digits4(const v4i (&d)[kDPhi], int v) {
 }
 
 // 5-digit value of byte v of the digit operands d[0..4]: sum_j d_j 128^(4-j).
-__device__ __forceinline__ long long digits5(const v4i (&d)[kDB], int v) {
+__device__ __forceinline__ double digits5(const v4i (&d)[kDB], int v) {
     const int hi = ((byte_of(d[0], v) * 128 + byte_of(d[1], v)) * 128 + byte_of(d[2], v)) * 128 + byte_of(d[3], v);
-    return static_cast<long long>(hi) * 128 + byte_of(d[4], v);
+    return fma(static_cast<double>(hi), 128.0, static_cast<double>(byte_of(d[4], v)));    // exact
 }
 
 // Signed 16-bit element v (0..15) of 32 bytes, and unsigned byte v of 16 bytes.
@@ -434,17 +460,18 @@ __global__ void __launch_bounds__(256) p_slice_kernel(const xq::MixedJob *__rest
 // Density rows (one row chunk I of one block per work-group, 256 threads = 4 waves): X = P_red Phi for the chunk's 32
 // rows on int8 MFMA, then the chunk's share of rho and grad rho at the block's points, stored in part[chunk][4][point].
 // Wave wv owns points 32 wv .. + 31; lane (lr, lh) owns point 32 wv + lr and the rows chunk_fun(lh, v) of chunk I.
-// Each step stages one column chunk of P_red's row panel (gathered) and that chunk's Phi digits (16-byte loads of the
-// contiguous DB chunk) in LDS, both fetched by all 256 threads into registers one step ahead.  The row chunks of a
+// Each step stages one column chunk of P_red's row panel, gathered by all 256 threads one step ahead, in one of two LDS
+// buffers (one barrier per step).  The matching Phi digits are a lane's own operands, contiguous over the wave in DB, and
+// are loaded into the registers of the current ones as soon as the products with them are issued.  The row chunks of a
 // block are consecutive items of one XCD, so that their work-groups run at about the same time and read the block's
 // Phi digit chunks, in the same order, through that XCD's L2: Phi comes from HBM about once per block instead of once
-// per row chunk.  Chunk I's digits, staged at step I, are kept in LDS for the epilogue.  52 KB of LDS and at most 168
-// VGPRs let three work-groups share a CU (four, at 128 VGPRs, were slower: 3.56 against 2.75 ms on (H2O)64).
+// per row chunk.  At most 168 VGPRs let three work-groups share a CU (four, at 128, spill: 2.53 against 2.31 ms on
+// (H2O)64).  Bound by latency and vector arithmetic: without the gathers it would take 1.98 ms, with grad Phi
+// from L2 2.23; the vector units are busy for a third of the time, the matrix cores for a fifth.  With Phi staged in LDS
+// as well, two barriers a step, and 64-bit integers in the epilogue it took 2.43 ms.
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
 density_rows_kernel(const xq::MixedJob *__restrict__ jobs, int nJobs, int interleaved) {
-    __shared__ __attribute__((aligned(16))) int sP[kDP][kC][kPRowDwords];   // [digit][row][K positions / 4]
-    __shared__ v4i sB[kChunkBytesB / 16];   // the step's Phi digits, in DB's order
-    __shared__ v4i sBI[kChunkBytesB / 16];  // chunk I's Phi digits, kept from step I for the epilogue
+    __shared__ __attribute__((aligned(16))) int sP[2][kDP][kC][kPRowDwords];   // [digit][row][K positions / 4]
     __shared__ int sPe[kC];
     __shared__ int sIdx[kIdxCache];
     // Work-group g runs on XCD x = g % 8 and takes slot g / 8 of that XCD's item list: the jobs' lists in job order, or,
@@ -489,51 +516,47 @@ density_rows_kernel(const xq::MixedJob *__restrict__ jobs, int nJobs, int interl
     v16i acc[kXOrders];
 #pragma unroll
     for (int s = 0; s < kXOrders; s++) acc[s] = v16i{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    // One chunk per step; the next step's P_red words and Phi digits are loaded into registers while the current
-    // step's products run.
-    constexpr int kPhiPerThread = kChunkBytesB / 16 / 256;
-    const v4i *phiSrc = reinterpret_cast<const v4i *>(DBb);
+    // One chunk per step; the next step's P_red words are loaded while the current step's products run, each of its Phi
+    // digits when the products with the current one are issued.
+    const v4i *__restrict__ phi = reinterpret_cast<const v4i *>(DBb) + 2 * p + lh;
     unsigned long long wd[4];
-    v4i ph[kPhiPerThread];
-    auto fetch = [&](int c) {
+    v4i bq[kDB];
+    auto fetch_p = [&](int c) {
 #pragma unroll
         for (int jj = 0; jj < 4; jj++) {
             const int k = kC * c + 8 * jj + s8;
             wd[jj] = (r < nb && k < nb) ? Pq[rowOff + idx[k]] : 0ull;
         }
-#pragma unroll
-        for (int i = 0; i < kPhiPerThread; i++)
-            ph[i] = phiSrc[static_cast<size_t>(c) * (kChunkBytesB / 16) + t + 256 * i];
     };
-    fetch(0);
-    for (int c = 0; c < nChunks; c++) {
-        __syncthreads();   // every wave is done with the previous chunk
+    auto step = [&](int c, auto more) {
+        int (&tile)[kDP][kC][kPRowDwords] = sP[c & 1];
+        unsigned digit[kDP];
+        words_to_digits(wd, digit);
 #pragma unroll
-        for (int i = 0; i < kPhiPerThread; i++) sB[t + 256 * i] = ph[i];
-        if (c == I) {
-#pragma unroll
-            for (int i = 0; i < kPhiPerThread; i++) sBI[t + 256 * i] = ph[i];
-        }
-#pragma unroll
-        for (int j = 0; j < kDP; j++) {
-            unsigned x = 0;
-#pragma unroll
-            for (int jj = 0; jj < 4; jj++) x |= (static_cast<unsigned>(wd[jj] >> (8 * j)) & 255u) << (8 * jj);
-            sP[j][srow][s8] = static_cast<int>(x);
-        }
+        for (int j = 0; j < kDP; j++) tile[j][srow][s8] = static_cast<int>(digit[j]);
+        // A wave writes this buffer again two steps on, after the next barrier, which every wave reaches done with it.
         __syncthreads();
-        if (c + 1 < nChunks) fetch(c + 1);
-        v4i a[kDP], bq[kDB];
+        if constexpr (more) {
+            fetch_p(c + 1);
+            phi += kChunkBytesB / 16;
+        }
+        v4i a[kDP];
 #pragma unroll
-        for (int j = 0; j < kDB; j++) bq[j] = sB[(j * kBlockSize + p) * 2 + lh];
+        for (int i = 0; i < kDP; i++) a[i] = *reinterpret_cast<const v4i *>(&tile[i][lr][4 * lh]);
 #pragma unroll
-        for (int j = 0; j < kDP; j++) a[j] = *reinterpret_cast<const v4i *>(&sP[j][lr][4 * lh]);
+        for (int j = kDB - 1; j >= 0; j--) {
 #pragma unroll
-        for (int i = 0; i < kDP; i++)
-#pragma unroll
-            for (int j = 0; j < kDB; j++)
+            for (int i = 0; i < kDP; i++)
                 if (i + j < kXOrders) acc[i + j] = mfma_i8(a[i], bq[j], acc[i + j]);
-    }
+            if constexpr (more) bq[j] = phi[j * kBlockSize * 2];
+        }
+    };
+    fetch_p(0);
+#pragma unroll
+    for (int j = 0; j < kDB; j++) bq[j] = phi[j * kBlockSize * 2];
+#pragma unroll 1
+    for (int c = 0; c + 1 < nChunks; c++) step(c, std::true_type{});
+    step(nChunks - 1, std::false_type{});
     // Epilogue: X for rows chunk_fun(lh, v) of chunk I at point p; Phi from the chunk's own digits, grad Phi from its
     // fixed point (the sums over v are scaled once).  X in FP64 first, so that the accumulators are free before the
     // epilogue's operands arrive.
@@ -541,15 +564,16 @@ density_rows_kernel(const xq::MixedJob *__restrict__ jobs, int nJobs, int interl
     double x[16];
 #pragma unroll
     for (int v = 0; v < 16; v++) {
-        const int s[kXOrders] = {acc[0][v], acc[1][v], acc[2][v], acc[3][v], acc[4][v]};
-        x[v] = ldexp(static_cast<double>(combine<kXOrders>(s)), sPe[chunk_fun(lh, v)] + eb - 7 * (kXOrders + 1));
+        x[v] = ldexp(combined(acc[0][v], acc[1][v], acc[2][v], acc[3][v], acc[4][v]),
+                     sPe[chunk_fun(lh, v)] + eb - 7 * (kXOrders + 1));
     }
-    v4i dI[kDB];   // the lane's Phi digits of chunk I (written to sBI before the last step's barrier)
+    v4i dI[kDB];   // the lane's Phi digits of chunk I
+    const v4i *__restrict__ phiI = reinterpret_cast<const v4i *>(DBb + static_cast<size_t>(I) * kChunkBytesB) + 2 * p + lh;
 #pragma unroll
-    for (int j = 0; j < kDB; j++) dI[j] = sBI[(j * kBlockSize + p) * 2 + lh];
+    for (int j = 0; j < kDB; j++) dI[j] = phiI[j * kBlockSize * 2];
     double sumR = 0.0, sumG[3] = {0.0, 0.0, 0.0};
 #pragma unroll
-    for (int v = 0; v < 16; v++) sumR += static_cast<double>(digits5(dI, v)) * x[v];
+    for (int v = 0; v < 16; v++) sumR += digits5(dI, v) * x[v];
 #pragma unroll
     for (int c = 0; c < 3; c++) {
         const size_t o = CI * kChunkGrad + (c * kBlockSize + p) * kC + 16 * lh;
