@@ -34,7 +34,9 @@ namespace {
 
 constexpr int kC = 32;                   // chunk rows
 constexpr int kChunk = 4096;             // doubles per chunk plane
-constexpr int kRowPitch = kC + 4;        // LDS row pitch of a staged P_red chunk in doubles (padded against bank conflicts)
+// LDS row pitch of a staged P_red chunk in doubles: odd, so that the operands' 16 rows lie in different banks (39: two rows
+// being written as well).  With 36, whose rows met in four banks, the density rows took 3.62 ms on (H2O)64, now 3.51.
+constexpr int kRowPitch = kC + 7;
 constexpr int kIdxCache = 1024;          // kept-function indices of a block cached in LDS by the density kernel
 
 __device__ __forceinline__ v4d mfma_f64(double a, double b, const v4d &c) {
@@ -84,11 +86,11 @@ __global__ void __launch_bounds__(256) f64_prepare_kernel(
 // step multiplies one 32 x 32 chunk of P_red, gathered by all threads and staged in one of two LDS buffers (one barrier per
 // step), with the matching Phi chunk, whose operands go straight to registers; the words of P_red are fetched one step
 // ahead, and each Phi operand for the next step as soon as its products of this step are issued, into the same registers:
-// four work-groups per CU instead of three with a second set of operand registers (3.62 ms against 4.13).  The row
+// four work-groups per CU instead of three with a second set of operand registers (3.62 ms against 4.13 then).  The row
 // chunks of a block are consecutive items of one XCD, so that Phi comes from HBM about once per block.
 // Bound by HBM (Phi and grad Phi once, 10.7 GB on (H2O)64, and the gathers of P_red) and the FP64 matrix cores (busy for
 // half of the time).  One work-group per block, which read Phi once per row chunk from HBM and waited for each panel of
-// gathers, took 8.26 ms on (H2O)64 (1.3e11 operations); this takes 3.62 ms and the functional 0.21 ms.
+// gathers, took 8.26 ms on (H2O)64 (1.3e11 operations); this takes 3.51 ms and the functional 0.21 ms.
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
 density_rows_kernel_f64(const MixedJob *__restrict__ jobs, int nJobs, int interleaved) {
     __shared__ double sP[2][kC][kRowPitch];

@@ -36,7 +36,7 @@ namespace {
 // larger batches than 131,072 rows took 3.6 ms off an (H2O)64 gradient call: fewer launches, each with its own tail.
 constexpr long long kBatchRows = 524288;
 constexpr int kC = 32;                           // rows per chunk (two 16-row MFMA tiles)
-constexpr int kRowPitch = kC + 4;                // LDS row pitch of a staged P_red chunk in doubles (padded against bank conflicts)
+constexpr int kRowPitch = kC + 7;                // LDS row pitch of a staged P_red chunk in doubles, odd against bank conflicts
 constexpr int kIdxCache = 1024;                  // kept-function indices cached in LDS
 constexpr int kGradCopies = 64;                  // copies of the gradient array that spread the atomics
 
@@ -52,8 +52,8 @@ __device__ __forceinline__ v4d mfma_f64(double a, double b, const v4d &c) {
 // a plane of rows of 128 points (rows >= nb are not read).  Each step multiplies one 32 x 32 chunk of P_red, gathered by
 // all threads and staged in one of two LDS buffers (one barrier per step), with 32 rows of Bp; the words of P_red are
 // fetched one step ahead, each operand of Bp for the next step as soon as its products of this step are issued.  Staged
-// panels of four chunks, each waited for, took 7.2 ms (X pass) and 9.3 ms (Z pass) per call on (H2O)64; this takes 3.8 and
-// 5.9 ms.
+// panels of four chunks, each waited for, took 7.2 ms (X pass) and 9.3 ms (Z pass) per call on (H2O)64; this takes 3.7 and
+// 5.7 ms.
 __device__ __forceinline__ void reduced_product(const double *__restrict__ P, int n, const int *idx, int nb,
                                                 const double *__restrict__ Bp, double (&sP)[2][kC][kRowPitch], int I,
                                                 v4d (&acc)[2][2]) {
