@@ -218,11 +218,63 @@ __global__ void __launch_bounds__(256) w_kernel_f64(const MixedJob *__restrict__
     }
 }
 
-// Fock kernel: one wave per lower-triangle tile (I, J <= I), four tiles per work-group, no LDS and no barriers; K runs
-// over the block's 128 points in steps of 4.  V += Phi_I W_J^T + W_I Phi_J^T with FP64 atomics.  Work-group g runs on XCD
-// g % 8; tiles are dealt so that each XCD takes a contiguous range of the tile list.
-__global__ void __launch_bounds__(256) fock_kernel_f64(const MixedJob *__restrict__ jobs, int nJobs, int groupsPerXcd,
+// The sums over a block's 128 points of one 32 x 32 tile, 32 steps of 4 points: Phi_I W_J^T, and, off the diagonal,
+// W_I Phi_J^T as well (on it that is the transpose).  Operands are fetched four steps ahead, each into the registers of the
+// one whose products have just been issued.
+template <bool kDiagonal>
+__device__ __forceinline__ void fock_tile_f64(const double *__restrict__ fI, const double *__restrict__ wI,
+                                              const double *__restrict__ fJ, const double *__restrict__ wJ,
+                                              v4d (&acc)[2][2]) {
+    constexpr int kAhead = 4;
+    double xf[kAhead][2], xw[kAhead][2], yf[kAhead][2], yw[kAhead][2];
+    auto load = [&](int k) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int o = (2 * k + h) * 64;
+            xf[k][h] = fI[o];
+            yw[k][h] = wJ[o];
+            if constexpr (!kDiagonal) {
+                xw[k][h] = wI[o];
+                yf[k][h] = fJ[o];
+            }
+        }
+    };
+    auto products = [&](int k) {
+#pragma unroll
+        for (int hm = 0; hm < 2; hm++)
+#pragma unroll
+            for (int hn = 0; hn < 2; hn++) {
+                acc[hm][hn] = mfma_f64(xf[k][hm], yw[k][hn], acc[hm][hn]);
+                if constexpr (!kDiagonal) acc[hm][hn] = mfma_f64(xw[k][hm], yf[k][hn], acc[hm][hn]);
+            }
+    };
+#pragma unroll
+    for (int k = 0; k < kAhead; k++) load(k);
+#pragma unroll 1
+    for (int s = kAhead; s < kBlockSize / 4; s += kAhead) {
+        fI += 2 * 64 * kAhead;
+        wI += 2 * 64 * kAhead;
+        fJ += 2 * 64 * kAhead;
+        wJ += 2 * 64 * kAhead;
+#pragma unroll
+        for (int k = 0; k < kAhead; k++) {
+            products(k);
+            load(k);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < kAhead; k++) products(k);
+}
+
+// Fock kernel: one wave per lower-triangle tile (I, J <= I), four tiles per work-group, no barriers.
+// V += Phi_I W_J^T + W_I Phi_J^T with FP64 atomics; on a diagonal tile the second term is the first one's transpose, taken
+// through LDS.  Work-group g runs on XCD g % 8; tiles are dealt so that each XCD takes a contiguous range of the tile list.
+// Bound by the FP64 matrix cores and the atomics, which go to memory.  Groups of four steps whose loads were each waited
+// for, and both products on the diagonal, took 3.79 ms on (H2O)64 and 27 us on one water; this takes 3.58 ms and
+// 19 us (four waves per SIMD; 3.68 ms with three).
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) fock_kernel_f64(const MixedJob *__restrict__ jobs, int nJobs, int groupsPerXcd,
                                                        int nGroups) {
+    __shared__ double sT[4][kC][kC + 1];
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6, l16 = lane & 15, l4 = lane >> 4;
     const int group = (blockIdx.x & 7) * groupsPerXcd + (blockIdx.x >> 3);
     if (group >= nGroups) return;
@@ -243,24 +295,26 @@ __global__ void __launch_bounds__(256) fock_kernel_f64(const MixedJob *__restric
     for (int hm = 0; hm < 2; hm++)
 #pragma unroll
         for (int hn = 0; hn < 2; hn++) acc[hm][hn] = v4d{0.0, 0.0, 0.0, 0.0};
-#pragma unroll 4
-    for (int s = 0; s < 32; s++) {
-        double xf[2], xw[2], yf[2], yw[2];
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const int o = (s * 2 + h) * 64;
-            xf[h] = fI[o];
-            xw[h] = wI[o];
-            yf[h] = fJ[o];
-            yw[h] = wJ[o];
-        }
+    if (I != J) {
+        fock_tile_f64<false>(fI, wI, fJ, wJ, acc);
+    } else {
+        fock_tile_f64<true>(fI, wI, fJ, wJ, acc);
+        double (&T)[kC][kC + 1] = sT[wv];
 #pragma unroll
         for (int hm = 0; hm < 2; hm++)
 #pragma unroll
-            for (int hn = 0; hn < 2; hn++) {
-                acc[hm][hn] = mfma_f64(xf[hm], yw[hn], acc[hm][hn]);   // Phi_I W_J^T
-                acc[hm][hn] = mfma_f64(xw[hm], yf[hn], acc[hm][hn]);   // W_I Phi_J^T
-            }
+            for (int hn = 0; hn < 2; hn++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) T[16 * hm + 4 * v + l4][16 * hn + l16] = acc[hm][hn][v];
+        // The wave's LDS accesses are in order; this keeps the compiler from moving them.
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int hm = 0; hm < 2; hm++)
+#pragma unroll
+            for (int hn = 0; hn < 2; hn++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) acc[hm][hn][v] += T[16 * hn + l16][16 * hm + 4 * v + l4];
     }
     const int n = job.n;
 #pragma unroll
