@@ -26,7 +26,10 @@ namespace xq {
 
 namespace {
 
-__global__ void expand_packed_kernel(int n, const double *__restrict__ packed, double *__restrict__ dense) {
+// The dense symmetric matrix of a packed triangle; with `cleared`, that n x n matrix to zero as well (V beside P: a launch
+// less per step).
+__global__ void expand_packed_kernel(int n, const double *__restrict__ packed, double *__restrict__ dense,
+                                     double *__restrict__ cleared) {
     const size_t total = static_cast<size_t>(n) * n;
     for (size_t e = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x; e < total;
          e += static_cast<size_t>(gridDim.x) * blockDim.x) {
@@ -34,10 +37,14 @@ __global__ void expand_packed_kernel(int n, const double *__restrict__ packed, d
         const int hi = i > j ? i : j, lo = i > j ? j : i;
         const double v = packed[static_cast<size_t>(hi) * (hi + 1) / 2 + lo];
         dense[e] = v;
+        if (cleared != nullptr) cleared[e] = 0.0;
     }
 }
 
-__global__ void pack_lower_kernel(int n, const double *__restrict__ dense, double *__restrict__ packed) {
+// The packed lower triangle of a dense matrix; with nB blocks, their sums (2 nB) and skip flags behind it, so that one copy
+// brings a step's results.
+__global__ void pack_lower_kernel(int n, const double *__restrict__ dense, double *__restrict__ packed, int nB,
+                                  const double *__restrict__ blockEN, const int *__restrict__ skip) {
     const size_t total = static_cast<size_t>(n) * (n + 1) / 2;
     for (size_t e = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x; e < total;
          e += static_cast<size_t>(gridDim.x) * blockDim.x) {
@@ -47,6 +54,13 @@ __global__ void pack_lower_kernel(int n, const double *__restrict__ dense, doubl
         while (static_cast<size_t>(i + 1) * (i + 2) / 2 <= e) i++;
         const int j = static_cast<int>(e - static_cast<size_t>(i) * (i + 1) / 2);
         packed[e] = dense[static_cast<size_t>(i) * n + j];
+    }
+    double *__restrict__ sums = packed + total;
+    int *__restrict__ flags = reinterpret_cast<int *>(sums + 2 * static_cast<size_t>(nB));
+    for (int b = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x); b < nB; b += static_cast<int>(gridDim.x * blockDim.x)) {
+        sums[2 * b] = blockEN[2 * b];
+        sums[2 * b + 1] = blockEN[2 * b + 1];
+        flags[b] = skip[b];
     }
 }
 
@@ -64,7 +78,7 @@ void launch_expand_P(xq_grid *g, hipStream_t s) {
     const size_t n = static_cast<size_t>(g->nFunctions);
     const int grid = static_cast<int>(std::min<size_t>((n * n + 255) / 256, 16384));
     hipLaunchKernelGGL(expand_packed_kernel, dim3(grid > 0 ? grid : 1), dim3(256), 0, s, g->nFunctions, g->d_packed,
-                       g->d_P);
+                       g->d_P, nullptr);
 }
 
 void launch_zero_V(xq_grid *g, hipStream_t s) {
@@ -76,7 +90,7 @@ void launch_zero_V(xq_grid *g, hipStream_t s) {
 void launch_expand(int n, const double *packed, double *dense, hipStream_t s) {
     const size_t nn = static_cast<size_t>(n) * n;
     const int grid = static_cast<int>(std::min<size_t>((nn + 255) / 256, 16384));
-    hipLaunchKernelGGL(expand_packed_kernel, dim3(grid > 0 ? grid : 1), dim3(256), 0, s, n, packed, dense);
+    hipLaunchKernelGGL(expand_packed_kernel, dim3(grid > 0 ? grid : 1), dim3(256), 0, s, n, packed, dense, nullptr);
 }
 
 void launch_zero(int n, double *dense, hipStream_t s) {
@@ -88,14 +102,22 @@ void launch_zero(int n, double *dense, hipStream_t s) {
 void launch_pack(int n, const double *dense, double *packed, hipStream_t s) {
     const size_t nPacked = static_cast<size_t>(n) * (n + 1) / 2;
     const int grid = static_cast<int>(std::min<size_t>((nPacked + 255) / 256, 16384));
-    hipLaunchKernelGGL(pack_lower_kernel, dim3(grid > 0 ? grid : 1), dim3(256), 0, s, n, dense, packed);
+    hipLaunchKernelGGL(pack_lower_kernel, dim3(grid > 0 ? grid : 1), dim3(256), 0, s, n, dense, packed, 0, nullptr,
+                       nullptr);
 }
 
 void launch_pack_V(xq_grid *g, hipStream_t s) {
     const size_t n = static_cast<size_t>(g->nFunctions), nPacked = n * (n + 1) / 2;
     const int grid = static_cast<int>(std::min<size_t>((nPacked + 255) / 256, 16384));
     hipLaunchKernelGGL(pack_lower_kernel, dim3(grid > 0 ? grid : 1), dim3(256), 0, s, g->nFunctions, g->d_V,
-                       g->d_packed);
+                       g->d_packed, 0, nullptr, nullptr);
+}
+
+void launch_pack_results(xq_grid *g, hipStream_t s) {
+    const size_t n = static_cast<size_t>(g->nFunctions), work = std::max<size_t>(n * (n + 1) / 2, g->nBlocks);
+    const int grid = static_cast<int>(std::min<size_t>((work + 255) / 256, 16384));
+    hipLaunchKernelGGL(pack_lower_kernel, dim3(grid > 0 ? grid : 1), dim3(256), 0, s, g->nFunctions, g->d_V,
+                       g->d_packed, g->nBlocks, g->d_blockEN, g->d_skip);
 }
 
 // f(begin, end) over 0 .. n - 1, cut between threads; what no thread could be started for runs here.
@@ -138,7 +160,7 @@ int upload_density(xq_grid *g, const double *Ppacked, hipStream_t s) {
     host_copy(g->h_stage, Ppacked, nPacked);
     XQ_CHECK(hipMemcpyAsync(g->d_packed, g->h_stage, nPacked * sizeof(double), hipMemcpyHostToDevice, s));
     const int grid = static_cast<int>(std::min<size_t>((n * n + 255) / 256, 16384));
-    hipLaunchKernelGGL(expand_packed_kernel, dim3(grid > 0 ? grid : 1), dim3(256), 0, s, g->nFunctions, g->d_packed, g->d_P);
+    hipLaunchKernelGGL(expand_packed_kernel, dim3(grid > 0 ? grid : 1), dim3(256), 0, s, g->nFunctions, g->d_packed, g->d_P, nullptr);
     XQ_CHECK(hipGetLastError());
     return kOK;
 }
@@ -147,8 +169,8 @@ int upload_density(xq_grid *g, const double *Ppacked, hipStream_t s) {
 // way releases what the set already holds, so the next call allocates it again from scratch.
 static void free_work_arrays(xq_grid *g) {
     if (g->h_stage != nullptr) { cache_host_free(g->h_stage); g->h_stage = nullptr; }
-    if (g->h_blockEN != nullptr) { cache_host_free(g->h_blockEN); g->h_blockEN = nullptr; }
-    if (g->h_skip != nullptr) { cache_host_free(g->h_skip); g->h_skip = nullptr; }
+    g->h_blockEN = nullptr;
+    g->h_skip = nullptr;
     dev_free(g, &g->d_P);
     dev_free(g, &g->d_V);
     dev_free(g, &g->d_packed);
@@ -166,23 +188,29 @@ void free_work(xq_grid *g) {
     free_work_arrays(g);
 }
 
+size_t result_bytes(const xq_grid *g) {
+    const size_t n = static_cast<size_t>(g->nFunctions), nB = static_cast<size_t>(g->nBlocks);
+    return (n * (n + 1) / 2 + 2 * nB) * sizeof(double) + nB * sizeof(int);
+}
+
 static int alloc_work_arrays(xq_grid *g) {
     const size_t n = static_cast<size_t>(g->nFunctions);
     XQ_TRY(dev_alloc(g, &g->d_P, n * n));
     XQ_TRY(dev_alloc(g, &g->d_V, n * n));
-    XQ_TRY(dev_alloc(g, &g->d_packed, n * (n + 1) / 2));
-    XQ_TRY(dev_alloc(g, &g->d_blockEN, 2 * static_cast<size_t>(g->nBlocks)));
-    XQ_TRY(dev_alloc(g, &g->d_skip, static_cast<size_t>(g->nBlocks)));
-    const size_t nb = static_cast<size_t>(g->nBlocks > 0 ? g->nBlocks : 1);
-    XQ_CHECK(cache_host_alloc(reinterpret_cast<void **>(&g->h_stage), n * (n + 1) / 2 * sizeof(double) + 8));
-    XQ_CHECK(cache_host_alloc(reinterpret_cast<void **>(&g->h_blockEN), 2 * nb * sizeof(double)));
-    XQ_CHECK(cache_host_alloc(reinterpret_cast<void **>(&g->h_skip), nb * sizeof(int)));
+    // The packed buffers have room for the block sums and the skip flags behind the matrix (launch_pack_results).
+    const size_t nPacked = n * (n + 1) / 2, nB = static_cast<size_t>(g->nBlocks);
+    XQ_TRY(dev_alloc(g, &g->d_packed, nPacked + 2 * nB + (nB + 1) / 2));
+    XQ_TRY(dev_alloc(g, &g->d_blockEN, 2 * nB));
+    XQ_TRY(dev_alloc(g, &g->d_skip, nB));
+    XQ_CHECK(cache_host_alloc(reinterpret_cast<void **>(&g->h_stage), result_bytes(g) + 8));
+    g->h_blockEN = g->h_stage + nPacked;
+    g->h_skip = reinterpret_cast<int *>(g->h_blockEN + 2 * nB);
     return kOK;
 }
 
 int ensure_work(xq_grid *g) {
     if (g->d_P != nullptr && g->d_V != nullptr && g->d_packed != nullptr && g->d_blockEN != nullptr &&
-        g->d_skip != nullptr && g->h_stage != nullptr && g->h_blockEN != nullptr && g->h_skip != nullptr)
+        g->d_skip != nullptr && g->h_stage != nullptr)
         return kOK;
     free_work_arrays(g);
     const int status = alloc_work_arrays(g);
@@ -273,8 +301,7 @@ static int integrate_jobs_queued(hipStream_t s, const StageEvents &ev, int nJobs
         const size_t n = static_cast<size_t>(g->nFunctions);
         const int grid = static_cast<int>(std::min<size_t>((n * n + 255) / 256, 16384));
         hipLaunchKernelGGL(expand_packed_kernel, dim3(grid > 0 ? grid : 1), dim3(256), 0, s, g->nFunctions, g->d_packed,
-                           g->d_P);
-        hipLaunchKernelGGL(zero_kernel, dim3(grid > 0 ? grid : 1), dim3(256), 0, s, n * n, g->d_V);
+                           g->d_P, g->d_V);
     }
     XQ_CHECK(hipGetLastError());
     if (precision == XQ_PRECISION_FP64) {
@@ -283,25 +310,13 @@ static int integrate_jobs_queued(hipStream_t s, const StageEvents &ev, int nJobs
         XQ_TRY(launch_mixed(s, ev, nJobs, grids, fs, h_table, d_table));
     }
     XQ_CHECK(hipGetLastError());
-    for (int j = 0; j < nJobs; j++) {
-        const xq_grid *g = grids[j];
-        const size_t n = static_cast<size_t>(g->nFunctions), nPacked = n * (n + 1) / 2;
-        const int pgrid = static_cast<int>(std::min<size_t>((nPacked + 255) / 256, 16384));
-        hipLaunchKernelGGL(pack_lower_kernel, dim3(pgrid > 0 ? pgrid : 1), dim3(256), 0, s, g->nFunctions, g->d_V,
-                           g->d_packed);
-    }
+    for (int j = 0; j < nJobs; j++) launch_pack_results(grids[j], s);
     XQ_CHECK(hipGetLastError());
     XQ_CHECK(hipEventRecord(ev.ev1, s));
     // Results into the pinned buffers (asynchronous DMAs ordered after the kernels), then one wait.
     for (int j = 0; j < nJobs; j++) {
         xq_grid *g = grids[j];
-        const size_t n = static_cast<size_t>(g->nFunctions), nPacked = n * (n + 1) / 2;
-        XQ_CHECK(hipMemcpyAsync(g->h_stage, g->d_packed, nPacked * sizeof(double), hipMemcpyDeviceToHost, s));
-        if (g->nBlocks > 0) {
-            XQ_CHECK(hipMemcpyAsync(g->h_blockEN, g->d_blockEN, 2 * g->nBlocks * sizeof(double), hipMemcpyDeviceToHost,
-                                    s));
-            XQ_CHECK(hipMemcpyAsync(g->h_skip, g->d_skip, g->nBlocks * sizeof(int), hipMemcpyDeviceToHost, s));
-        }
+        XQ_CHECK(hipMemcpyAsync(g->h_stage, g->d_packed, result_bytes(g), hipMemcpyDeviceToHost, s));
     }
     XQ_CHECK(hipStreamSynchronize(s));
     double bfv = 0.0, bfs = 0.0, bfp = 0.0, rhoBytes = 0.0, fockBytes = 0.0, productBytes = 0.0;

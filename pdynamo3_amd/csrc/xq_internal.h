@@ -293,6 +293,10 @@ int upload_density(xq_grid *g, const double *Ppacked, hipStream_t s);
 // four; smaller arrays take less than starting the threads).
 void host_copy(double *to, const double *from, size_t n);
 void host_add(double *to, const double *from, size_t n);
+// A step's results behind each other in d_packed (packed V, the block sums, the skip flags), and their bytes; h_stage takes
+// them with one copy, and h_blockEN and h_skip point into it.
+void launch_pack_results(xq_grid *g, hipStream_t s);
+size_t result_bytes(const xq_grid *g);
 void free_mixed(xq_grid *g);
 int alloc_step_mixed(xq_grid *g, StepArrays *a);
 void free_step_mixed(xq_grid *g, StepArrays *a);

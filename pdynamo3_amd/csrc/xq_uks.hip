@@ -151,20 +151,14 @@ int integrate_uks(xq_grid *g, int nIDs, const int *ids, const double *Pa, const 
         status = mixed ? launch_mixed(s, ev, 2, grids, fs2, h_tab + 2, d_tab + 2, kStageFock, fock)
                        : launch_f64(s, ev, 2, grids, fs2, h_tab + 2, d_tab + 2, kStageFock, fock);
         if (status != kOK) break;
-        launch_pack(n, g->d_V, g->d_packed, s);
+        launch_pack_results(g, s);
         launch_pack(n, Vbd, packedB, s);
         if ((status = check(hipGetLastError(), "pack")) != kOK) break;
         if ((status = check(hipEventRecord(g->ev1, s), "event")) != kOK) break;
-        if ((status = check(hipMemcpyAsync(g->h_stage, g->d_packed, nPacked * sizeof(double), hipMemcpyDeviceToHost, s),
-                            "copy V alpha")) != kOK) break;
+        if ((status = check(hipMemcpyAsync(g->h_stage, g->d_packed, result_bytes(g), hipMemcpyDeviceToHost, s),
+                            "copy V alpha, block sums and skips")) != kOK) break;
         if ((status = check(hipMemcpyAsync(stageB, packedB, nPacked * sizeof(double), hipMemcpyDeviceToHost, s),
                             "copy V beta")) != kOK) break;
-        if (g->nBlocks > 0) {
-            if ((status = check(hipMemcpyAsync(g->h_blockEN, g->d_blockEN, 2 * g->nBlocks * sizeof(double),
-                                               hipMemcpyDeviceToHost, s), "copy block sums")) != kOK) break;
-            if ((status = check(hipMemcpyAsync(g->h_skip, g->d_skip, g->nBlocks * sizeof(int), hipMemcpyDeviceToHost, s),
-                                "copy skips")) != kOK) break;
-        }
         if ((status = check(hipStreamSynchronize(s), "unrestricted quadrature")) != kOK) break;
         host_add(Va, g->h_stage, nPacked);
         host_add(Vb, stageB, nPacked);
