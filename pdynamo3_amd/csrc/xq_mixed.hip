@@ -294,7 +294,7 @@ __global__ void __launch_bounds__(256) union_rows_kernel(const int4 *__restrict_
 // One union chunk per work-group (256 threads): EA, DA, GHU and GLU of the chunk's 32 union rows from the FP64 values of
 // the block's kept rows (zero for the rows the block does not keep).  Each plane's 32 rows are read in order into LDS, from
 // which thread (q, lane) takes its 16 points of one row; reading those 16 points from memory took 2.14 ms on (H2O)24
-// (2.7 GB in, 1.1 GB out) where this takes 1.08 ms.
+// (2.7 GB in, 1.1 GB out) where this takes 0.76 ms (1.08 without a plane fetched ahead).
 __global__ void __launch_bounds__(256) fock_operand_prepare_kernel(
     const xq::DevBlock *__restrict__ blocks, const int *__restrict__ uChunkBlock, const int *__restrict__ uRow,
     const double *__restrict__ f, const double *__restrict__ fx, const double *__restrict__ fy,
@@ -309,17 +309,25 @@ __global__ void __launch_bounds__(256) fock_operand_prepare_kernel(
     if (t < kC) sRow[t] = uRow[C * kC + t];
     for (int k = t; k < 3 * kBlockSize; k += 256) sE[k / kBlockSize][k % kBlockSize] = EG[static_cast<size_t>(b) * 3 * kBlockSize + k];
     __syncthreads();
-    // Plane a's rows into LDS: two rows at a time, a thread per point.
-    auto stage = [&](const double *__restrict__ a) {
+    // A plane's rows, two at a time, a thread per point: into registers, while the plane before is cut into digits, then
+    // into LDS.
+    double next[kC / 2];
+    auto fetch = [&](const double *__restrict__ a) {
 #pragma unroll
         for (int r = 0; r < kC; r += 2) {
-            const int i = r + (t >> 7), k = sRow[i];
-            sv[i][t & (kBlockSize - 1)] = k >= 0 ? a[(R + k) * kBlockSize + (t & (kBlockSize - 1))] : 0.0;
+            const int k = sRow[r + (t >> 7)];
+            next[r / 2] = k >= 0 ? a[(R + k) * kBlockSize + (t & (kBlockSize - 1))] : 0.0;
         }
+    };
+    auto stage = [&]() {
+#pragma unroll
+        for (int r = 0; r < kC; r += 2) sv[r + (t >> 7)][t & (kBlockSize - 1)] = next[r / 2];
         __syncthreads();
     };
+    fetch(f);
+    stage();
+    fetch(fx);
     const double *mine = &sv[lr][kC * q + 16 * lh];
-    stage(f);
     // EA: the row's largest value, over the 8 threads (q, lh) that share it.
     double m = 0.0;
 #pragma unroll
@@ -346,7 +354,8 @@ __global__ void __launch_bounds__(256) fock_operand_prepare_kernel(
 #pragma unroll 1
     for (int c = 0; c < 3; c++) {
         __syncthreads();      // every thread is done with the plane before
-        stage(grads[c]);
+        stage();
+        if (c < 2) fetch(grads[c + 1]);
         int Q[16];
 #pragma unroll
         for (int k = 0; k < 16; k++) Q[k] = grad_encode<kGradBitsW>(mine[k], sE[c][kC * q + 16 * lh + k]);
@@ -370,7 +379,8 @@ __global__ void __launch_bounds__(256) fock_operand_prepare_kernel(
 
 // One chunk per work-group (256 threads): DB and GF from the FP64 values of the chunk's rows.  Each plane's 32 rows are read
 // in order into LDS, and consecutive threads write consecutive 16-byte pieces of the operands; threads that each wrote 64
-// bytes of their own took 1.32 ms on (H2O)24 (2.5 GB in, 1.4 GB out) where this takes 1.17 ms.
+// bytes of their own took 1.32 ms on (H2O)24 (2.5 GB in, 1.4 GB out) where this takes 0.88 ms (1.13
+// without a plane fetched ahead).
 __global__ void __launch_bounds__(256) density_operand_prepare_kernel(
     const xq::DevBlock *__restrict__ blocks, const int *__restrict__ chunkOffset, const int *__restrict__ chunkBlock,
     const double *__restrict__ f, const double *__restrict__ fx, const double *__restrict__ fy,
@@ -382,15 +392,24 @@ __global__ void __launch_bounds__(256) density_operand_prepare_kernel(
     const xq::DevBlock blk = blocks[b];
     const int nb = blk.nKept, rc = static_cast<int>(C) - chunkOffset[b], t = threadIdx.x;
     const size_t R = static_cast<size_t>(blk.vOffset) + static_cast<size_t>(kC) * rc;
-    auto stage = [&](const double *__restrict__ a) {
+    // A plane's rows, two at a time, a thread per point: into registers, while the plane before is cut into digits, then
+    // into LDS.
+    double next[kC / 2];
+    auto fetch = [&](const double *__restrict__ a) {
 #pragma unroll
         for (int r = 0; r < kC; r += 2) {
             const int i = r + (t >> 7), p = t & (kBlockSize - 1);
-            sv[i][p] = kC * rc + i < nb ? a[(R + i) * kBlockSize + p] : 0.0;
+            next[r / 2] = kC * rc + i < nb ? a[(R + i) * kBlockSize + p] : 0.0;
         }
+    };
+    auto stage = [&]() {
+#pragma unroll
+        for (int r = 0; r < kC; r += 2) sv[r + (t >> 7)][t & (kBlockSize - 1)] = next[r / 2];
         __syncthreads();
     };
-    stage(f);
+    fetch(f);
+    stage();
+    fetch(fx);
     // DB: thread = (point p, half h) with the 16 rows chunk_fun(h, 0..15).
     {
         const int p = t >> 1, h = t & 1;
@@ -413,7 +432,8 @@ __global__ void __launch_bounds__(256) density_operand_prepare_kernel(
 #pragma unroll 1
     for (int c = 0; c < 3; c++) {
         __syncthreads();      // every thread is done with the plane before
-        stage(grads[c]);
+        stage();
+        if (c < 2) fetch(grads[c + 1]);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const int p = 32 * i + (t >> 3);
