@@ -300,14 +300,17 @@ __global__ void __launch_bounds__(kBlockSize) basis_eval_kernel(
     }
 }
 
-// Values, gradients and second derivatives of one shell (GaussianBasisIntegrals_f1Op1.c:203-331): with e2 = 4 sum c a^2 e^{-a r^2},
-// d2/dx2 phi = (i(i-1) x^{i-2} e0 + (2i+1) x^i e1 + x^{i+2} e2) y^j z^k and
-// d2/dxdy phi = (i j x^{i-1} y^{j-1} e0 + (i x^{i-1} y^{j+1} + j x^{i+1} y^{j-1}) e1 + x^{i+1} y^{j+1} e2) z^k; out[0..9] = phi, x, y,
-// z, xx, xy, xz, yy, yz, zz (nBasis values each, spherical = c2s^T Cartesian).
+// sum_r H_r A_r over a shell's functions r at one point, added to out: H_r the function's Hessian
+// (GaussianBasisIntegrals_f1Op1.c:203-331), with e2 = 4 sum c a^2 e^{-a r^2}
+//     d2/dx2 phi = (i(i-1) x^{i-2} e0 + (2i+1) x^i e1 + x^{i+2} e2) y^j z^k,
+//     d2/dxdy phi = (i j x^{i-1} y^{j-1} e0 + (i x^{i-1} y^{j+1} + j x^{i+1} y^{j-1}) e1 + x^{i+1} y^{j+1} e2) z^k,
+// and A_r a vector.  The vectors are transformed to the Cartesian functions (where the shell's functions are spherical), whose Hessians are then used one
+// by one.
 template <int LL, int LH, bool SPH>
-__device__ __forceinline__ void shell_eval2(const xq::DevShell &sh, const double *__restrict__ coef,
-                                            const double *__restrict__ trans, double dx, double dy, double dz,
-                                            double (*out)[SPH ? ShellDims<LL, LH>::nSph : ShellDims<LL, LH>::nCBF]) {
+__device__ __forceinline__ void shell_second(const xq::DevShell &sh, const double *__restrict__ coef,
+                                             const double *__restrict__ trans, double dx, double dy, double dz,
+                                             const double (&A)[3][SPH ? ShellDims<LL, LH>::nSph : ShellDims<LL, LH>::nCBF],
+                                             double (&out)[3]) {
     constexpr int NC = ShellDims<LL, LH>::nCBF;
     constexpr int NB = SPH ? ShellDims<LL, LH>::nSph : NC;
     constexpr int C0 = cart_offset(LL);
@@ -335,85 +338,144 @@ __device__ __forceinline__ void shell_eval2(const xq::DevShell &sh, const double
         X1[i] = i * X0[i - 1]; Y1[i] = i * Y0[i - 1]; Z1[i] = i * Z0[i - 1];
         X2[i] = i * X1[i - 1]; Y2[i] = i * Y1[i - 1]; Z2[i] = i * Z1[i - 1];
     }
-    double g[10][NC];
 #pragma unroll
     for (int c = 0; c < NC; c++) {
+        double B[3];
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            if (SPH) {
+                const double *T = trans + sh.trans;
+                B[d] = 0.0;
+#pragma unroll
+                for (int r = 0; r < NB; r++) B[d] += T[c * NB + r] * A[d][r];
+            } else {
+                B[d] = A[d][c];
+            }
+        }
         const int i = kCart.x[C0 + c], j = kCart.y[C0 + c], k = kCart.z[C0 + c];
         const double E0 = e0[c], E1 = -2.0 * e1[c], E2 = 4.0 * e2[c];
-        g[0][c] = X0[i] * Y0[j] * Z0[k] * E0;
-        g[1][c] = (X1[i] * E0 + X0[i + 1] * E1) * Y0[j] * Z0[k];
-        g[2][c] = (Y1[j] * E0 + Y0[j + 1] * E1) * X0[i] * Z0[k];
-        g[3][c] = (Z1[k] * E0 + Z0[k + 1] * E1) * X0[i] * Y0[j];
-        g[4][c] = (X2[i] * E0 + (dx * X1[i] + X1[i + 1]) * E1 + X0[i + 2] * E2) * Y0[j] * Z0[k];
-        g[5][c] = (X1[i] * Y1[j] * E0 + (X1[i] * Y0[j + 1] + X0[i + 1] * Y1[j]) * E1 + X0[i + 1] * Y0[j + 1] * E2) * Z0[k];
-        g[6][c] = (X1[i] * Z1[k] * E0 + (X1[i] * Z0[k + 1] + X0[i + 1] * Z1[k]) * E1 + X0[i + 1] * Z0[k + 1] * E2) * Y0[j];
-        g[7][c] = (Y2[j] * E0 + (dy * Y1[j] + Y1[j + 1]) * E1 + Y0[j + 2] * E2) * X0[i] * Z0[k];
-        g[8][c] = (Y1[j] * Z1[k] * E0 + (Y1[j] * Z0[k + 1] + Y0[j + 1] * Z1[k]) * E1 + Y0[j + 1] * Z0[k + 1] * E2) * X0[i];
-        g[9][c] = (Z2[k] * E0 + (dz * Z1[k] + Z1[k + 1]) * E1 + Z0[k + 2] * E2) * X0[i] * Y0[j];
-    }
-#pragma unroll
-    for (int d = 0; d < 10; d++) {
-        if (SPH) {
-            const double *T = trans + sh.trans;
-#pragma unroll
-            for (int s = 0; s < NB; s++) {
-                double a = 0.0;
-#pragma unroll
-                for (int c = 0; c < NC; c++) a += T[c * NB + s] * g[d][c];
-                out[d][s] = a;
-            }
-        } else {
-#pragma unroll
-            for (int s = 0; s < NB; s++) out[d][s] = g[d][s];
-        }
+        const double xx = (X2[i] * E0 + (dx * X1[i] + X1[i + 1]) * E1 + X0[i + 2] * E2) * Y0[j] * Z0[k];
+        const double xy = (X1[i] * Y1[j] * E0 + (X1[i] * Y0[j + 1] + X0[i + 1] * Y1[j]) * E1 + X0[i + 1] * Y0[j + 1] * E2) * Z0[k];
+        const double xz = (X1[i] * Z1[k] * E0 + (X1[i] * Z0[k + 1] + X0[i + 1] * Z1[k]) * E1 + X0[i + 1] * Z0[k + 1] * E2) * Y0[j];
+        const double yy = (Y2[j] * E0 + (dy * Y1[j] + Y1[j + 1]) * E1 + Y0[j + 2] * E2) * X0[i] * Z0[k];
+        const double yz = (Y1[j] * Z1[k] * E0 + (Y1[j] * Z0[k + 1] + Y0[j + 1] * Z1[k]) * E1 + Y0[j + 1] * Z0[k + 1] * E2) * X0[i];
+        const double zz = (Z2[k] * E0 + (dz * Z1[k] + Z1[k + 1]) * E1 + Z0[k + 2] * E2) * X0[i] * Y0[j];
+        out[0] += xx * B[0] + xy * B[1] + xz * B[2];
+        out[1] += xy * B[0] + yy * B[1] + yz * B[2];
+        out[2] += xz * B[0] + yz * B[1] + zz * B[2];
     }
 }
 
-// Dispatch on the shell type; calls body(N, out), N the shell's functions as a compile-time constant.
-template <typename Body>
-__device__ __forceinline__ void with_shell2(const xq::DevShell &sh, bool sph, const double *coef, const double *trans,
-                                            double dx, double dy, double dz, Body body) {
-    for_shell_type(sh, sph, [&](auto ll, auto lh, auto s) {
-        constexpr int N = s ? ShellDims<ll, lh>::nSph : ShellDims<ll, lh>::nCBF;
-        double out[10][N];
-        shell_eval2<ll, lh, s>(sh, coef, trans, dx, dy, dz, out);
-        body(std::integral_constant<int, N>{}, out);
-    });
+// The kept rows h nKept / S .. (h + 1) nKept / S - 1 of a block, S = gridDim.y and h = blockIdx.y.
+__device__ __forceinline__ void row_range(int nKept, int &k0, int &k1) {
+    const long long S = gridDim.y, h = blockIdx.y;
+    k0 = static_cast<int>(h * nKept / S);
+    k1 = static_cast<int>((h + 1) * nKept / S);
 }
 
-// Values and first and second derivatives of the kept functions of blocks b0 + blockIdx.x into rows
-// [vOffset - rowBase, + nKept) of the ten planes out[0..9] (row stride kBlockSize; zero past a block's points).
-__global__ void __launch_bounds__(kBlockSize) basis_eval2_kernel(
+// Values and first derivatives of the kept functions of blocks b0 + blockIdx.x into rows [vOffset - rowBase, + nKept) of the
+// planes out[0..3] (row stride kBlockSize; zero past a block's points).  A shell that straddles two work-groups' rows is
+// evaluated by both.
+__global__ void __launch_bounds__(kBlockSize) basis_planes_kernel(
     int b0, long long rowBase, const xq::DevBlock *__restrict__ blocks, const double *__restrict__ px,
     const double *__restrict__ py, const double *__restrict__ pz, const xq::DevShell *__restrict__ shells,
     const int *__restrict__ shellOf, const double *__restrict__ coef, const double *__restrict__ trans, int spherical,
-    const int *__restrict__ idx, xq::Planes10 out) {
-    const int b = b0 + static_cast<int>(blockIdx.x);
-    const xq::DevBlock blk = blocks[b];
+    const int *__restrict__ idx, xq::Planes4 out) {
+    const xq::DevBlock blk = blocks[b0 + static_cast<int>(blockIdx.x)];
     const int t = threadIdx.x;
     const bool valid = t < blk.nPoints;
     const double x = valid ? px[blk.pStart + t] : 0.0, y = valid ? py[blk.pStart + t] : 0.0,
                  z = valid ? pz[blk.pStart + t] : 0.0;
     const int *kept = idx + blk.iOffset;
-    // Work-group (b, h) writes the kept rows h nKept / S .. (h + 1) nKept / S - 1 (S = gridDim.y); a shell that
-    // straddles two ranges is evaluated by both.
-    const int S = static_cast<int>(gridDim.y), h = static_cast<int>(blockIdx.y);
-    const int k1 = static_cast<int>((static_cast<long long>(h) + 1) * blk.nKept / S);
-    int k = static_cast<int>(static_cast<long long>(h) * blk.nKept / S);
+    int k, k1;
+    row_range(blk.nKept, k, k1);
     while (k < k1) {
         const xq::DevShell &sh = shells[shellOf[kept[k]]];
-        with_shell2(sh, spherical != 0, coef, trans, x - sh.x, y - sh.y, z - sh.z, [&](auto n, const auto &v) {
+        with_shell<true>(sh, spherical != 0, coef, trans, x - sh.x, y - sh.y, z - sh.z,
+                         [&](auto n, const auto &v, const auto &vx, const auto &vy, const auto &vz) {
 #pragma unroll
             for (int j = 0; j < n; j++) {
                 if (k < k1 && kept[k] == sh.fStart + j) {
                     const size_t o = static_cast<size_t>(blk.vOffset - rowBase + k) * kBlockSize + t;
-#pragma unroll
-                    for (int d = 0; d < 10; d++) out.p[d][o] = valid ? v[d][j] : 0.0;
+                    out.p[0][o] = valid ? v[j] : 0.0;
+                    out.p[1][o] = valid ? vx[j] : 0.0;
+                    out.p[2][o] = valid ? vy[j] : 0.0;
+                    out.p[3][o] = valid ? vz[j] : 0.0;
                     k++;
                 }
             }
         });
     }
+}
+
+// The second derivatives' part of the XC gradients of blocks b0 + blockIdx.x: for each kept function r with its atom m,
+// sum_p sum_s X^s_rp H_rp a^s_p (H the function's Hessian at point p, a^s the spins' coefficients coef[..][1..3]) is
+// subtracted from the gradient of m and added to that of the block's atom.  The Hessians are used where they are
+// evaluated, for all spins at once; a thread sums its point over an atom's functions before the wave is reduced.  Bound by
+// FP64 arithmetic.  With ten planes of values and derivatives written and the second ones read by the Z pass, the two
+// took 10.7 ms on (H2O)64; four planes, this kernel (3.2 ms) and the Z pass without them take 9.3 ms.
+__global__ void __launch_bounds__(kBlockSize) second_terms_kernel(
+    int b0, long long rowBase, const xq::DevBlock *__restrict__ blocks, const double *__restrict__ px,
+    const double *__restrict__ py, const double *__restrict__ pz, const xq::DevShell *__restrict__ shells,
+    const int *__restrict__ shellOf, const double *__restrict__ coef, const double *__restrict__ trans, int spherical,
+    const int *__restrict__ idx, const double *__restrict__ X0, const double *__restrict__ X1, int nSpins,
+    const double *__restrict__ pointCoef, const int *__restrict__ skip, int nAtoms, int nCopies, double *__restrict__ copies) {
+    const int local = static_cast<int>(blockIdx.x), b = b0 + local;
+    if (skip[local]) return;
+    const xq::DevBlock blk = blocks[b];
+    const int t = threadIdx.x, lane = t & 63;
+    const bool valid = t < blk.nPoints;
+    const double x = valid ? px[blk.pStart + t] : 0.0, y = valid ? py[blk.pStart + t] : 0.0,
+                 z = valid ? pz[blk.pStart + t] : 0.0;
+    double a0[3], a1[3];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        const double *q = pointCoef + (static_cast<size_t>(local) * 4 * nSpins + 1 + d) * kBlockSize + t;
+        a0[d] = valid ? q[0] : 0.0;
+        a1[d] = valid && nSpins == 2 ? q[4 * kBlockSize] : 0.0;
+    }
+    const int *kept = idx + blk.iOffset;
+    double *grad = copies + static_cast<size_t>((b + static_cast<int>(blockIdx.y)) % nCopies) * 3 * nAtoms;
+    double c[3] = {0.0, 0.0, 0.0}, total[3] = {0.0, 0.0, 0.0};
+    int atom = -1;
+    auto flush = [&]() {
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            double e = c[d];
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) e += __shfl_xor(e, o, 64);
+            if (lane == 0) atomicAdd(&grad[3 * atom + d], -e);
+            total[d] += e;
+            c[d] = 0.0;
+        }
+    };
+    int k, k1;
+    row_range(blk.nKept, k, k1);
+    while (k < k1) {
+        const xq::DevShell &sh = shells[shellOf[kept[k]]];
+        if (sh.atom != atom) {
+            if (atom >= 0) flush();
+            atom = sh.atom;
+        }
+        for_shell_type(sh, spherical != 0, [&](auto ll, auto lh, auto s) {
+            constexpr int N = s ? ShellDims<ll, lh>::nSph : ShellDims<ll, lh>::nCBF;
+            double A[3][N];
+#pragma unroll
+            for (int j = 0; j < N; j++) {
+                const bool has = k < k1 && kept[k] == sh.fStart + j;
+                const size_t o = static_cast<size_t>(blk.vOffset - rowBase + k) * kBlockSize + t;
+                const double x0 = has && valid ? X0[o] : 0.0, x1 = has && valid && nSpins == 2 ? X1[o] : 0.0;
+#pragma unroll
+                for (int d = 0; d < 3; d++) A[d][j] = x0 * a0[d] + x1 * a1[d];
+                k += has ? 1 : 0;
+            }
+            shell_second<ll, lh, s>(sh, coef, trans, x - sh.x, y - sh.y, z - sh.z, A, c);
+        });
+    }
+    if (atom >= 0) flush();
+    if (lane == 0)
+#pragma unroll
+        for (int d = 0; d < 3; d++) atomicAdd(&grad[3 * blk.atom + d], total[d]);
 }
 
 }  // namespace
@@ -642,20 +704,38 @@ int set_basis(xq_grid *g, int nSpec, const double *spec, int spherical, int prec
 }
 
 
-// Basis values, gradients and second derivatives of blocks [b0, b1) into the planes (rows from the blocks' value-row offsets
-// less rowBase), for the XC gradients.
-int eval_basis2(xq_grid *g, int b0, int b1, long long rowBase, const Planes10 &out, hipStream_t s) {
+// Work-groups per block of the two launches below, each a part of its kept rows: the blocks' rows are evaluated one shell
+// after another, so a launch would otherwise last as long as its largest block.
+constexpr unsigned kRowParts = 4;
+
+static int shell_of_functions(xq_grid *g) {
+    if (g->d_shellOf != nullptr) return kOK;
+    XQ_TRY(dev_alloc(g, &g->d_shellOf, g->h_shellOf.size()));
+    XQ_CHECK(hipMemcpyAsync(g->d_shellOf, g->h_shellOf.data(), g->h_shellOf.size() * sizeof(int), hipMemcpyHostToDevice,
+                            g->stream));
+    XQ_CHECK(hipStreamSynchronize(g->stream));
+    return kOK;
+}
+
+// Basis values and gradients of blocks [b0, b1) into the planes (rows from the blocks' value-row offsets less rowBase), for
+// the XC gradients.
+int eval_planes(xq_grid *g, int b0, int b1, long long rowBase, const Planes4 &out, hipStream_t s) {
     if (b1 <= b0) return kOK;
-    if (g->d_shellOf == nullptr) {
-        XQ_TRY(dev_alloc(g, &g->d_shellOf, g->h_shellOf.size()));
-        XQ_CHECK(hipMemcpyAsync(g->d_shellOf, g->h_shellOf.data(), g->h_shellOf.size() * sizeof(int), hipMemcpyHostToDevice,
-                                g->stream));
-        XQ_CHECK(hipStreamSynchronize(g->stream));
-    }
-    // Four work-groups per block, each a quarter of its kept rows: the blocks' rows are evaluated one shell after another,
-    // so a launch would otherwise last as long as its largest block.
-    hipLaunchKernelGGL(basis_eval2_kernel, dim3(b1 - b0, 4), dim3(kBlockSize), 0, s, b0, rowBase, g->d_blocks, g->d_x, g->d_y,
-                       g->d_z, g->d_shells, g->d_shellOf, g->d_coef, g->d_trans, g->spherical, g->d_idx, out);
+    XQ_TRY(shell_of_functions(g));
+    hipLaunchKernelGGL(basis_planes_kernel, dim3(b1 - b0, kRowParts), dim3(kBlockSize), 0, s, b0, rowBase, g->d_blocks,
+                       g->d_x, g->d_y, g->d_z, g->d_shells, g->d_shellOf, g->d_coef, g->d_trans, g->spherical, g->d_idx, out);
+    XQ_CHECK(hipGetLastError());
+    return kOK;
+}
+
+// The second derivatives' part of the XC gradients of blocks [b0, b1), added to nCopies copies of the gradients.
+int second_derivative_terms(xq_grid *g, int b0, int b1, long long rowBase, int spins, const double *X0, const double *X1,
+                            const double *pointCoef, const int *skip, int nCopies, double *copies, hipStream_t s) {
+    if (b1 <= b0) return kOK;
+    XQ_TRY(shell_of_functions(g));
+    hipLaunchKernelGGL(second_terms_kernel, dim3(b1 - b0, kRowParts), dim3(kBlockSize), 0, s, b0, rowBase, g->d_blocks,
+                       g->d_x, g->d_y, g->d_z, g->d_shells, g->d_shellOf, g->d_coef, g->d_trans, g->spherical, g->d_idx,
+                       X0, X1, spins, pointCoef, skip, g->nAtoms, nCopies, copies);
     XQ_CHECK(hipGetLastError());
     return kOK;
 }

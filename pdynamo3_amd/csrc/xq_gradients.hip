@@ -14,10 +14,11 @@
 //   vrho_s and the sigma coefficient 4 vsigma_ss grad rho_s + 2 vsigma_ab grad rho_t (t the other spin).
 // The weight terms (DFTGridWeights_Derivatives) follow per point from eXC (weight_gradient_kernel, xq_grid.hip).
 //
-// Device layout: the basis data of a batch of consecutive blocks in ten planes of rows of 128 points (as the set-up's FP64
-// values), plus X and U planes per spin; batches keep the scratch bounded.  The products P_red Phi and P_red U run on
+// Device layout: the values and first derivatives of a batch of consecutive blocks in four planes of rows of 128 points (as
+// the set-up's FP64 values), plus X and U planes per spin; batches keep the scratch bounded.  The products P_red Phi and P_red U run on
 // FP64 MFMA with P_red staged in LDS, as in the FP64 quadrature's density kernel, one work-group per row chunk of a
-// block and spin; per batch: the X pass, the per-block functional (which forms U), the Z pass.
+// block and spin; per batch: the X pass, the per-block functional (which forms U), the Z pass, and the second
+// derivatives' terms from X (second_terms_kernel, xq_basis.hip).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -32,7 +33,7 @@ namespace xq {
 
 namespace {
 
-// Rows of basis data per batch (12 or 14 planes of 128 doubles per row: about 6.4 or 7.5 GB).  Four times fewer,
+// Rows of basis data per batch (6 or 8 planes of 128 doubles per row: about 3.2 or 4.3 GB).  Four times fewer,
 // larger batches than 131,072 rows took 3.6 ms off an (H2O)64 gradient call: fewer launches, each with its own tail.
 constexpr long long kBatchRows = 524288;
 constexpr int kC = 32;                           // rows per chunk (two 16-row MFMA tiles)
@@ -53,7 +54,7 @@ __device__ __forceinline__ v4d mfma_f64(double a, double b, const v4d &c) {
 // all threads and staged in one of two LDS buffers (one barrier per step), with 32 rows of Bp; the words of P_red are
 // fetched one step ahead, each operand of Bp for the next step as soon as its products of this step are issued.  Staged
 // panels of four chunks, each waited for, took 7.2 ms (X pass) and 9.3 ms (Z pass) per call on (H2O)64; this takes 3.7 and
-// 5.7 ms.
+// 4.1 ms (the Z pass without the second derivatives, which it read then).
 __device__ __forceinline__ void reduced_product(const double *__restrict__ P, int n, const int *idx, int nb,
                                                 const double *__restrict__ Bp, double (&sP)[2][kC][kRowPitch], int I,
                                                 v4d (&acc)[2][2]) {
@@ -120,11 +121,11 @@ struct XcdRanges {
 //   grad_functional_kernel (one work-group per block): rho and grad rho as the sums of the shares in chunk order, the
 //     block skip, the functional, eXC and the coefficients (u0, c) per point, and U_s = u0 Phi + c . grad Phi for the
 //     block's rows;
-//   grad_rows_z_kernel: per spin, Z rows of chunk I = P_s U_s and the per-row terms of chunk I.
+//   grad_rows_z_kernel: per spin, Z rows of chunk I = P_s U_s and the terms Z grad phi of chunk I.
 // The two row-chunk kernels take spin blockIdx.y of nSpins.
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) grad_rows_x_kernel(
     const int4 *__restrict__ items, XcdRanges xr, long long rowBase, const DevBlock *__restrict__ blocks,
-    const int *__restrict__ idxAll, int n, const double *__restrict__ P0, const double *__restrict__ P1, Planes10 B,
+    const int *__restrict__ idxAll, int n, const double *__restrict__ P0, const double *__restrict__ P1, Planes4 B,
     double *__restrict__ Xp0, double *__restrict__ Xp1, double *__restrict__ part, int nSpins) {
     __shared__ double sP[2][kC][kRowPitch];
     __shared__ int sIdx[kIdxCache];
@@ -191,7 +192,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) g
 template <int kSpins>
 __global__ void __launch_bounds__(256) grad_functional_kernel(
     const int2 *__restrict__ blockList, long long rowBase, const DevBlock *__restrict__ blocks,
-    const double *__restrict__ w, FunctionalSet fs, double rhoTol, Planes10 B, const double *__restrict__ part,
+    const double *__restrict__ w, FunctionalSet fs, double rhoTol, Planes4 B, const double *__restrict__ part,
     double *__restrict__ Up0, double *__restrict__ Up1, double *__restrict__ coef, int *__restrict__ skipOut,
     double *__restrict__ eXC) {
     __shared__ double sCoef[4 * kSpins][kBlockSize];
@@ -296,12 +297,10 @@ __global__ void __launch_bounds__(256) grad_functional_kernel(
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) grad_rows_z_kernel(
     const int4 *__restrict__ items, XcdRanges xr, long long rowBase, const DevBlock *__restrict__ blocks,
     const int *__restrict__ idxAll, const int *__restrict__ atomOf, int n, const double *__restrict__ P0,
-    const double *__restrict__ P1, Planes10 B, const double *__restrict__ Xp0, const double *__restrict__ Xp1,
-    const double *__restrict__ Up0, const double *__restrict__ Up1, const double *__restrict__ coef,
+    const double *__restrict__ P1, Planes4 B, const double *__restrict__ Up0, const double *__restrict__ Up1,
     const int *__restrict__ skip, double *__restrict__ gradCopies, int nAtoms, int nSpins) {
     __shared__ double sP[2][kC][kRowPitch];
     __shared__ int sIdx[kIdxCache];
-    __shared__ double sCoef[3][kBlockSize];
     __shared__ double sRed[4][kC][3];
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
     if (slot >= xr.start[xcd + 1] - xr.start[xcd]) return;
@@ -314,22 +313,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) g
     const int *idxG = idxAll + blk.iOffset;
     const int sp = blockIdx.y;
     for (int k = t; k < nb && k < kIdxCache; k += 256) sIdx[k] = idxG[k];
-    if (t < kBlockSize) {
-#pragma unroll
-        for (int k = 0; k < 3; k++)
-            sCoef[k][t] = coef[(static_cast<size_t>(local) * 4 * nSpins + 4 * sp + 1 + k) * kBlockSize + t];
-    }
     __syncthreads();
     const int *idx = nb <= kIdxCache ? sIdx : idxG;
     const size_t R0 = static_cast<size_t>(blk.vOffset - rowBase) * kBlockSize;
     const double *Fx = B.p[1] + R0, *Fy = B.p[2] + R0, *Fz = B.p[3] + R0;
-    const double *Hxx = B.p[4] + R0, *Hxy = B.p[5] + R0, *Hxz = B.p[6] + R0, *Hyy = B.p[7] + R0, *Hyz = B.p[8] + R0,
-                 *Hzz = B.p[9] + R0;
     double *grad = gradCopies + static_cast<size_t>((b + sp) % kGradCopies) * 3 * nAtoms;
     double gs[3] = {0.0, 0.0, 0.0};
     {
-        const double *X = (sp == 0 ? Xp0 : Xp1) + R0;
-        const double *sA = sCoef[0], *sB = sCoef[1], *sC = sCoef[2];
         v4d acc[2][2];
         reduced_product(sp == 0 ? P0 : P1, n, idx, nb, (sp == 0 ? Up0 : Up1) + R0, sP, I, acc);
         double c[2][4][3];
@@ -345,12 +335,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) g
                         const int p = kC * wv + 16 * hn + l16;
                         if (p < np) {
                             const size_t o = static_cast<size_t>(i) * kBlockSize + p;
-                            const double z = acc[hm][hn][v], x = X[o];
-                            const double ax = sA[p], ay = sB[p], az = sC[p];
-                            const double hxy = Hxy[o], hxz = Hxz[o], hyz = Hyz[o];
-                            c[hm][v][0] += z * Fx[o] + x * (Hxx[o] * ax + hxy * ay + hxz * az);
-                            c[hm][v][1] += z * Fy[o] + x * (hxy * ax + Hyy[o] * ay + hyz * az);
-                            c[hm][v][2] += z * Fz[o] + x * (hxz * ax + hyz * ay + Hzz[o] * az);
+                            const double z = acc[hm][hn][v];
+                            c[hm][v][0] += z * Fx[o];
+                            c[hm][v][1] += z * Fy[o];
+                            c[hm][v][2] += z * Fz[o];
                         }
                     }
                 }
@@ -447,9 +435,9 @@ int gradients_on_device(xq_grid *g, const FunctionalSet &fs, int spins, const do
     const long long batchRows = std::max(kBatchRows, maxRows);
     std::vector<double> zeros(3 * static_cast<size_t>(nA), 0.0);
     std::vector<double> zeroCopies(zeros.size() * kGradCopies, 0.0);
-    // Ten basis planes, X and U per spin.
-    const int nPlanes = 10 + 2 * spins;
-    double *planes[14] = {};
+    // Four basis planes, X and U per spin.
+    const int nPlanes = 4 + 2 * spins;
+    double *planes[8] = {};
     double *d_grad = nullptr, *d_eXC = nullptr, *d_copies = nullptr, *d_part = nullptr, *d_coef = nullptr;
     int *d_atomOf = nullptr, *d_skip = nullptr;
     int4 *d_items = nullptr;
@@ -523,14 +511,14 @@ int gradients_on_device(xq_grid *g, const FunctionalSet &fs, int spins, const do
                             "copy items")) != kOK) break;
         if ((status = check(hipMemcpyAsync(d_blockList, blockList.data(), blockList.size() * sizeof(int2),
                                            hipMemcpyHostToDevice, s), "copy block list")) != kOK) break;
-        Planes10 B;
-        for (int k = 0; k < 10; k++) B.p[k] = planes[k];
-        double *Xa = planes[10], *Xb = spins == 2 ? planes[11] : planes[10];
-        double *Ua = planes[10 + spins], *Ub = spins == 2 ? planes[13] : Ua;
+        Planes4 B;
+        for (int k = 0; k < 4; k++) B.p[k] = planes[k];
+        double *Xa = planes[4], *Xb = spins == 2 ? planes[5] : planes[4];
+        double *Ua = planes[4 + spins], *Ub = spins == 2 ? planes[7] : Ua;
         for (size_t k = 0; k < batches.size() && status == kOK; k++) {
             const int b0 = batches[k].first, b1 = batches[k].second;
             const long long rowBase = g->blocks[b0].vOffset;
-            if ((status = eval_basis2(g, b0, b1, rowBase, B, s)) != kOK) break;
+            if ((status = eval_planes(g, b0, b1, rowBase, B, s)) != kOK) break;
             const XcdRanges &xr = ranges[k];
             int perXcd = 0;
             for (int x = 0; x < 8; x++) perXcd = std::max(perXcd, xr.start[x + 1] - xr.start[x]);
@@ -548,9 +536,10 @@ int gradients_on_device(xq_grid *g, const FunctionalSet &fs, int spins, const do
                                    g->d_w, fs, g->rhoTol, B, d_part, Ua, Ub, d_coef, d_skip, d_eXC);
             if (perXcd > 0)
                 hipLaunchKernelGGL(grad_rows_z_kernel, dim3(8 * perXcd, spins), dim3(256), 0, s, it, xr, rowBase,
-                                   g->d_blocks, g->d_idx, d_atomOf, g->nFunctions, d_P0, P1, B, Xa, Xb, Ua, Ub, d_coef,
-                                   d_skip, d_copies, nA, spins);
-            status = check(hipGetLastError(), "direct gradient kernels");
+                                   g->d_blocks, g->d_idx, d_atomOf, g->nFunctions, d_P0, P1, B, Ua, Ub, d_skip, d_copies,
+                                   nA, spins);
+            if ((status = check(hipGetLastError(), "direct gradient kernels")) != kOK) break;
+            status = second_derivative_terms(g, b0, b1, rowBase, spins, Xa, Xb, d_coef, d_skip, kGradCopies, d_copies, s);
         }
         if (status != kOK) break;
         const int nEntries = static_cast<int>(zeros.size());

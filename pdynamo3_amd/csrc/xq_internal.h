@@ -275,11 +275,13 @@ void free_f64(xq_grid *g);
 void free_basis(xq_grid *g);
 void free_work(xq_grid *g);
 int prepare_mixed(xq_grid *g, const double *f, const double *fx, const double *fy, const double *fz);
-// Ten FP64 planes of basis data (phi, its three first and six second derivatives), rows of kBlockSize points.
-struct Planes10 {
-    double *p[10];
+// Four FP64 planes of basis data (phi and its first derivatives), rows of kBlockSize points.
+struct Planes4 {
+    double *p[4];
 };
-int eval_basis2(xq_grid *g, int b0, int b1, long long rowBase, const Planes10 &out, hipStream_t s);
+int eval_planes(xq_grid *g, int b0, int b1, long long rowBase, const Planes4 &out, hipStream_t s);
+int second_derivative_terms(xq_grid *g, int b0, int b1, long long rowBase, int spins, const double *X0, const double *X1,
+                            const double *pointCoef, const int *skip, int nCopies, double *copies, hipStream_t s);
 int gradients(xq_grid *g, int nIDs, const int *ids, const double *Ppacked, double *grad);
 int gradients_uks(xq_grid *g, int nIDs, const int *ids, const double *Pa, const double *Pb, double *grad);
 int weight_gradients(xq_grid *g, const double *d_eXC, double *d_grad, hipStream_t s);
