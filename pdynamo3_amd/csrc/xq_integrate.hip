@@ -113,11 +113,23 @@ void launch_pack_V(xq_grid *g, hipStream_t s) {
                        g->d_packed, 0, nullptr, nullptr);
 }
 
+// Results up to this size are written to the pinned buffer by the packing kernel itself: a copy of 16 KB or more starts
+// later than three small ones and costs 10 us a step ((H2O)2, 20 KB: 160 -> 150 us; (H2O)16, 0.45 MB: 911 -> 901 us).
+// Matrices of many MB go through the copy engine.
+constexpr size_t kDirectResultBytes = size_t(1) << 19;
+
 void launch_pack_results(xq_grid *g, hipStream_t s) {
     const size_t n = static_cast<size_t>(g->nFunctions), work = std::max<size_t>(n * (n + 1) / 2, g->nBlocks);
     const int grid = static_cast<int>(std::min<size_t>((work + 255) / 256, 16384));
-    hipLaunchKernelGGL(pack_lower_kernel, dim3(grid > 0 ? grid : 1), dim3(256), 0, s, g->nFunctions, g->d_V,
-                       g->d_packed, g->nBlocks, g->d_blockEN, g->d_skip);
+    double *out = result_bytes(g) <= kDirectResultBytes ? g->h_stage : g->d_packed;
+    hipLaunchKernelGGL(pack_lower_kernel, dim3(grid > 0 ? grid : 1), dim3(256), 0, s, g->nFunctions, g->d_V, out, g->nBlocks,
+                       g->d_blockEN, g->d_skip);
+}
+
+int copy_results(xq_grid *g, hipStream_t s) {
+    if (result_bytes(g) > kDirectResultBytes)
+        XQ_CHECK(hipMemcpyAsync(g->h_stage, g->d_packed, result_bytes(g), hipMemcpyDeviceToHost, s));
+    return kOK;
 }
 
 // f(begin, end) over 0 .. n - 1, cut between threads; what no thread could be started for runs here.
@@ -313,11 +325,8 @@ static int integrate_jobs_queued(hipStream_t s, const StageEvents &ev, int nJobs
     for (int j = 0; j < nJobs; j++) launch_pack_results(grids[j], s);
     XQ_CHECK(hipGetLastError());
     XQ_CHECK(hipEventRecord(ev.ev1, s));
-    // Results into the pinned buffers (asynchronous DMAs ordered after the kernels), then one wait.
-    for (int j = 0; j < nJobs; j++) {
-        xq_grid *g = grids[j];
-        XQ_CHECK(hipMemcpyAsync(g->h_stage, g->d_packed, result_bytes(g), hipMemcpyDeviceToHost, s));
-    }
+    // Results into the pinned buffers, ordered after the kernels, then one wait.
+    for (int j = 0; j < nJobs; j++) XQ_TRY(copy_results(grids[j], s));
     XQ_CHECK(hipStreamSynchronize(s));
     double bfv = 0.0, bfs = 0.0, bfp = 0.0, rhoBytes = 0.0, fockBytes = 0.0, productBytes = 0.0;
     long long skipped = 0;

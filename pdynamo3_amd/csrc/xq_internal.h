@@ -295,10 +295,11 @@ int upload_density(xq_grid *g, const double *Ppacked, hipStream_t s);
 // four; smaller arrays take less than starting the threads).
 void host_copy(double *to, const double *from, size_t n);
 void host_add(double *to, const double *from, size_t n);
-// A step's results behind each other in d_packed (packed V, the block sums, the skip flags), and their bytes; h_stage takes
-// them with one copy, and h_blockEN and h_skip point into it.
-void launch_pack_results(xq_grid *g, hipStream_t s);
+// A step's results behind each other (packed V, the block sums, the skip flags; result_bytes) in h_stage, into which h_blockEN
+// and h_skip point: written there by the packing kernel, or, when large, in d_packed and copied once.
 size_t result_bytes(const xq_grid *g);
+void launch_pack_results(xq_grid *g, hipStream_t s);
+int copy_results(xq_grid *g, hipStream_t s);
 void free_mixed(xq_grid *g);
 int alloc_step_mixed(xq_grid *g, StepArrays *a);
 void free_step_mixed(xq_grid *g, StepArrays *a);

@@ -155,8 +155,7 @@ int integrate_uks(xq_grid *g, int nIDs, const int *ids, const double *Pa, const 
         launch_pack(n, Vbd, packedB, s);
         if ((status = check(hipGetLastError(), "pack")) != kOK) break;
         if ((status = check(hipEventRecord(g->ev1, s), "event")) != kOK) break;
-        if ((status = check(hipMemcpyAsync(g->h_stage, g->d_packed, result_bytes(g), hipMemcpyDeviceToHost, s),
-                            "copy V alpha, block sums and skips")) != kOK) break;
+        if ((status = copy_results(g, s)) != kOK) break;
         if ((status = check(hipMemcpyAsync(stageB, packedB, nPacked * sizeof(double), hipMemcpyDeviceToHost, s),
                             "copy V beta")) != kOK) break;
         if ((status = check(hipStreamSynchronize(s), "unrestricted quadrature")) != kOK) break;
