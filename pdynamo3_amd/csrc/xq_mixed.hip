@@ -485,10 +485,11 @@ __global__ void __launch_bounds__(256) p_slice_kernel(const xq::MixedJob *__rest
 // are loaded into the registers of the current ones as soon as the products with them are issued.  The row chunks of a
 // block are consecutive items of one XCD, so that their work-groups run at about the same time and read the block's
 // Phi digit chunks, in the same order, through that XCD's L2: Phi comes from HBM about once per block instead of once
-// per row chunk.  At most 168 VGPRs let three work-groups share a CU (four, at 128, spill: 2.53 against 2.31 ms on
-// (H2O)64).  Bound by latency and vector arithmetic: without the gathers it would take 1.98 ms, with grad Phi
-// from L2 2.23; the vector units are busy for a third of the time, the matrix cores for a fifth.  With Phi staged in LDS
-// as well, two barriers a step, and 64-bit integers in the epilogue it took 2.43 ms.
+// per row chunk.  Chunk I's digits stay in registers from step I on (2.26 ms on (H2O)64; read again for the epilogue, with
+// 10% more traffic, 2.31).  At most 168 VGPRs let three work-groups share a CU (four, at 128, spill: 2.53 ms).  Bound by
+// latency and vector arithmetic: of 2.31 ms, gathers that hit the cache save 0.33 and grad Phi from L2 0.1; the vector
+// units are busy for a third of the time, the matrix cores for a fifth.  With Phi staged in LDS as well, two barriers a
+// step, and 64-bit integers in the epilogue it took 2.43 ms.
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
 density_rows_kernel(const xq::MixedJob *__restrict__ jobs, int nJobs, int interleaved) {
     __shared__ __attribute__((aligned(16))) int sP[2][kDP][kC][kPRowDwords];   // [digit][row][K positions / 4]
@@ -540,7 +541,7 @@ density_rows_kernel(const xq::MixedJob *__restrict__ jobs, int nJobs, int interl
     // digits when the products with the current one are issued.
     const v4i *__restrict__ phi = reinterpret_cast<const v4i *>(DBb) + 2 * p + lh;
     unsigned long long wd[4];
-    v4i bq[kDB];
+    v4i bq[kDB], dI[kDB];   // the step's Phi digits, and those of chunk I for the epilogue
     auto fetch_p = [&](int c) {
 #pragma unroll
         for (int jj = 0; jj < 4; jj++) {
@@ -559,6 +560,10 @@ density_rows_kernel(const xq::MixedJob *__restrict__ jobs, int nJobs, int interl
         if constexpr (more) {
             fetch_p(c + 1);
             phi += kChunkBytesB / 16;
+        }
+        if (c == I) {
+#pragma unroll
+            for (int j = 0; j < kDB; j++) dI[j] = bq[j];
         }
         v4i a[kDP];
 #pragma unroll
@@ -587,10 +592,6 @@ density_rows_kernel(const xq::MixedJob *__restrict__ jobs, int nJobs, int interl
         x[v] = ldexp(combined(acc[0][v], acc[1][v], acc[2][v], acc[3][v], acc[4][v]),
                      sPe[chunk_fun(lh, v)] + eb - 7 * (kXOrders + 1));
     }
-    v4i dI[kDB];   // the lane's Phi digits of chunk I
-    const v4i *__restrict__ phiI = reinterpret_cast<const v4i *>(DBb + static_cast<size_t>(I) * kChunkBytesB) + 2 * p + lh;
-#pragma unroll
-    for (int j = 0; j < kDB; j++) dI[j] = phiI[j * kBlockSize * 2];
     double sumR = 0.0, sumG[3] = {0.0, 0.0, 0.0};
 #pragma unroll
     for (int v = 0; v < 16; v++) sumR += digits5(dI, v) * x[v];
