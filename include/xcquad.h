@@ -121,6 +121,10 @@ const char *xq_last_error       ( void ) ;
 !  paths (status 7) and check that the handle is usable afterwards. */
 void        xq_test_fail_allocations ( long long count ) ;
 
+/* Test hook, no counterpart in the reference: the library's check that the runtime has device memory left (6 GB, before the
+!  integrals and the dense steps of an SCF) sees `bytes` free, and what it releases itself; a negative value ends that. */
+void        xq_test_free_memory ( long long bytes ) ;
+
 /* Batched quadratures for a request loop.  No counterpart in the reference (its integrator takes one molecule per call):
 !  the quadratures of several handles (one per job, each with its own P, V and functional) run on the batch's stream, and
 !  each mixed-precision stage is one launch over all the jobs' blocks.  Every job's results are those of xq_integrate

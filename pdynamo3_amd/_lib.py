@@ -40,6 +40,7 @@ SIGNATURES = {
                                           ctypes.POINTER(_dp), _dp]),
     "xq_batch_free": (None, [_vp]),
     "xq_test_fail_allocations": (None, [ctypes.c_longlong]),
+    "xq_test_free_memory": (None, [ctypes.c_longlong]),
 }
 
 # . The SCF wrapper's integrals (include/qcscf.h), in the same library.

@@ -80,6 +80,8 @@ int aufbau(qs_dense *h, const double *fockF, int nOccupied, double *densityP, do
                           h->B, n), "dgemm F X");
     QS_BLAS(rocblas_dgemm(h->blas, rocblas_operation_none, rocblas_operation_none, n, n, n, &one, h->X, n, h->B, n, &zero,
                           h->C, n), "dgemm X F X");
+    // The eigensolver's kernels have private memory; what idle blocks hold of it is released.
+    (void)xq::make_runtime_room("qs_dense_aufbau");
     // Eigenvectors of C in its columns (lower triangle read), eigenvalues ascending.
     QS_BLAS(rocsolver_dsyevd(h->blas, rocblas_evect_original, rocblas_fill_lower, n, h->C, n, h->w, h->e, h->info),
             "rocsolver_dsyevd");

@@ -437,6 +437,7 @@ int qs_one_electron(qs_basis *basis, double *S, double *T, double *V) {
                                                      hipMemcpyHostToDevice, s), "copy pairs");
     if (status == kOK) status = check(hipMemcpyAsync(d_atoms, atoms.data(), atoms.size() * sizeof(double),
                                                      hipMemcpyHostToDevice, s), "copy atoms");
+    if (status == kOK && !set.items.empty()) status = xq::make_runtime_room("one-electron integrals");
     if (status == kOK) status = launch_records(basis, set, d_items, d_records, s);
     if (status == kOK)
         status = for_classes(set, d_items, "one-electron kernels", [&](auto la, auto lb, PairItem *items, int n) {
@@ -560,6 +561,7 @@ int qs_fit_create(const qs_basis *orbital, const qs_basis *fitBasis, qs_fit **ou
                                           "copy rows");
         if (status == kOK) status = check(hipMemcpy(d_items, set.items.data(), set.items.size() * sizeof(PairItem),
                                                     hipMemcpyHostToDevice), "copy pairs");
+        if (status == kOK && !fitSorted.empty()) status = xq::make_runtime_room("fit integrals");
         if (status == kOK) status = launch_records(orbital, set, d_items, d_records, F->stream);
         launch.records = d_records;
         launch.B = F->d_B;
@@ -607,6 +609,7 @@ int qs_fit_matrix(qs_fit *fit, double *M) {
                                                      hipMemcpyHostToDevice, s), "copy fit shells");
     if (status == kOK) status = check(hipMemcpyAsync(d_column, fit->column.data(), nFit * sizeof(int),
                                                      hipMemcpyHostToDevice, s), "copy columns");
+    if (status == kOK && !set.items.empty()) status = xq::make_runtime_room("fit matrix");
     if (status == kOK) status = launch_records(basis, set, d_items, d_records, s);
     FitLaunch launch = fit->launch;
     launch.oShells = basis->d_shells;

@@ -5,8 +5,8 @@
 // takes the smallest cached block of at least its size and at most a quarter larger (sizes are rounded up to 512 bytes,
 // and to 2 MiB above 1 MiB), so a loop whose jobs come and go reuses device memory without runtime calls.  When
 // hipMalloc fails, every cached block is released (hipFree) and the allocation is tried once more; they are released as
-// well before an allocation that would leave less than kRuntimeBytes of free device memory.  A block is cached only after
-// the work that used it has completed: every caller synchronises the owning stream before it frees.
+// well where the runtime may need memory of its own (make_runtime_room).  A block is cached only after the work that used
+// it has completed: every caller synchronises the owning stream before it frees.
 // Pinned host blocks (the staging of P and V) are cached the same way, since hipHostFree synchronises the device too.
 #include <hip/hip_runtime.h>
 
@@ -32,8 +32,9 @@ std::multimap<size_t, void *> g_hostCached;        // pinned host blocks, as abo
 std::unordered_map<void *, size_t> g_hostLive;
 
 // Device memory left to the runtime, which allocates the private memory of a kernel at its dispatch (rocSOLVER's kernels have
-// some) and aborts the process when it cannot: idle blocks must not hold it.
+// some) and aborts the process when it cannot.
 constexpr size_t kRuntimeBytes = size_t(6) << 30;
+long long g_testFree = -1;                         // test hook: the free device memory that make_runtime_room sees (-1: its own)
 
 size_t rounded(size_t bytes) {
     if (bytes == 0) bytes = 1;
@@ -43,6 +44,7 @@ size_t rounded(size_t bytes) {
 
 void release_cached_locked() {
     for (auto &kv : g_cached) (void)hipFree(kv.second);
+    if (g_testFree >= 0) g_testFree += static_cast<long long>(g_cachedBytes);
     g_cached.clear();
     g_cachedBytes = 0;
 }
@@ -64,9 +66,6 @@ hipError_t cache_alloc(void **ptr, size_t bytes) {
         g_cached.erase(it);
         return hipSuccess;
     }
-    size_t freeB = 0, totalB = 0;
-    if (!g_cached.empty() && hipMemGetInfo(&freeB, &totalB) == hipSuccess && freeB < size + kRuntimeBytes)
-        release_cached_locked();
     hipError_t e = hipMalloc(ptr, size);
     if (e != hipSuccess && !g_cached.empty()) {
         (void)hipGetLastError();
@@ -137,9 +136,24 @@ void cache_fail_after(long long count) {
     g_failAfter = count;
 }
 
-void cache_release() {
+void cache_test_free(long long bytes) {
     std::lock_guard<std::mutex> lock(g_mutex);
-    release_cached_locked();
+    g_testFree = bytes;
+}
+
+int make_runtime_room(const char *what) {
+    std::lock_guard<std::mutex> lock(g_mutex);
+    size_t freeB = 0, totalB = 0;
+    for (bool released = false;; released = true) {
+        if (g_testFree >= 0) freeB = static_cast<size_t>(g_testFree);
+        else XQ_CHECK(hipMemGetInfo(&freeB, &totalB));
+        if (freeB >= kRuntimeBytes) return kOK;
+        if (released || g_cached.empty()) break;
+        release_cached_locked();
+    }
+    set_error(std::string(what) + ": " + std::to_string(freeB >> 20) + " MiB of device memory free, " +
+              std::to_string(kRuntimeBytes >> 20) + " MiB needed by the runtime");
+    return kOutOfMemory;
 }
 
 }  // namespace xq

@@ -293,4 +293,6 @@ const char *xq_last_error(void) { return g_lastError.c_str(); }
 
 void xq_test_fail_allocations(long long count) { cache_fail_after(count); }
 
+void xq_test_free_memory(long long bytes) { cache_test_free(bytes); }
+
 }  // extern "C"

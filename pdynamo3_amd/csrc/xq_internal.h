@@ -185,14 +185,18 @@ namespace xq {
 // Process-wide caching allocator (xq_alloc.hip): blocks freed by the library are kept for reuse instead of being
 // returned with hipFree, which synchronises the device.  The caller must have completed all work on a block before it
 // frees it; cache_free returns the bytes that were requested for the block (0 for a pointer it does not know).
-// cache_idle_bytes: bytes held idle; cache_release: hipFree every idle block.
+// cache_idle_bytes: bytes held idle.
 hipError_t cache_alloc(void **ptr, size_t bytes);
 size_t cache_free(void *ptr);
 hipError_t cache_host_alloc(void **ptr, size_t bytes);   // pinned host memory, cached the same way
 void cache_host_free(void *ptr);
 size_t cache_idle_bytes();
-void cache_release();
 void cache_fail_after(long long count);   // test hook: after `count` more device allocations, one fails (-1 disarms)
+void cache_test_free(long long bytes);    // test hook: the free device memory make_runtime_room sees (-1: the device's)
+// Room for the private memory of library kernels, which the runtime allocates at their dispatch: releases the cache's idle
+// blocks if less than 6 GB of device memory are free, and returns kOutOfMemory (with `what` in the message) if there is
+// still less.  An SCF's integrals, which come before its dense steps, refuse then; the dense steps release only.
+int make_runtime_room(const char *what);
 // Allocation helpers that account device bytes on the handle.  Every stage synchronises the handle's stream before it
 // frees what it allocated.
 template <typename T>
