@@ -49,7 +49,8 @@ int  qs_fit_create   ( const qs_basis *orbital, const qs_basis *fit, qs_fit **ou
 int  qs_fit_matrix   ( qs_fit *fit, double *M ) ;
 /* b_P = sum_mn P_mn (mn|P) for a packed density P (nFit values). */
 int  qs_fit_b        ( qs_fit *fit, const double *densityP, double *b ) ;
-/* F_mn += sum_P c_P (mn|P) (packed F, INCREMENTED; c holds nFit values). */
+/* F_mn += sum_P c_P (mn|P) (packed F, INCREMENTED; c holds nFit values).  Calls of qs_fit_b and qs_fit_fock on one handle
+!  from several threads run one after the other. */
 int  qs_fit_fock     ( qs_fit *fit, const double *c, double *fockF ) ;
 /* Device bytes qs_fit_create would allocate for the orbital basis (spec, spherical) and the fit basis (fitSpec,
 !  fitSpherical) on the given atoms, computed on the host with the same pair screen: admission control for a request loop.

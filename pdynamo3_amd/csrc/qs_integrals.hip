@@ -271,6 +271,7 @@ struct qs_fit {
     qs::QShell *d_fitSorted = nullptr;
     std::vector<int> column;           // stored column of each fit function
     double *staging = nullptr;         // pinned: b or c in the order of the columns (nFit), then packed P or F
+    std::mutex step;                   // held while a call's matrices are in the staging and the device arrays
     const qs_basis *orbital = nullptr, *fit = nullptr;
     double *d_B = nullptr;
     long long *d_rowPacked = nullptr;
@@ -654,6 +655,7 @@ int qs_fit_b(qs_fit *fit, const double *P, double *b) {
         for (int k = 0; k < fit->nFit; k++) b[k] = 0.0;
         return kOK;
     }
+    std::lock_guard<std::mutex> lock(fit->step);
     hipStream_t s = fit->stream;
     double *packed = fit->staging + fit->nFit;
     xq::host_copy(packed, P, nPacked);
@@ -678,6 +680,7 @@ int qs_fit_fock(qs_fit *fit, const double *c, double *Fock) {
     if (fit == nullptr || c == nullptr || Fock == nullptr) { set_error("invalid fit arguments"); return kInvalidArgument; }
     const size_t nPacked = static_cast<size_t>(fit->nOrbital) * (fit->nOrbital + 1) / 2;
     if (fit->rows == 0) return kOK;
+    std::lock_guard<std::mutex> lock(fit->step);
     hipStream_t s = fit->stream;
     double *packed = fit->staging + fit->nFit;
     for (int k = 0; k < fit->nFit; k++) fit->staging[fit->column[k]] = c[k];
