@@ -22,6 +22,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstring>
 #include <mutex>
@@ -302,6 +303,15 @@ void qs_release(T **p) {
     if (*p != nullptr) { (void)xq::cache_free(*p); *p = nullptr; }
 }
 
+// An array with at least `count` elements; one that is too small is replaced (the work on it must be done).
+template <typename T>
+int qs_room(T **p, size_t *room, size_t count) {
+    if (*p != nullptr && count <= *room) return kOK;
+    qs_release(p);
+    *room = count;
+    return qs_alloc(p, count);
+}
+
 // Shell pairs sorted by class, and where each class starts; doubles of all their records.
 struct PairSet {
     std::vector<PairItem> items;
@@ -314,15 +324,29 @@ int pair_class(const QShell &a, const QShell &b) {
     return la * (la + 1) / 2 + lb;
 }
 
-// The pairs by class, in their order within a class; row: the first row of each pair's electron-fit integrals, or empty.
-PairSet pair_set(const QBasis *b, const std::vector<QPair> &pairs, const std::vector<long long> &row) {
+// Doubles of the records a set may hold where its pairs may be fewer (256 MB): the records have room for every primitive
+// pair, 50 KB for each pair of 6-31G* waters, and those of all pairs would grow with the square of the molecule
+// (6 GB for 500 waters).  One set covers up to about 100 waters.
+constexpr long long kSliceDoubles = 1LL << 25;
+
+// The pairs first .. last - 1 by class, in their order within a class, last the number of pairs or the first whose records
+// would pass `limit` doubles (at least one is taken); row: the first row of each pair's electron-fit integrals, or empty.
+PairSet pair_set(const QBasis *b, const std::vector<QPair> &pairs, const std::vector<long long> &row, size_t first = 0,
+                 size_t *last = nullptr, long long limit = LLONG_MAX) {
     PairSet set;
-    set.items.resize(pairs.size());
-    for (const QPair &q : pairs) set.start[pair_class(b->shells[q.x], b->shells[q.y]) + 1]++;
+    size_t end = first;
+    for (long long doubles = 0; end < pairs.size(); end++) {
+        const QShell &A = b->shells[pairs[end].x], &B = b->shells[pairs[end].y];
+        doubles += record_room(A, B);
+        if (doubles > limit && end > first) break;
+        set.start[pair_class(A, B) + 1]++;
+    }
+    if (last != nullptr) *last = end;
+    set.items.resize(end - first);
     for (int c = 0; c < 6; c++) set.start[c + 1] += set.start[c];
     int at[6];
     for (int c = 0; c < 6; c++) at[c] = set.start[c];
-    for (size_t k = 0; k < pairs.size(); k++) {
+    for (size_t k = first; k < end; k++) {
         const QShell &A = b->shells[pairs[k].x], &B = b->shells[pairs[k].y];
         set.items[at[pair_class(A, B)]++] =
             pair_item(b->shells.data(), pairs[k].x, pairs[k].y, row.empty() ? 0 : row[k], set.doubles);
@@ -419,7 +443,7 @@ int qs_one_electron(qs_basis *basis, double *S, double *T, double *V) {
         return kInvalidArgument;
     }
     const size_t n = static_cast<size_t>(basis->nFunctions), size = n * (n + 1) / 2;
-    const PairSet set = pair_set(basis, shell_pairs(basis, false), {});
+    const std::vector<QPair> pairs = shell_pairs(basis, false);
     std::vector<double> atoms(4 * static_cast<size_t>(basis->nAtoms));
     for (int a = 0; a < basis->nAtoms; a++) {
         for (int c = 0; c < 3; c++) atoms[4 * a + c] = basis->xyz[3 * a + c];
@@ -427,26 +451,33 @@ int qs_one_electron(qs_basis *basis, double *S, double *T, double *V) {
     }
     PairItem *d_items = nullptr;
     double *d_records = nullptr, *d_atoms = nullptr, *d_S = nullptr, *d_T = nullptr, *d_V = nullptr;
-    int status = qs_alloc(&d_items, set.items.size());
-    if (status == kOK) status = qs_alloc(&d_records, static_cast<size_t>(set.doubles));
-    if (status == kOK) status = qs_alloc(&d_atoms, atoms.size());
+    int status = qs_alloc(&d_atoms, atoms.size());
     if (status == kOK) status = qs_alloc(&d_S, size);
     if (status == kOK) status = qs_alloc(&d_T, size);
     if (status == kOK) status = qs_alloc(&d_V, size);
     hipStream_t s = basis->stream;
-    if (status == kOK) status = check(hipMemcpyAsync(d_items, set.items.data(), set.items.size() * sizeof(PairItem),
-                                                     hipMemcpyHostToDevice, s), "copy pairs");
     if (status == kOK) status = check(hipMemcpyAsync(d_atoms, atoms.data(), atoms.size() * sizeof(double),
                                                      hipMemcpyHostToDevice, s), "copy atoms");
-    if (status == kOK && !set.items.empty()) status = xq::make_runtime_room("one-electron integrals");
-    if (status == kOK) status = launch_records(basis, set, d_items, d_records, s);
-    if (status == kOK)
+    PairSet set;        // one slice after another, each done before the next takes its place
+    size_t room[2] = {0, 0};
+    for (size_t first = 0, last = 0; status == kOK && first < pairs.size(); first = last) {
+        if (first > 0) status = check(hipStreamSynchronize(s), "one-electron integrals");
+        if (status != kOK) break;
+        set = pair_set(basis, pairs, {}, first, &last, kSliceDoubles);
+        status = qs_room(&d_items, &room[0], set.items.size());
+        if (status == kOK) status = qs_room(&d_records, &room[1], static_cast<size_t>(set.doubles));
+        if (status == kOK) status = check(hipMemcpyAsync(d_items, set.items.data(), set.items.size() * sizeof(PairItem),
+                                                         hipMemcpyHostToDevice, s), "copy pairs");
+        if (status == kOK && first == 0) status = xq::make_runtime_room("one-electron integrals");
+        if (status == kOK) status = launch_records(basis, set, d_items, d_records, s);
+        if (status != kOK) break;
         status = for_classes(set, d_items, "one-electron kernels", [&](auto la, auto lb, PairItem *items, int n) {
             hipLaunchKernelGGL((overlap_kinetic_kernel<la, lb>), groups(n, kThreads), dim3(kThreads), 0, s, n, items,
                                basis->d_shells, basis->d_exps, basis->d_coefs, basis->spherical, d_S, d_T);
             hipLaunchKernelGGL((nuclear_kernel<la, lb>), groups(n, 4), dim3(256), 0, s, n, items, basis->d_shells,
                                d_records, basis->nAtoms, d_atoms, basis->spherical, d_V);
         });
+    }
     if (status == kOK) status = check(hipMemcpyAsync(S, d_S, size * sizeof(double), hipMemcpyDeviceToHost, s), "copy S");
     if (status == kOK) status = check(hipMemcpyAsync(T, d_T, size * sizeof(double), hipMemcpyDeviceToHost, s), "copy T");
     if (status == kOK) status = check(hipMemcpyAsync(V, d_V, size * sizeof(double), hipMemcpyDeviceToHost, s), "copy V");

@@ -1,0 +1,68 @@
+"""Integrals of molecules whose pair records do not fit in one slice: the device memory a call takes beside its results, and
+values that do not depend on where the slices are cut (the atoms in reverse order, whose pairs fall into other slices)."""
+
+import ctypes
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+GB = 1 << 30
+
+
+def _free():
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert ctypes.CDLL("libamdhip64.so").hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def _lattice(waters):
+    """Waters 6 bohr apart on a cubic lattice, each turned a little against the one before."""
+    from pdynamo3_amd import molecules
+    Z, xyz = molecules.water()
+    Z, xyz = np.asarray(Z, dtype=np.int32), np.asarray(xyz).reshape(-1, 3)
+    side, out = int(np.ceil(waters ** (1.0 / 3.0))), []
+    for k in range(waters):
+        c, s = np.cos(0.37 * k), np.sin(0.37 * k)
+        turn = np.array([[c, -s, 0.0], [s, c, 0.0], [0.0, 0.0, 1.0]])
+        out.append(xyz @ turn.T + 6.0 * np.array([k % side, k // side % side, k // side ** 2]))
+    return np.tile(Z, waters), np.concatenate(out)
+
+
+def _functions(Z, spec_of):
+    return np.array([spec_of[int(z)] for z in Z])
+
+
+def _reversed_places(Z, per_element):
+    """Places of the functions, in the order of the reversed atoms."""
+    first = np.concatenate([[0], np.cumsum(_functions(Z, per_element))])
+    return np.concatenate([np.arange(first[a], first[a + 1]) for a in range(Z.size - 1, -1, -1)])
+
+
+def _dense(packed, n):
+    out = np.zeros((n, n))
+    out[np.tril_indices(n)] = packed
+    return out + np.tril(out, -1).T
+
+
+def test_one_electron_of_300_waters():
+    from pdynamo3_amd import basis, scf
+    Z, xyz = _lattice(300)
+    data = basis.load_basis()
+    spec = basis.element_spec(data, Z)
+    g = scf.GPUIntegrals(Z, xyz, spec, False, None)
+    before = _free()
+    got = g.one_electron()
+    taken = before - _free()
+    n = g.n
+    g.close()
+    print("functions", n, "device memory taken", taken / GB)
+    assert taken < 1.2 * GB                     # S, T and V are 0.4 GB
+    places = _reversed_places(Z, {z: basis.number_of_functions(data, np.array([z], dtype=np.int32), False) for z in (1, 8)})
+    g = scf.GPUIntegrals(Z[::-1].copy(), xyz[::-1].copy(), spec, False, None)
+    other = g.one_electron()
+    g.close()
+    for a, b in zip(got, other):
+        A = _dense(a, n)[np.ix_(places, places)]
+        assert np.max(np.abs(A - _dense(b, n))) <= 1e-12 * np.max(np.abs(A))
