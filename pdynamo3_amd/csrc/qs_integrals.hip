@@ -134,14 +134,14 @@ __global__ void __launch_bounds__(256) nuclear_kernel(int nPairs, const PairItem
 
 // ------------------------------------------------------------------------------------------------------------------------
 // Fit matrix: its integrals are the electron-fit integrals of pairs of a fit shell with the unit shell (qs_kernels.h), dense
-// with the fit functions' stored columns; here the lower triangle is packed, with the functions' own integrals in the last
-// row.  One thread per entry, and per fit shell.
+// with the fit functions' stored columns; here the lower triangle of the rows p0 .. p1 - 1 is packed, with the functions' own
+// integrals in the last row.  One thread per entry, and per fit shell.
 // ------------------------------------------------------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) fit_matrix_pack_kernel(int nFit, const double *__restrict__ dense,
+__global__ void __launch_bounds__(256) fit_matrix_pack_kernel(int nFit, int p0, int p1, const double *__restrict__ dense,
                                                               const int *__restrict__ column, double *__restrict__ M) {
     const int q = blockIdx.x * 256 + threadIdx.x;
-    for (int p = blockIdx.y; p < nFit; p += gridDim.y)
-        if (q <= p) M[packed_index(p, q)] = dense[static_cast<size_t>(p) * nFit + column[q]];
+    for (int p = p0 + static_cast<int>(blockIdx.y); p < p1; p += gridDim.y)
+        if (q <= p) M[packed_index(p, q)] = dense[static_cast<size_t>(p - p0) * nFit + column[q]];
 }
 
 template <int LA>
@@ -323,6 +323,10 @@ int pair_class(const QShell &a, const QShell &b) {
     const int la = std::max(a.l, b.l), lb = std::min(a.l, b.l);
     return la * (la + 1) / 2 + lb;
 }
+
+// Doubles of the dense rows of the fit matrix that are held at once (256 MB; all of them up to about 150 waters' fit
+// functions): as a whole they would take twice the packed result's memory beside it.
+constexpr long long kSlabDoubles = 1LL << 25;
 
 // Doubles of the records a set may hold where its pairs may be fewer (256 MB): the records have room for every primitive
 // pair, 50 KB for each pair of 6-31G* waters, and those of all pairs would grow with the square of the molecule
@@ -617,39 +621,60 @@ int qs_fit_matrix(qs_fit *fit, double *M) {
     if (fit == nullptr || M == nullptr) { set_error("invalid fit matrix arguments"); return kInvalidArgument; }
     const size_t nFit = static_cast<size_t>(fit->nFit), size = (nFit + 1) * (nFit + 2) / 2;
     const qs_basis *basis = fit->fit;
-    // One pair of every fit shell with the unit shell; a shell's rows are its functions.
-    std::vector<QPair> pairs(basis->shells.size());
-    std::vector<long long> row(pairs.size());
-    for (size_t k = 0; k < pairs.size(); k++) {
-        pairs[k] = QPair{static_cast<int>(k), static_cast<int>(basis->shells.size())};
-        row[k] = basis->shells[k].f0;
-    }
     QBasis withUnit;
     withUnit.shells = basis->shells;
     withUnit.shells.push_back(unit_shell(static_cast<int>(basis->exps.size())));
-    const PairSet set = pair_set(&withUnit, pairs, row);
+    // Slabs of consecutive fit shells, whose functions are consecutive rows: the first shell of each, and the end.
+    const int nShells = static_cast<int>(basis->shells.size());
+    const long long slabRows = std::max<long long>(1, kSlabDoubles / std::max(1, fit->nFit));
+    std::vector<int> slab(1, 0);
+    long long rows = 0, mostRows = 0;
+    for (int k = 0; k < nShells; k++) {
+        if (rows > 0 && rows + basis->shells[k].nf > slabRows) {
+            slab.push_back(k);
+            rows = 0;
+        }
+        rows += basis->shells[k].nf;
+        mostRows = std::max(mostRows, rows);
+    }
+    slab.push_back(nShells);
     PairItem *d_items = nullptr;
     double *d_records = nullptr, *d_dense = nullptr, *d_M = nullptr;
     int *d_column = nullptr;
     const hipStream_t s = fit->stream;
     int status = qs_alloc(&d_M, size);
-    if (status == kOK) status = qs_alloc(&d_dense, nFit * nFit);
+    if (status == kOK) status = qs_alloc(&d_dense, static_cast<size_t>(mostRows) * nFit);
     if (status == kOK) status = qs_alloc(&d_column, nFit);
-    if (status == kOK) status = qs_alloc(&d_items, set.items.size());
-    if (status == kOK) status = qs_alloc(&d_records, static_cast<size_t>(set.doubles));
-    if (status == kOK) status = check(hipMemcpyAsync(d_items, set.items.data(), set.items.size() * sizeof(PairItem),
-                                                     hipMemcpyHostToDevice, s), "copy fit shells");
     if (status == kOK) status = check(hipMemcpyAsync(d_column, fit->column.data(), nFit * sizeof(int),
                                                      hipMemcpyHostToDevice, s), "copy columns");
-    if (status == kOK && !set.items.empty()) status = xq::make_runtime_room("fit matrix");
-    if (status == kOK) status = launch_records(basis, set, d_items, d_records, s);
+    if (status == kOK && nShells > 0) status = xq::make_runtime_room("fit matrix");
     FitLaunch launch = fit->launch;
     launch.oShells = basis->d_shells;
     launch.oSpherical = basis->spherical;
-    launch.records = d_records;
     launch.cut = -1.0;
     launch.B = d_dense;
-    if (status == kOK)
+    PairSet set;        // one slab after another, each done before the next takes its place
+    size_t room[2] = {0, 0};
+    for (size_t b = 0; status == kOK && nShells > 0 && b + 1 < slab.size(); b++) {
+        if (b > 0) status = check(hipStreamSynchronize(s), "fit matrix");
+        if (status != kOK) break;
+        // One pair of every fit shell of the slab with the unit shell; a shell's rows are its functions.
+        const int k0 = slab[b], k1 = slab[b + 1], p0 = basis->shells[k0].f0,
+                  p1 = basis->shells[k1 - 1].f0 + basis->shells[k1 - 1].nf;
+        std::vector<QPair> pairs;
+        std::vector<long long> row;
+        for (int k = k0; k < k1; k++) {
+            pairs.push_back(QPair{k, nShells});
+            row.push_back(basis->shells[k].f0 - p0);
+        }
+        set = pair_set(&withUnit, pairs, row);
+        status = qs_room(&d_items, &room[0], set.items.size());
+        if (status == kOK) status = qs_room(&d_records, &room[1], static_cast<size_t>(set.doubles));
+        if (status == kOK) status = check(hipMemcpyAsync(d_items, set.items.data(), set.items.size() * sizeof(PairItem),
+                                                         hipMemcpyHostToDevice, s), "copy fit shells");
+        if (status == kOK) status = launch_records(basis, set, d_items, d_records, s);
+        if (status != kOK) break;
+        launch.records = d_records;
         status = for_classes(set, d_items, "fit matrix kernels", [&](auto la, auto lb, PairItem *items, int n) {
             if constexpr (lb == 0) {     // the unit shell is the second of every pair
                 launch_fit<la, 0, 0>(launch, items, n);
@@ -660,10 +685,10 @@ int qs_fit_matrix(qs_fit *fit, double *M) {
                                    d_M + nFit * (nFit + 1) / 2);
             }
         });
-    if (status == kOK && nFit > 0) {
+        if (status != kOK) break;
         hipLaunchKernelGGL(fit_matrix_pack_kernel, dim3(static_cast<unsigned>((nFit + 255) / 256),
-                                                        static_cast<unsigned>(std::min<size_t>(nFit, 65535))),
-                           dim3(256), 0, s, fit->nFit, d_dense, d_column, d_M);
+                                                        static_cast<unsigned>(std::min(p1 - p0, 65535))),
+                           dim3(256), 0, s, fit->nFit, p0, p1, d_dense, d_column, d_M);
         status = check(hipGetLastError(), "fit_matrix_pack_kernel");
     }
     const int drained = check(hipStreamSynchronize(s), "fit matrix");

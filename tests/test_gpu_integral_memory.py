@@ -66,3 +66,30 @@ def test_one_electron_of_300_waters():
     for a, b in zip(got, other):
         A = _dense(a, n)[np.ix_(places, places)]
         assert np.max(np.abs(A - _dense(b, n))) <= 1e-12 * np.max(np.abs(A))
+
+
+def test_fit_matrix_of_250_waters():
+    """One tight s function per atom as the orbital basis: the fit integrals themselves stay small."""
+    from pdynamo3_amd import basis, scf
+    Z, xyz = _lattice(250)
+    shell = {"lLow": 0, "lHigh": 0, "exponents": [50.0], "coefficients": [[1.0]]}
+    spec = basis.element_spec({"label": "s", "elements": {z: {"shells": [shell]} for z in ("1", "8")}}, Z)
+    data = basis.load_basis("dgauss-a1-dftjfit")
+    fit = basis.element_spec(data, Z)
+    g = scf.GPUIntegrals(Z, xyz, spec, False, fit)
+    before = _free()
+    got = g.fit_matrix()
+    taken = before - _free()
+    n = g.n_fit
+    g.close()
+    print("fit functions", n, "device memory taken", taken / GB)
+    assert taken < 0.75 * GB                    # the packed matrix is 0.4 GB
+    places = _reversed_places(Z, {z: basis.number_of_functions(data, np.array([z], dtype=np.int32), True) for z in (1, 8)})
+    places = np.concatenate([places, [n]])
+    g = scf.GPUIntegrals(Z[::-1].copy(), xyz[::-1].copy(), spec, False, fit)
+    other = g.fit_matrix()
+    g.close()
+    A = _dense(got, n + 1)
+    A = A[np.ix_(places, places)]
+    B = _dense(other, n + 1)
+    assert np.max(np.abs(A - B)) <= 1e-12 * np.max(np.abs(A))
