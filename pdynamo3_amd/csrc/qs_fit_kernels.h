@@ -4,6 +4,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "qs_kernels.h"
 
 namespace qs {
@@ -29,6 +31,9 @@ template <int LA, int LB, int LC>
 void launch_fit(const FitLaunch &f, const PairItem *items, int n);
 
 #ifdef QS_FIT_KERNELS
+
+// Waves of one launch: a launch holds less than 2^32 threads.
+constexpr int kLaunchWaves = 1 << 25;
 
 // One wave per pair and 64 fit shells of an angular momentum, components M0 .. M0 + NM - 1 of the shells.  The pair's
 // records are read as scalars, and a lane holds its fit shell's Hermite integrals and its part of the block in registers
@@ -68,13 +73,16 @@ void launch_fit(const FitLaunch &f, const PairItem *items, int n) {
     constexpr int NM = fit_group<LA, LB, LC>();
     const int shells = f.first[LC + 1] - f.first[LC];
     if (shells == 0 || n == 0) return;
-    const long long waves = static_cast<long long>(n) * ((shells + 63) / 64);
-    const dim3 grid(static_cast<unsigned>((waves + 3) / 4));
-    static_for<cartesians(LC) / NM>([&](auto group) {
-        hipLaunchKernelGGL((fit_integrals_kernel<LA, LB, LC, group * NM, NM>), grid, dim3(256), 0, f.stream, n, items,
-                           f.oShells, f.oSpherical, f.records, shells, f.fShells + f.first[LC], f.fSpherical, f.fExps,
-                           f.fCoefs, f.boys, f.column[LC], f.nFit, f.cut, f.B);
-    });
+    const int chunks = (shells + 63) / 64, most = std::max(1, kLaunchWaves / chunks);
+    for (int k = 0; k < n; k += most) {
+        const int m = std::min(most, n - k);
+        const dim3 grid(static_cast<unsigned>((static_cast<long long>(m) * chunks + 3) / 4));
+        static_for<cartesians(LC) / NM>([&](auto group) {
+            hipLaunchKernelGGL((fit_integrals_kernel<LA, LB, LC, group * NM, NM>), grid, dim3(256), 0, f.stream, m, items + k,
+                               f.oShells, f.oSpherical, f.records, shells, f.fShells + f.first[LC], f.fSpherical, f.fExps,
+                               f.fCoefs, f.boys, f.column[LC], f.nFit, f.cut, f.B);
+        });
+    }
 }
 
 #endif

@@ -1,5 +1,6 @@
 """Integrals of molecules whose pair records do not fit in one slice: the device memory a call takes beside its results, and
-values that do not depend on where the slices are cut (the atoms in reverse order, whose pairs fall into other slices)."""
+values that do not depend on where the slices are cut (the atoms in reverse order, whose pairs fall into other slices).
+Electron-fit integrals that one launch cannot hold, against their closed form."""
 
 import ctypes
 
@@ -93,3 +94,38 @@ def test_fit_matrix_of_250_waters():
     A = A[np.ix_(places, places)]
     B = _dense(other, n + 1)
     assert np.max(np.abs(A - B)) <= 1e-12 * np.max(np.abs(A))
+
+
+def test_fit_integrals_beyond_one_launch():
+    """One s function on each of 11,700 H atoms and one s fit function on an O atom: 68 million shell pairs, a wave each.
+    (ab|c) = 2 pi^(5/2) / (p g sqrt(p + g)) c_a c_b c_c exp(-a R^2 / 2) F_0(T), p = 2 a, T = p g / (p + g) |P - C|^2."""
+    from scipy.special import erf
+    from pdynamo3_amd import basis, scf
+    n, a, g = 11700, 0.1, 1.0
+    rng = np.random.default_rng(8)
+    xyz = np.concatenate([np.zeros((1, 3)), rng.uniform(-4.0, 4.0, (n, 3))])
+    Z = np.array([8] + [1] * n, dtype=np.int32)
+
+    def spec(on, exponent):
+        shell = {"lLow": 0, "lHigh": 0, "exponents": [exponent], "coefficients": [[1.0]]}
+        return basis.element_spec({"label": "s", "elements": {z: {"shells": [shell] if z == on else []} for z in ("1", "8")}}, Z)
+
+    ints = scf.GPUIntegrals(Z, xyz, spec("1", a), False, spec("8", g))
+    pairs = n * (n + 1) // 2
+    assert ints.n_fit == 1 and ints.stats()["fit_rows"] == pairs > 1 << 26
+    F = np.zeros(pairs)
+    ints.fit_fock(np.ones(1), F)
+    ints.close()
+    k = np.concatenate([rng.integers(0, pairs, 200000), np.arange(1000), pairs - 1 - np.arange(1000),
+                        (1 << 25) + np.arange(-500, 500), (1 << 26) + np.arange(-500, 500)])
+    i = ((np.sqrt(8.0 * k + 1.0) - 1.0) / 2.0).astype(np.int64)
+    i += (i + 1) * (i + 2) // 2 <= k
+    i -= i * (i + 1) // 2 > k
+    j = k - i * (i + 1) // 2
+    assert np.all((0 <= j) & (j <= i))
+    A, B = xyz[1 + i], xyz[1 + j]
+    p, norm = 2.0 * a, (2.0 * a / np.pi) ** 1.5 * (2.0 * g / np.pi) ** 0.75
+    T = p * g / (p + g) * np.sum((0.5 * (A + B)) ** 2, axis=1)
+    F0 = 0.5 * np.sqrt(np.pi / T) * erf(np.sqrt(T))
+    want = norm * 2.0 * np.pi ** 2.5 / (p * g * np.sqrt(p + g)) * np.exp(-0.5 * a * np.sum((A - B) ** 2, axis=1)) * F0
+    assert np.max(np.abs(F[k] - want)) < 1e-12
