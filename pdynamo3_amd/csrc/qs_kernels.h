@@ -101,8 +101,9 @@ struct PairClass {
     static constexpr int na = cartesians(LA), nb = cartesians(LB), size = table.size;
 };
 
-// Primitive pairs whose prefactor c_a c_b exp(-mu R^2) is below this are left out of a pair's records: their integrals
-// are below 1e-16 for any exponents and distances of a basis (the kept ones' smallest are 1e-12).
+// Primitive pairs are left out of a pair's records when their integrals with a unit charge are below about this.  An
+// integral is at most the prefactor |c_a c_b| exp(-mu R^2) times 2 pi / p for a nucleus (pi^(5/2) / (p g sqrt(p + g)), c_c
+// in it, for a fit function), times a power of lengths, R between the centres and p^(-1/2) of the product, that is la + lb.
 constexpr double kPrimitiveScreen = 1.0e-24;
 
 // The records of a pair (A of LA, B of LB) at out, size doubles apart; returns their number.
@@ -118,7 +119,9 @@ QS_HD int pair_records(const QShell &A, const QShell &B, const double *__restric
         for (int qb = 0; qb < B.nPrim; qb++) {
             const double a = exps[A.prim + qa], b = exps[B.prim + qb], p = a + b, ip = 1.0 / p, h = 0.5 * ip;
             const double K = coefs[A.prim + qa] * coefs[B.prim + qb] * exp(-a * b * ip * r2);
-            if (fabs(K) < kPrimitiveScreen) continue;
+            double bound = fabs(K) * fmax(1.0, ip) * fmax(1.0, ip);
+            static_for<(LA + LB + 1) / 2>([&](auto) { bound *= fmax(1.0, r2 + ip); });
+            if (bound < kPrimitiveScreen) continue;
             double *rec = out + static_cast<long long>(n) * C::size;
             n++;
             rec[0] = p;
