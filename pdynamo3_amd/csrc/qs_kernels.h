@@ -493,10 +493,10 @@ inline PairItem pair_item(const QShell *shells, int a, int b, long long row, lon
 }
 // Doubles of a pair's records, all its primitive pairs kept.
 inline long long record_room(const QShell &A, const QShell &B) {
-    long long size = 0;
-    with_pair_class(A.l > B.l ? A.l : B.l, A.l > B.l ? B.l : A.l,
-                    [&](auto la, auto lb) { size = PairClass<la, lb>::size; });
-    return size * A.nPrim * B.nPrim;
+    static constexpr long long size[3][3] = {{PairClass<0, 0>::size, PairClass<1, 0>::size, PairClass<2, 0>::size},
+                                             {PairClass<1, 0>::size, PairClass<1, 1>::size, PairClass<2, 1>::size},
+                                             {PairClass<2, 0>::size, PairClass<2, 1>::size, PairClass<2, 2>::size}};
+    return size[A.l][B.l] * A.nPrim * B.nPrim;
 }
 
 // The unit function as an s shell whose one primitive, of exponent 0 and coefficient 1, is at prim: a pair with it is the
