@@ -91,11 +91,11 @@ __device__ __forceinline__ v16i mfma_i8(const v4i &a, const v4i &b, const v16i &
 
 // The D digits of x in a group of power of two e.  The integer Q = round(x 2^(7D - e)) is exact in FP64; its first four digits
 // come from one 32-bit word and a fifth from the remainder, so that nothing is converted to 64-bit integers (which takes
-// about ten instructions).
+// about ten instructions).  A NaN has the digits of zero (fmin alone would make it the largest magnitude).
 template <int D>
 __device__ __forceinline__ void slice(double x, int e, signed char *d) {
     static_assert(D == 4 || D == 5, "four digits fill one word");
-    const double Q = rint(ldexp(x, 7 * D - e));
+    const double Q = x == x ? rint(ldexp(x, 7 * D - e)) : 0.0;
     // |x| < 2^e, so |Q| <= 2^(7D); the one value that rounds up to 2^(7D) is clamped to the largest D-digit magnitude.
     const double a = fmin(fabs(Q), static_cast<double>((1ull << (7 * D)) - 1ull));
     const int s = Q < 0.0 ? -1 : 0;      // (digit ^ s) - s is the digit with Q's sign
@@ -181,11 +181,11 @@ __device__ __forceinline__ int ubyte_of(const v4i &x, int v) {
 // Element v (0..15) of sixteen int32 held in four 16-byte operands.
 __device__ __forceinline__ double int_of(const v4i (&g)[4], int v) { return static_cast<double>(g[v >> 2][v & 3]); }
 
-// B-bit fixed point of g with |g| < 2^e: round(g 2^(B - e)) in [-(2^B - 1), 2^B - 1] (B <= 31).
+// B-bit fixed point of g with |g| < 2^e: round(g 2^(B - e)) in [-(2^B - 1), 2^B - 1] (B <= 31); zero for a NaN.
 template <int B>
 __device__ __forceinline__ int grad_encode(double g, int e) {
     constexpr double lim = static_cast<double>((1ll << B) - 1);
-    return static_cast<int>(fmin(fmax(rint(ldexp(g, B - e)), -lim), lim));
+    return g == g ? static_cast<int>(fmin(fmax(rint(ldexp(g, B - e)), -lim), lim)) : 0;
 }
 
 // Row of a chunk held at density position 16 h + v (K position 4 q + j holds row 8 j + q).
