@@ -1,7 +1,6 @@
 // The integral work items of the SCF wrapper (a shell pair, a fit shell pair or a shell pair with a fit shell each), as host
 // and device functions: the GPU kernels of qs_integrals.hip call them, and a host build of this header checks the same
-// code against the compiled reference on the CPU.  The mathematics is in qs_md.h; the Boys table and the c2s transformation
-// come in as arguments.
+// code against the compiled reference on the CPU.  The mathematics is in qs_md.h; the Boys table comes in as an argument.
 //
 // The one-electron and electron-fit integrals are templates over the shells' angular momenta ("classes", la >= lb: a pair
 // whose first shell has the lower one swaps the roles of its shells), so that every loop over Cartesian components and
@@ -165,7 +164,10 @@ QS_HD int pair_records(const QShell &A, const QShell &B, const double *__restric
     return n;
 }
 
-// F_L(T) .. F_0(T) as boys (qs_md.h), the order fixed; row L of the table is read once.
+// Boys function F_L(T) .. F_0(T) from the table F[k][n] = F_n(k step), n < kBoysTable: a Taylor expansion of F_L about the
+// nearest tabulated T (|dT| <= step / 2, kBoysTaylor + 1 terms) and downward recursion F_n = (2 T F_n+1 + exp(-T)) / (2n + 1);
+// beyond the table, F_0 = sqrt(pi / T) / 2 and upward recursion F_n+1 = ((2n + 1) F_n - exp(-T)) / (2T), which is stable for
+// large T.
 template <int L>
 QS_HD void boys_of(double T, const double *__restrict__ table, double (&F)[L + 1]) {
     if (T < kBoysTMax) {
@@ -198,7 +200,7 @@ QS_HD void boys_of(double T, const double *__restrict__ table, double (&F)[L + 1
     }
 }
 
-// R_tuv (t + u + v <= L) of hermite_r (qs_md.h) times scale, at R[(t * (L + 1) + u) * (L + 1) + v].
+// Hermite integrals R_tuv (t + u + v <= L; qs_md.h) times scale, at R[(t * (L + 1) + u) * (L + 1) + v].
 constexpr int hermite_steps(int L) {
     int c = 0;
     for (int n = L - 1; n >= 0; n--)
@@ -515,9 +517,20 @@ QS_HD long long pair_row(const PairItem &it, int i, int j, int ma, int mb) {
 }
 
 // ------------------------------------------------------------------------------------------------------------------------
-// One whole work item on the host, for the CPU check of the code above (not part of the GPU build).
+// One whole work item on the host, for the CPU check of the code above (not part of the GPU build).  The unnamed arguments
+// are c2s transformations, which the unrolled forms have as constants.
 // ------------------------------------------------------------------------------------------------------------------------
 #ifndef __HIPCC__
+// F_0 .. F_m (m <= kMaxR) by the fixed-order function of the kernels.
+inline void boys(int m, double T, const double *table, double *F) {
+    static_for<kMaxR + 1>([&](auto l) {
+        if (m != l) return;
+        double f[l + 1];
+        boys_of<l>(T, table, f);
+        for (int n = 0; n <= l; n++) F[n] = f[n];
+    });
+}
+
 // Overlap, kinetic and electron-nuclear blocks of shell pair k (A >= B), written into the packed matrices (mu >= nu).
 inline void one_electron_pair(int k, const QPair *pairs, const QShell *shells, const double *exps, const double *coefs,
                               int nAtoms, const double *atoms, int spherical, const double *boysTable, const double *,

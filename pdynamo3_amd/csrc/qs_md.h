@@ -40,28 +40,4 @@ constexpr double kBoysStep = 0.05;             // table spacing in T
 constexpr int kBoysPoints = 801;               // T = 0 .. 40
 constexpr double kBoysTMax = kBoysStep * (kBoysPoints - 1);
 
-// Boys function F_0 .. F_m (m <= kMaxR) at T from the table F[k][n] = F_n(k step), n < kBoysTable: a Taylor expansion of
-// F_m about the nearest tabulated T (|dT| <= step / 2, kBoysTaylor + 1 terms) and downward recursion
-// F_n = (2 T F_n+1 + exp(-T)) / (2n + 1); beyond the table, F_0 = sqrt(pi / T) / 2 and upward recursion
-// F_n+1 = ((2n + 1) F_n - exp(-T)) / (2T), which is stable for large T.
-QS_HD void boys(int m, double T, const double *__restrict__ table, double *F) {
-    if (T < kBoysTMax) {
-        const int k = static_cast<int>(T / kBoysStep + 0.5);
-        const double d = T - k * kBoysStep;
-        const double *row = table + k * kBoysTable;
-        double s = 0.0, term = 1.0;
-        for (int j = 0; j <= kBoysTaylor; j++) {
-            s += row[m + j] * term;
-            term *= -d / (j + 1);
-        }
-        F[m] = s;
-        const double e = exp(-T);
-        for (int n = m - 1; n >= 0; n--) F[n] = (2.0 * T * F[n + 1] + e) / (2 * n + 1);
-    } else {
-        const double e = exp(-T);
-        F[0] = 0.5 * sqrt(M_PI / T);
-        for (int n = 0; n < m; n++) F[n + 1] = ((2 * n + 1) * F[n] - e) / (2.0 * T);
-    }
-}
-
 }  // namespace qs

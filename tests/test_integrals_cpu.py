@@ -69,3 +69,19 @@ def test_attraction_of_distant_diffuse_pairs(host, exponent):
             want = f * _attraction(exponent, A, u, exponent, B, v, nuclei)
             got = V[i * (i + 1) // 2 + j]
             assert abs(got - want) <= 1e-8 * abs(want) + 1e-22, (u, v, got, want)
+
+
+@pytest.mark.parametrize("order", range(7))
+def test_boys_function_between_its_table_points(host, order):
+    """Every order by the kernels' own code, at the table's points (0.05 apart), midway between them and at both sides of its
+    end (T = 40), against Gauss-Legendre of t^2n exp(-T t^2) in pieces."""
+    t, w = np.polynomial.legendre.leggauss(40)
+    for T in (0.0, 0.025, 0.025 - 1e-12, 0.05, 1.225, 7.775, 19.975, 39.975, 40.0 - 1e-9, 40.0, 40.0 + 1e-9, 40.025, 300.0):
+        F = np.zeros(order + 1)
+        host.qsh_boys(order, ctypes.c_double(T), _lib.dptr(F))
+        edges = np.linspace(0.0, min(1.0, 7.0 / np.sqrt(max(T, 1e-300))), 6)     # exp(-49) beyond
+        for n in range(order + 1):
+            want = sum(0.5 * (b - a) * np.sum(w * (0.5 * (a + b) + 0.5 * (b - a) * t) ** (2 * n) *
+                                              np.exp(-T * (0.5 * (a + b) + 0.5 * (b - a) * t) ** 2))
+                       for a, b in zip(edges[:-1], edges[1:]))
+            assert abs(F[n] - want) <= 2e-14 * want, (T, n, F[n], want)
