@@ -15,12 +15,11 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
-#include <system_error>
-#include <thread>
 #include <vector>
 
 #include "xq_functional.h"
 #include "xq_internal.h"
+#include "xq_ranges.h"
 
 namespace xq {
 
@@ -130,30 +129,6 @@ int copy_results(xq_grid *g, hipStream_t s) {
     if (result_bytes(g) > kDirectResultBytes)
         XQ_CHECK(hipMemcpyAsync(g->h_stage, g->d_packed, result_bytes(g), hipMemcpyDeviceToHost, s));
     return kOK;
-}
-
-// f(begin, end) over 0 .. n - 1, cut between threads; what no thread could be started for runs here.
-template <typename F>
-static void in_ranges(size_t n, F f) {
-    constexpr size_t kPerThread = size_t{1} << 18;      // doubles: 2 MB
-    const size_t parts = std::min<size_t>({4, n / kPerThread, std::max<size_t>(1, std::thread::hardware_concurrency())});
-    if (parts <= 1) { f(size_t{0}, n); return; }
-    std::thread threads[3];
-    size_t done = n / parts;            // the first part is this thread's
-    const size_t own = done;
-    for (size_t k = 1; k < parts; k++) {
-        const size_t end = n * (k + 1) / parts;
-        try {
-            threads[k - 1] = std::thread(f, done, end);
-        } catch (const std::system_error &) {
-            break;
-        }
-        done = end;
-    }
-    f(size_t{0}, own);
-    f(done, n);
-    for (std::thread &t : threads)
-        if (t.joinable()) t.join();
 }
 
 void host_copy(double *to, const double *from, size_t n) {
