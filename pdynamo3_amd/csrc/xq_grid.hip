@@ -260,7 +260,8 @@ struct PairRow {
 
 // Share of the largest cell product at a point below which an atom's product does not count: in the sum of the products, and
 // in the derivatives, where a factor s = c y^11 P (y = 1 - nu) near its zero has a derivative of 11 s / y, so that a dropped
-// term is below 1e-16 of the point's energy over a bond length.
+// term is below 1e-16 of the point's energy over a bond length.  With 2^-80 gradients and weights are the same to 2e-15 and
+// (H2O)64 gradients take 39.6 instead of 35.1 ms.
 constexpr double kCellScreen = 0x1p-64;
 
 // Candidate points of one radial shell and their Becke weights w = 4 pi w_r w_ang P_A / sum_i P_i (DFTGrid.c:158-211,

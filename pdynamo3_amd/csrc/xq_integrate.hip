@@ -105,16 +105,10 @@ void launch_pack(int n, const double *dense, double *packed, hipStream_t s) {
                        nullptr);
 }
 
-void launch_pack_V(xq_grid *g, hipStream_t s) {
-    const size_t n = static_cast<size_t>(g->nFunctions), nPacked = n * (n + 1) / 2;
-    const int grid = static_cast<int>(std::min<size_t>((nPacked + 255) / 256, 16384));
-    hipLaunchKernelGGL(pack_lower_kernel, dim3(grid > 0 ? grid : 1), dim3(256), 0, s, g->nFunctions, g->d_V,
-                       g->d_packed, 0, nullptr, nullptr);
-}
-
-// Results up to this size are written to the pinned buffer by the packing kernel itself: a copy of 16 KB or more starts
-// later than three small ones and costs 10 us a step ((H2O)2, 20 KB: 160 -> 150 us; (H2O)16, 0.45 MB: 911 -> 901 us).
-// Matrices of many MB go through the copy engine.
+// Results up to this size are written to the pinned buffer by the packing kernel itself, which saves starting a copy: about
+// 10 us a step at every size measured, against a copy of the same results (6 KB: 142 against 155 us; 362 KB: 961 against
+// 970; 566 KB: 1247 against 1255; 3.2 MB: 3716 to 3741 against 3720).  Above the line that is less than 1% of a step, lost
+// in its noise at 3 MB, and matrices of many MB would keep the packing kernel at the rate of PCIe.
 constexpr size_t kDirectResultBytes = size_t(1) << 19;
 
 void launch_pack_results(xq_grid *g, hipStream_t s) {

@@ -260,7 +260,6 @@ int integrate_uks(xq_grid *g, int nIDs, const int *ids, const double *Pa, const 
                   double *Va, double *Vb, double *stats);
 void launch_expand_P(xq_grid *g, hipStream_t s);
 void launch_zero_V(xq_grid *g, hipStream_t s);
-void launch_pack_V(xq_grid *g, hipStream_t s);
 // The same on explicit arrays: packed lower triangle -> dense n x n, zero n x n, dense -> packed.
 void launch_expand(int n, const double *packed, double *dense, hipStream_t s);
 void launch_zero(int n, double *dense, hipStream_t s);

@@ -6,8 +6,8 @@
 //     x = 2^e sum_k d_k 2^(-7(k+1)) + r,   |r| <= 2^(e - 7D - 1)   (one round-to-nearest, unbiased).
 // A product of two sliced groups is sum_{k,l} 2^(-7(k+l+2)) sum d_k d_l.  The inner sums are int8 GEMMs with int32
 // accumulation (v_mfma_i32_32x32x32_i8), exact for the sizes used here, and products of equal order k + l share one
-// accumulator.  The accumulators of one result combine exactly into a 64-bit integer, sum_s acc_s 128^(S-1-s), which is
-// converted to FP64 once and scaled by the two groups' powers of two.  Only r and the dropped products (order above the
+// accumulator.  The accumulators of one result, sum_s acc_s 128^(S-1-s), combine exactly, in a 64-bit integer (V) or in two
+// FP64 parts (X), and are rounded to FP64 once and scaled by the two groups' powers of two.  Only r and the dropped products (order above the
 // kept one) differ from FP64, both bounded relative to the groups' powers of two.
 //
 //   X = P_red Phi           P: 5 digits per element, one power of two per row of P (sliced once per step).
