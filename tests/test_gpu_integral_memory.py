@@ -13,9 +13,14 @@ GB = 1 << 30
 
 
 def _free():
-    free, total = ctypes.c_size_t(), ctypes.c_size_t()
-    assert ctypes.CDLL("libamdhip64.so").hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
-    return free.value
+    """Free device memory as the runtime that this library is linked with sees it (torch may have brought another)."""
+    with open("/proc/self/maps") as maps:
+        paths = sorted({line.split()[-1] for line in maps if "libamdhip64" in line})
+    for path in paths:
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        if ctypes.CDLL(path).hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0:
+            return free.value
+    raise AssertionError("no runtime with a device among {}".format(paths))
 
 
 def _lattice(waters):
