@@ -338,12 +338,15 @@ constexpr long long kSliceDoubles = 1LL << 25;
 PairSet pair_set(const QBasis *b, const std::vector<QPair> &pairs, const std::vector<long long> &row, size_t first = 0,
                  size_t *last = nullptr, long long limit = LLONG_MAX) {
     PairSet set;
+    // A pair's records have six doubles or more.
+    std::vector<unsigned char> cls(std::min<size_t>(pairs.size() - first, static_cast<size_t>(limit / 6) + 1));
     size_t end = first;
     for (long long doubles = 0; end < pairs.size(); end++) {
         const QShell &A = b->shells[pairs[end].x], &B = b->shells[pairs[end].y];
         doubles += record_room(A, B);
         if (doubles > limit && end > first) break;
-        set.start[pair_class(A, B) + 1]++;
+        cls[end - first] = static_cast<unsigned char>(pair_class(A, B));
+        set.start[cls[end - first] + 1]++;
     }
     if (last != nullptr) *last = end;
     set.items.resize(end - first);
@@ -352,7 +355,7 @@ PairSet pair_set(const QBasis *b, const std::vector<QPair> &pairs, const std::ve
     for (int c = 0; c < 6; c++) at[c] = set.start[c];
     for (size_t k = first; k < end; k++) {
         const QShell &A = b->shells[pairs[k].x], &B = b->shells[pairs[k].y];
-        set.items[at[pair_class(A, B)]++] =
+        set.items[at[cls[k - first]]++] =
             pair_item(b->shells.data(), pairs[k].x, pairs[k].y, row.empty() ? 0 : row[k], set.doubles);
         set.doubles += record_room(A, B);
     }
