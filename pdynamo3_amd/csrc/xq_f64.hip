@@ -270,8 +270,8 @@ __device__ __forceinline__ void fock_tile_f64(const double *__restrict__ fI, con
 // V += Phi_I W_J^T + W_I Phi_J^T with FP64 atomics; on a diagonal tile the second term is the first one's transpose, taken
 // through LDS.  Work-group g runs on XCD g % 8; tiles are dealt so that each XCD takes a contiguous range of the tile list.
 // Bound by the FP64 matrix cores and the atomics, which go to memory.  Groups of four steps whose loads were each waited
-// for, and both products on the diagonal, took 3.79 ms on (H2O)64 and 27 us on one water; this takes 3.58 ms and
-// 19 us (four waves per SIMD; 3.68 ms with three).
+// for, and both products on the diagonal, took 3.99 and 4.03 ms in two runs on (H2O)64 and 27 us on one water; this takes
+// 3.87 and 3.72 ms on the same box and 19 us (four waves per SIMD; three took 3% more).
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) fock_kernel_f64(const MixedJob *__restrict__ jobs, int nJobs, int groupsPerXcd,
                                                        int nGroups) {
     __shared__ double sT[4][kC][kC + 1];

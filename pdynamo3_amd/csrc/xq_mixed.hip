@@ -485,11 +485,11 @@ __global__ void __launch_bounds__(256) p_slice_kernel(const xq::MixedJob *__rest
 // are loaded into the registers of the current ones as soon as the products with them are issued.  The row chunks of a
 // block are consecutive items of one XCD, so that their work-groups run at about the same time and read the block's
 // Phi digit chunks, in the same order, through that XCD's L2: Phi comes from HBM about once per block instead of once
-// per row chunk.  Chunk I's digits stay in registers from step I on (2.26 ms on (H2O)64; read again for the epilogue, with
-// 10% more traffic, 2.31).  At most 168 VGPRs let three work-groups share a CU (four, at 128, spill: 2.53 ms).  Bound by
-// latency and vector arithmetic: of 2.31 ms, gathers that hit the cache save 0.33 and grad Phi from L2 0.1; the vector
+// per row chunk.  Chunk I's digits stay in registers from step I on (2.28 ms on (H2O)64; read again for the epilogue, with
+// 10% more traffic, 2% more).  At most 168 VGPRs let three work-groups share a CU (four, at 128, spill: 2.5 ms).  Bound by
+// latency and vector arithmetic: of 2.3 ms, gathers that hit the cache save 0.33 and grad Phi from L2 0.1; the vector
 // units are busy for a third of the time, the matrix cores for a fifth.  With Phi staged in LDS as well, two barriers a
-// step, and 64-bit integers in the epilogue it took 2.43 ms.
+// step, and 64-bit integers in the epilogue it took 2.38 ms on the same box.
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
 density_rows_kernel(const xq::MixedJob *__restrict__ jobs, int nJobs, int interleaved) {
     __shared__ __attribute__((aligned(16))) int sP[2][kDP][kC][kPRowDwords];   // [digit][row][K positions / 4]
