@@ -111,16 +111,18 @@ void launch_pack(int n, const double *dense, double *packed, hipStream_t s) {
 // in its noise at 3 MB, and matrices of many MB would keep the packing kernel at the rate of PCIe.
 constexpr size_t kDirectResultBytes = size_t(1) << 19;
 
+bool direct_results(const xq_grid *g) { return result_bytes(g) <= kDirectResultBytes; }
+
 void launch_pack_results(xq_grid *g, hipStream_t s) {
     const size_t n = static_cast<size_t>(g->nFunctions), work = std::max<size_t>(n * (n + 1) / 2, g->nBlocks);
     const int grid = static_cast<int>(std::min<size_t>((work + 255) / 256, 16384));
-    double *out = result_bytes(g) <= kDirectResultBytes ? g->h_stage : g->d_packed;
+    double *out = direct_results(g) ? g->h_stage : g->d_packed;
     hipLaunchKernelGGL(pack_lower_kernel, dim3(grid > 0 ? grid : 1), dim3(256), 0, s, g->nFunctions, g->d_V, out, g->nBlocks,
                        g->d_blockEN, g->d_skip);
 }
 
 int copy_results(xq_grid *g, hipStream_t s) {
-    if (result_bytes(g) > kDirectResultBytes)
+    if (!direct_results(g))
         XQ_CHECK(hipMemcpyAsync(g->h_stage, g->d_packed, result_bytes(g), hipMemcpyDeviceToHost, s));
     return kOK;
 }

@@ -301,6 +301,7 @@ void host_add(double *to, const double *from, size_t n);
 // A step's results behind each other (packed V, the block sums, the skip flags; result_bytes) in h_stage, into which h_blockEN
 // and h_skip point: written there by the packing kernel, or, when large, in d_packed and copied once.
 size_t result_bytes(const xq_grid *g);
+bool direct_results(const xq_grid *g);      // small enough to be written by the packing kernel
 void launch_pack_results(xq_grid *g, hipStream_t s);
 int copy_results(xq_grid *g, hipStream_t s);
 void free_mixed(xq_grid *g);
