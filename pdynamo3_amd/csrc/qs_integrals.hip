@@ -462,6 +462,7 @@ int qs_one_electron(qs_basis *basis, double *S, double *T, double *V) {
     if (status == kOK) status = qs_alloc(&d_S, size);
     if (status == kOK) status = qs_alloc(&d_T, size);
     if (status == kOK) status = qs_alloc(&d_V, size);
+    if (status == kOK && !pairs.empty()) status = xq::make_runtime_room("one-electron integrals");
     hipStream_t s = basis->stream;
     if (status == kOK) status = check(hipMemcpyAsync(d_atoms, atoms.data(), atoms.size() * sizeof(double),
                                                      hipMemcpyHostToDevice, s), "copy atoms");
@@ -475,7 +476,6 @@ int qs_one_electron(qs_basis *basis, double *S, double *T, double *V) {
         if (status == kOK) status = qs_room(&d_records, &room[1], static_cast<size_t>(set.doubles));
         if (status == kOK) status = check(hipMemcpyAsync(d_items, set.items.data(), set.items.size() * sizeof(PairItem),
                                                          hipMemcpyHostToDevice, s), "copy pairs");
-        if (status == kOK && first == 0) status = xq::make_runtime_room("one-electron integrals");
         if (status == kOK) status = launch_records(basis, set, d_items, d_records, s);
         if (status != kOK) break;
         status = for_classes(set, d_items, "one-electron kernels", [&](auto la, auto lb, PairItem *items, int n) {
@@ -648,9 +648,9 @@ int qs_fit_matrix(qs_fit *fit, double *M) {
     int status = qs_alloc(&d_M, size);
     if (status == kOK) status = qs_alloc(&d_dense, static_cast<size_t>(mostRows) * nFit);
     if (status == kOK) status = qs_alloc(&d_column, nFit);
+    if (status == kOK && nShells > 0) status = xq::make_runtime_room("fit matrix");
     if (status == kOK) status = check(hipMemcpyAsync(d_column, fit->column.data(), nFit * sizeof(int),
                                                      hipMemcpyHostToDevice, s), "copy columns");
-    if (status == kOK && nShells > 0) status = xq::make_runtime_room("fit matrix");
     FitLaunch launch = fit->launch;
     launch.oShells = basis->d_shells;
     launch.oSpherical = basis->spherical;

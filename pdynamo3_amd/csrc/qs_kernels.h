@@ -118,9 +118,10 @@ QS_HD int pair_records(const QShell &A, const QShell &B, const double *__restric
         for (int qb = 0; qb < B.nPrim; qb++) {
             const double a = exps[A.prim + qa], b = exps[B.prim + qb], p = a + b, ip = 1.0 / p, h = 0.5 * ip;
             const double K = coefs[A.prim + qa] * coefs[B.prim + qb] * exp(-a * b * ip * r2);
-            double bound = fabs(K) * fmax(1.0, ip) * fmax(1.0, ip);
-            static_for<(LA + LB + 1) / 2>([&](auto) { bound *= fmax(1.0, r2 + ip); });
-            if (bound < kPrimitiveScreen) continue;
+            const double q = fmax(1.0, ip);
+            double bound = q * q;           // formed while the exponential is
+            static_for<(LA + LB + 1) / 2>([&](auto) { bound *= r2 + q; });
+            if (bound * fabs(K) < kPrimitiveScreen) continue;
             double *rec = out + static_cast<long long>(n) * C::size;
             n++;
             rec[0] = p;
