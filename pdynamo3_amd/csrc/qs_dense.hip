@@ -80,8 +80,6 @@ int aufbau(qs_dense *h, const double *fockF, int nOccupied, double *densityP, do
                           h->B, n), "dgemm F X");
     QS_BLAS(rocblas_dgemm(h->blas, rocblas_operation_none, rocblas_operation_none, n, n, n, &one, h->X, n, h->B, n, &zero,
                           h->C, n), "dgemm X F X");
-    // The eigensolver's kernels have private memory; what idle blocks hold of it is released.
-    (void)xq::make_runtime_room("qs_dense_aufbau");
     // Eigenvectors of C in its columns (lower triangle read), eigenvalues ascending.
     QS_BLAS(rocsolver_dsyevd(h->blas, rocblas_evect_original, rocblas_fill_lower, n, h->C, n, h->w, h->e, h->info),
             "rocsolver_dsyevd");
@@ -195,6 +193,8 @@ int qs_dense_aufbau(qs_dense *h, const double *fockF, int nOccupied, double *den
         return xq::kInvalidArgument;
     }
     XQ_TRY(check_device(h));
+    // The libraries' kernels have private memory (the eigensolver's do); what idle blocks hold of it is released.
+    (void)xq::make_runtime_room("qs_dense_aufbau");
     // The stream is drained on every return, so that no queued copy touches the caller's arrays afterwards.
     const int status = aufbau(h, fockF, nOccupied, densityP, orbitalEnergies);
     (void)hipStreamSynchronize(h->stream);
@@ -207,6 +207,7 @@ int qs_dense_commutator(qs_dense *h, const double *fockF, const double *densityP
         return xq::kInvalidArgument;
     }
     XQ_TRY(check_device(h));
+    (void)xq::make_runtime_room("qs_dense_commutator");
     const int status = commutator(h, fockF, densityP, error);
     (void)hipStreamSynchronize(h->stream);
     return status;

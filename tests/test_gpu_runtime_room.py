@@ -66,19 +66,22 @@ def test_idle_blocks_make_room(free_memory):
     g.close()
 
 
-def test_dense_steps_release_idle_blocks_and_go_on(free_memory):
+@pytest.mark.parametrize("step", ["aufbau", "commutator"])
+def test_dense_steps_release_idle_blocks_and_go_on(free_memory, step):
     from pdynamo3_amd import scf
     n = 64
     rng = np.random.default_rng(3)
     F = rng.standard_normal((n, n))
     d = scf.DeviceDenseSteps(np.eye(n), scf.pack(np.eye(n)))
-    want = d.aufbau(scf.pack(F + F.T), 20)
+    call = {"aufbau": lambda: d.aufbau(scf.pack(F + F.T), 20),
+            "commutator": lambda: [d.commutator(scf.pack(F + F.T), scf.pack(F @ F.T))]}[step]
+    want = call()
     Z, xyz, spec, fit = _system()
     scf.GPUIntegrals(Z, xyz, spec, False, fit).close()
     g = scf.GPUIntegrals(Z, xyz, spec, False, None)
     free_memory(0)
-    got = d.aufbau(scf.pack(F + F.T), 20)           # nothing idle is left
-    assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+    for a, b in zip(call(), want):                  # nothing idle is left
+        assert np.array_equal(a, b)
     free_memory(ROOM - 512)
     _refused(g.one_electron)
     d.close()
